@@ -29,9 +29,11 @@ from .uvu import Block, Path, UVUGenerator
 
 
 class UVUDirectGenerator(UVUGenerator):
+    _allow_shared = False      # one weight vector for all rows: uvu_shared.py
+
     def __init__(self, problem: TPProblem, kind: str = "tp", waves_per_eu: int = 0, vector_stores: bool = True):
         super().__init__(problem, kind)
-        if (kind == "conv_det" and not getattr(self, "_allow_det", False)) or self.shared:
+        if (kind == "conv_det" and not getattr(self, "_allow_det", False)) or (self.shared and not self._allow_shared):
             raise NotImplementedError("direct schedule: batch product with per-row weights and atomic convolution")
         self.waves_per_eu = waves_per_eu
         # False: outputs are written with dword-aligned record stores only (for callers whose
@@ -285,7 +287,7 @@ class UVUDirectGenerator(UVUGenerator):
                 E("const u64 rowc = rv ? row : n - 1;")    # idle lanes work on the last row once more
                 rc = "rowc"
             E(f"const T* __restrict__ Yr = Y + {rc} * {self.D2};")
-            E(f"const T* __restrict__ Wr = W + {rc} * {self.WN};")
+            E("const T* __restrict__ Wr = W" + ("" if self.shared else f" + {rc} * {self.WN}") + ";")
             if self.uniform_rows:
                 self.xrow_of = self.zrow_of = (lambda r: ("row", "true"))
             else:

@@ -59,8 +59,9 @@ def _on_device(device):
 def select_generator(config: TPProblem):
     """The kernel generator of a batch tensor product: MFMA kernels for uvw with shared weights (vector-ALU
     kernels with a row per lane when the weights are few and the multiplicities small),
-    streaming vector-ALU kernels for uvw with per-row weights, the persistent two-stage dW
-    reduction for uvu with shared weights, register-direct streaming kernels otherwise."""
+    streaming vector-ALU kernels for uvw with per-row weights, register-direct streaming kernels for uvu, with
+    dW sums held in registers across rows when the weights are shared (dW partial rows in memory and LDS-staged
+    loads where those sums do not fit)."""
     mode = validate_problem(config)
     if mode == "uvw" and config.shared_weights:
         from .codegen.uvw import UVWGenerator
@@ -71,7 +72,8 @@ def select_generator(config: TPProblem):
         from .codegen.uvw_batched import UVWBatchedGenerator
         return UVWBatchedGenerator(config)
     if config.shared_weights:
-        return UVUGenerator(config, "tp")
+        from .codegen.uvu_shared import UVUSharedGenerator
+        return UVUSharedGenerator(config) if UVUSharedGenerator.suits(config) else UVUGenerator(config, "tp")
     return UVUDirectGenerator(config, "tp")
 
 
@@ -161,7 +163,7 @@ class TensorProduct(TensorProductBase):
         if not aligned and isinstance(self.generator, UVUDirectGenerator):
             # rare: a caller-supplied tensor that is not 16-byte aligned -> kernels without vector stores
             if self._internal_unaligned is None:
-                g = UVUDirectGenerator(self.config, "tp", vector_stores=False)
+                g = type(self.generator)(self.config, vector_stores=False)
                 fwd, bwd, _ = g.plan()
                 self._internal_unaligned = rt.TPImpl(rt.compile_source(g.render()), _make_steps(fwd, self._step_flags),
                                                      _make_steps(bwd, self._step_flags))
