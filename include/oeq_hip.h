@@ -110,6 +110,18 @@ int  oeq_tp_backward(oeq_tp* tp, uint64_t num_products, const void* L1_in, void*
                      const void* L2_in, void* L2_grad, const void* weights, void* weights_grad,
                      const void* L3_grad, void* workspace, void* stream);
 
+/* Double backward of the product in one call.  `tp` was created from the code object of the double backward with its
+ * launch plan as `backward_steps` (and no forward steps); every step is launched with
+ *   (uint64_t n, const void* L1, const void* L2, const void* W, const void* L3g, const void* L1g_cot,
+ *    const void* L2g_cot, const void* Wg_cot, void* L1_grad, void* L2_grad, void* W_grad, void* L3g_grad).
+ * `*_cot` are the cotangents of the backward's three outputs, `*_grad` the gradients of its four inputs.  The
+ * reference composes these from four backward and three forward calls
+ * (implementations/TensorProductBase.py:281-298). */
+int  oeq_tp_double_backward(oeq_tp* tp, uint64_t num_products, const void* L1_in, const void* L2_in,
+                            const void* weights, const void* L3_grad, const void* L1_grad_cot,
+                            const void* L2_grad_cot, const void* weights_grad_cot, void* L1_out, void* L2_out,
+                            void* weights_out, void* L3_grad_out, void* stream);
+
 /* -------------------------------------------------------- fused convolution */
 /* Replaces JITConvImpl (extension/convolution.hpp:94-176).  rows = receivers (scatter
  * target), cols = senders (gather source), both int64[nnz].  Forward steps receive

@@ -1,6 +1,7 @@
 """Shared pieces of the gfx950 kernel generator: source emitter, literals, Jinja environment."""
 from __future__ import annotations
 
+import functools
 import pathlib
 from typing import Iterable, List
 
@@ -11,7 +12,9 @@ TEMPLATE_DIR = pathlib.Path(__file__).resolve().parent / "templates"
 WAVE = 64
 
 
+@functools.lru_cache(maxsize=1)
 def jinja_env() -> jinja2.Environment:
+    """One environment for the process: parsing the templates again took half of a generator's ``render``."""
     env = jinja2.Environment(loader=jinja2.FileSystemLoader(str(TEMPLATE_DIR)),
                              trim_blocks=True, lstrip_blocks=True, undefined=jinja2.StrictUndefined,
                              keep_trailing_newline=True)
@@ -41,6 +44,9 @@ class Emitter:
         self.level = indent
 
     def __call__(self, text: str = "") -> None:
+        if "\n" not in text:
+            self.lines.append(("    " * self.level + text) if text else "")
+            return
         for line in text.split("\n"):
             self.lines.append(("    " * self.level + line) if line else "")
 

@@ -287,6 +287,17 @@ int oeq_tp_backward(oeq_tp* tp, uint64_t n, const void* L1, void* L1g, const voi
     return 0;
 }
 
+int oeq_tp_double_backward(oeq_tp* tp, uint64_t n, const void* L1, const void* L2, const void* W, const void* L3g,
+                           const void* L1c, const void* L2c, const void* Wc, void* L1o, void* L2o, void* Wo, void* L3o,
+                           void* stream) {
+    if (!tp) return fail("null handle");
+    if (tp->bwd.empty()) return fail("this operator was built without a double backward plan");
+    void* args[] = {&n, &L1, &L2, &W, &L3g, &L1c, &L2c, &Wc, &L1o, &L2o, &Wo, &L3o};
+    for (auto& s : tp->bwd)
+        if (launch(s, n, 0, args, stream)) return 1;
+    return 0;
+}
+
 // ------------------------------------------------------------------- conv
 static int noalloc_scratch(void** out);
 

@@ -173,6 +173,11 @@ class TPProblem:
         self.irrep_dtype = irrep_dtype
         self.weight_dtype = weight_dtype
 
+    def signature(self) -> tuple:
+        """Everything a kernel's source depends on, as a hashable value."""
+        return (str(self.irreps_in1), str(self.irreps_in2), str(self.irreps_out), tuple(self.instructions),
+                self.shared_weights, np.dtype(self.irrep_dtype).str)
+
     # ------------------------------------------------------------------
     def weight_range_and_shape_for_instruction(self, instruction: int) -> Tuple[int, int, tuple]:
         t = self.instructions[instruction]

@@ -7,6 +7,7 @@ been built, loading raises.
 """
 from __future__ import annotations
 
+import collections
 import ctypes as C
 import hashlib
 import os
@@ -89,6 +90,7 @@ def lib() -> C.CDLL:
             "oeq_tp_destroy": (None, [vp]),
             "oeq_tp_forward": (C.c_int, [vp, u64, vp, vp, vp, vp, vp, vp]),
             "oeq_tp_backward": (C.c_int, [vp, u64, vp, vp, vp, vp, vp, vp, vp, vp, vp]),
+            "oeq_tp_double_backward": (C.c_int, [vp, u64, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]),
             "oeq_conv_create": (C.c_int, [vp, sz, C.POINTER(Step), C.c_int, C.POINTER(Step), C.c_int, C.POINTER(vp)]),
             "oeq_conv_destroy": (None, [vp]),
             "oeq_conv_forward": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, u64, u64, vp, vp, vp]),
@@ -121,7 +123,7 @@ def lib() -> C.CDLL:
 
 EXPORTED_SYMBOLS = [
     "oeq_last_error", "oeq_device_props", "oeq_device_count", "oeq_compile", "oeq_free", "oeq_hiprtc_version",
-    "oeq_tp_create", "oeq_tp_destroy", "oeq_tp_forward", "oeq_tp_backward",
+    "oeq_tp_create", "oeq_tp_destroy", "oeq_tp_forward", "oeq_tp_backward", "oeq_tp_double_backward",
     "oeq_conv_create", "oeq_conv_destroy", "oeq_conv_forward", "oeq_conv_backward",
     "oeq_conv_forward_ex", "oeq_conv_backward_ex", "oeq_conv_set_forward_workspace", "oeq_conv_forward_noalloc",
     "oeq_module_load", "oeq_module_unload", "oeq_module_launch",
@@ -187,6 +189,29 @@ def compile_source(source: str, arch: str = TARGET_ARCH, options: Sequence[str] 
     return blob
 
 
+# Code objects of kernel sets that operators build on first need (double backward), by what their source depends on:
+# operators of one problem - the layers of a model - then render and look up that source once.  Bounded; the entries are
+# plain bytes, every operator loads its own module from them.
+_VARIANTS: "collections.OrderedDict[tuple, bytes]" = collections.OrderedDict()
+_VARIANTS_MAX = 64
+_variants_lock = threading.Lock()
+
+
+def variant_code(key: tuple, render) -> bytes:
+    """Code object of the source that ``render()`` gives, remembered by ``key`` (everything the source depends on)."""
+    with _variants_lock:
+        code = _VARIANTS.get(key)
+        if code is not None:
+            _VARIANTS.move_to_end(key)
+            return code
+    code = compile_source(render())
+    with _variants_lock:
+        _VARIANTS[key] = code
+        while len(_VARIANTS) > _VARIANTS_MAX:
+            _VARIANTS.popitem(last=False)
+    return code
+
+
 def kernel_metadata(code: bytes) -> dict:
     """{kernel name: metadata} from the AMDGPU note of a code object: ``.vgpr_count``, ``.agpr_count``,
     ``.sgpr_count``, ``.private_segment_fixed_size`` (scratch bytes per lane: register spills),
@@ -241,6 +266,10 @@ class TPImpl:
 
     def backward(self, n, L1, L1g, L2, L2g, W, Wg, L3g, workspace=0, stream=0):
         _check(lib().oeq_tp_backward(self._h, n, L1, L1g, L2, L2g, W, Wg, L3g, workspace, stream))
+
+    def double_backward(self, n, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, stream=0):
+        """Of a handle created from a double backward's code object with its plan as the backward steps."""
+        _check(lib().oeq_tp_double_backward(self._h, n, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, stream))
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None

@@ -19,6 +19,7 @@ from . import runtime as rt
 from .autograd_glue import double_backward_terms
 from .codegen.uvu import UVUGenerator
 from .codegen.uvu_direct import UVUDirectGenerator
+from .codegen.uvu_double import UVUDoubleGenerator
 from .codegen.uvw_batched import UVWBatchedGenerator
 from .problem import TPProblem
 from .weight_order import WeightReorder
@@ -128,6 +129,9 @@ class TensorProduct(TensorProductBase):
         self._dims = (self.L1.dim, self.L2.dim, self.L3.dim, config.weight_numel)
         self._workspaces = {}                 # (device, stream) -> scratch tensor (fixed size, never regrown)
         self._internal_unaligned = None       # kernels without 16-byte vector stores, compiled on first need
+        # double backward in one launch: kernels by alignment of the outputs, compiled on first need
+        self._double_generator = UVUDoubleGenerator if mode == "uvu" and UVUDoubleGenerator.suits(config) else None
+        self._double = {}
 
         self._reorder = WeightReorder(config)
         self.reorder_weights_e3nn_to_oeq = self._reorder.e3nn_to_oeq
@@ -190,6 +194,19 @@ class TensorProduct(TensorProductBase):
         impl = self._pick(L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad)
         impl.backward(int(batch_size), L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad,
                       self._workspace_ptr(stream), self._stream() if stream is None else stream)
+
+    def double_backward_raw(self, batch_size, L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot,
+                            L1_out, L2_out, weights_out, L3_grad_out, stream=None) -> None:
+        """Gradients of the backward's inputs (x, y, w, dz) for cotangents of its outputs, in one launch
+        (``_double_generator`` must exist for the problem)."""
+        aligned = L1_out % 16 == 0 and L3_grad_out % 16 == 0
+        impl = self._double.get(aligned)
+        if impl is None:
+            g = self._double_generator(self.config, vector_stores=aligned)
+            code = rt.variant_code(("tp double", self.config.signature(), aligned, g.one_block_ahead()), g.render)
+            impl = self._double[aligned] = rt.TPImpl(code, [], _make_steps(g.plan()))
+        impl.double_backward(int(batch_size), L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot,
+                             L1_out, L2_out, weights_out, L3_grad_out, self._stream() if stream is None else stream)
 
     # ------------------------------------------------- numpy entry points (tests)
     def forward_cpu(self, L1_in, L2_in, L3_out, weights) -> None:
@@ -271,9 +288,30 @@ class TensorProduct(TensorProductBase):
         def setup_context_double_backward(ctx, inputs, output):
             ctx.L1_in, ctx.L2_in, ctx.weights, ctx.L3_grad = inputs
 
+        fused = None
+        if self._double_generator is not None:
+            @torch.library.custom_op(f"openequivariance_amd::tp_double_backward{self.tp_id}", mutates_args=(),
+                                     device_types="cuda")
+            def fused(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, L3_grad: torch.Tensor,
+                      L1_cot: torch.Tensor, L2_cot: torch.Tensor, weights_cot: torch.Tensor) -> typing.List[torch.Tensor]:
+                x, y, w, g, a, b, v = _contiguous(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot)
+                self._check_inputs(x, y, w, g)
+                self._check_inputs(a, b, v)
+                if a.shape != x.shape or a.device != x.device:
+                    raise ValueError("the cotangents must match the operands' batch and device")
+                out = [torch.empty_like(t) for t in (x, y, w, g)]
+                with _on_device(x.device):
+                    self.double_backward_raw(x.shape[0], *(t.data_ptr() for t in (x, y, w, g, a, b, v, *out)),
+                                             stream=self._stream(x.device.index))
+                return out
+
+            @fused.register_fake
+            def _(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot):
+                return [t.new_empty(*t.shape) for t in (L1_in, L2_in, weights, L3_grad)]
+
         def double_backward(ctx, grad_output):
             return double_backward_terms(forward, backward_helper, ctx.L1_in, ctx.L2_in, ctx.weights, ctx.L3_grad,
-                                         grad_output[0], grad_output[1], grad_output[2])
+                                         grad_output[0], grad_output[1], grad_output[2], fused=fused)
 
         backward_helper.register_autograd(double_backward, setup_context=setup_context_double_backward)
 
