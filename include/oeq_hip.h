@@ -172,6 +172,20 @@ int  oeq_conv_backward_ex(oeq_conv* conv, const void* L1_in, void* L1_grad, cons
                           const void* rows, const void* cols, uint64_t nnz, uint64_t node_count,
                           void* workspace, const void* transpose_perm, void* stream, uint32_t call_flags);
 
+/* Double backward of the convolution in one call.  `conv` was created from the code object of the double backward with
+ * its launch plan as `backward_steps` (and no forward steps); every step is launched with
+ *   (const void* L1, const void* L2, const void* W, const void* L3g, const void* L1g_cot, const void* L2g_cot,
+ *    const void* Wg_cot, void* L1_grad, void* L2_grad, void* W_grad, void* L3g_grad, const int64_t* rows,
+ *    const int64_t* cols, uint64_t nnz, uint64_t node_count, void* workspace, const int64_t* transpose_perm).
+ * `*_cot` are the cotangents of the backward's three outputs, `*_grad` the gradients of its four inputs (all written
+ * whole).  The reference composes these from four backward and three forward calls
+ * (implementations/convolution/ConvolutionBase.py:618-636 and :691-709). */
+int  oeq_conv_double_backward(oeq_conv* conv, const void* L1_in, const void* L2_in, const void* weights,
+                              const void* L3_grad, const void* L1_grad_cot, const void* L2_grad_cot,
+                              const void* weights_grad_cot, void* L1_out, void* L2_out, void* weights_out,
+                              void* L3_grad_out, const void* rows, const void* cols, uint64_t nnz,
+                              uint64_t node_count, void* workspace, const void* transpose_perm, void* stream);
+
 /* Workspace bytes the forward steps use when every node is walked by one wavefront (no pieces):
  * fixed_bytes + bytes_per_node * node_count + bytes_per_edge * nnz.  The host sets it from the plan it
  * built the operator with; oeq_conv_forward_noalloc checks graphs against it.  (The reference sizes

@@ -42,6 +42,21 @@ class UVUDetGenerator(UVUDirectGenerator):
     SPLIT_TARGET = {"float": 64, "double": 24}
     FWD_SPLIT_WORDS = {"float": 100, "double": 32}
     FWD_COHERENT = True
+    FWD_STAGE_WAVES = 16          # wavefronts per CU that the LDS stage of the forward must leave room for
+    FWD_STAGE_OPERANDS = 26       # words per edge and lane from which several chunks per node are staged, too
+    # What one edge brings, as (kernel argument, register prefix): weight rows, second-operand rows, and the rows
+    # of its sender.  The double backward (uvu_conv_double.py) walks the same loops with each operand's cotangent beside it.
+    EDGE_W = (("W", "We_"),)
+    EDGE_Y = (("Y", "y"),)
+    NODE_X = (("X", "x"),)
+    NODE_OUT = "Z"                # what the receiver-side pass writes
+    CALL_FWD_ARGS = ("const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ W, T* __restrict__ Z, \\\n"
+                     "    const IDX* __restrict__ rows, const IDX* __restrict__ cols, u64 nnz, u64 node_count, \\\n"
+                     "    void* __restrict__ ws, const IDX* __restrict__ tperm")
+    CALL_BWD_ARGS = ("const T* __restrict__ X, T* __restrict__ Xg, const T* __restrict__ Y, T* __restrict__ Yg, \\\n"
+                     "    const T* __restrict__ W, T* __restrict__ Wg, const T* __restrict__ G, \\\n"
+                     "    const IDX* __restrict__ rows, const IDX* __restrict__ cols, u64 nnz, u64 node_count, \\\n"
+                     "    void* __restrict__ ws, const IDX* __restrict__ tperm")
     # int64 words of one on-the-fly grouping of the edges in the workspace: group pointers and fill cursors
     # (node_count + 1 each), the position list (nnz), the counters (node_count + 1) and the ticket of the
     # counting kernel
@@ -87,14 +102,14 @@ class UVUDetGenerator(UVUDirectGenerator):
         # dZ and W; launch 0 writes dX, the later ones add to it; dY goes through per-(chunk, group) partials).
         def words_of(outs):
             ps = [p for p in self.paths if p.o.idx in outs]
-            return (sum(self.out[i].D for i in outs) + sum(p.mv for p in ps)
-                    + len({p.b.off + v * p.b.D + j for p in ps for v in range(p.mv) for (_, j) in p.pairs}))
+            return (sum(self.out[i].D for i in outs) + len(self.EDGE_W) * sum(p.mv for p in ps)
+                    + len(self.EDGE_Y) * len({p.b.off + v * p.b.D + j for p in ps for v in range(p.mv) for (_, j) in p.pairs}))
         words = words_of(self.used_out)
         H = 1
         split = tunables.current.det_split                      # 0: never; a number: threshold for A/B runs
-        limit = split if split else self.SPLIT_WORDS
+        limit = split if split else self.split_limit()
         if words > limit and split != 0 and allow_split:
-            H = min(len(self.used_out), -(-words // self.SPLIT_TARGET[self.T]))
+            H = min(len(self.used_out), self.sender_launches(words, limit))
         self.out_groups = [[] for _ in range(H)]
         for oi in sorted(self.used_out, key=lambda i: -(self.out[i].D + len(self.paths_into(i)))):
             min(self.out_groups, key=words_of).append(oi)
@@ -122,7 +137,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         # (LDS-DMA), which leaves room for a third wavefront per SIMD; see emit_staged_loop
         def stage_words_of(outs):
             return WAVE * (sum(self.dma_stride(w) for i in outs for _, w in self.dma_pieces(self.out[i].D))
-                           + sum(p.mv for p in self.paths if p.o.idx in outs) + 1)
+                           + len(self.EDGE_W) * sum(p.mv for p in self.paths if p.o.idx in outs) + len(self.EDGE_Y))
         self.stage_words = max(stage_words_of(g_) for g_ in self.out_groups)      # of the largest group
         lds = tunables.current.det_lds if lds is None else lds
         stage_waves = (160 * 1024) // (4 * self.stage_words * 4)        # wavefronts per SIMD the stage leaves room for
@@ -143,10 +158,11 @@ class UVUDetGenerator(UVUDirectGenerator):
         # 0.640 ms on the 128-channel MACE problem and 3.65 -> 3.49 ms on 256 channels with outputs of either
         # parity; with 22 words, 256 channels and 13 paths, 2.583 -> 2.596 ms; not over a position list built on the
         # fly - the unsorted MACE forward went 0.741 -> 0.775 ms)
-        fwd_operands = sum(self.in1[i].D for i in self.used_in1) + sum(p.mv for p in self.paths)
+        fwd_operands = (len(self.NODE_X) * sum(self.in1[i].D for i in self.used_in1)
+                        + len(self.EDGE_W) * sum(p.mv for p in self.paths))
         self.lds_forward = (self.T == "float" and self.P >= self.D2 and lds is not False
-                            and (self.NCH == 1 or (fwd_operands >= 26 and not forward_perm) or lds is True)
-                            and 16 * (fwd_words + self.lds_elems) * 4 <= 160 * 1024)
+                            and (self.NCH == 1 or (fwd_operands >= self.FWD_STAGE_OPERANDS and not forward_perm) or lds is True)
+                            and self.FWD_STAGE_WAVES * (fwd_words + self.lds_elems) * 4 <= 160 * 1024)
         # Forward: the sums of every output block of a node stay in registers across its edge list.  Beyond
         # FWD_SPLIT_WORDS words per lane the loop spilled them (5000 nodes, 150 000 edges, fp32 / fp64: 30 paths and 102
         # words 0.68 / 3.33 ms, 68 paths and 312 words 19.6 / 44.6 ms), so the output blocks are dealt into groups, one
@@ -179,6 +195,14 @@ class UVUDetGenerator(UVUDirectGenerator):
         self.LONG = max(0, int(tunables.current.long_node)) if long_node is None else int(long_node)
         # byte offset (C expression) of the piece area in the workspace: counters, then partial rows
         self.piece_base = f"((({self.flags_off} + 4ull * ((nnz + 255) / 256)) + 255ull) & ~255ull)"
+
+    def split_limit(self) -> int:
+        """Words per edge up to which the sender-side pass is one launch."""
+        return self.SPLIT_WORDS
+
+    def sender_launches(self, words: int, limit: int) -> int:
+        """Its launches when the ``words`` per edge are more than ``limit``."""
+        return -(-words // self.SPLIT_TARGET[self.T])
 
     def dealt_groups(self, n: int, words_of):
         """The output blocks in n groups of about equal ``words_of``, largest block first."""
@@ -584,10 +608,10 @@ class UVUDetGenerator(UVUDirectGenerator):
         # in flight (software pipelining hides the gather latency, which dominates when a node has few
         # edges and few wavefronts are resident)
         names = []
-        for i in self.used_in1:
-            names += [f"x{i}_{m}" for m in range(self.in1[i].D)]
-        names += [f"We_{p.t}_{v}" for p in self.paths for v in range(p.mv)]
-        names += [f"y{f}" for f in self.used_y]
+        for _, x in self.NODE_X:
+            for i in self.used_in1:
+                names += [f"{x}{i}_{m}" for m in range(self.in1[i].D)]
+        names += self._edge_names()
         def load_idx(E, it, q):
             """Edge position, sender (clamped) and validity of iteration ``it`` into index set q."""
             E("{")
@@ -613,34 +637,61 @@ class UVUDetGenerator(UVUDirectGenerator):
             E("{")
             E.level += 1
             E(f"const u64 e = I{q}e, sndc = I{q}n; const bool rv = I{q}rv;")
-            E(f"const T* __restrict__ Yr = Y + e * {self.D2};")
-            E(f"const T* __restrict__ Wr = W + e * {self.WN};")
-            for f in self.used_y:
-                E(f"S{h}y{f} = {self.ld('Yr', f)};")
-            for i in self.used_in1:
-                a = self.in1[i]
-                E(f"{{ const T* __restrict__ p_ = X + sndc * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D}; "
-                  + " ".join(f"S{h}x{i}_{m} = p_[{m}];" for m in range(a.D)) + " }")
-                # everything an edge adds is proportional to x: zero it for idle lanes
-                E(f"if (!({self.act(a)})) {{ " + " ".join(f"S{h}x{i}_{m} = (T)0;" for m in range(a.D)) + " }")
-            for p in self.paths:
-                for v in range(p.mv):
-                    E(f"S{h}We_{p.t}_{v} = {self.ld('Wr', self.widx(p, self.uclamp(p.a, 0), v))};")
+            self._edge_rows(E)
+            self._load_edge_y(E, h)
+            for src, x in self.NODE_X:
+                for i in self.used_in1:
+                    a = self.in1[i]
+                    E(f"{{ const T* __restrict__ p_ = {src} + sndc * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D}; "
+                      + " ".join(f"S{h}{x}{i}_{m} = p_[{m}];" for m in range(a.D)) + " }")
+                    # everything an edge adds is proportional to x: zero it for idle lanes
+                    E(f"if (!({self.act(a)})) {{ " + " ".join(f"S{h}{x}{i}_{m} = (T)0;" for m in range(a.D)) + " }")
+            self._load_edge_w(E, h)
             E.level -= 1
             E("}")
 
         def compute(E, h):
             for oi in self.used_out:
-                self.emit_forward_block(E, self.out[oi], "Wr", zname=f"z{oi}_", declare=False)
+                self.emit_receiver_block(E, self.out[oi], f"z{oi}_")
         if self.lds_forward:
             self._emit_staged_forward(E, compute)
         else:
             self.emit_pingpong_loop(E, names, load_idx, load, compute)
         E("const bool rv = nv;")
-        self.emit_node_output(E, self.out, self.used_out, lambda o: [f"z{o.idx}_{k}" for k in range(o.D)], "Z", self.D3,
+        self.emit_node_output(E, self.out, self.used_out, lambda o: [f"z{o.idx}_{k}" for k in range(o.D)], self.NODE_OUT, self.D3,
                               via_lds=True, zero_unused=(h == 0), add_existing=False,
                               elsewhere={oi for g_ in self.fwd_groups for oi in g_} - set(self.used_out))
         return E.text()
+
+    # ---- operands of one edge (shared by both directions)
+    def _edge_names(self):
+        return ([f"{w}{p.t}_{v}" for _, w in self.EDGE_W for p in self.paths for v in range(p.mv)]
+                + [f"{y}{f}" for _, y in self.EDGE_Y for f in self.used_y])
+
+    def _edge_rows(self, E: Emitter) -> None:
+        for src, _ in self.EDGE_Y:
+            E(f"const T* __restrict__ {src}r = {src} + e * {self.D2};")
+        for src, _ in self.EDGE_W:
+            E(f"const T* __restrict__ {src}r = {src} + e * {self.WN};")
+
+    def _load_edge_y(self, E: Emitter, h) -> None:
+        for src, y in self.EDGE_Y:
+            for f in self.used_y:
+                E(f"S{h}{y}{f} = {self.ld(src + 'r', f)};")
+
+    def _load_edge_w(self, E: Emitter, h) -> None:
+        for src, w in self.EDGE_W:
+            for p in self.paths:
+                for v in range(p.mv):
+                    E(f"S{h}{w}{p.t}_{v} = {self.ld(src + 'r', self.widx(p, self.uclamp(p.a, 0), v))};")
+
+    def emit_receiver_block(self, E: Emitter, o, zname: str) -> None:
+        """What an edge adds to block ``o`` of its receiver's row (sums {zname}{k})."""
+        self.emit_forward_block(E, o, "Wr", zname=zname, declare=False)
+
+    def emit_sender_block(self, E: Emitter, o, sink) -> None:
+        """What an edge adds to dx and dy through output block ``o`` (g{k} = dZ of its receiver), and its dW."""
+        self.emit_backward_block(E, o, "Wr", sink)
 
     def uclamp(self, blk, c) -> str:
         return "u" if self.full(blk) else f"min(u, {blk.mul - 1})"
@@ -835,12 +886,12 @@ class UVUDetGenerator(UVUDirectGenerator):
         E("const u64 nodec = nv ? node : 0;")
         for i in self.used_in1:
             a = self.in1[i]
-            self.emit_record_load(E, [f"x{i}_{m}" for m in range(a.D)],
-                                  f"X + nodec * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D}", self.act(a), zero=True)
+            for src, x in self.NODE_X:
+                self.emit_record_load(E, [f"{x}{i}_{m}" for m in range(a.D)],
+                                      f"{src} + nodec * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D}", self.act(a), zero=True)
             E("T " + ", ".join(f"dx{i}_{m} = (T)0" for m in range(a.D)) + ";")
         names = [f"G{oi}_{k}" for oi in self.used_out for k in range(self.out[oi].D)]
-        names += [f"We_{p.t}_{v}" for p in self.paths for v in range(p.mv)]
-        names += [f"y{f}" for f in self.used_y]
+        names += self._edge_names()
         def load_idx(E, it, q):
             """Edge id, receiver (clamped) and validity of iteration ``it`` into index set q: a chain of two
             dependent loads (position list, then the edge's receiver), kept off the data loads' critical path."""
@@ -861,13 +912,9 @@ class UVUDetGenerator(UVUDirectGenerator):
             E("{")
             E.level += 1
             E(f"const u64 e = I{q}e, rcvc = I{q}n; const bool rv = I{q}rv;")
-            E(f"const T* __restrict__ Yr = Y + e * {self.D2};")
-            E(f"const T* __restrict__ Wr = W + e * {self.WN};")
-            for f in self.used_y:
-                E(f"S{h}y{f} = {self.ld('Yr', f)};")
-            for p in self.paths:
-                for v in range(p.mv):
-                    E(f"S{h}We_{p.t}_{v} = {self.ld('Wr', self.widx(p, self.uclamp(p.a, 0), v))};")
+            self._edge_rows(E)
+            self._load_edge_y(E, h)
+            self._load_edge_w(E, h)
             for oi in self.used_out:
                 o = self.out[oi]
                 E(f"{{ const T* __restrict__ p_ = G + rcvc * {self.D3} + {o.off} + {self.uclamp(o, 0)} * {o.D}; "
@@ -894,7 +941,7 @@ class UVUDetGenerator(UVUDirectGenerator):
                         E(f"  pw_{p.t}_{v} = {expr};")
                     else:
                         E(f"  if ({self.act(p.a)}) {self.st('Wgr', self.widx(p, 'u', v), expr)}")
-                self.emit_backward_block(E, o, "Wr", sink)
+                self.emit_sender_block(E, o, sink)
                 E.level -= 1
                 E("}")
             self.emit_dy_sum(E)
@@ -922,58 +969,75 @@ class UVUDetGenerator(UVUDirectGenerator):
     def _forward_slabs(self):
         """(slabs, words) of the forward stage: X records of the sender, path weights, Y."""
         slabs, off = [], 0
-        for i in self.used_in1:
-            for k0, w in self.dma_pieces(self.in1[i].D):
-                slabs.append(("X", i, k0, w, off))
-                off += WAVE * self.dma_stride(w)
-        for p in self.paths:
-            for v in range(p.mv):
-                slabs.append(("W", (p, v), 0, 1, off))
-                off += WAVE
-        return slabs, off + WAVE
+        for src, _ in self.NODE_X:
+            for i in self.used_in1:
+                for k0, w in self.dma_pieces(self.in1[i].D):
+                    slabs.append((src, i, k0, w, off))
+                    off += WAVE * self.dma_stride(w)
+        off = self._edge_slabs(slabs, off)
+        return slabs, off + WAVE * len(self.EDGE_Y)
+
+    def _edge_slabs(self, slabs, off: int) -> int:
+        """One slab per weight of an edge, behind ``off``; the second-operand slabs follow at the returned offset."""
+        for src, _ in self.EDGE_W:
+            for p in self.paths:
+                for v in range(p.mv):
+                    slabs.append((src, (p, v), 0, 1, off))
+                    off += WAVE
+        return off
+
+    def _edge_dma(self, E: Emitter, slabs, y_off: int, nt: int) -> None:
+        for src, _ in self.EDGE_W:
+            E(f"const T* __restrict__ {src}r = {src} + e * {self.WN};")
+        for q, (src, _) in enumerate(self.EDGE_Y):
+            E(f"OEQ_DMA(4, {nt}, {src} + e * {self.D2} + min(ul, {self.D2 - 1}), stage + {y_off + q * WAVE});")
+        for src, _ in self.EDGE_W:
+            for kind, key, k0, w, so in slabs:
+                if kind == src:
+                    p, v = key
+                    E(f"OEQ_DMA(4, {nt}, {src}r + {self.widx(p, self.uclamp(p.a, 0), v)}, stage + {so});")
+
+    def _edge_readback(self, E: Emitter, slabs, y_off: int) -> None:
+        for q, (_, y) in enumerate(self.EDGE_Y):
+            for f in self.used_y:
+                E(f"const T {y}{f} = stage[{y_off + q * WAVE} + sub * {self.P} + {f}];")
+        for src, name in self.EDGE_W:
+            for kind, key, k0, w, so in slabs:
+                if kind == src:
+                    p, v = key
+                    E(f"const T {name}{p.t}_{v} = stage[{so} + lane];")
 
     def _emit_staged_forward(self, E: Emitter, compute) -> None:
         nt = 2 if self.nontemporal else 0
         slabs, words = self._forward_slabs()
-        y_off = words - WAVE
+        y_off = words - WAVE * len(self.EDGE_Y)
         E(f"__shared__ __attribute__((aligned(16))) T stage[{words}];")
 
         def dma(E, e, n):
             E("{")
             E.level += 1
             E(f"const u64 e = {e}, sndc = {n};")
-            E(f"const T* __restrict__ Wr = W + e * {self.WN};")
-            E(f"OEQ_DMA(4, {nt}, Y + e * {self.D2} + min(ul, {self.D2 - 1}), stage + {y_off});")
+            self._edge_dma(E, slabs, y_off, nt)
             for kind, key, k0, w, so in slabs:
-                if kind == "W":
-                    p, v = key
-                    E(f"OEQ_DMA(4, {nt}, Wr + {self.widx(p, self.uclamp(p.a, 0), v)}, stage + {so});")
-            for kind, key, k0, w, so in slabs:
-                if kind == "X":
+                if kind in dict(self.NODE_X):
                     a = self.in1[key]
-                    E(f"OEQ_DMA({4 * w}, 0, X + sndc * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D} + {k0}, stage + {so});")
+                    E(f"OEQ_DMA({4 * w}, 0, {kind} + sndc * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D} + {k0}, stage + {so});")
             E.level -= 1
             E("}")
 
         def readback(E):
             E("const bool rv = cur_rv;")
-            for f in self.used_y:
-                E(f"const T y{f} = stage[{y_off} + sub * {self.P} + {f}];")
-            for kind, key, k0, w, so in slabs:
-                if kind == "W":
-                    p, v = key
-                    E(f"const T We_{p.t}_{v} = stage[{so} + lane];")
+            self._edge_readback(E, slabs, y_off)
             for i in self.used_in1:
                 a = self.in1[i]
-                parts = []
-                for kind, key, k0, w, so in slabs:
-                    if kind == "X" and key == i:
-                        parts += [f"stage[{so} + lane * {self.dma_stride(w)} + {r}]" for r in range(w)]
                 # everything an edge adds is proportional to x: zero it for idle lanes
                 # (read unconditionally, then masked: a conditional expression would put a branch around every LDS read)
                 E(f"const bool a{i}_ = {self.act(a)};")
-                E("const T " + ", ".join(f"xr{i}_{m} = {parts[m]}" for m in range(a.D)) + ";")
-                E("const T " + ", ".join(f"x{i}_{m} = a{i}_ ? xr{i}_{m} : (T)0" for m in range(a.D)) + ";")
+                for src, x in self.NODE_X:
+                    parts = [f"stage[{so} + lane * {self.dma_stride(w)} + {r}]" for kind, key, k0, w, so in slabs
+                             if kind == src and key == i for r in range(w)]
+                    E("const T " + ", ".join(f"{x}r{i}_{m} = {parts[m]}" for m in range(a.D)) + ";")
+                    E("const T " + ", ".join(f"{x}{i}_{m} = a{i}_ ? {x}r{i}_{m} : (T)0" for m in range(a.D)) + ";")
         self.emit_staged_loop(E, self.edge_pos, "eperm" if self.forward_perm else None, "cols", dma, readback, compute)
 
     def _emit_staged_backward(self, E: Emitter, compute, grp: int = 0) -> None:
@@ -985,12 +1049,8 @@ class UVUDetGenerator(UVUDirectGenerator):
             for k0, w in self.dma_pieces(self.out[oi].D):
                 slabs.append(("G", oi, k0, w, off))
                 off += WAVE * self.dma_stride(w)
-        for p in self.paths:
-            for v in range(p.mv):
-                slabs.append(("W", (p, v), 0, 1, off))
-                off += WAVE
-        y_off = off
-        off += WAVE
+        y_off = self._edge_slabs(slabs, off)
+        off = y_off + WAVE * len(self.EDGE_Y)
         assert off <= self.stage_words
         E(f"__shared__ __attribute__((aligned(16))) T stage[{off}];")
 
@@ -998,12 +1058,7 @@ class UVUDetGenerator(UVUDirectGenerator):
             E("{")
             E.level += 1
             E(f"const u64 e = {e}, rcvc = {n};")
-            E(f"const T* __restrict__ Wr = W + e * {self.WN};")
-            E(f"OEQ_DMA(4, {nt}, Y + e * {self.D2} + min(ul, {self.D2 - 1}), stage + {y_off});")
-            for kind, key, k0, w, so in slabs:
-                if kind == "W":
-                    p, v = key
-                    E(f"OEQ_DMA(4, {nt}, Wr + {self.widx(p, self.uclamp(p.a, 0), v)}, stage + {so});")
+            self._edge_dma(E, slabs, y_off, nt)
             for kind, key, k0, w, so in slabs:
                 if kind == "G":
                     o = self.out[key]
@@ -1013,12 +1068,7 @@ class UVUDetGenerator(UVUDirectGenerator):
 
         def readback(E):
             E("rv = cur_rv;")
-            for f in self.used_y:
-                E(f"const T y{f} = stage[{y_off} + sub * {self.P} + {f}];")
-            for kind, key, k0, w, so in slabs:
-                if kind == "W":
-                    p, v = key
-                    E(f"const T We_{p.t}_{v} = stage[{so} + lane];")
+            self._edge_readback(E, slabs, y_off)
             for oi in self.used_out:
                 o = self.out[oi]
                 parts = []

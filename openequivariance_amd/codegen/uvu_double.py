@@ -31,18 +31,21 @@ class DoubleArithmetic:
 
     def emit_double_block(self, E: Emitter, o: Block, zname: str, dw_sink, declare: bool = True) -> None:
         """Given g{k} = dZ[o][u, k], the weights ``w{t}_{v}`` and their cotangents ``ww{t}_{v}`` in registers: adds to
-        gx{a}_{i}, gy{f} and {zname}{k}, and hands every second gradient of a weight to ``dw_sink``."""
+        dx{a}_{i}, dy{f} and {zname}{k}, and hands every second gradient of a weight to ``dw_sink``.  Without ``zname``
+        only the former, without ``dw_sink`` only the sums {zname}{k} (no g{k} needed)."""
         if declare:
             E("T " + ", ".join(f"{zname}{k} = (T)0" for k in range(o.D)) + ";")
         for p in self.paths_into(o.idx):
             E(f"{{ // path {p.t}: l = {p.a.l} x {p.b.l} -> {p.o.l}")
             E.level += 1
-            self._emit_cg_products(E, p)
+            if dw_sink:
+                self._emit_cg_products(E, p)
             for v in range(p.mv):
                 E("{")
                 E.level += 1
-                self._emit_double_pairs(E, p, v, zname)
-                dw_sink(E, p, v, "dw")
+                self._emit_double_pairs(E, p, v, zname, bool(dw_sink))
+                if dw_sink:
+                    dw_sink(E, p, v, "dw")
                 E.level -= 1
                 E("}")
             E.level -= 1
@@ -50,39 +53,47 @@ class DoubleArithmetic:
 
     def emit_settle(self, E: Emitter, oi: int) -> None:
         """The sums an output block has added to are final here: the stores behind a block sit in branches, and the
-        compiler otherwise moves the additions to gx and gy past them, with every operand alive until the end."""
+        compiler otherwise moves the additions to dx and dy past them, with every operand alive until the end."""
         ps = self.paths_into(oi)
-        names = [f"gx{i}_{m}" for i in sorted({p.a.idx for p in ps}) for m in range(self.in1[i].D)]
-        names += [f"gy{f}" for f in sorted({p.b.off + v * p.b.D + j for p in ps for v in range(p.mv) for (_, j) in p.pairs})]
+        names = [f"dx{i}_{m}" for i in sorted({p.a.idx for p in ps}) for m in range(self.in1[i].D)]
+        names += [f"dy{f}" for f in sorted({p.b.off + v * p.b.D + j for p in ps for v in range(p.mv) for (_, j) in p.pairs})]
         E(" ".join(f"OEQ_OPAQUE({n});" for n in names))
 
-    def _emit_double_pairs(self, E: Emitter, p: Path, v: int, zname: str) -> None:
+    def _emit_double_pairs(self, E: Emitter, p: Path, v: int, zname: str, first: bool) -> None:
+        """The (i, j) pairs of one path: with ``first`` the sums proportional to dZ (dw, dx, dy), with ``zname`` those
+        of the gradient of dZ."""
         by_i = {}
         for (i, j), ks in sorted(p.pairs.items()):
             by_i.setdefault(i, []).append((j, ks))
         w, ww, X = f"w{p.t}_{v}", f"ww{p.t}_{v}", p.a.idx
         f = lambda j: p.b.off + v * p.b.D + j
-        E("T dw = (T)0;")
+        if first:
+            E("T dw = (T)0;")
         for i, lst in sorted(by_i.items()):
-            E(f"{{ const T wx = {w} * x{X}_{i}, pi = oeq_fma({w}, a{X}_{i}, {ww} * x{X}_{i});")
+            wx = f"wx = {w} * x{X}_{i}, " if zname else ""
+            E(f"{{ const T {wx}pi = oeq_fma({w}, a{X}_{i}, {ww} * x{X}_{i});")
             E.level += 1
-            E("T t, tb;")
+            if first:
+                E("T t, tb;")
             for n_, (j, ks) in enumerate(lst):
                 E("{")
-                if len(ks) == 1:
-                    E(f"  const T s = {'-' if ks[0][1] < 0 else ''}{self._cg_names[self._cg_key(*ks[0])]};")
-                else:
-                    E(f"  T s = {self.lit(ks[0][1])} * g{ks[0][0]};")
-                    for k, val in ks[1:]:
-                        E(f"  s = oeq_fma({self.lit(val)}, g{k}, s);")
                 y, b = f"y{f(j)}", f"b{f(j)}"
-                E(f"  t = s * {y}; tb = s * {b};" if n_ == 0 else f"  t = oeq_fma(s, {y}, t); tb = oeq_fma(s, {b}, tb);")
-                E(f"  gy{f(j)} = oeq_fma(s, pi, gy{f(j)});")
-                E(f"  const T q = oeq_fma(wx, {b}, pi * {y});")
-                E("  " + " ".join(f"{zname}{k} = oeq_fma({self.lit(val)}, q, {zname}{k});" for k, val in ks))
+                if first:
+                    if len(ks) == 1:
+                        E(f"  const T s = {'-' if ks[0][1] < 0 else ''}{self._cg_names[self._cg_key(*ks[0])]};")
+                    else:
+                        E(f"  T s = {self.lit(ks[0][1])} * g{ks[0][0]};")
+                        for k, val in ks[1:]:
+                            E(f"  s = oeq_fma({self.lit(val)}, g{k}, s);")
+                    E(f"  t = s * {y}; tb = s * {b};" if n_ == 0 else f"  t = oeq_fma(s, {y}, t); tb = oeq_fma(s, {b}, tb);")
+                    E(f"  dy{f(j)} = oeq_fma(s, pi, dy{f(j)});")
+                if zname:
+                    E(f"  const T q = oeq_fma(wx, {b}, pi * {y});")
+                    E("  " + " ".join(f"{zname}{k} = oeq_fma({self.lit(val)}, q, {zname}{k});" for k, val in ks))
                 E("}")
-            E(f"dw = oeq_fma(a{X}_{i}, t, dw); dw = oeq_fma(x{X}_{i}, tb, dw);")
-            E(f"gx{X}_{i} = oeq_fma({w}, tb, gx{X}_{i}); gx{X}_{i} = oeq_fma({ww}, t, gx{X}_{i});")
+            if first:
+                E(f"dw = oeq_fma(a{X}_{i}, t, dw); dw = oeq_fma(x{X}_{i}, tb, dw);")
+                E(f"dx{X}_{i} = oeq_fma({w}, tb, dx{X}_{i}); dx{X}_{i} = oeq_fma({ww}, t, dx{X}_{i});")
             E.level -= 1
             E("}")
 
@@ -123,7 +134,7 @@ class UVUDoubleGenerator(DoubleArithmetic, UVUDirectGenerator):
         E(f"T* __restrict__ Wgr = Wg + {rc} * {self.WN};")
         for f in self.used_y:
             E(f"const T y{f} = Yr[{f}], b{f} = Br[{f}];")
-            E(f"T gy{f} = (T)0;")
+            E(f"T dy{f} = (T)0;")
         if self.NCH == 1:
             E("{")
             E.level += 1
@@ -138,11 +149,11 @@ class UVUDoubleGenerator(DoubleArithmetic, UVUDirectGenerator):
         E.level -= 1
         E("}")
         for f in self.used_y:
-            E(f"gy{f} = {'oeq_wave_sum63' if self.P == WAVE else f'oeq_group_sum<{self.P}>'}(gy{f});")
+            E(f"dy{f} = {'oeq_wave_sum63' if self.P == WAVE else f'oeq_group_sum<{self.P}>'}(dy{f});")
         E(f"if ({'lane == 63' if self.P == WAVE else 'ul == 0'}) {{")
         E(f"    T* __restrict__ Ygr = Yg + {rc} * {self.D2};")
         for f in range(self.D2):
-            E(f"    Ygr[{f}] = " + (f"gy{f};" if f in self.used_y else "(T)0;"))
+            E(f"    Ygr[{f}] = " + (f"dy{f};" if f in self.used_y else "(T)0;"))
         E("}")
         return E.text()
 
@@ -152,11 +163,11 @@ class UVUDoubleGenerator(DoubleArithmetic, UVUDirectGenerator):
             for src, name in (("X", "x"), ("A", "a")):
                 self.emit_record_load(E, [f"{name}{i}_{m}" for m in range(blk.D)],
                                       f"{src} + (u64){rc} * {self.D1} + {blk.off} + {self.uclamp(blk, c)} * {blk.D}", self.act_c(blk, c))
-            E("T " + ", ".join(f"gx{i}_{m} = (T)0" for m in range(blk.D)) + ";")
+            E("T " + ", ".join(f"dx{i}_{m} = (T)0" for m in range(blk.D)) + ";")
 
         def fetch(oi):
             o = self.out[oi]
-            # everything a lane adds up across lanes (gy) is proportional to dZ: zero for idle lanes
+            # everything a lane adds up across lanes (dy) is proportional to dZ: zero for idle lanes
             self.emit_record_load(E, [f"G{oi}_{k}" for k in range(o.D)],
                                   f"G + (u64){rc} * {self.D3} + {o.off} + {self.uclamp(o, c)} * {o.D}", self.act(o), zero=True)
             for p in self.paths_into(oi):
@@ -191,7 +202,7 @@ class UVUDoubleGenerator(DoubleArithmetic, UVUDirectGenerator):
             if a.dim == 0:
                 continue
             if a.idx in self.used_in1:
-                self.emit_block_store(E, a, [f"gx{a.idx}_{m}" for m in range(a.D)], "Xg", self.D1, rc, self.xrow_of, "store",
+                self.emit_block_store(E, a, [f"dx{a.idx}_{m}" for m in range(a.D)], "Xg", self.D1, rc, self.xrow_of, "store",
                                       via_lds=self.dx_through_slot(a))
             else:
                 self.emit_record_store(E, ["(T)0"] * a.D, f"Xg + (u64){rc} * {self.D1} + {a.off} + u * {a.D}", self.act(a))

@@ -34,6 +34,7 @@ from .uvu_recv import UVURecvGenerator
 class UVUSortedGenerator:
     kind = "conv_atomic"
     SCAN_THREADS = 1024
+    SEGMENTED = UVUDetGenerator      # what walks the groups
 
     # dX values per edge from which the grouped backward is the starting choice.  Measured with the grouping
     # rebuilt on every call: 288 per edge - atomic 202 us, grouped 200 us, a tie; 2304 per edge - atomic
@@ -50,14 +51,14 @@ class UVUSortedGenerator:
     def __init__(self, problem: TPProblem, vector_stores: bool = True, grouped_backward=None, idx_ctype: str = "i64",
                  recv_backward=None):
         self.problem = problem
-        self.fwd = UVUDetGenerator(problem, forward_perm=True, vector_stores=vector_stores, idx_ctype=idx_ctype)
+        self.fwd = self.SEGMENTED(problem, forward_perm=True, vector_stores=vector_stores, idx_ctype=idx_ctype)
         if grouped_backward is None:
             forced = tunables.current.conv_backward               # "grouped" / "atomic": A/B runs
             grouped_backward = (forced == "grouped") if forced else self.fwd.D1 >= self.ATOMIC_BACKWARD_MAX_D1
         self.grouped_backward = grouped_backward
         self.recv_backward = False
         if grouped_backward:
-            self.bwd = UVUDetGenerator(problem, backward_perm=True, vector_stores=vector_stores, idx_ctype=idx_ctype)
+            self.bwd = self.SEGMENTED(problem, backward_perm=True, vector_stores=vector_stores, idx_ctype=idx_ctype)
             if recv_backward is not False and (recv_backward or self.fwd.D3 >= self.RECV_ORDER_MIN_RATIO * self.fwd.D1):
                 # long dZ rows: the two-pass backward in receiver order (pass 1 over the receiver grouping, which the
                 # backward then builds as well; pass 2 over the sender grouping), where pass 1 can stage its operands

@@ -23,12 +23,13 @@ import torch
 from . import runtime as rt
 from . import tunables
 from .autograd_glue import double_backward_terms
+from .codegen.uvu_conv_double import conv_double_generator
 from .codegen.uvu_det import UVUDetGenerator
 from .codegen.uvu_direct import UVUDirectGenerator
 from .codegen.uvu_recv import UVURecvGenerator
 from .codegen.uvu_sorted import UVUSortedGenerator
 from .problem import TPProblem
-from .tensor_product import _contiguous, _make_steps, _on_device, validate_problem
+from .tensor_product import _capturing, _contiguous, _make_steps, _on_device, validate_problem
 from .weight_order import WeightReorder
 from .wigner import wigner_3j
 
@@ -206,6 +207,7 @@ class TensorProductConv:
                          and tunables.current.conv_backward is None)
         self.graph_cache = tunables.current.graph_cache if graph_cache is None else bool(graph_cache)
         self._internal_unaligned = None
+        self._double = None                   # kernels of the double backward, compiled on first need
         self._reorder = WeightReorder(config)
         self.reorder_weights_e3nn_to_oeq = self._reorder.e3nn_to_oeq
         self.reorder_weights_oeq_to_e3nn = self._reorder.oeq_to_e3nn
@@ -241,6 +243,23 @@ class TensorProductConv:
             for rec in self._workspaces.values():            # the workspace may have to grow: sizes are re-checked per call
                 rec.bwd_key = None
         return self._bwd_variants[name]
+
+    def _double_usable(self) -> bool:
+        """Not under stream capture before its code object is loaded: the first-order kernels are, and the second
+        derivatives are composed from them there."""
+        return self._double is not None or not _capturing()
+
+    def _double_impl(self) -> "rt.ConvImpl":
+        """Kernel set of the fused double backward; its steps share the operator's workspace."""
+        if self._double is None:
+            idx = "i64" if self.idx_dtype == np.int64 else "int"
+            g = conv_double_generator(self.config, self.deterministic, idx)
+            code = rt.variant_code(("conv double", self.config.signature(), self.deterministic, idx, g.variant()), g.render)
+            need = rt.STEP_NEEDS_WORKSPACE | (rt.STEP_NEEDS_TPERM if self.deterministic else 0)
+            impl = rt.ConvImpl(code, [], _make_steps(g.steps(), need))
+            self._ws_fns.append(g.plan()[2])
+            self._double = impl
+        return self._double
 
     @staticmethod
     def name():
@@ -374,6 +393,25 @@ class TensorProductConv:
                               nnz, node_count, workspace, transpose_perm,
                               self._stream() if stream is None else stream, prepared, counters_zero)
 
+    def double_backward_rawptrs(self, L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot, L1_out, L2_out,
+                                weights_out, L3_grad_out, rows, cols, nnz, node_count, transpose_perm=0, stream=None):
+        """Gradients of the backward's inputs (x, y, w, dz) for cotangents of its outputs, in two passes over the edges
+        (codegen/uvu_conv_double.py).  Builds both graph preparations anew in the operator's scratch for the stream, so
+        neither the forward's nor the backward's cached one is valid afterwards."""
+        nnz, node_count = int(nnz), int(node_count)
+        if self.deterministic and nnz > 0 and not transpose_perm:
+            raise ValueError("the deterministic double backward needs transpose_perm (a device pointer), got 0")
+        if any(int(p) % 16 for p in (L1_out, L3_grad_out)):
+            raise ValueError("the double backward writes 16-byte vectors: its node outputs must be 16-byte aligned")
+        impl = self._double_impl()
+        rec = self._workspace_record(nnz, node_count, stream)
+        if torch.cuda.is_current_stream_capturing():
+            rec.captured = True
+        rec.fwd_key = rec.bwd_key = rec.zero_fwd = rec.zero_bwd = None
+        impl.double_backward(L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot, L1_out, L2_out,
+                             weights_out, L3_grad_out, rows, cols, nnz, node_count, rec.buffer.data_ptr(), transpose_perm,
+                             self._stream() if stream is None else stream)
+
     def _time_backward_variants(self, run, names=("atomic", "grouped"), repeats: int = 3) -> str:
         """Fastest of the backward variants on the caller's own tensors: one untimed call each (compilation,
         graph preparation), then the best of ``repeats`` timed calls between HIP events."""
@@ -505,6 +543,37 @@ class TensorProductConv:
         def _(L1_in, L2_in, weights, L3_grad, *index):
             return [L1_in.new_empty(*L1_in.shape), L2_in.new_empty(*L2_in.shape), weights.new_empty(*weights.shape)]
 
+        def double_impl(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, rows, cols, tperm):
+            x, y, w, g, a, b, v, rows, cols, tperm = _contiguous(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot,
+                                                                 rows, cols, tperm)
+            self._check(x, y, w, rows, cols, tperm, g)
+            self._check(a, b, v, rows, cols, tperm)
+            if a.shape != x.shape or a.device != x.device:
+                raise ValueError("the cotangents must match the operands' nodes and device")
+            out = [torch.empty_like(t) for t in (x, y, w, g)]
+            with _on_device(x.device):
+                self.double_backward_rawptrs(*(t.data_ptr() for t in (x, y, w, g, a, b, v, *out, rows, cols)), rows.shape[0],
+                                             x.shape[0], tperm.data_ptr() if tperm is not None else 0,
+                                             stream=self._stream(x.device.index))
+            return out
+
+        if not det:
+            @torch.library.custom_op(f"openequivariance_amd::conv_double_backward{cid}", mutates_args=(), device_types="cuda")
+            def fused(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, L3_grad: torch.Tensor,
+                      L1_cot: torch.Tensor, L2_cot: torch.Tensor, weights_cot: torch.Tensor, rows: torch.Tensor,
+                      cols: torch.Tensor) -> typing.List[torch.Tensor]:
+                return double_impl(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, rows, cols, None)
+        else:
+            @torch.library.custom_op(f"openequivariance_amd::conv_double_backward{cid}", mutates_args=(), device_types="cuda")
+            def fused(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, L3_grad: torch.Tensor,
+                      L1_cot: torch.Tensor, L2_cot: torch.Tensor, weights_cot: torch.Tensor, rows: torch.Tensor,
+                      cols: torch.Tensor, transpose_perm: torch.Tensor) -> typing.List[torch.Tensor]:
+                return double_impl(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, rows, cols, transpose_perm)
+
+        @fused.register_fake
+        def _(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, *index):
+            return [t.new_empty(*t.shape) for t in (L1_in, L2_in, weights, L3_grad)]
+
         def setup_context(ctx, inputs, output):
             ctx.L1_in, ctx.L2_in, ctx.weights, *ctx.index = inputs
 
@@ -519,7 +588,8 @@ class TensorProductConv:
 
         def double_backward(ctx, grad_output):
             terms = double_backward_terms(forward, backward_helper, ctx.L1_in, ctx.L2_in, ctx.weights, ctx.L3_grad,
-                                          grad_output[0], grad_output[1], grad_output[2], tuple(ctx.index))
+                                          grad_output[0], grad_output[1], grad_output[2], tuple(ctx.index),
+                                          fused=fused if self._double_usable() else None)
             return terms + (None,) * len(ctx.index)
 
         backward_helper.register_autograd(double_backward, setup_context=setup_context_double_backward)

@@ -51,6 +51,11 @@ def _contiguous(*tensors):
     return tuple(t if t is None or t.is_contiguous() else t.contiguous() for t in tensors)
 
 
+def _capturing() -> bool:
+    """torch's current stream is recording a graph (never on a machine without a GPU)."""
+    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+
+
 def _on_device(device):
     """Context that makes ``device`` current: nothing at all when it already is (the usual case; entering
     torch.cuda.device costs several microseconds per call)."""
@@ -311,7 +316,9 @@ class TensorProduct(TensorProductBase):
 
         def double_backward(ctx, grad_output):
             return double_backward_terms(forward, backward_helper, ctx.L1_in, ctx.L2_in, ctx.weights, ctx.L3_grad,
-                                         grad_output[0], grad_output[1], grad_output[2], fused=fused)
+                                         grad_output[0], grad_output[1], grad_output[2],
+                                         # (its code object is loaded on first use, which a stream capture must not do)
+                                         fused=fused if self._double or not _capturing() else None)
 
         backward_helper.register_autograd(double_backward, setup_context=setup_context_double_backward)
 
