@@ -59,6 +59,7 @@ class WPath:
     v: int = 0                      # which copy of the second operand this path contracts with ...
     mv: int = 1                     # ... out of this many (the instruction's weights are [u][v][w])
     poff: int = 0                   # offset of this path's [u][w] slice in the dense dW partial rows
+    gs: int = 4                     # forward K steps fetched at a time
 
     @property
     def mu(self) -> int:
@@ -69,8 +70,8 @@ class WPath:
         return self.o.mul
 
     @property
-    def SU(self) -> int:            # K steps over u (forward): whole blocks of 16 channels, 4 steps each
-        return 4 * _ceil(self.mu, 16)
+    def SU(self) -> int:            # K steps over u (forward): blocks of 16 channels, 4 steps each (step s: channels 4 g + s)
+        return 4 * (self.mu // 16) + self.gs * _ceil(min(4, self.mu % 16), self.gs)
 
     @property
     def SW(self) -> int:            # K steps over w (backward dX)
@@ -94,6 +95,8 @@ class UVWGenerator:
     # w tiles.  (48 instead of 80, for a third wavefront per SIMD, measured slower on 64x0e+64x1o+64x2e: fp32
     # 0.329 -> 0.376 ms, fp64 0.566 -> 0.694 ms - the CG part of a tile is then computed once per range.)
     FWD_ACC_LIMIT = 80
+    FWD_PIPELINE = {4: (4, 1), 8: (1, 3)}
+    BWD_LDS_LIMIT = 80 * 1024    # dZ tile of the backward: two workgroups per compute unit (gfx950: 160 KB)
 
     def __init__(self, problem: TPProblem):
         self.problem = problem
@@ -107,7 +110,7 @@ class UVWGenerator:
         # MI355X: fp32 4 / 1, fp64 1 / 3; a loop written out on alternating register sets, so that nothing is
         # copied between sets, has 0.9 instead of 2.1 vector-ALU instructions per MFMA and measured 0.341
         # against 0.331 ms; larger groups for the cheap work items 0.361 - 0.422 against 0.359 ms)
-        self.fwd_group, self.fwd_unroll = (4, 1) if self.T == "float" else (1, 3)
+        self.fwd_group, self.fwd_unroll = self.FWD_PIPELINE[self.itemsize]
         # Tile shape: 16 x 16 x 4 in both types.  The fp32 forward on v_mfma_f32_32x32x2_f32 (32 batch rows per
         # tile, half the weight-operand loads per FLOP) passed the same parity tests and measured 0.371 ms (w
         # ranges of at most 96 accumulator registers, two wavefronts per SIMD) and 0.374 ms (whole output
@@ -136,7 +139,8 @@ class UVWGenerator:
             # it is emitted as mv paths over single-copy blocks (reference: loop_unroll_tp.cuh:48-60 walks v)
             for v in range(b.mul):
                 bv = Block(b.idx, 1, b.l, b.off + v * b.D)
-                p = WPath(len(self.paths), a, bv, o, ins.path_weight, woff, v=v, mv=b.mul, poff=woff + v * a.mul * o.mul)
+                p = WPath(len(self.paths), a, bv, o, ins.path_weight, woff, v=v, mv=b.mul, poff=woff + v * a.mul * o.mul,
+                          gs=self.fwd_group)
                 for i, j, k in np.argwhere(np.abs(c) > 1e-14):
                     p.pairs.setdefault((int(i), int(j)), []).append((int(k), float(c[i, j, k])))
                 self.paths.append(p)
@@ -180,7 +184,8 @@ class UVWGenerator:
         # backward dX/dY: the 16-row dZ tile is staged in LDS when it fits (row stride padded against bank
         # conflicts of the B-operand reads: lanes c = 0..15 read 16 different rows at the same column)
         self.bwd_rs = self._pick_row_stride()
-        self.bwd_lds = 16 * self.bwd_rs * self.itemsize <= 80 * 1024    # gfx950: 160 KB per CU
+        self.bwd_groups = [list(self.used_in1)]          # in1 blocks by group of wavefronts (one group: four wavefronts a tile)
+        self.bwd_lds = 16 * self.bwd_rs * self.itemsize <= self.BWD_LDS_LIMIT
         # packed weight copies in the workspace
         pos = 0
         for p in self.paths:
@@ -482,9 +487,19 @@ class UVWGenerator:
             E("}")
 
     # ====================================================== backward: dX, dY
+    # wavefronts of a workgroup: one per 16-channel u-subtile
+    backward_threads = 256
+
     def backward_body(self) -> str:
         E = Emitter()
-        E("const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;")
+        NT_, groups = self.backward_threads, self.bwd_groups
+        if len(groups) == 1:
+            E("const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;")
+        else:
+            E("const int lane = threadIdx.x & 63, grp = threadIdx.x >> 8, c = lane & 15, g = lane >> 4;")
+            # (opaque: a compiler that sees wave < 4 drops the branches that keep an item's two halves apart, and spills)
+            E("int wave = (threadIdx.x >> 6) & 3;")
+            E("OEQ_OPAQUE(wave);")
         E("const u64 row0 = (u64)blockIdx.x * 16;")
         E("if (row0 >= n) return;")
         E("const u64 rowB = min(row0 + (u64)c, n - 1);")
@@ -492,7 +507,7 @@ class UVWGenerator:
         E("const T* __restrict__ wsT = (const T*)ws;")
         E(f"const T* __restrict__ Xr = X + rowB * {self.D1};")
         E(f"const T* __restrict__ Gr = G + rowB * {self.D3};")
-        E(f"__shared__ T dyl[4 * 16 * {max(1, self.D2)}];")
+        E(f"__shared__ T dyl[{NT_ // 64} * 16 * {max(1, self.D2)}];")
         if self.bwd_lds:
             # the dZ tile goes to LDS once per workgroup (coalesced, one HBM round trip), and every
             # wavefront reads its MFMA B operands from there
@@ -502,34 +517,49 @@ class UVWGenerator:
             if self.D3 % VW == 0:
                 # 16-byte vectors, all requested before the first one is written to LDS
                 NV, RV = 16 * self.D3 // VW, self.D3 // VW
-                NQ = _ceil(NV, 256)
+                NQ = _ceil(NV, NT_)
                 E("if ((((unsigned long long)G) & 15ull) == 0) {")
                 E.level += 1
                 E(f"VT gv[{NQ}];")
                 for q in range(NQ):
-                    idx = f"(int)threadIdx.x + {256 * q}"
-                    guard = "" if 256 * (q + 1) <= NV else f"if ({idx} < {NV}) "
+                    idx = f"(int)threadIdx.x + {NT_ * q}"
+                    guard = "" if NT_ * (q + 1) <= NV else f"if ({idx} < {NV}) "
                     E(f"{guard}{{ const int r_ = ({idx}) / {RV}, v_ = ({idx}) - r_ * {RV}; "
                       f"gv[{q}] = *(const VT*)(G + min(row0 + (u64)r_, n - 1) * {self.D3} + v_ * {VW}); }}")
                 for q in range(NQ):
-                    idx = f"(int)threadIdx.x + {256 * q}"
-                    guard = "" if 256 * (q + 1) <= NV else f"if ({idx} < {NV}) "
+                    idx = f"(int)threadIdx.x + {NT_ * q}"
+                    guard = "" if NT_ * (q + 1) <= NV else f"if ({idx} < {NV}) "
                     E(f"{guard}{{ const int r_ = ({idx}) / {RV}, v_ = ({idx}) - r_ * {RV}; T* __restrict__ d_ = gl + r_ * {RS} + v_ * {VW}; "
                       + " ".join(f"d_[{i}] = gv[{q}][{i}];" for i in range(VW)) + " }")
                 E.level -= 1
                 E("} else")
-            E(f"for (int q = threadIdx.x; q < 16 * {self.D3}; q += 256) {{")
+            E(f"for (int q = threadIdx.x; q < 16 * {self.D3}; q += {NT_}) {{")
             E(f"    const int r_ = q / {self.D3}, col_ = q - r_ * {self.D3};")
             E(f"    gl[r_ * {RS} + col_] = G[min(row0 + (u64)r_, n - 1) * {self.D3} + col_];")
             E("}")
         for f in self.used_y:
             E(f"const T y{f} = Y[rowB * {self.D2} + {f}];")
             E(f"T dy{f} = (T)0;")
+        if len(groups) == 1:
+            self._backward_items(E, self.used_in1, synced=False)
+        else:
+            E("oeq_block_sync();")
+            for k_, ins in enumerate(groups):
+                E(f"if (grp == {k_}) {{   // in1 blocks {ins}")
+                E.level += 1
+                self._backward_items(E, ins, synced=True)
+                E.level -= 1
+                E("}")
+        self._backward_tail(E)
+        return E.text()
+
+    def _backward_items(self, E: Emitter, in1, synced: bool) -> None:
+        """The work of one wavefront on the in1 blocks ``in1`` (all of them, or those of its group of wavefronts)."""
         # X records and dX accumulators of this wavefront: u-subtiles mt = wave + 4q, rows r of the
         # accumulator tile.  X is read once for all paths that consume the block.  With the dZ tile in
         # LDS the work is ordered by in1 block, so only one block's X and dX are live at a time (plus the
         # next block's X, requested one block ahead); otherwise everything is loaded here.
-        for ai in self.used_in1:
+        for ai in in1:
             a = self.in1[ai]
             for q in range(_ceil(_ceil(a.mul, 16), 4)):
                 for r in range(4):
@@ -557,9 +587,9 @@ class UVWGenerator:
                 E("}")
         by_in1 = self.bwd_lds
         if by_in1:
-            load_x(E, self.used_in1[0])
+            load_x(E, in1[0])
         else:
-            for ai in self.used_in1:
+            for ai in in1:
                 load_x(E, ai)
         # Work list of this wavefront: (output block, path, u-subtile group).  The packed weight
         # fragments (MFMA A operand) of the next item are fetched into a second register set while
@@ -567,10 +597,10 @@ class UVWGenerator:
         # as the last matrix-core step of the current one is issued, so that neither L2 nor HBM
         # latency sits between two items.
         if by_in1:
-            items = [(p.o.idx, p, q) for ai in self.used_in1 for p in self.paths_from(ai) for q in range(_ceil(p.NTU, 4))]
+            items = [(p.o.idx, p, q) for ai in in1 for p in self.paths_from(ai) for q in range(_ceil(p.NTU, 4))]
         else:
             items = [(oi, p, q) for oi in self.used_out for p in self.paths_into(oi) for q in range(_ceil(p.NTU, 4))]
-        max_sw = max(_ceil(self.out[oi].mul, 4) for oi in self.used_out)
+        max_sw = max(_ceil(self.out[oi].mul, 4) for oi in {it[0] for it in items})
         NSETS = 1          # register sets of packed weight fragments (a second set, fetched one item ahead, measured no gain)
         E("T " + ", ".join(f"af{b_}_{s_}" for b_ in range(NSETS) for s_ in range(max_sw)) + ";")
 
@@ -591,7 +621,9 @@ class UVWGenerator:
                 if o.mul % 4 != 0:
                     E(f"if ({4 * s_} + g >= {o.mul}) {{ " + " ".join(f"gz{oi}_{s_}_{k} = (T)0;" for k in range(o.D)) + " }")
 
-        if self.bwd_lds:
+        if synced:
+            pass
+        elif self.bwd_lds:
             E("oeq_block_sync();")
         else:
             for oi in self.used_out:
@@ -610,10 +642,10 @@ class UVWGenerator:
             # sinking the vector-ALU halves of all items below the matrix-core work, which would keep
             # every accumulator alive and halve the occupancy.
             cond = f"wave + {4 * q} < {p.NTU}"
-            if by_in1 and (j == 0 or items[j - 1][1].a.idx != a.idx):
-                nxt = self.used_in1.index(a.idx) + 1
-                if nxt < len(self.used_in1):
-                    load_x(E, self.used_in1[nxt])
+            if by_in1 and not synced and (j == 0 or items[j - 1][1].a.idx != a.idx):
+                nxt = in1.index(a.idx) + 1
+                if nxt < len(in1):
+                    load_x(E, in1[nxt])
             if j + 1 < len(items) and NSETS == 2:
                 load_a(E, j + 1)
             for k in range(o.D):
@@ -656,34 +688,47 @@ class UVWGenerator:
             E("}")
             if by_in1 and (j + 1 == len(items) or items[j + 1][1].a.idx != a.idx):
                 store_dx(E, a.idx)
-        # ---- dX stores
+                if synced and j + 1 < len(items):        # (several groups: no registers for a block ahead)
+                    load_x(E, items[j + 1][1].a.idx)
+        if not by_in1:
+            for ai in in1:
+                store_dx(E, ai)
+
+    def _backward_tail(self, E: Emitter) -> None:
+        W_ = self.backward_threads // 64
+        wave = "wave" if len(self.bwd_groups) == 1 else "(threadIdx.x >> 6)"
+        # ---- blocks of dX that no path reads
         for a in self.in1:
             if a.dim == 0:
                 continue
             if a.idx not in self.used_in1:
-                E(f"if (wave == 0 && bvalid) for (int q = g; q < {a.dim}; q += 4) Xg[(row0 + c) * {self.D1} + {a.off} + q] = (T)0;")
-            elif not by_in1:
-                store_dx(E, a.idx)
+                E(f"if ({wave} == 0 && bvalid) for (int q = g; q < {a.dim}; q += 4) Xg[(row0 + c) * {self.D1} + {a.off} + q] = (T)0;")
         # ---- dY: sum over the 4 lane groups (channels), then over the 4 wavefronts, fixed order
         for f in self.used_y:
             E(f"dy{f} += oeq_shfl_xor(dy{f}, 16);")
             E(f"dy{f} += oeq_shfl_xor(dy{f}, 32);")
         E("if (g == 0) {")
         for f in range(self.D2):
-            E(f"    dyl[(wave * 16 + c) * {self.D2} + {f}] = " + (f"dy{f};" if f in self.used_y else "(T)0;"))
+            E(f"    dyl[({wave} * 16 + c) * {self.D2} + {f}] = " + (f"dy{f};" if f in self.used_y else "(T)0;"))
         E("}")
         E("oeq_block_sync();")
-        E(f"if (wave == 0 && g == 0 && bvalid) {{")
-        E(f"    for (int f = 0; f < {self.D2}; ++f)")
-        E(f"        Yg[(row0 + c) * {self.D2} + f] = ((dyl[c * {self.D2} + f] + dyl[(16 + c) * {self.D2} + f]) + dyl[(32 + c) * {self.D2} + f]) + dyl[(48 + c) * {self.D2} + f];")
+        E(f"if ({wave} == 0 && g == 0 && bvalid) {{")
+        E(f"    for (int f = 0; f < {self.D2}; ++f) {{")
+        E(f"        T s_ = dyl[c * {self.D2} + f];")
+        E(f"        for (int w_ = 1; w_ < {W_}; ++w_) s_ += dyl[(16 * w_ + c) * {self.D2} + f];")
+        E(f"        Yg[(row0 + c) * {self.D2} + f] = s_;")
+        E("    }")
         E("}")
-        return E.text()
 
     # ============================================================ backward: dW
     # accumulator registers (32-bit) live in one pass of the dW kernel.  fp64: the 352 accumulators of the
     # 64-channel benchmark problem in one pass leave one wavefront per SIMD and no room for anything else;
     # two passes of 192 + 160 measured 0.70 -> 0.63 ms for that kernel, three or more passes lose again
     DW_ACC_BUDGET = {4: 352, 8: 192}
+
+    @property
+    def dw_threads(self) -> int:
+        return 256 * self.dw_groups
 
     def dw_passes(self):
         """(wavefront group, [(path, first w tile, end w tile), ...]) of the passes of the dW kernel.  The
@@ -936,8 +981,8 @@ class UVWGenerator:
         fwd = [dict(kernel="prep_forward", num_threads=256, grid_kind=FIXED, num_blocks=self.prep_blocks),
                dict(kernel="forward", num_threads=64, grid_kind=ROW, work_per_block=16, grid_y=len(self.fwd_items))]
         bwd = [dict(kernel="prep_backward", num_threads=256, grid_kind=FIXED, num_blocks=self.prep_blocks),
-               dict(kernel="backward", num_threads=256, grid_kind=ROW, work_per_block=16),
-               dict(kernel="backward_dw", num_threads=256 * self.dw_groups, grid_kind=FIXED,
+               dict(kernel="backward", num_threads=self.backward_threads, grid_kind=ROW, work_per_block=16),
+               dict(kernel="backward_dw", num_threads=self.dw_threads, grid_kind=FIXED,
                     num_blocks=self.DW_WORKGROUPS),
                dict(kernel="backward_reduce", num_threads=256, grid_kind=FIXED, num_blocks=_ceil(self.WN, 256))]
         return fwd, bwd, (lambda nnz=0, nodes=0: self.ws_elems * self.itemsize)

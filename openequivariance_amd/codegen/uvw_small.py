@@ -1,0 +1,217 @@
+"""Dense "uvw" tensor products with shared weights on batches of few rows (same contraction and packing as
+:mod:`.uvw`; reference: templates/loop_unroll_tp.cuh:74-78, :184, :209).
+
+The kernels of :mod:`.uvw` give a 16-row tile to one workgroup and a whole output block to one wavefront, and let every
+dW workgroup walk all paths.  With fewer tiles than the chip has places for them, the longest of those serial chains is
+the time of a launch.  Here the same work is cut finer:
+
+* forward: output blocks in ranges of w tiles of at most ``FWD_ACC_LIMIT`` accumulators per work item;
+* backward dX/dY: the in1 blocks of a tile are dealt to two or four groups of four wavefronts, which share the dZ tile;
+* backward dW: a workgroup holds ONE path (or a range of its w tiles) and walks a share of the batch given by the path's
+  cost; its 16 wavefronts are u-subtiles x phases of the batch, combined through LDS, so that the launch leaves 15 to 80
+  partial rows of a path instead of 256 of all paths.
+
+Bound: latency of the operand loads, four wavefronts per SIMD hide what one did not.  50x0e+50x1o+50x1e+50x2o+50x2e with
+one scalar, fp64, 4097 rows (kernel times, us): dX/dY 41 -> 30, dW 35 -> 19, reduction 16.7 -> 4.6; fp32 backward of that
+product as a whole 65 -> 46.  64x0e+64x1o+64x2e, 500 rows: forward 29 -> 20 and backward 57 -> 29 in fp32, 44 -> 30 and
+81 -> 44 in fp64.
+"""
+from __future__ import annotations
+
+from typing import List
+
+from ..problem import TPProblem
+from .common import Emitter
+from .uvw import UVWGenerator, _ceil
+
+
+class UVWSmallGenerator(UVWGenerator):
+    FWD_ACC_LIMIT = 40           # accumulator tiles x 4 of one forward work item (two w tiles of an l = 2 block)
+    BWD_LDS_LIMIT = 144 * 1024   # the dZ tile may fill a compute unit: there is one workgroup for each at most
+    FWD_PIPELINE = {4: (4, 2), 8: (1, 4)}
+    DW_WAVES = 16
+    DW_REGISTERS = 88            # of 128 a lane has with 16 wavefronts: accumulators, operands and one T of a dW unit
+
+    def __init__(self, problem: TPProblem):
+        super().__init__(problem)
+        words = self.itemsize // 4
+        # in1 blocks of the backward by group of wavefronts, balanced by matrix-core steps.  fp64 takes 256 registers a
+        # lane (two groups), fp32 about 120 (four)
+        cost = {a: sum(p.o.D * p.SW * p.NTU for p in self.paths_from(a)) for a in self.used_in1}
+        groups: List[List[int]] = [[] for _ in range(min(4 if words == 1 else 2, len(cost)))]
+        if self.bwd_lds:
+            for a in sorted(cost, key=lambda k: -cost[k]):
+                min(groups, key=lambda m: sum(cost[k] for k in m)).append(a)
+            self.bwd_groups = [sorted(m) for m in groups]
+        # dW units: (path, first w tile, end w tile, wavefronts along u)
+        self.units = []
+        for p in self.paths:
+            uw = 4 if p.NTU >= 3 else p.NTU
+            q = _ceil(p.NTU, uw)
+            fixed = words * (q * p.a.D + p.o.D + 9)
+            per_w = words * (4 * q + p.o.D)
+            step = max(1, min(p.NTW, (self.DW_REGISTERS - fixed) // per_w, 16 // (q * words)))
+            step = _ceil(p.NTW, _ceil(p.NTW, step))
+            self.units += [(p, lo, min(p.NTW, lo + step), uw) for lo in range(0, p.NTW, step)]
+            self.dw_fits = getattr(self, "dw_fits", True) and fixed + step * per_w <= self.DW_REGISTERS + 24
+        # workgroups per unit, by its time on a compute unit: matrix-core cycles plus what a step costs beside them
+        cyc = 32 if words == 1 else 64
+        load = [uw * (_ceil(p.NTU, uw) * (hi - lo) * p.o.D * cyc + 100) for p, lo, hi, uw in self.units]
+        share = [max(1, int(self.DW_WORKGROUPS * l / sum(load))) for l in load]
+        for k in sorted(range(len(load)), key=lambda k: -load[k] / share[k])[:max(0, self.DW_WORKGROUPS - sum(share))]:
+            share[k] = min(self.DW_WORKGROUPS, share[k] + 1)
+        self.chunks = share
+        self.unit_off, pos = [], self.PART_OFF
+        for (p, lo, hi, _), ch in zip(self.units, share):
+            self.unit_off.append(pos)
+            pos += ch * p.mu * self._width(p, lo, hi)
+        assert pos <= self.ws_elems, "the partial rows of few workgroups per path outgrow those of all paths"
+
+    @staticmethod
+    def row_limits(g: UVWGenerator):
+        """Largest batch (forward, backward) these kernels take from ``g``'s.  Forward, 64 channels: fp32 8192 rows 50 -> 42
+        us, 65 536 rows 194 -> 234; fp64 2000 rows 47 -> 34, 4097 rows 50 -> 53.  Backward, where a block is read by several
+        paths, each of which fetches it here (64 channels, 3.9 times): 4097 rows 73 -> 60 us in fp32 and 118 -> 104 in fp64, 8192
+        rows 81 -> 84 and 131 -> 149; where every block has one path (50 channels) 65 536 rows still gain, 512 -> 459
+        and 803 -> 619."""
+        fetched = sum(p.a.dim + p.o.dim for p in g.paths)
+        once = sum(g.in1[a].dim for a in g.used_in1) + sum(g.out[o].dim for o in g.used_out)
+        return (8192 if g.itemsize == 4 else 2048), (65536 if fetched <= 1.25 * once else 5120)
+
+    @staticmethod
+    def _width(p, lo, hi) -> int:
+        return min(p.mw, 16 * hi) - 16 * lo
+
+    @classmethod
+    def create(cls, problem: TPProblem):
+        """The generator, or None where a dW unit does not fit its registers or no launch would be cut finer."""
+        try:
+            g = cls(problem)
+        except NotImplementedError:
+            return None
+        return g if g.dw_fits and g.bwd_lds else None
+
+    def forward_attr(self) -> str:
+        return " __attribute__((amdgpu_waves_per_eu(2)))"
+
+    def backward_attr(self) -> str:
+        return ""
+
+    @property
+    def backward_threads(self) -> int:
+        return 256 * len(self.bwd_groups)
+
+    @property
+    def dw_threads(self) -> int:
+        return 64 * self.DW_WAVES
+
+    # ============================================================ backward: dW
+    def _live_chunks(self, k: int) -> str:
+        """Workgroups of unit k that have rows to walk (the rest leave no partial row)."""
+        per = 4 * (self.DW_WAVES // self.units[k][3])
+        return f"(int)min((u64){self.chunks[k]}, (n + {per - 1}) / {per})"
+
+    def backward_dw_body(self) -> str:
+        E = Emitter()
+        PH = lambda uw: self.DW_WAVES // uw
+        slots = max(uw * (PH(uw) // 2) * _ceil(p.NTU, uw) * (hi - lo) * 256 for p, lo, hi, uw in self.units)
+        E("const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;")
+        E(f"__shared__ T comb[{max(1, slots)}];")
+        first = 0
+        for k, (p, lo, hi, uw) in enumerate(self.units):
+            Q, ph, D = _ceil(p.NTU, uw), PH(uw), p.o.D
+            cells = [(q, nt) for q in range(Q) for nt in range(lo, hi)]
+            E(f"{'else ' if k else ''}if (blockIdx.x < {first + self.chunks[k]}) {{ // path {p.t}, w tiles {lo} .. {hi - 1} of {p.NTW}")
+            E.level += 1
+            E(f"const int chunk = blockIdx.x - {first}, live = {self._live_chunks(k)};")
+            E("if (chunk >= live) return;")
+            E(f"const int uwv = wv % {uw}, ph = wv / {uw};")
+            for q, nt in cells:
+                E(f"V4 acc{q}_{nt} = {{0, 0, 0, 0}};")
+            E("#pragma unroll 1")
+            E(f"for (u64 s = (u64)(chunk * {ph} + ph); s < (n + 3) / 4; s += (u64)(live * {ph})) {{")
+            E.level += 1
+            E("const u64 b = 4 * s + g;          // batch row of this lane for both operands")
+            E("const bool bv = b < n;")
+            E("const u64 bc = bv ? b : n - 1;")
+            for f in sorted({p.b.off + j for (_, j) in p.pairs}):
+                E(f"T y{f} = Y[bc * {self.D2} + {f}];")
+            E(f"const T* __restrict__ Xr = X + bc * {self.D1} + {p.a.off};")
+            E(f"const T* __restrict__ Gr = G + bc * {self.D3} + {p.o.off};")
+            for q in range(Q):
+                uexp = f"16 * (uwv + {uw * q}) + c"
+                ucl = uexp if p.mu % (16 * uw) == 0 else f"min({uexp}, {p.mu - 1})"
+                E("T " + ", ".join(f"x{q}_{i}" for i in range(p.a.D)) + ";")
+                E(f"{{ const T* __restrict__ xp = Xr + ({ucl}) * {p.a.D}; " + " ".join(f"x{q}_{i} = xp[{i}];" for i in range(p.a.D)) + " }")
+            for nt in range(lo, hi):
+                wexp = f"{16 * nt} + c"
+                wcl = wexp if p.mw % 16 == 0 else f"min({wexp}, {p.mw - 1})"
+                E("T " + ", ".join(f"g{nt}_{k_}" for k_ in range(D)) + ";")
+                E(f"{{ const T* __restrict__ gp = Gr + ({wcl}) * {D}; " + " ".join(f"g{nt}_{k_} = gp[{k_}];" for k_ in range(D)) + " }")
+            E("if (!bv) { " + " ".join(f"y{f} = (T)0;" for f in sorted({p.b.off + j for (_, j) in p.pairs})) + " }     // rows past the end: T = 0 there")
+            for q in range(Q):
+                if p.mu % (16 * uw) != 0:
+                    E(f"if (16 * (uwv + {uw * q}) + c >= {p.mu}) {{ " + " ".join(f"x{q}_{i} = (T)0;" for i in range(p.a.D)) + " }")
+                E("{")
+                E.level += 1
+                self.emit_cg_forward(E, p, f"x{q}_", "y", "t")
+                for nt in range(lo, hi):
+                    for k_ in range(D):
+                        E(f"acc{q}_{nt} = oeq_mfma(t{k_}, g{nt}_{k_}, acc{q}_{nt});")
+                E.level -= 1
+                E("}")
+            E.level -= 1
+            E("}")
+            # phases of the batch, summed pairwise in a fixed order
+            half = ph // 2
+            while half >= 1:
+                E(f"if (ph >= {half} && ph < {2 * half}) {{ T* __restrict__ d_ = comb + ((ph - {half}) * {uw} + uwv) * {len(cells) * 256} + lane;")
+                for i, (q, nt) in enumerate(cells):
+                    E("    " + " ".join(f"d_[{256 * i + 64 * r}] = acc{q}_{nt}[{r}];" for r in range(4)))
+                E("}")
+                E("oeq_block_sync();")
+                E(f"if (ph < {half}) {{ const T* __restrict__ d_ = comb + (ph * {uw} + uwv) * {len(cells) * 256} + lane;")
+                for i, (q, nt) in enumerate(cells):
+                    E("    " + " ".join(f"acc{q}_{nt}[{r}] += d_[{256 * i + 64 * r}];" for r in range(4)))
+                E("}")
+                if half > 1:
+                    E("oeq_block_sync();")
+                half //= 2
+            width = self._width(p, lo, hi)
+            E(f"if (ph == 0) {{ T* __restrict__ part = (T*)ws + {self.unit_off[k]} + (u64)chunk * {p.mu * width};")
+            for q, nt in cells:
+                for r in range(4):
+                    E(f"    {{ const int u = 16 * (uwv + {uw * q}) + {self.row(r)}; const int w = {16 * (nt - lo)} + c;")
+                    E(f"      if (u < {p.mu} && w < {width}) part[u * {width} + w] = acc{q}_{nt}[{r}]; }}")
+            E("}")
+            E.level -= 1
+            E("}")
+            first += self.chunks[k]
+        return E.text()
+
+    def reduce_body(self) -> str:
+        E = Emitter()
+        # 64 weights a workgroup, its four wavefronts take every fourth partial row
+        E("const int q = blockIdx.x * 64 + (threadIdx.x & 63), sl = threadIdx.x >> 6;")
+        E("__shared__ T sums[192];")
+        E("const T* __restrict__ part = (const T*)ws;")
+        E("int live = 0, size = 0, dst = 0;")
+        pos = 0
+        for k, (p, lo, hi, _) in enumerate(self.units):
+            width = self._width(p, lo, hi)
+            size = p.mu * width
+            E(f"{'else ' if k else ''}if (q < {pos + size}) {{ const int e = q - {pos}; const int u = e / {width}; const int w = {16 * lo} + e - u * {width};")
+            E(f"    live = {self._live_chunks(k)}; size = {size}; part += {self.unit_off[k]} + e; dst = {self.oeq_index(p, 'u', 'w')}; }}")
+            pos += size
+        E("T acc = (T)0;")
+        E("for (int b = sl; b < live; b += 4) acc += part[(u64)b * size];")
+        E("if (sl > 0) sums[(sl - 1) * 64 + (threadIdx.x & 63)] = acc;")
+        E("oeq_block_sync();")
+        E(f"if (sl == 0 && q < {pos}) Wg[dst] = ((acc + sums[threadIdx.x]) + sums[64 + threadIdx.x]) + sums[128 + threadIdx.x];")
+        return E.text()
+
+    def plan(self):
+        fwd, bwd, ws = super().plan()
+        bwd[2]["num_blocks"] = sum(self.chunks)
+        bwd[3]["num_blocks"] = _ceil(self.WN, 64)
+        return fwd, bwd, ws

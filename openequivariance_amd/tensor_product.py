@@ -20,6 +20,8 @@ from .autograd_glue import double_backward_terms
 from .codegen.uvu import UVUGenerator
 from .codegen.uvu_direct import UVUDirectGenerator
 from .codegen.uvu_double import UVUDoubleGenerator
+from .codegen.uvw import UVWGenerator
+from .codegen.uvw_small import UVWSmallGenerator
 from .codegen.uvw_batched import UVWBatchedGenerator
 from .problem import TPProblem
 from .weight_order import WeightReorder
@@ -70,7 +72,6 @@ def select_generator(config: TPProblem):
     loads where those sums do not fit)."""
     mode = validate_problem(config)
     if mode == "uvw" and config.shared_weights:
-        from .codegen.uvw import UVWGenerator
         from .codegen.uvw_rows import UVWRowsGenerator
         # a few hundred weights on multiplicities far below a 16 x 16 tile: one row per lane on the vector ALU
         return UVWRowsGenerator(config) if UVWRowsGenerator.suits(config) else UVWGenerator(config)
@@ -134,6 +135,9 @@ class TensorProduct(TensorProductBase):
         self._dims = (self.L1.dim, self.L2.dim, self.L3.dim, config.weight_numel)
         self._workspaces = {}                 # (device, stream) -> scratch tensor (fixed size, never regrown)
         self._internal_unaligned = None       # kernels without 16-byte vector stores, compiled on first need
+        # dense uvw: largest batch (forward, backward) of the kernels for few rows, which are compiled on first need
+        self._few_rows = None
+        self._few_rows_limits = UVWSmallGenerator.row_limits(self.generator) if type(self.generator) is UVWGenerator else (0, 0)
         # double backward in one launch: kernels by alignment of the outputs, compiled on first need
         self._double_generator = UVUDoubleGenerator if mode == "uvu" and UVUDoubleGenerator.suits(config) else None
         self._double = {}
@@ -187,16 +191,31 @@ class TensorProduct(TensorProductBase):
             return self._internal_unaligned
         return self.internal
 
+    def _pick_rows(self, batch: int, backward: bool):
+        """The kernels for few rows where ``batch`` is one, else None (under stream capture also while their code object
+        is not loaded)."""
+        if not 0 < batch <= self._few_rows_limits[backward]:
+            return None
+        if self._few_rows is None and not _capturing():
+            g = UVWSmallGenerator.create(self.config)
+            if g is None:                     # a problem whose units do not fit their registers or LDS
+                self._few_rows_limits = (0, 0)
+                return None
+            code = rt.variant_code(("uvw few rows", self.config.signature()), g.render)
+            fwd, bwd, _ = g.plan()
+            self._few_rows = rt.TPImpl(code, _make_steps(fwd, self._step_flags), _make_steps(bwd, self._step_flags))
+        return self._few_rows
+
     def forward_raw(self, batch, L1_in, L2_in, L3_out, weights, stream=None) -> None:
         """Device pointers as integers (reference: TensorProductBase.py:41-49)."""
-        impl = self._pick(L1_in, L2_in, L3_out, weights)
+        impl = self._pick_rows(int(batch), False) or self._pick(L1_in, L2_in, L3_out, weights)
         impl.exec_tensor_product(int(batch), L1_in, L2_in, L3_out, weights, self._workspace_ptr(stream),
                                  self._stream() if stream is None else stream)
 
     def backward_raw(self, batch_size, L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad,
                      stream=None) -> None:
         """reference: TensorProductBase.py:51-61."""
-        impl = self._pick(L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad)
+        impl = self._pick_rows(int(batch_size), True) or self._pick(L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad)
         impl.backward(int(batch_size), L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad,
                       self._workspace_ptr(stream), self._stream() if stream is None else stream)
 

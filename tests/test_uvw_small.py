@@ -1,0 +1,72 @@
+"""Dense uvw kernels for batches of few rows: emulated on the CPU and, on the GPU, against the oracle and the kernels for
+large batches at the edges of tiles, of a workgroup's share of the batch and of the dispatch."""
+import numpy as np
+import pytest
+
+import common
+from host_emu import emu
+from openequivariance_amd.codegen.uvw import UVWGenerator
+from openequivariance_amd.codegen.uvw_small import UVWSmallGenerator
+from oracle import tp as otp
+from oracle import weights as ow
+
+# one, two, three and five 16-channel subtiles, outputs of one to three w tiles, every degree up to 2
+MIXED = ("33x0e+7x1o+20x2e", "1x0e+1x1o+1x2e", "18x0e+35x1o+5x2e")
+BOTH = ("50x0e+50x1o+50x1e+50x2o+50x2e", "1x0e", "50x0e+50x1o+50x1e+50x2o+50x2e")
+
+
+def rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+# a sum of n products in any order errs by at most n units of the last place of the largest partial sum: 33 x 3 terms an
+# output element and 37 rows x 5 a weight, six operations each in front of them
+TOL = {np.float32: 200 * 6.0e-8, np.float64: 200 * 1.2e-16}
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, 21), (np.float64, 2)])
+def test_emulated(dtype, n, monkeypatch):
+    monkeypatch.setattr(UVWGenerator, "DW_WORKGROUPS", 7)
+    monkeypatch.setattr(UVWSmallGenerator, "DW_WAVES", 4)
+    prob, oprob = common.fully_connected(("18x0e+3x1o", "1x0e+1x1o", "17x0e+5x1o"), shared=True, dtype=dtype)
+    g = UVWSmallGenerator.create(prob)
+    assert len(g.bwd_groups) == 2 and max(g.chunks) > 1
+    X, Y, We, G = common.tp_inputs(prob, n, 9, dtype, w_scale=0.3)
+    W = ow.e3nn_to_oeq(oprob, We)
+    fwd, bwd, ws = g.plan()
+    assert ws() <= UVWGenerator(prob).plan()[2]()
+    out = emu.run_tp(g, fwd, X, Y, W, ws_bytes=ws())
+    assert rel(out["Z"], otp.forward(oprob, X, Y, We)) < TOL[dtype]
+    out = emu.run_tp(g, bwd, X, Y, W, G, ws_bytes=ws())
+    dX, dY, dW = otp.backward(oprob, X, Y, We, G)
+    assert rel(out["Xg"], dX) < TOL[dtype] and rel(out["Yg"], dY) < TOL[dtype]
+    assert rel(ow.oeq_to_e3nn(oprob, out["Wg"]), dW) < TOL[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("irreps", [MIXED, BOTH, common.DENSE], ids=["mixed", "both", "dense"])
+def test_on_the_gpu(cuda, irreps, dtype):
+    import torch
+    import openequivariance_amd as oeq
+    prob, oprob = common.fully_connected(irreps, shared=True, dtype=dtype)
+    tp = oeq.TensorProduct(prob, torch_op=True)
+    limits = tp._few_rows_limits
+    assert limits[1] == (65536 if irreps is BOTH else 5120)
+    for n in (1, 16, 37, 2049, 4097, 5120, 5121):
+        X, Y, We, G = common.tp_inputs(prob, n, n, dtype, w_scale=0.3)
+        x, y, w, g = (torch.tensor(a, device=cuda) for a in (X, Y, ow.e3nn_to_oeq(oprob, We), G))
+        assert [tp._pick_rows(n, back) is None for back in (False, True)] == [n > limit for limit in limits]
+        got = [tp.forward(x, y, w), *tp.backward_helper(x, y, w, g)]
+        if n <= 37:
+            ref = [otp.forward(oprob, X, Y, We), *otp.backward(oprob, X, Y, We, G)]
+            ref[3] = ow.e3nn_to_oeq(oprob, ref[3])
+            tol = TOL[dtype]
+        else:
+            # the kernels for large batches; a weight gradient is a sum over the batch in another order
+            tp._few_rows_limits = (0, 0)
+            ref = [t.cpu().numpy() for t in (tp.forward(x, y, w), *tp.backward_helper(x, y, w, g))]
+            tp._few_rows_limits, tol = limits, 4 * TOL[dtype]
+        for a, b in zip(got, ref):
+            assert rel(a.cpu().numpy(), b) < tol
+        assert all(torch.equal(a, b) for a, b in zip(got[1:], tp.backward_helper(x, y, w, g)))
