@@ -1,9 +1,10 @@
-"""In-tree build of the C-ABI runtime library ``liboeq_hip.so`` with hipcc.
+"""In-tree build of the C-ABI runtime library ``liboeq_hip.so`` with hipcc and of the torch operators' autograd kernels
+``liboeq_torch.so`` (host code only) with the C++ compiler.
 
 ``python -m openequivariance_amd.build_ext`` (or ``__graft_entry__.build()``)
-compiles ``csrc/oeq_hip.cpp`` for gfx950 and leaves the shared object next to
-the sources, where :mod:`openequivariance_amd.runtime` loads it from.  The
-library is never built implicitly at import time.
+compiles ``csrc/oeq_hip.cpp`` for gfx950 and ``csrc/oeq_torch.cpp`` against the installed torch and leaves the shared
+objects next to the sources, where :mod:`openequivariance_amd.runtime` and :mod:`openequivariance_amd.autograd_glue` load
+them from.  The libraries are never built implicitly at import time.
 """
 from __future__ import annotations
 
@@ -16,6 +17,7 @@ import sys
 PKG_DIR = pathlib.Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = CSRC / "liboeq_hip.so"
+TORCH_LIB_PATH = CSRC / "liboeq_torch.so"
 ROCM = pathlib.Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 
 # -packed-fp32-ops is switched off for every device compilation of this project
@@ -41,7 +43,25 @@ def build_native(verbose: bool = True) -> pathlib.Path:
         raise RuntimeError(f"hipcc failed:\n{res.stdout}\n{res.stderr}")
     if verbose and res.stderr.strip():
         print(res.stderr, file=sys.stderr)
+    build_torch_ops(verbose)
     return LIB_PATH
+
+
+def build_torch_ops(verbose: bool = True) -> pathlib.Path:
+    import torch
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no C++ compiler found (g++ or c++)")
+    root = pathlib.Path(torch.__file__).resolve().parent
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{root / 'include'}", f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+           str(CSRC / "oeq_torch.cpp"), "-o", str(TORCH_LIB_PATH), f"-L{root / 'lib'}", "-ltorch", "-ltorch_cpu", "-lc10"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cxx} failed:\n{res.stdout}\n{res.stderr}")
+    return TORCH_LIB_PATH
 
 
 if __name__ == "__main__":

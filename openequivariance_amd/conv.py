@@ -22,7 +22,7 @@ import torch
 
 from . import runtime as rt
 from . import tunables
-from .autograd_glue import double_backward_terms
+from .autograd_glue import define_derivatives, define_operator, double_backward_terms
 from .codegen.uvu_conv_double import conv_double_generator
 from .codegen.uvu_det import UVUDetGenerator
 from .codegen.uvu_direct import UVUDirectGenerator
@@ -344,7 +344,10 @@ class TensorProductConv:
     def _pick(self, *ptrs):
         """The forward kernels write Z with 16-byte vector stores; a misaligned tensor (rare: a view
         with an odd storage offset) gets a variant without them, compiled on first need."""
-        if any(int(p) % 16 for p in ptrs):
+        bits = 0
+        for p in ptrs:
+            bits |= int(p)
+        if bits % 16:
             if self._internal_unaligned is None:
                 g = select_conv_generator(self.config, self.deterministic, vector_stores=False, idx_dtype=self.idx_dtype)
                 self._internal_unaligned = self._build(g)
@@ -511,37 +514,21 @@ class TensorProductConv:
                         lambda name: bwd_run(x, y, w, g, rows, cols, tperm, E, N, name))
                 return bwd_run(x, y, w, g, rows, cols, tperm, E, N, self._bwd_choice[size_class])
 
-        # the two variants differ only in the trailing transpose_perm argument, which torch's operator
-        # schemas need spelled out
-        if not det:
-            @torch.library.custom_op(f"openequivariance_amd::conv_forward{cid}", mutates_args=(), device_types="cuda")
-            def forward(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, rows: torch.Tensor,
-                        cols: torch.Tensor) -> torch.Tensor:
-                return fwd_impl(L1_in, L2_in, weights, rows, cols, None)
+        # the two variants differ only in the trailing transpose_perm argument, which the operators' schemas spell out
+        operands = ("L1_in", "L2_in", "weights")
+        index = ("rows", "cols", "transpose_perm") if det else ("rows", "cols")
+        tperm_of = (lambda index: index) if det else (lambda index: (*index, None))
 
-            @torch.library.custom_op(f"openequivariance_amd::conv_backward{cid}", mutates_args=(), device_types="cuda")
-            def backward_helper(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, L3_grad: torch.Tensor,
-                                rows: torch.Tensor, cols: torch.Tensor) -> typing.List[torch.Tensor]:
-                return bwd_impl(L1_in, L2_in, weights, L3_grad, rows, cols, None)
-        else:
-            @torch.library.custom_op(f"openequivariance_amd::conv_forward{cid}", mutates_args=(), device_types="cuda")
-            def forward(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, rows: torch.Tensor,
-                        cols: torch.Tensor, transpose_perm: torch.Tensor) -> torch.Tensor:
-                return fwd_impl(L1_in, L2_in, weights, rows, cols, transpose_perm)
+        def like(*tensors):
+            return [t.new_empty(*t.shape) for t in tensors]
 
-            @torch.library.custom_op(f"openequivariance_amd::conv_backward{cid}", mutates_args=(), device_types="cuda")
-            def backward_helper(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, L3_grad: torch.Tensor,
-                                rows: torch.Tensor, cols: torch.Tensor,
-                                transpose_perm: torch.Tensor) -> typing.List[torch.Tensor]:
-                return bwd_impl(L1_in, L2_in, weights, L3_grad, rows, cols, transpose_perm)
-
-        @forward.register_fake
-        def _(L1_in, L2_in, weights, *index):
-            return L1_in.new_empty(L1_in.shape[0], L3_dim)
-
-        @backward_helper.register_fake
-        def _(L1_in, L2_in, weights, L3_grad, *index):
-            return [L1_in.new_empty(*L1_in.shape), L2_in.new_empty(*L2_in.shape), weights.new_empty(*weights.shape)]
+        forward = define_operator(
+            f"conv_forward{cid}", operands + index, "Tensor", lambda x, y, w, *index: fwd_impl(x, y, w, *tperm_of(index)),
+            lambda L1_in, L2_in, weights, *index: L1_in.new_empty(L1_in.shape[0], L3_dim))
+        backward_helper = define_operator(
+            f"conv_backward{cid}", (*operands, "L3_grad", *index), "Tensor[]",
+            lambda x, y, w, g, *index: bwd_impl(x, y, w, g, *tperm_of(index)),
+            lambda L1_in, L2_in, weights, L3_grad, *index: like(L1_in, L2_in, weights))
 
         def double_impl(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, rows, cols, tperm):
             x, y, w, g, a, b, v, rows, cols, tperm = _contiguous(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot,
@@ -557,42 +544,16 @@ class TensorProductConv:
                                              stream=self._stream(x.device.index))
             return out
 
-        if not det:
-            @torch.library.custom_op(f"openequivariance_amd::conv_double_backward{cid}", mutates_args=(), device_types="cuda")
-            def fused(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, L3_grad: torch.Tensor,
-                      L1_cot: torch.Tensor, L2_cot: torch.Tensor, weights_cot: torch.Tensor, rows: torch.Tensor,
-                      cols: torch.Tensor) -> typing.List[torch.Tensor]:
-                return double_impl(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, rows, cols, None)
-        else:
-            @torch.library.custom_op(f"openequivariance_amd::conv_double_backward{cid}", mutates_args=(), device_types="cuda")
-            def fused(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, L3_grad: torch.Tensor,
-                      L1_cot: torch.Tensor, L2_cot: torch.Tensor, weights_cot: torch.Tensor, rows: torch.Tensor,
-                      cols: torch.Tensor, transpose_perm: torch.Tensor) -> typing.List[torch.Tensor]:
-                return double_impl(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, rows, cols, transpose_perm)
+        fused = define_operator(
+            f"conv_double_backward{cid}", (*operands, "L3_grad", "L1_cot", "L2_cot", "weights_cot", *index), "Tensor[]",
+            lambda x, y, w, g, a, b, v, *index: double_impl(x, y, w, g, a, b, v, *tperm_of(index)),
+            lambda L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, *index: like(L1_in, L2_in, weights, L3_grad))
 
-        @fused.register_fake
-        def _(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, *index):
-            return [t.new_empty(*t.shape) for t in (L1_in, L2_in, weights, L3_grad)]
+        def double_backward(x, y, w, g, a, b, v, *index):
+            return list(double_backward_terms(forward, backward_helper, x, y, w, g, a, b, v, index,
+                                              fused=fused if self._double_usable() else None))
 
-        def setup_context(ctx, inputs, output):
-            ctx.L1_in, ctx.L2_in, ctx.weights, *ctx.index = inputs
-
-        def backward(ctx, grad_output):
-            r = backward_helper(ctx.L1_in, ctx.L2_in, ctx.weights, grad_output, *ctx.index)
-            return (r[0], r[1], r[2]) + (None,) * len(ctx.index)
-
-        forward.register_autograd(backward, setup_context=setup_context)
-
-        def setup_context_double_backward(ctx, inputs, output):
-            ctx.L1_in, ctx.L2_in, ctx.weights, ctx.L3_grad, *ctx.index = inputs
-
-        def double_backward(ctx, grad_output):
-            terms = double_backward_terms(forward, backward_helper, ctx.L1_in, ctx.L2_in, ctx.weights, ctx.L3_grad,
-                                          grad_output[0], grad_output[1], grad_output[2], tuple(ctx.index),
-                                          fused=fused if self._double_usable() else None)
-            return terms + (None,) * len(ctx.index)
-
-        backward_helper.register_autograd(double_backward, setup_context=setup_context_double_backward)
+        define_derivatives(f"conv_forward{cid}", f"conv_backward{cid}", operands + index, double_backward)
         self.forward = forward
         self.backward_helper = backward_helper
 

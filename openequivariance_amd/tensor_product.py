@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from . import runtime as rt
-from .autograd_glue import double_backward_terms
+from .autograd_glue import define_derivatives, define_operator, double_backward_terms
 from .codegen.uvu import UVUGenerator
 from .codegen.uvu_direct import UVUDirectGenerator
 from .codegen.uvu_double import UVUDoubleGenerator
@@ -172,8 +172,10 @@ class TensorProduct(TensorProductBase):
         return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device_index is None else device_index)
 
     def _pick(self, *ptrs):
-        aligned = all(int(p) % 16 == 0 for p in ptrs)
-        if not aligned and isinstance(self.generator, UVUDirectGenerator):
+        bits = 0
+        for p in ptrs:
+            bits |= int(p)
+        if bits % 16 and isinstance(self.generator, UVUDirectGenerator):
             # rare: a caller-supplied tensor that is not 16-byte aligned -> kernels without vector stores
             if self._internal_unaligned is None:
                 g = type(self.generator)(self.config, vector_stores=False)
@@ -181,7 +183,7 @@ class TensorProduct(TensorProductBase):
                 self._internal_unaligned = rt.TPImpl(rt.compile_source(g.render()), _make_steps(fwd, self._step_flags),
                                                      _make_steps(bwd, self._step_flags))
             return self._internal_unaligned
-        if isinstance(self.generator, UVWBatchedGenerator) and self.generator.pairs and any(int(p) % 8 for p in ptrs):
+        if isinstance(self.generator, UVWBatchedGenerator) and self.generator.pairs and bits % 8:
             # the same for the per-row-weights uvw kernels, which move fp32 weights two words at a time
             if self._internal_unaligned is None:
                 g = UVWBatchedGenerator(self.config, pairs=False)
@@ -265,10 +267,11 @@ class TensorProduct(TensorProductBase):
     def _setup_torch_custom_op(self) -> None:
         """reference: TensorProductBase.py:234-298 (forward, backward, double backward)."""
         L3_dim = self.L3.dim
-        shared = self.config.shared_weights
 
-        @torch.library.custom_op(f"openequivariance_amd::tp_forward{self.tp_id}", mutates_args=(), device_types="cuda")
-        def forward(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor) -> torch.Tensor:
+        operands = ("L1_in", "L2_in", "weights")
+        tp_id = self.tp_id
+
+        def forward_impl(L1_in, L2_in, weights):
             x, y, w = _contiguous(L1_in, L2_in, weights)
             self._check_inputs(x, y, w)
             out = torch.empty((x.shape[0], L3_dim), dtype=x.dtype, device=x.device)
@@ -277,15 +280,12 @@ class TensorProduct(TensorProductBase):
                                  self._stream(x.device.index))
             return out
 
-        @forward.register_fake
-        def _(L1_in, L2_in, weights):
+        def forward_fake(L1_in, L2_in, weights):
             return L1_in.new_empty(L1_in.shape[0], L3_dim)
 
-        self.forward = forward
+        forward = self.forward = define_operator(f"tp_forward{tp_id}", operands, "Tensor", forward_impl, forward_fake)
 
-        @torch.library.custom_op(f"openequivariance_amd::tp_grad_helper{self.tp_id}", mutates_args=(), device_types="cuda")
-        def backward_helper(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor,
-                            L3_grad: torch.Tensor) -> typing.List[torch.Tensor]:
+        def backward_impl(L1_in, L2_in, weights, L3_grad):
             x, y, w, g = _contiguous(L1_in, L2_in, weights, L3_grad)
             self._check_inputs(x, y, w, g)
             xg, yg, wg = torch.empty_like(x), torch.empty_like(y), torch.empty_like(w)
@@ -294,30 +294,16 @@ class TensorProduct(TensorProductBase):
                                   w.data_ptr(), wg.data_ptr(), g.data_ptr(), self._stream(x.device.index))
             return [xg, yg, wg]
 
-        @backward_helper.register_fake
-        def _(L1_in, L2_in, weights, L3_grad):
-            return [L1_in.new_empty(*L1_in.shape), L2_in.new_empty(*L2_in.shape), weights.new_empty(*weights.shape)]
+        def like(*tensors):
+            return [t.new_empty(*t.shape) for t in tensors]
 
-        self.backward_helper = backward_helper
-
-        def setup_context(ctx, inputs, output):
-            ctx.L1_in, ctx.L2_in, ctx.weights = inputs
-
-        def backward(ctx, grad_output):
-            r = backward_helper(ctx.L1_in, ctx.L2_in, ctx.weights, grad_output)
-            return r[0], r[1], r[2]
-
-        forward.register_autograd(backward, setup_context=setup_context)
-
-        def setup_context_double_backward(ctx, inputs, output):
-            ctx.L1_in, ctx.L2_in, ctx.weights, ctx.L3_grad = inputs
+        backward_helper = self.backward_helper = define_operator(
+            f"tp_grad_helper{tp_id}", (*operands, "L3_grad"), "Tensor[]", backward_impl,
+            lambda L1_in, L2_in, weights, L3_grad: like(L1_in, L2_in, weights))
 
         fused = None
         if self._double_generator is not None:
-            @torch.library.custom_op(f"openequivariance_amd::tp_double_backward{self.tp_id}", mutates_args=(),
-                                     device_types="cuda")
-            def fused(L1_in: torch.Tensor, L2_in: torch.Tensor, weights: torch.Tensor, L3_grad: torch.Tensor,
-                      L1_cot: torch.Tensor, L2_cot: torch.Tensor, weights_cot: torch.Tensor) -> typing.List[torch.Tensor]:
+            def double_impl(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot):
                 x, y, w, g, a, b, v = _contiguous(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot)
                 self._check_inputs(x, y, w, g)
                 self._check_inputs(a, b, v)
@@ -329,17 +315,16 @@ class TensorProduct(TensorProductBase):
                                              stream=self._stream(x.device.index))
                 return out
 
-            @fused.register_fake
-            def _(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot):
-                return [t.new_empty(*t.shape) for t in (L1_in, L2_in, weights, L3_grad)]
+            fused = define_operator(
+                f"tp_double_backward{tp_id}", (*operands, "L3_grad", "L1_cot", "L2_cot", "weights_cot"), "Tensor[]", double_impl,
+                lambda L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot: like(L1_in, L2_in, weights, L3_grad))
 
-        def double_backward(ctx, grad_output):
-            return double_backward_terms(forward, backward_helper, ctx.L1_in, ctx.L2_in, ctx.weights, ctx.L3_grad,
-                                         grad_output[0], grad_output[1], grad_output[2],
-                                         # (its code object is loaded on first use, which a stream capture must not do)
-                                         fused=fused if self._double or not _capturing() else None)
+        def double_backward(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot):
+            return list(double_backward_terms(forward, backward_helper, L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot,
+                                              # (its code object is loaded on first use, which a stream capture must not do)
+                                              fused=fused if self._double or not _capturing() else None))
 
-        backward_helper.register_autograd(double_backward, setup_context=setup_context_double_backward)
+        define_derivatives(f"tp_forward{tp_id}", f"tp_grad_helper{tp_id}", operands, double_backward)
 
     def _check_inputs(self, x, y, w, g=None) -> None:
         """Shapes, dtypes and devices, before anything is launched (the kernels dereference every
