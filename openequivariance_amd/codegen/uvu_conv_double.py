@@ -49,6 +49,7 @@ class UVUDetDoubleGenerator(_DoublePlan, DoubleArithmetic, UVUDetGenerator):
     # Receiver pass staged through LDS where the multiplicity fits one chunk (32 channels, 11 paths: 109 registers, 96
     # staged; several chunks, 100 / 128 channels: 415 / 420, 441 / 447)
     FWD_STAGE_WAVES = 8
+    F64_STAGE_WORDS = 0
     FWD_STAGE_OPERANDS = 1 << 30
     # ... and one launch up to 48 words of sums in fp64 (38 words: 197, in two 224; 42 words: 566 and 566; 102 words in
     # groups of 32 / 48 / 64: 900 / 879 / 843)

@@ -37,6 +37,7 @@ from .uvu_direct import UVUDirectGenerator
 class UVUDetGenerator(UVUDirectGenerator):
     _allow_det = True
     SPLIT_WORDS = 80
+    F64_STAGE_WORDS = 45          # operand words per edge from which an fp64 backward is staged through LDS (0: never)
     # words per group when the backward is split (fp64, 5000 nodes / 150 000 edges, 64 -> 24 words per group: 17 paths
     # at 128 channels 3.12 -> 2.52 ms, 68 paths 9.38 -> 7.56 ms, 30 paths 2.11 -> 1.98 and 1.27 -> 1.33 ms)
     SPLIT_TARGET = {"float": 64, "double": 24}
@@ -136,18 +137,28 @@ class UVUDetGenerator(UVUDirectGenerator):
         # backward operands of the next edge travel global -> LDS without passing through registers
         # (LDS-DMA), which leaves room for a third wavefront per SIMD; see emit_staged_loop
         def stage_words_of(outs):
-            return WAVE * (sum(self.dma_stride(w) for i in outs for _, w in self.dma_pieces(self.out[i].D))
-                           + len(self.EDGE_W) * sum(p.mv for p in self.paths if p.o.idx in outs) + len(self.EDGE_Y))
+            return WAVE * (sum(self.dma_stride(w) for i in outs for _, w in self.record_transfers(self.out[i].D))
+                           + len(self.EDGE_W) * self.itemsize // 4 * sum(p.mv for p in self.paths if p.o.idx in outs) + len(self.EDGE_Y))
         self.stage_words = max(stage_words_of(g_) for g_ in self.out_groups)      # of the largest group
         lds = tunables.current.det_lds if lds is None else lds
         stage_waves = (160 * 1024) // (4 * self.stage_words * 4)        # wavefronts per SIMD the stage leaves room for
         # one chunk per node: also at two wavefronts per SIMD (the register pipeline then has one); chunked
         # problems only when three fit (config 5, two: 1 % slower than the register pipeline)
         small = self.NCH == 1 and H == 1
-        fits = self.T == "float" and self.P >= self.D2 and (stage_waves >= 3 or (small and stage_waves >= 2))
-        self.lds_backward = fits and lds is not False
-        if self.lds_backward:
-            self.waves_per_eu = min(3, stage_waves)
+        if self.T == "float":
+            fits = self.P >= self.D2 and (stage_waves >= 3 or (small and stage_waves >= 2))
+        else:
+            # fp64, values as pairs of 4-byte words: where a launch with register loads takes more than 256 registers, one
+            # wavefront per SIMD.  Backward, register loads against staged (1000 - 3000 nodes, 30 000 - 60 000 edges): 55
+            # words 32 channels 104 / 89 us, 64 channels 289 / 257, 128 channels 371 / 346; six groups of 24 words 335 / 271.
+            # Below, the loads' own registers are free: 25 words 142 / 158 us, 36 words 186 / 203
+            fits = (self.P >= 2 * self.D2 and stage_waves >= 1 and bool(self.F64_STAGE_WORDS)
+                    and (words >= self.F64_STAGE_WORDS or H > 1))
+        self.lds_backward = fits and self.T == "float" and lds is not False
+        self.staged_f64 = fits and self.T == "double" and lds is not False
+        self.staged_backward = self.lds_backward or self.staged_f64
+        if self.staged_backward:
+            self.waves_per_eu = min(3 if self.T == "float" else 2, stage_waves)
         elif self.prefetch_backward:
             # two register sets: hold the allocation to what two wavefronts per SIMD leave each (256 registers)
             self.waves_per_eu = 2
@@ -160,6 +171,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         # fly - the unsorted MACE forward went 0.741 -> 0.775 ms)
         fwd_operands = (len(self.NODE_X) * sum(self.in1[i].D for i in self.used_in1)
                         + len(self.EDGE_W) * sum(p.mv for p in self.paths))
+        # (fp64 keeps the register pipeline: 100 channels 57 against 76 us, 64 channels of either parity 83 against 106)
         self.lds_forward = (self.T == "float" and self.P >= self.D2 and lds is not False
                             and (self.NCH == 1 or (fwd_operands >= self.FWD_STAGE_OPERANDS and not forward_perm) or lds is True)
                             and self.FWD_STAGE_WAVES * (fwd_words + self.lds_elems) * 4 <= 160 * 1024)
@@ -183,7 +195,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         # the regrouped backward arithmetic (see UVUGenerator.regroup_pairs) where registers are to spare: measured
         # on one GPU in one process, 32 channels (LDS-staged loop) 0.165 against 0.170 ms with it, 256 channels
         # (two register sets, 256 registers) 7.78 against 7.61 ms
-        self.regroup_pairs = self.lds_backward
+        self.regroup_pairs = self.staged_backward
         # A node whose edge list is longer than LONG times the mean (at least PIECE_MIN_EDGES) is not walked
         # by its own wavefront: the edge list is cut at multiples of that length, and every piece of a long
         # node is walked by one of the wavefronts launched behind the nodes (two per tile of the list: the
@@ -937,7 +949,7 @@ class UVUDetGenerator(UVUDirectGenerator):
                     E(f"const T g{k} = G{oi}_{k};")
 
                 def sink(E, p, v, expr):
-                    if self.lds_backward:          # stored at the top of the next iteration (flush)
+                    if self.staged_backward:       # stored at the top of the next iteration (flush)
                         E(f"  pw_{p.t}_{v} = {expr};")
                     else:
                         E(f"  if ({self.act(p.a)}) {self.st('Wgr', self.widx(p, 'u', v), expr)}")
@@ -945,7 +957,7 @@ class UVUDetGenerator(UVUDirectGenerator):
                 E.level -= 1
                 E("}")
             self.emit_dy_sum(E)
-            if self.lds_backward:
+            if self.staged_backward:
                 E(" ".join(f"pdy{f} = dy{f};" for f in self.used_y) + " pe = e; pv = rv;")
                 return
             writer = "ul == 0" if self.P < 64 else "lane == 63"
@@ -957,7 +969,7 @@ class UVUDetGenerator(UVUDirectGenerator):
             for f in range(self.D2):
                 E(f"    Ygr[{f}] = " + (f"dy{f};" if f in self.used_y else "(T)0;"))
             E("}")
-        if self.lds_backward:
+        if self.staged_backward:
             self._emit_staged_backward(E, compute, grp)
         else:
             self.emit_pingpong_loop(E, names, load_idx, load, compute, prefetch_first=self.prefetch_backward)
@@ -971,47 +983,80 @@ class UVUDetGenerator(UVUDirectGenerator):
         slabs, off = [], 0
         for src, _ in self.NODE_X:
             for i in self.used_in1:
-                for k0, w in self.dma_pieces(self.in1[i].D):
+                for k0, w in self.record_transfers(self.in1[i].D):
                     slabs.append((src, i, k0, w, off))
                     off += WAVE * self.dma_stride(w)
         off = self._edge_slabs(slabs, off)
         return slabs, off + WAVE * len(self.EDGE_Y)
 
     def _edge_slabs(self, slabs, off: int) -> int:
-        """One slab per weight of an edge, behind ``off``; the second-operand slabs follow at the returned offset."""
+        """One slab per weight of an edge (two in fp64), behind ``off``; the second-operand slabs follow at the returned
+        offset."""
         for src, _ in self.EDGE_W:
             for p in self.paths:
                 for v in range(p.mv):
-                    slabs.append((src, (p, v), 0, 1, off))
-                    off += WAVE
+                    for k0, w in self.record_transfers(1):
+                        slabs.append((src, (p, v), k0, w, off))
+                        off += WAVE
         return off
+
+    # The stage is an array of 4-byte words in both types.
+    def record_transfers(self, D: int):
+        """Transfers of a record of D values; in fp64 two values at a time, an odd one as its two halves."""
+        if self.itemsize == 4:
+            return self.dma_pieces(D)
+        return [(4 * q, 4) for q in range(D // 2)] + [(2 * D - 2, 1), (2 * D - 1, 1)] * (D % 2)
+
+    def stage_type(self) -> str:
+        return "T" if self.itemsize == 4 else "float"
+
+    def words_at(self, address: str) -> str:
+        return address if self.itemsize == 4 else f"(const float*)({address})"
+
+    def staged_record(self, slabs, kind, key):
+        """The values of this lane's record from its slabs."""
+        at = {}
+        for kind_, key_, k0, w, so in slabs:
+            if kind_ == kind and key_ == key:
+                for r in range(w):
+                    at[k0 + r] = (so, w, f"{so} + lane" + (f" * {self.dma_stride(w)} + {r}" if w > 1 else ""))
+        if self.itemsize == 4:
+            return [f"stage[{at[m][2]}]" for m in sorted(at)]
+        return [f"oeq_lds_f64(stage + {at[m][2]})" if at[m][1] == 4 else f"oeq_f64_words(stage[{at[m][2]}], stage[{at[m + 1][2]}])"
+                for m in sorted(at) if m % 2 == 0]
+
+    def emit_y_dma(self, E: Emitter, src: str, at: int, nt: int) -> None:
+        """One lane a word of the second operand; a row's group of lanes has at least as many as it has words."""
+        E(f"OEQ_DMA(4, {nt}, {self.words_at(f'{src} + e * {self.D2}')} + min(ul, {self.D2 * self.itemsize // 4 - 1}), stage + {at});")
+
+    def staged_y(self, f: int, at: int) -> str:
+        return f"stage[{at} + sub * {self.P} + {f}]" if self.itemsize == 4 else f"oeq_lds_f64(stage + {at} + sub * {self.P} + {2 * f})"
 
     def _edge_dma(self, E: Emitter, slabs, y_off: int, nt: int) -> None:
         for src, _ in self.EDGE_W:
             E(f"const T* __restrict__ {src}r = {src} + e * {self.WN};")
         for q, (src, _) in enumerate(self.EDGE_Y):
-            E(f"OEQ_DMA(4, {nt}, {src} + e * {self.D2} + min(ul, {self.D2 - 1}), stage + {y_off + q * WAVE});")
+            self.emit_y_dma(E, src, y_off + q * WAVE, nt)
         for src, _ in self.EDGE_W:
             for kind, key, k0, w, so in slabs:
                 if kind == src:
                     p, v = key
-                    E(f"OEQ_DMA(4, {nt}, {src}r + {self.widx(p, self.uclamp(p.a, 0), v)}, stage + {so});")
+                    E(f"OEQ_DMA(4, {nt}, {self.words_at(f'{src}r + {self.widx(p, self.uclamp(p.a, 0), v)}')} + {k0}, stage + {so});")
 
     def _edge_readback(self, E: Emitter, slabs, y_off: int) -> None:
         for q, (_, y) in enumerate(self.EDGE_Y):
             for f in self.used_y:
-                E(f"const T {y}{f} = stage[{y_off + q * WAVE} + sub * {self.P} + {f}];")
+                E(f"const T {y}{f} = {self.staged_y(f, y_off + q * WAVE)};")
         for src, name in self.EDGE_W:
-            for kind, key, k0, w, so in slabs:
-                if kind == src:
-                    p, v = key
-                    E(f"const T {name}{p.t}_{v} = stage[{so} + lane];")
+            for p in self.paths:
+                for v in range(p.mv):
+                    E(f"const T {name}{p.t}_{v} = {self.staged_record(slabs, src, (p, v))[0]};")
 
     def _emit_staged_forward(self, E: Emitter, compute) -> None:
         nt = 2 if self.nontemporal else 0
         slabs, words = self._forward_slabs()
         y_off = words - WAVE * len(self.EDGE_Y)
-        E(f"__shared__ __attribute__((aligned(16))) T stage[{words}];")
+        E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{words}];")
 
         def dma(E, e, n):
             E("{")
@@ -1021,7 +1066,7 @@ class UVUDetGenerator(UVUDirectGenerator):
             for kind, key, k0, w, so in slabs:
                 if kind in dict(self.NODE_X):
                     a = self.in1[key]
-                    E(f"OEQ_DMA({4 * w}, 0, {kind} + sndc * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D} + {k0}, stage + {so});")
+                    E(f"OEQ_DMA({4 * w}, 0, {self.words_at(f'{kind} + sndc * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D}')} + {k0}, stage + {so});")
             E.level -= 1
             E("}")
 
@@ -1034,8 +1079,7 @@ class UVUDetGenerator(UVUDirectGenerator):
                 # (read unconditionally, then masked: a conditional expression would put a branch around every LDS read)
                 E(f"const bool a{i}_ = {self.act(a)};")
                 for src, x in self.NODE_X:
-                    parts = [f"stage[{so} + lane * {self.dma_stride(w)} + {r}]" for kind, key, k0, w, so in slabs
-                             if kind == src and key == i for r in range(w)]
+                    parts = self.staged_record(slabs, src, i)
                     E("const T " + ", ".join(f"{x}r{i}_{m} = {parts[m]}" for m in range(a.D)) + ";")
                     E("const T " + ", ".join(f"{x}{i}_{m} = a{i}_ ? {x}r{i}_{m} : (T)0" for m in range(a.D)) + ";")
         self.emit_staged_loop(E, self.edge_pos, "eperm" if self.forward_perm else None, "cols", dma, readback, compute)
@@ -1046,13 +1090,13 @@ class UVUDetGenerator(UVUDirectGenerator):
         nt = 2 if self.nontemporal else 0          # cache policy bit "nt" for the streamed operands
         slabs, off = [], 0                         # (kind, key, first word, words, slab offset)
         for oi in self.used_out:
-            for k0, w in self.dma_pieces(self.out[oi].D):
+            for k0, w in self.record_transfers(self.out[oi].D):
                 slabs.append(("G", oi, k0, w, off))
                 off += WAVE * self.dma_stride(w)
         y_off = self._edge_slabs(slabs, off)
         off = y_off + WAVE * len(self.EDGE_Y)
         assert off <= self.stage_words
-        E(f"__shared__ __attribute__((aligned(16))) T stage[{off}];")
+        E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{off}];")
 
         def dma(E, e, n):
             E("{")
@@ -1062,7 +1106,7 @@ class UVUDetGenerator(UVUDirectGenerator):
             for kind, key, k0, w, so in slabs:
                 if kind == "G":
                     o = self.out[key]
-                    E(f"OEQ_DMA({4 * w}, 0, G + rcvc * {self.D3} + {o.off} + {self.uclamp(o, 0)} * {o.D} + {k0}, stage + {so});")
+                    E(f"OEQ_DMA({4 * w}, 0, {self.words_at(f'G + rcvc * {self.D3} + {o.off} + {self.uclamp(o, 0)} * {o.D}')} + {k0}, stage + {so});")
             E.level -= 1
             E("}")
 
@@ -1071,10 +1115,7 @@ class UVUDetGenerator(UVUDirectGenerator):
             self._edge_readback(E, slabs, y_off)
             for oi in self.used_out:
                 o = self.out[oi]
-                parts = []
-                for kind, key, k0, w, so in slabs:
-                    if kind == "G" and key == oi:
-                        parts += [f"stage[{so} + lane * {self.dma_stride(w)} + {r}]" for r in range(w)]
+                parts = self.staged_record(slabs, "G", oi)
                 # every gradient of an edge is proportional to dZ: zero it for idle lanes
                 # (read unconditionally, then masked: a conditional expression would put a branch around every LDS read)
                 E(f"const bool a{oi}_ = {self.act(o)};")

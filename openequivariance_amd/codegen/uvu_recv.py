@@ -86,9 +86,6 @@ class UVURecvGenerator(UVUDetGenerator):
         # wavefronts per SIMD).
         self.can_stage = self.T == "float" and self.P >= self.D2      # (the Y slab holds one word per lane of a row's group)
         self.staged_edges = self.can_stage and (True if staged is None else bool(staged))
-        self.regroup_pairs = bool(self.REGROUP_STAGED and self.staged_edges)
-        if self.staged_edges:
-            self.waves_hint = 0
         # Pass 1 in several launches when the dZ row of a receiver is too long to hold beside an edge's operands
         # (312 words per lane with 68 paths: 512 registers and scratch): the output blocks are grouped so that no
         # in1 block is read by paths of two groups, hence every launch writes words of the per-edge dX rows that
@@ -103,11 +100,18 @@ class UVURecvGenerator(UVUDetGenerator):
             if recv_split is None else recv_split
         self.recv_groups = self._disjoint_groups(limit)
         self.HR = len(self.recv_groups)
-        # pass 1 with register loads is worth choosing (fp64 only): every launch holds few
-        # enough dZ words to leave room for an edge's operands and results
+        # receiver order is worth choosing in fp64: every launch of pass 1 holds few enough dZ words to leave room for an
+        # edge's operands and results
         self.register_loads_fit = (self.T == "double" and not self.staged_edges and
                                    max(sum(self.out[i].D for i in g_) for g_ in self.recv_groups)
                                    <= self.RECV_SPLIT_WORDS_REGISTER_LOADS["double"])
+        # Such launches go through the stage as well, an edge's operands as 4-byte words: 334 registers and one wavefront per
+        # SIMD become 210 and two (17 paths at 128 channels, 10 000 nodes / 300 000 edges: forward + backward 6.56 -> 5.73 ms)
+        self.staged_f64 = (self.register_loads_fit and self.P >= 2 * self.D2 and (True if staged is None else bool(staged)))
+        self.uses_stage = self.staged_edges or self.staged_f64
+        self.regroup_pairs = bool(self.REGROUP_STAGED and self.uses_stage)
+        if self.uses_stage:
+            self.waves_hint = 0
         self.dy_slots = self.NCH * self.HR
         if not backward_perm:
             self.dypart_off = "(2 * (node_count + 1) + node_count) * sizeof(i64)"
@@ -190,7 +194,7 @@ class UVURecvGenerator(UVUDetGenerator):
         R, P, NCH = self.R, self.P, self.NCH
         self.emit_lane_direct(E, lds=False)
         with self._group(h, self.recv_groups):
-            return self._edges_body_staged(E, h) if self.staged_edges else self._edges_body_registers(E, h)
+            return self._edges_body_staged(E, h) if self.uses_stage else self._edges_body_registers(E, h)
 
     def _edges_body_registers(self, E: Emitter, grp: int = 0) -> str:
         R, P, NCH = self.R, self.P, self.NCH
@@ -384,7 +388,7 @@ class UVURecvGenerator(UVUDetGenerator):
         E("i64 cur_rcv = -1, rawR = -1, rcv0 = -1;")
         slabs, words = self._forward_slabs()
         y_off = words - 64
-        E(f"__shared__ __attribute__((aligned(16))) T stage[{words}];")
+        E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{words}];")
         res = [f"pw_{p.t}_{v}" for p in self.paths for v in range(p.mv)] + [f"pdy{f}" for f in self.used_y] \
             + [f"pdx{i}_{m}" for i in self.used_in1 for m in range(self.in1[i].D)]
         E("T " + ", ".join(f"{n} = (T)0" for n in res) + "; u64 pe = 0; bool pv = false, pev = false;")
@@ -395,15 +399,15 @@ class UVURecvGenerator(UVUDetGenerator):
             E(f"const u64 e = {e}, sndc = {n};")
             E("rawR = rows[e];")
             E(f"const T* __restrict__ Wr = W + e * {self.WN};")
-            E(f"OEQ_DMA(4, {nt}, Y + e * {self.D2} + min(ul, {self.D2 - 1}), stage + {y_off});")
+            self.emit_y_dma(E, "Y", y_off, nt)
             for kind, key, k0, w, so in slabs:
                 if kind == "W":
                     p, v = key
-                    E(f"OEQ_DMA(4, {nt}, Wr + {self.widx(p, self.uclamp(p.a, 0), v)}, stage + {so});")
+                    E(f"OEQ_DMA(4, {nt}, {self.words_at(f'Wr + {self.widx(p, self.uclamp(p.a, 0), v)}')} + {k0}, stage + {so});")
             for kind, key, k0, w, so in slabs:
                 if kind == "X":
                     a = self.in1[key]
-                    E(f"OEQ_DMA({4 * w}, 0, X + sndc * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D} + {k0}, stage + {so});")
+                    E(f"OEQ_DMA({4 * w}, 0, {self.words_at(f'X + sndc * {self.D1} + {a.off} + {self.uclamp(a, 0)} * {a.D}')} + {k0}, stage + {so});")
             E.level -= 1
             E("}")
 
@@ -414,17 +418,13 @@ class UVURecvGenerator(UVUDetGenerator):
             E(f"const bool cur_ev = {self.edge_pos('it')} < len;")
             E("rv = cur_rv && rcv0 >= 0 && rcv0 < (i64)node_count;")
             for f in self.used_y:
-                E(f"const T y{f} = stage[{y_off} + sub * {P} + {f}];")
-            for kind, key, k0, w, so in slabs:
-                if kind == "W":
-                    p, v = key
-                    E(f"const T We_{p.t}_{v} = stage[{so} + lane];")
+                E(f"const T y{f} = {self.staged_y(f, y_off)};")
+            for p in self.paths:
+                for v in range(p.mv):
+                    E(f"const T We_{p.t}_{v} = {self.staged_record(slabs, 'W', (p, v))[0]};")
             for i in self.used_in1:
                 a = self.in1[i]
-                parts = []
-                for kind, key, k0, w, so in slabs:
-                    if kind == "X" and key == i:
-                        parts += [f"stage[{so} + lane * {self.dma_stride(w)} + {r}]" for r in range(w)]
+                parts = self.staged_record(slabs, "X", i)
                 # dW and dY of an edge are proportional to x: zero it for idle lanes and invalid edges
                 E(f"const bool a{i}_ = {self.act(a)};")
                 E("const T " + ", ".join(f"xr{i}_{m} = {parts[m]}" for m in range(a.D)) + ";")

@@ -75,6 +75,8 @@ static inline i64 oeq_lds_claim(i64* slot, i64 key) { std::lock_guard<std::mutex
 static inline void oeq_st_agent(T* p, T v) { *p = v; }
 static inline T oeq_ld_agent(const T* p) { return *p; }
 static inline int oeq_lds_add(int* p, int v) { std::lock_guard<std::mutex> g(g_atomic_mutex); const int o = *p; *p += v; return o; }
+static inline T oeq_lds_f64(const float* p) { T v; memcpy(&v, p, sizeof(T)); return v; }
+static inline T oeq_f64_words(float lo, float hi) { float w[2] = {lo, hi}; T v; memcpy(&v, w, sizeof(T)); return v; }
 static inline void oeq_wait_vm() {}
 static inline void oeq_wait_lds() {}
 static inline T oeq_wave_sum63(T v) { g_xT[threadIdx.x] = v; oeq_sync(); T t = 0; for (int i = 0; i < 64; ++i) t += g_xT[(threadIdx.x & ~63) + i]; oeq_sync(); return t; }
