@@ -95,7 +95,7 @@ class UVWGenerator:
     # w tiles.  (48 instead of 80, for a third wavefront per SIMD, measured slower on 64x0e+64x1o+64x2e: fp32
     # 0.329 -> 0.376 ms, fp64 0.566 -> 0.694 ms - the CG part of a tile is then computed once per range.)
     FWD_ACC_LIMIT = 80
-    FWD_PIPELINE = {4: (4, 1), 8: (1, 3)}
+    FWD_PIPELINE = {4: (4, 2), 8: (1, 3)}
     BWD_LDS_LIMIT = 80 * 1024    # dZ tile of the backward: two workgroups per compute unit (gfx950: 160 KB)
 
     def __init__(self, problem: TPProblem):
@@ -106,10 +106,12 @@ class UVWGenerator:
         self.shared = bool(problem.shared_weights)
         if not self.shared and not getattr(self, "_allow_batched", False):
             raise NotImplementedError("this generator handles shared weights; see uvw_batched.py for per-row weights")
-        # forward K loop: steps fetched per batch of loads, and unroll factor of the batch loop (measured on
-        # MI355X: fp32 4 / 1, fp64 1 / 3; a loop written out on alternating register sets, so that nothing is
+        # forward K loop: steps fetched per batch of loads, and unroll factor of the batch loop.  Measured on MI355X, 100 000
+        # rows, fp32 4 / 1 against 4 / 2: 64 channels 304 / 297 us, 20 channels 102 / 95, 100 -> 30 channels 142 / 142; with
+        # one path per block (50 channels) 259 / 265, hence the exception below.  fp64 1 / 3 against 2 / 2 and 1 / 4: 540 /
+        # 623 / 641.  (A loop written out on alternating register sets, so that nothing is
         # copied between sets, has 0.9 instead of 2.1 vector-ALU instructions per MFMA and measured 0.341
-        # against 0.331 ms; larger groups for the cheap work items 0.361 - 0.422 against 0.359 ms)
+        # against 0.331 ms; larger groups for the cheap work items 0.361 - 0.422 against 0.359 ms.)
         self.fwd_group, self.fwd_unroll = self.FWD_PIPELINE[self.itemsize]
         # Tile shape: 16 x 16 x 4 in both types.  The fp32 forward on v_mfma_f32_32x32x2_f32 (32 batch rows per
         # tile, half the weight-operand loads per FLOP) passed the same parity tests and measured 0.371 ms (w
@@ -147,6 +149,8 @@ class UVWGenerator:
             woff += a.mul * b.mul * o.mul
         if not self.paths:
             raise ValueError("Tensor product problem has no valid instructions!")
+        if self.itemsize == 4 and max(len(self.paths_into(p.o.idx)) for p in self.paths) == 1:
+            self.fwd_unroll = 1
         self.used_in1 = sorted({p.a.idx for p in self.paths})
         self.used_out = sorted({p.o.idx for p in self.paths})
         self.used_y = sorted({p.b.off + j for p in self.paths for (_, j) in p.pairs})
