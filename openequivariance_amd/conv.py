@@ -23,7 +23,7 @@ import torch
 from . import runtime as rt
 from . import tunables
 from .autograd_glue import define_derivatives, define_operator, double_backward_terms
-from .codegen.uvu_conv_double import conv_double_generator
+from .codegen.uvu_conv_double import UVUDetDoubleGenerator, conv_double_generator
 from .codegen.uvu_det import UVUDetGenerator
 from .codegen.uvu_direct import UVUDirectGenerator
 from .codegen.uvu_recv import UVURecvGenerator
@@ -253,11 +253,15 @@ class TensorProductConv:
         """Kernel set of the fused double backward; its steps share the operator's workspace."""
         if self._double is None:
             idx = "i64" if self.idx_dtype == np.int64 else "int"
-            g = conv_double_generator(self.config, self.deterministic, idx)
-            code = rt.variant_code(("conv double", self.config.signature(), self.deterministic, idx, g.variant()), g.render)
+
+            def build():
+                g = conv_double_generator(self.config, self.deterministic, idx)
+                return g.render(), (g.steps(), g.plan()[2])
             need = rt.STEP_NEEDS_WORKSPACE | (rt.STEP_NEEDS_TPERM if self.deterministic else 0)
-            impl = rt.ConvImpl(code, [], _make_steps(g.steps(), need))
-            self._ws_fns.append(g.plan()[2])
+            impl, (_, ws) = rt.variant(("conv double", self.config.signature(), self.deterministic, idx,
+                                        UVUDetDoubleGenerator.variant()), torch.cuda.current_device(), build,
+                                       lambda code, plan: rt.ConvImpl(code, [], _make_steps(plan[0], need)))
+            self._ws_fns.append(ws)
             self._double = impl
         return self._double
 

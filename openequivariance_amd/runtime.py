@@ -13,6 +13,7 @@ import hashlib
 import os
 import pathlib
 import threading
+import weakref
 from typing import List, Optional, Sequence
 
 from . import tunables
@@ -190,27 +191,34 @@ def compile_source(source: str, arch: str = TARGET_ARCH, options: Sequence[str] 
     return blob
 
 
-# Code objects of kernel sets that operators build on first need (double backward), by what their source depends on:
-# operators of one problem - the layers of a model - then render and look up that source once.  Bounded; the entries are
-# plain bytes, every operator loads its own module from them.
-_VARIANTS: "collections.OrderedDict[tuple, bytes]" = collections.OrderedDict()
+# Kernel sets that operators build on first need (double backward, batches of few rows), by what they depend on.  Operators
+# of one problem - the layers of a model - plan, render and look up the source once (bounded: code objects and launch
+# plans), and share one loaded module per device for as long as one of them holds it: a launch changes nothing in it.
+_VARIANTS: "collections.OrderedDict[tuple, tuple]" = collections.OrderedDict()
 _VARIANTS_MAX = 64
-_variants_lock = threading.Lock()
+_LOADED: "weakref.WeakValueDictionary[tuple, object]" = weakref.WeakValueDictionary()
+_variants_lock = threading.RLock()
 
 
-def variant_code(key: tuple, render) -> bytes:
-    """Code object of the source that ``render()`` gives, remembered by ``key`` (everything the source depends on)."""
+def variant(key: tuple, device: int, build, load):
+    """(handle, plan) where ``build()`` gives (source, plan) and ``load(code object, plan)`` the handle on ``device``;
+    ``key`` is everything they depend on.  A source of None: there is no such kernel set, and no handle."""
     with _variants_lock:
-        code = _VARIANTS.get(key)
-        if code is not None:
+        got = _VARIANTS.get(key)
+        if got is None:
+            source, plan = build()
+            got = _VARIANTS[key] = (None if source is None else compile_source(source), plan)
+            if len(_VARIANTS) > _VARIANTS_MAX:
+                _VARIANTS.popitem(last=False)
+        else:
             _VARIANTS.move_to_end(key)
-            return code
-    code = compile_source(render())
-    with _variants_lock:
-        _VARIANTS[key] = code
-        while len(_VARIANTS) > _VARIANTS_MAX:
-            _VARIANTS.popitem(last=False)
-    return code
+        code, plan = got
+        if code is None:
+            return None, plan
+        handle = _LOADED.get((key, device))
+        if handle is None:
+            handle = _LOADED[(key, device)] = load(code, plan)
+        return handle, plan
 
 
 def kernel_metadata(code: bytes) -> dict:

@@ -199,13 +199,14 @@ class TensorProduct(TensorProductBase):
         if not 0 < batch <= self._few_rows_limits[backward]:
             return None
         if self._few_rows is None and not _capturing():
-            g = UVWSmallGenerator.create(self.config)
-            if g is None:                     # a problem whose units do not fit their registers or LDS
+            def build():
+                g = UVWSmallGenerator.create(self.config)
+                return (None, None) if g is None else (g.render(), g.plan()[:2])
+            impl, _ = rt.variant(("uvw few rows", self.config.signature()), torch.cuda.current_device(), build,
+                                 lambda code, plan: rt.TPImpl(code, *(_make_steps(steps, self._step_flags) for steps in plan)))
+            if impl is None:                  # a problem whose units do not fit their registers or LDS
                 self._few_rows_limits = (0, 0)
-                return None
-            code = rt.variant_code(("uvw few rows", self.config.signature()), g.render)
-            fwd, bwd, _ = g.plan()
-            self._few_rows = rt.TPImpl(code, _make_steps(fwd, self._step_flags), _make_steps(bwd, self._step_flags))
+            self._few_rows = impl
         return self._few_rows
 
     def forward_raw(self, batch, L1_in, L2_in, L3_out, weights, stream=None) -> None:
@@ -228,9 +229,12 @@ class TensorProduct(TensorProductBase):
         aligned = L1_out % 16 == 0 and L3_grad_out % 16 == 0
         impl = self._double.get(aligned)
         if impl is None:
-            g = self._double_generator(self.config, vector_stores=aligned)
-            code = rt.variant_code(("tp double", self.config.signature(), aligned, g.one_block_ahead()), g.render)
-            impl = self._double[aligned] = rt.TPImpl(code, [], _make_steps(g.plan()))
+            def build():
+                g = self._double_generator(self.config, vector_stores=aligned)
+                return g.render(), g.plan()
+            impl, _ = rt.variant(("tp double", self.config.signature(), aligned, self._double_generator.ONE_BLOCK_AHEAD),
+                                 torch.cuda.current_device(), build, lambda code, plan: rt.TPImpl(code, [], _make_steps(plan)))
+            self._double[aligned] = impl
         impl.double_backward(int(batch_size), L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot,
                              L1_out, L2_out, weights_out, L3_grad_out, self._stream() if stream is None else stream)
 
