@@ -28,6 +28,7 @@ from .uvw import UVWGenerator, _ceil
 class UVWSmallGenerator(UVWGenerator):
     FWD_ACC_LIMIT = 40           # accumulator tiles x 4 of one forward work item (two w tiles of an l = 2 block)
     BWD_LDS_LIMIT = 144 * 1024   # the dZ tile may fill a compute unit: there is one workgroup for each at most
+    LDS_BYTES = 160 * 1024       # of a compute unit: what a kernel's arrays together may take (see lds_bytes)
     FWD_PIPELINE = {4: (4, 2), 8: (1, 4)}
     DW_WAVES = 16
     DW_REGISTERS = 88            # of 128 a lane has with 16 wavefronts: accumulators, operands and one T of a dW unit
@@ -84,12 +85,23 @@ class UVWSmallGenerator(UVWGenerator):
 
     @classmethod
     def create(cls, problem: TPProblem):
-        """The generator, or None where a dW unit does not fit its registers or no launch would be cut finer."""
+        """The generator, or None where a dW unit does not fit its registers, a kernel's arrays do not fit LDS together or
+        no launch would be cut finer."""
         try:
             g = cls(problem)
         except NotImplementedError:
             return None
-        return g if g.dw_fits and g.bwd_lds else None
+        return g if g.dw_fits and g.bwd_lds and g.lds_bytes() <= cls.LDS_BYTES else None
+
+    def lds_bytes(self) -> int:
+        """LDS of the largest kernel: the backward's dZ tile beside a dY patch per wavefront (1 KB per word of the second
+        operand with 16 wavefronts: from 17 words on a tile within BWD_LDS_LIMIT can be too much), or the dW phases."""
+        patches = self.backward_threads // 64 * 16 * max(1, self.D2)
+        return max(16 * self.bwd_rs + patches, self._phase_elems()) * self.itemsize
+
+    def _phase_elems(self) -> int:
+        """What the dW phases of a workgroup hand over to each other, of the largest unit."""
+        return max(uw * (self.DW_WAVES // uw // 2) * _ceil(p.NTU, uw) * (hi - lo) * 256 for p, lo, hi, uw in self.units)
 
     def forward_attr(self) -> str:
         return " __attribute__((amdgpu_waves_per_eu(2)))"
@@ -114,9 +126,8 @@ class UVWSmallGenerator(UVWGenerator):
     def backward_dw_body(self) -> str:
         E = Emitter()
         PH = lambda uw: self.DW_WAVES // uw
-        slots = max(uw * (PH(uw) // 2) * _ceil(p.NTU, uw) * (hi - lo) * 256 for p, lo, hi, uw in self.units)
         E("const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;")
-        E(f"__shared__ T comb[{max(1, slots)}];")
+        E(f"__shared__ T comb[{max(1, self._phase_elems())}];")
         first = 0
         for k, (p, lo, hi, uw) in enumerate(self.units):
             Q, ph, D = _ceil(p.NTU, uw), PH(uw), p.o.D

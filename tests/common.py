@@ -112,3 +112,15 @@ def conv_reference_on_valid_edges(otp, oprob, X, Y, W, G, rows, cols, valid):
     dY, dW = np.zeros_like(Y, dtype=np.float64), np.zeros_like(W, dtype=np.float64)
     dY[valid], dW[valid] = dYv, dWv
     return Z, dX, dY, dW
+
+
+def lds_bytes(source, itemsize):
+    """{kernel: bytes} of the LDS arrays that a generated source declares."""
+    import re
+    size = {"T": itemsize, "float": 4, "double": 8, "int": 4, "i64": 8, "u64": 8}
+    out = {}
+    for body in re.split(r'extern "C" __global__', source)[1:]:
+        arrays = re.findall(r"__shared__ (?:__attribute__\(\(aligned\(16\)\)\) )?(\w+) \w+\[([\d *]+)\];", body)
+        assert len(arrays) == body.count("__shared__")
+        out[re.search(r"void (\w+)\s*\(", body).group(1)] = sum(size[t] * eval(n) for t, n in arrays)
+    return out

@@ -43,6 +43,59 @@ def test_emulated(dtype, n, monkeypatch):
     assert rel(ow.oeq_to_e3nn(oprob, out["Wg"]), dW) < TOL[dtype]
 
 
+def natural(mul, lmax):
+    return "+".join(f"{mul}x{l}{'eo'[l % 2]}" for l in range(lmax + 1))
+
+
+# second operands of 16 to 108 words beside wide outputs: the dZ tile and the wavefronts' dY patches share 160 KB of LDS
+WIDE = {
+    "16_words": (np.float32, (natural(16, 2), natural(1, 3), natural(240, 2)), True),
+    "25_words": (np.float32, (natural(16, 4), natural(1, 4), natural(88, 4)), False),
+    "25_words_f64": (np.float64, (natural(16, 2), natural(1, 4), natural(124, 2)), False),
+    "36_words_f64": (np.float64, (natural(16, 3), natural(1, 5), natural(64, 3)), False),
+    "copies_f64": (np.float64, ("16x0e+16x1o", "3x0e+3x1o+3x2e", "120x0e+120x1o+120x2e"), False),
+    "copies": (np.float32, (natural(16, 2), natural(12, 2), natural(144, 2)), False),
+    "copies_narrow": (np.float32, (natural(16, 2), natural(12, 2), natural(136, 2)), True),
+}
+
+
+@pytest.mark.parametrize("case", sorted(WIDE))
+def test_arrays_fit_lds_together(case):
+    dtype, irreps, taken = WIDE[case]
+    prob, _ = common.fully_connected(irreps, shared=True, dtype=dtype)
+    g = UVWSmallGenerator.create(prob)
+    assert (g is not None) == taken
+    used = common.lds_bytes((g or UVWSmallGenerator(prob)).render(), np.dtype(dtype).itemsize)
+    assert (max(used.values()) <= 160 * 1024) == taken
+    assert (g or UVWSmallGenerator(prob)).lds_bytes() == max(used["backward"], used["backward_dw"])
+
+
+def test_source_that_nearly_fills_lds_builds():
+    from openequivariance_amd import runtime as rt
+    dtype, irreps, _ = WIDE["16_words"]
+    g = UVWSmallGenerator.create(common.fully_connected(irreps, shared=True, dtype=dtype)[0])
+    assert g.lds_bytes() > 144 * 1024
+    assert rt.kernel_metadata(rt.compile_source(g.render()))["backward"][".group_segment_fixed_size"] == g.lds_bytes()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["16_words", "copies_f64"])
+def test_wide_second_operands_on_the_gpu(cuda, case):
+    import torch
+    import openequivariance_amd as oeq
+    dtype, irreps, taken = WIDE[case]
+    prob, oprob = common.fully_connected(irreps, shared=True, dtype=dtype)
+    tp = oeq.TensorProduct(prob, torch_op=True)
+    X, Y, We, G = common.tp_inputs(prob, 19, 4, dtype, w_scale=0.3)
+    x, y, w, g = (torch.tensor(a, device=cuda) for a in (X, Y, ow.e3nn_to_oeq(oprob, We), G))
+    got = [tp.forward(x, y, w), *tp.backward_helper(x, y, w, g)]
+    assert (tp._few_rows is not None) == taken
+    ref = [otp.forward(oprob, X, Y, We), *otp.backward(oprob, X, Y, We, G)]
+    ref[3] = ow.e3nn_to_oeq(oprob, ref[3])
+    for a, b in zip(got, ref):
+        assert rel(a.cpu().numpy(), b) < 4 * TOL[dtype]      # (sums of up to four times the terms of the products above)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("irreps", [MIXED, BOTH, common.DENSE], ids=["mixed", "both", "dense"])
