@@ -28,14 +28,16 @@ class UVUSharedGenerator(UVUDirectGenerator):
     TILE_ROWS = 4             # rows per wavefront between two barriers when several wavefronts share a row
     # registers (32-bit) of dW sums and weights a wavefront may hold across its rows
     HELD_REGISTERS = 128
+    LDS_BYTES = 160 * 1024    # of a compute unit: what the backward's arrays together may take (see lds_bytes)
 
     @classmethod
     def suits(cls, problem: TPProblem) -> bool:
-        """dW sums and weights of a channel fit the registers, and a row's chunks fit one workgroup."""
+        """dW sums and weights of a channel fit the registers, and a row's chunks one workgroup and its LDS."""
         muls = [problem.irreps_in2[i.i_in2].mul for i in problem.instructions]
         words = 2 * sum(muls) * (2 if problem.irrep_dtype().itemsize == 8 else 1)
         widest = max(mul for mul, _ in list(problem.irreps_in1) + list(problem.irreps_out))
-        return max(muls) <= 8 and words <= cls.HELD_REGISTERS and widest <= 16 * WAVE
+        return (max(muls) <= 8 and words <= cls.HELD_REGISTERS and widest <= 16 * WAVE
+                and cls(problem).lds_bytes() <= cls.LDS_BYTES)
 
     def __init__(self, problem: TPProblem, vector_stores: bool = True):
         super().__init__(problem, "tp", vector_stores=vector_stores)
@@ -49,6 +51,16 @@ class UVUSharedGenerator(UVUDirectGenerator):
         full = all(self.full(b) for b in self.in1 + self.out if b.dim)
         self.max_workgroups = self.MAX_WORKGROUPS or (256 if self.T == "double" else 512 if full else 768)
         self.bwd_slot = any(self.dx_through_slot(self.in1[i]) for i in self.used_in1)
+
+    def lds_bytes(self) -> int:
+        """LDS of the backward: the wavefronts' dX slots, the chunks' dY (which a row of 1024 channels in fp64 fills with 160
+        words of the second operand, used or not) and the fold of the dW sums."""
+        elems = self.waves * self.lds_elems if self.bwd_slot else 0
+        if self.NCH > 1:
+            elems += 2 * self.slots * self.TILE_ROWS * self.NCH * self.D2
+        if self.slots > 1:
+            elems += min(self.FOLD_PATHS, sum(p.mv for p in self.paths)) * self.waves * WAVE
+        return elems * self.itemsize
 
     def describe(self) -> str:
         return super().describe() + " shared weights"

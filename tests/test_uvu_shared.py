@@ -51,6 +51,29 @@ def test_generated_source(case, monkeypatch):
             assert rel_err(got, ref) < 2e-6      # fp32 sums of at most 130 rows x 7 words against fp64
 
 
+# wide second operands beside the sixteen or eight wavefronts of a row: (dtype, in1 = out, in2, taken)
+WIDE = {
+    "144_words": (np.float64, "1024x0e+1024x1o", "+".join(f"1x{l}e" for l in range(12)), True),
+    "169_words": (np.float64, "1024x0e+1024x1o", "+".join(f"1x{l}e" for l in range(13)), False),
+    "392_words": (np.float64, "512x0e+512x1o", "+".join(f"8x{l}e" for l in range(7)), False),
+    "392_words_fp32": (np.float32, "512x0e+512x1o", "+".join(f"8x{l}e" for l in range(7)), True),
+    "dx_slots": (np.float64, "1024x6e", "+".join(f"1x{l}e" for l in range(8)), False),
+}
+
+
+@pytest.mark.parametrize("case", sorted(WIDE))
+def test_arrays_fit_lds_together(case):
+    dtype, irreps, in2, taken = WIDE[case]
+    prob = oeq.TPProblem(irreps, in2, irreps, [(0, 0, 0, "uvu", True), (0, 2, 0, "uvu", True)] if case == "dx_slots" else
+                         [(0, 0, 0, "uvu", True), (1, 0, 1, "uvu", True)], shared_weights=True, internal_weights=False,
+                         irrep_dtype=dtype, weight_dtype=dtype)
+    g = select_generator(prob)
+    assert (type(g) is UVUSharedGenerator) == taken
+    used = common.lds_bytes(UVUSharedGenerator(prob).render(), np.dtype(dtype).itemsize)["backward"]
+    assert used == UVUSharedGenerator(prob).lds_bytes() and (used <= 160 * 1024) == taken
+    assert max(common.lds_bytes(g.render(), np.dtype(dtype).itemsize).values()) <= 160 * 1024
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("case", sorted(CASES))
