@@ -48,11 +48,15 @@ struct Call {
     const variable_list& index;
 };
 
+// Where a node keeps argument i.  Each by itself, not as a list: torch's compiled autograd makes inputs of its graph only of
+// tensors that are entries of saved_data themselves.
+std::string slot(size_t i) { return "t" + std::to_string(i); }
+
 variable_list run_forward(AutogradContext* ctx, const variable_list& tensors, const Call& call) {
     const Rule& r = rule(call.id);
     // (kept as data of the node, not as saved variables: the operators' arguments are not checked for changes in place)
-    ctx->saved_data["tensors"] = c10::List<at::Tensor>(tensors);
-    ctx->saved_data["index"] = c10::List<at::Tensor>(call.index);
+    for (size_t i = 0; i < tensors.size(); ++i) ctx->saved_data[slot(i)] = tensors[i];
+    for (size_t i = 0; i < call.index.size(); ++i) ctx->saved_data[slot(tensors.size() + i)] = call.index[i];
     ctx->saved_data["rule"] = call.id;
     torch::jit::Stack stack;
     stack.reserve(tensors.size() + call.index.size());
@@ -65,15 +69,15 @@ variable_list run_forward(AutogradContext* ctx, const variable_list& tensors, co
 
 variable_list run_backward(AutogradContext* ctx, const variable_list& grads) {
     const Rule& r = rule(ctx->saved_data["rule"].toInt());
-    const auto tensors = ctx->saved_data["tensors"].toTensorVector(), index = ctx->saved_data["index"].toTensorVector();
+    const size_t n = r.op.schema().arguments().size();
     torch::jit::Stack stack;
-    stack.reserve(tensors.size() + grads.size() + index.size());
-    for (const auto& t : tensors) stack.emplace_back(t);
+    stack.reserve(n + grads.size());
+    for (size_t i = 0; i < r.differentiable; ++i) stack.push_back(ctx->saved_data.at(slot(i)));
     for (const auto& t : grads) stack.emplace_back(t);
-    for (const auto& t : index) stack.emplace_back(t);
+    for (size_t i = r.differentiable; i < n; ++i) stack.push_back(ctx->saved_data.at(slot(i)));
     r.next.callBoxed(&stack);
     variable_list out = stack.back().toTensorVector();
-    TORCH_CHECK(out.size() == tensors.size(), "a derivative returned ", out.size(), " gradients for ", tensors.size(), " tensors");
+    TORCH_CHECK(out.size() == r.differentiable, "a derivative returned ", out.size(), " gradients for ", r.differentiable, " tensors");
     out.emplace_back();                                     // nothing for the Call
     return out;
 }

@@ -1,5 +1,7 @@
 """The C++ autograd kernels of the torch operators, on a trilinear product defined for the CPU through the same registration
 as the operators: derivatives of three orders, graphs that are not asked for, and the transforms of torch around them."""
+import contextlib
+
 import pytest
 import torch
 
@@ -94,3 +96,29 @@ def test_transforms(ops, data):
     assert torch.allclose(many[1], 2 * reference(*plain, *index))
     torch.library.opcheck(ops[0], (x, y, w, *index), test_utils=("test_schema", "test_faketensor", "test_autograd_registration"))
     torch.library.opcheck(ops[1], (x, y, w, x.detach(), *index), test_utils=("test_schema", "test_faketensor", "test_autograd_registration"))
+
+
+def test_compiled_autograd(ops, data):
+    """Backward passes as torch records and compiles them, of two operators whose nodes differ only in their rule."""
+    (args, index), compiler = data, torch.compile(backend="aot_eager")
+    negative = define_operator("glue_negative", OPERANDS + INDEX, "Tensor", lambda *a: -2 * ops[0](*a), lambda x, *rest: like(x)[0], "CPU")
+    negative_backward = define_operator("glue_negative_backward", (*OPERANDS, "L3_grad", *INDEX), "Tensor[]",
+                                        lambda *a: [-2 * t for t in ops[1](*a)], lambda x, y, w, *rest: like(x, y, w), "CPU")
+    define_derivatives("glue_negative", "glue_negative_backward", OPERANDS + INDEX,
+                       lambda x, y, w, g, a, b, v, *index: list(double_backward_terms(negative, negative_backward, x, y, w, g, a, b, v, index)))
+    import torch._dynamo.compiled_autograd as compiled_autograd
+
+    def gradients(f, around):
+        first, got = torch.autograd.grad(f(*args, *index).sin().sum(), args, create_graph=True), []
+        for loss in (f(*args, *index).sin().sum(), sum(t.square().sum() for t in first)):      # both kinds of node
+            with around():
+                loss.backward()
+            got += [t.grad for t in args]
+            for t in args:
+                t.grad = None
+        return got
+
+    for op, scale in ((ops[0], 1), (negative, -2)) * 2:
+        got = gradients(op, lambda: compiled_autograd._enable(compiler))
+        want = gradients(lambda *a: scale * reference(*a), contextlib.nullcontext)
+        assert all(torch.allclose(a, b, rtol=1e-12, atol=1e-12) for a, b in zip(got, want))
