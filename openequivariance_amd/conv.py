@@ -29,7 +29,7 @@ from .codegen.uvu_direct import UVUDirectGenerator
 from .codegen.uvu_recv import UVURecvGenerator
 from .codegen.uvu_sorted import UVUSortedGenerator
 from .problem import TPProblem
-from .tensor_product import _capturing, _contiguous, _make_steps, _on_device, validate_problem
+from .tensor_product import _contiguous, _make_steps, _on_device, validate_problem
 from .weight_order import WeightReorder
 from .wigner import wigner_3j
 
@@ -207,7 +207,11 @@ class TensorProductConv:
                          and tunables.current.conv_backward is None)
         self.graph_cache = tunables.current.graph_cache if graph_cache is None else bool(graph_cache)
         self._internal_unaligned = None
-        self._double = None                   # kernels of the double backward, compiled on first need
+        # Kernels of the double backward and its workspace function.  The operator torch differentiates has them from the
+        # start, so that the first call does not wait for the compiler; the first call makes them `_double` and lets the
+        # workspace, until then sized for the first-order kernels, grow for them.
+        self._double = None
+        self._double_built = self._double_kernels() if torch_op else None
         self._reorder = WeightReorder(config)
         self.reorder_weights_e3nn_to_oeq = self._reorder.e3nn_to_oeq
         self.reorder_weights_oeq_to_e3nn = self._reorder.oeq_to_e3nn
@@ -245,22 +249,26 @@ class TensorProductConv:
         return self._bwd_variants[name]
 
     def _double_usable(self) -> bool:
-        """Not under stream capture before its code object is loaded: the first-order kernels are, and the second
-        derivatives are composed from them there."""
-        return self._double is not None or not _capturing()
+        """Not under stream capture before its first use, which lets the workspace grow: the first-order kernels have
+        theirs, and the second derivatives are composed from them there."""
+        return self._double is not None or not torch.cuda.is_current_stream_capturing()
+
+    def _double_kernels(self):
+        """(kernel set, workspace function) of the fused double backward; its steps share the operator's workspace."""
+        idx = "i64" if self.idx_dtype == np.int64 else "int"
+
+        def build():
+            g = conv_double_generator(self.config, self.deterministic, idx)
+            return g.render(), (g.steps(), g.plan()[2])
+        need = rt.STEP_NEEDS_WORKSPACE | (rt.STEP_NEEDS_TPERM if self.deterministic else 0)
+        impl, (_, ws) = rt.variant(("conv double", self.config.signature(), self.deterministic, idx,
+                                    UVUDetDoubleGenerator.variant()), torch.cuda.current_device(), build,
+                                   lambda code, plan: rt.ConvImpl(code, [], _make_steps(plan[0], need)))
+        return impl, ws
 
     def _double_impl(self) -> "rt.ConvImpl":
-        """Kernel set of the fused double backward; its steps share the operator's workspace."""
         if self._double is None:
-            idx = "i64" if self.idx_dtype == np.int64 else "int"
-
-            def build():
-                g = conv_double_generator(self.config, self.deterministic, idx)
-                return g.render(), (g.steps(), g.plan()[2])
-            need = rt.STEP_NEEDS_WORKSPACE | (rt.STEP_NEEDS_TPERM if self.deterministic else 0)
-            impl, (_, ws) = rt.variant(("conv double", self.config.signature(), self.deterministic, idx,
-                                        UVUDetDoubleGenerator.variant()), torch.cuda.current_device(), build,
-                                       lambda code, plan: rt.ConvImpl(code, [], _make_steps(plan[0], need)))
+            impl, ws = self._double_built = self._double_built or self._double_kernels()
             self._ws_fns.append(ws)
             self._double = impl
         return self._double

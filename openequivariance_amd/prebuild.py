@@ -11,6 +11,10 @@ import time
 import numpy as np
 
 from . import runtime as rt
+from .codegen.uvu_conv_double import conv_double_generator
+from .codegen.uvu_double import UVUDoubleGenerator
+from .codegen.uvw import UVWGenerator
+from .codegen.uvw_small import UVWSmallGenerator
 from .conv import select_conv_generator
 from .problem import ChannelwiseTPP, FullyConnectedTPProblem, TPProblem
 from .tensor_product import select_generator
@@ -19,28 +23,44 @@ from .workloads import DENSE, DIFFDOCK_L2, LARGE, MACE, MACE_ALL, NEQUIP, TETRIS
 
 
 def benchmark_generators():
-    """(label, generator) for every kernel set the benchmark workloads and the smoke test use,
-    chosen by the same selection functions as the operators."""
+    """(label, generator) for every kernel set the operators of the benchmark workloads and of the smoke test are
+    constructed with, chosen by the same selection functions."""
     readme = TPProblem("1x2e", "1x3e", "1x2e", [(0, 0, 0, "uvu", True)], shared_weights=False, internal_weights=False)
-    gens = [("readme/tp", select_generator(readme)),
-            ("mace/tp", select_generator(ChannelwiseTPP(*MACE))),
-            ("mace-all-parities/tp", select_generator(ChannelwiseTPP(*MACE_ALL))),
-            ("nequip/tp", select_generator(ChannelwiseTPP(*NEQUIP)))]
+    gens = []
+
+    def tp(label, problem):
+        g = select_generator(problem)
+        gens.append((label, g))
+        if type(g) is UVWGenerator:
+            few = UVWSmallGenerator.create(problem)
+            if few is not None:
+                gens.append((label + " few rows", few))
+        elif problem.instructions[0].connection_mode == "uvu" and UVUDoubleGenerator.suits(problem):
+            gens.append((label + " double backward", UVUDoubleGenerator(problem)))
+
+    def conv(label, problem, deterministic):
+        gens.append((label, select_conv_generator(problem, deterministic)))
+        gens.append((label + " double backward", conv_double_generator(problem, deterministic)))
+
+    tp("readme/tp", readme)
+    tp("mace/tp", ChannelwiseTPP(*MACE))
+    tp("mace-all-parities/tp", ChannelwiseTPP(*MACE_ALL))
+    tp("nequip/tp", ChannelwiseTPP(*NEQUIP))
     for label, irreps in (("nequip", NEQUIP), ("large", LARGE), ("mace", MACE)):
         for det in (False, True):
-            gens.append((f"{label}/conv_{'det' if det else 'atomic'}", select_conv_generator(ChannelwiseTPP(*irreps), det)))
+            conv(f"{label}/conv_{'det' if det else 'atomic'}", ChannelwiseTPP(*irreps), det)
     for det in (False, True):
         p = ChannelwiseTPP(*MACE, irrep_dtype=np.float64, weight_dtype=np.float64)
-        gens.append((f"mace/conv_{'det' if det else 'atomic'}/float64", select_conv_generator(p, det)))
-    gens.append(("benzene/conv_det", select_conv_generator(get_workload("benzene_conv_det").problem(), True)))
+        conv(f"mace/conv_{'det' if det else 'atomic'}/float64", p, det)
+    conv("benzene/conv_det", get_workload("benzene_conv_det").problem(), True)
     for dt in (np.float32, np.float64):
         p = FullyConnectedTPProblem(*DENSE, shared_weights=True, internal_weights=False, irrep_dtype=dt, weight_dtype=dt)
-        gens.append((f"dense/uvw/{np.dtype(dt).name}", select_generator(p)))
+        tp(f"dense/uvw/{np.dtype(dt).name}", p)
         p = FullyConnectedTPProblem(*DIFFDOCK_L2, shared_weights=False, internal_weights=False, irrep_dtype=dt, weight_dtype=dt)
-        gens.append((f"diffdock/uvw per-row weights/{np.dtype(dt).name}", select_generator(p)))
+        tp(f"diffdock/uvw per-row weights/{np.dtype(dt).name}", p)
         for which, irreps in TETRIS_POLY.items():
             p = FullyConnectedTPProblem(*irreps, shared_weights=True, internal_weights=False, irrep_dtype=dt, weight_dtype=dt)
-            gens.append((f"tetris-poly-{which}/uvw few weights/{np.dtype(dt).name}", select_generator(p)))
+            tp(f"tetris-poly-{which}/uvw few weights/{np.dtype(dt).name}", p)
     return gens
 
 

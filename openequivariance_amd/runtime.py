@@ -191,7 +191,7 @@ def compile_source(source: str, arch: str = TARGET_ARCH, options: Sequence[str] 
     return blob
 
 
-# Kernel sets that operators build on first need (double backward, batches of few rows), by what they depend on.  Operators
+# Kernel sets of an operator beside its main one (double backward, batches of few rows), by what they depend on.  Operators
 # of one problem - the layers of a model - plan, render and look up the source once (bounded: code objects and launch
 # plans), and share one loaded module per device for as long as one of them holds it: a launch changes nothing in it.
 _VARIANTS: "collections.OrderedDict[tuple, tuple]" = collections.OrderedDict()

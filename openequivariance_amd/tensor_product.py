@@ -53,11 +53,6 @@ def _contiguous(*tensors):
     return tuple(t if t is None or t.is_contiguous() else t.contiguous() for t in tensors)
 
 
-def _capturing() -> bool:
-    """torch's current stream is recording a graph (never on a machine without a GPU)."""
-    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
-
-
 def _on_device(device):
     """Context that makes ``device`` current: nothing at all when it already is (the usual case; entering
     torch.cuda.device costs several microseconds per call)."""
@@ -135,12 +130,14 @@ class TensorProduct(TensorProductBase):
         self._dims = (self.L1.dim, self.L2.dim, self.L3.dim, config.weight_numel)
         self._workspaces = {}                 # (device, stream) -> scratch tensor (fixed size, never regrown)
         self._internal_unaligned = None       # kernels without 16-byte vector stores, compiled on first need
-        # dense uvw: largest batch (forward, backward) of the kernels for few rows, which are compiled on first need
-        self._few_rows = None
-        self._few_rows_limits = UVWSmallGenerator.row_limits(self.generator) if type(self.generator) is UVWGenerator else (0, 0)
-        # double backward in one launch: kernels by alignment of the outputs, compiled on first need
+        # dense uvw: kernels for few rows and their largest batch (forward, backward).  Built here like the double backward's,
+        # not by the call that first needs them: that call would wait for the compiler, and a stream capture cannot
+        self._few_rows, self._few_rows_limits = self._few_row_kernels()
+        # double backward in one launch: kernels by alignment of the outputs (misaligned ones are compiled on first need)
         self._double_generator = UVUDoubleGenerator if mode == "uvu" and UVUDoubleGenerator.suits(config) else None
         self._double = {}
+        if torch_op and self._double_generator is not None:
+            self._double[True] = self._double_kernels(True)
 
         self._reorder = WeightReorder(config)
         self.reorder_weights_e3nn_to_oeq = self._reorder.e3nn_to_oeq
@@ -194,20 +191,29 @@ class TensorProduct(TensorProductBase):
         return self.internal
 
     def _pick_rows(self, batch: int, backward: bool):
-        """The kernels for few rows where ``batch`` is one, else None (under stream capture also while their code object
-        is not loaded)."""
-        if not 0 < batch <= self._few_rows_limits[backward]:
-            return None
-        if self._few_rows is None and not _capturing():
-            def build():
-                g = UVWSmallGenerator.create(self.config)
-                return (None, None) if g is None else (g.render(), g.plan()[:2])
-            impl, _ = rt.variant(("uvw few rows", self.config.signature()), torch.cuda.current_device(), build,
-                                 lambda code, plan: rt.TPImpl(code, *(_make_steps(steps, self._step_flags) for steps in plan)))
-            if impl is None:                  # a problem whose units do not fit their registers or LDS
-                self._few_rows_limits = (0, 0)
-            self._few_rows = impl
-        return self._few_rows
+        """The kernels for few rows where ``batch`` is one, else None."""
+        return self._few_rows if 0 < batch <= self._few_rows_limits[backward] else None
+
+    def _few_row_kernels(self):
+        """(kernel set, limits) of the kernels for few rows of a dense uvw product."""
+        none = None, (0, 0)
+        if type(self.generator) is not UVWGenerator:
+            return none
+
+        def build():
+            g = UVWSmallGenerator.create(self.config)
+            return (None, None) if g is None else (g.render(), g.plan()[:2])
+        impl, _ = rt.variant(("uvw few rows", self.config.signature()), torch.cuda.current_device(), build,
+                             lambda code, plan: rt.TPImpl(code, *(_make_steps(steps, self._step_flags) for steps in plan)))
+        # (None: a problem whose units do not fit their registers or LDS)
+        return none if impl is None else (impl, UVWSmallGenerator.row_limits(self.generator))
+
+    def _double_kernels(self, aligned: bool) -> "rt.TPImpl":
+        def build():
+            g = self._double_generator(self.config, vector_stores=aligned)
+            return g.render(), g.plan()
+        return rt.variant(("tp double", self.config.signature(), aligned, self._double_generator.ONE_BLOCK_AHEAD),
+                          torch.cuda.current_device(), build, lambda code, plan: rt.TPImpl(code, [], _make_steps(plan)))[0]
 
     def forward_raw(self, batch, L1_in, L2_in, L3_out, weights, stream=None) -> None:
         """Device pointers as integers (reference: TensorProductBase.py:41-49)."""
@@ -229,12 +235,7 @@ class TensorProduct(TensorProductBase):
         aligned = L1_out % 16 == 0 and L3_grad_out % 16 == 0
         impl = self._double.get(aligned)
         if impl is None:
-            def build():
-                g = self._double_generator(self.config, vector_stores=aligned)
-                return g.render(), g.plan()
-            impl, _ = rt.variant(("tp double", self.config.signature(), aligned, self._double_generator.ONE_BLOCK_AHEAD),
-                                 torch.cuda.current_device(), build, lambda code, plan: rt.TPImpl(code, [], _make_steps(plan)))
-            self._double[aligned] = impl
+            impl = self._double[aligned] = self._double_kernels(aligned)
         impl.double_backward(int(batch_size), L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot,
                              L1_out, L2_out, weights_out, L3_grad_out, self._stream() if stream is None else stream)
 
@@ -325,8 +326,7 @@ class TensorProduct(TensorProductBase):
 
         def double_backward(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot):
             return list(double_backward_terms(forward, backward_helper, L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot,
-                                              # (its code object is loaded on first use, which a stream capture must not do)
-                                              fused=fused if self._double or not _capturing() else None))
+                                              fused=fused))
 
         define_derivatives(f"tp_forward{tp_id}", f"tp_grad_helper{tp_id}", operands, double_backward)
 

@@ -1,6 +1,12 @@
-"""Kernel sets built on first need are planned and compiled once, loaded once per device, and unloaded with their last owner."""
+"""Kernel sets beside an operator's main one are planned and compiled once, loaded once per device and unloaded with their
+last owner; an operator has them when it is constructed."""
 import gc
 
+import pytest
+import torch
+
+import common
+import openequivariance_amd as oeq
 from openequivariance_amd import runtime as rt
 
 
@@ -29,3 +35,45 @@ def test_shared_while_held(monkeypatch):
     assert len(rt._VARIANTS) == rt._VARIANTS_MAX and get(1)[0] is a and built.count(1) == 2 and len(held) == rt._VARIANTS_MAX
     for key in [k for k in rt._VARIANTS if k[0] == "test"]:
         del rt._VARIANTS[key]
+
+
+class Impl:
+    def __init__(self, code, *steps):
+        self.code = code
+
+    def set_forward_workspace(self, *model):
+        pass
+
+
+@pytest.mark.parametrize("case", ["uvu", "uvu_raw", "uvw", "conv", "conv_sorted"])
+def test_no_call_waits_for_the_compiler(case, monkeypatch):
+    """The kernel sets of second derivatives and of batches of few rows are compiled and loaded with the operator."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(rt, "compile_source", lambda source, *a, **k: source.encode())
+    monkeypatch.setattr(rt, "TPImpl", Impl)
+    monkeypatch.setattr(rt, "ConvImpl", Impl)
+    monkeypatch.setattr(rt, "_VARIANTS", type(rt._VARIANTS)())
+    monkeypatch.setattr(rt, "_LOADED", type(rt._LOADED)())
+    if case == "uvw":
+        op = oeq.TensorProduct(common.fully_connected(common.DENSE, shared=True)[0], torch_op=False)
+    elif case.startswith("uvu"):
+        op = oeq.TensorProduct(common.channelwise(common.NEQUIP)[0], torch_op=case == "uvu")
+    else:
+        op = oeq.TensorProductConv(common.channelwise(common.NEQUIP)[0], torch_op=True, deterministic=case == "conv_sorted")
+    kinds = [key[0] for key in rt._VARIANTS]
+    assert kinds == {"uvu": ["tp double"], "uvu_raw": [], "uvw": ["uvw few rows"]}.get(case, ["conv double"])
+
+    def refuse(*a):
+        raise AssertionError("compiled inside a call")
+    monkeypatch.setattr(rt, "compile_source", refuse)
+    if case == "uvw":
+        limits = op._few_rows_limits
+        assert [op._pick_rows(n, back) is not None for back in (False, True) for n in (0, 1, limits[back], limits[back] + 1)] \
+            == [False, True, True, False] * 2
+    elif case == "uvu":
+        assert op._double[True].code
+    elif case.startswith("conv"):
+        before = op._ws_bytes(5000, 300)
+        assert op._double_usable() and op._double_impl().code
+        assert op._ws_bytes(5000, 300) >= before and len(op._ws_fns) == 2 and op._double_impl() is op._double
