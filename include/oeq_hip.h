@@ -186,6 +186,15 @@ int  oeq_conv_double_backward(oeq_conv* conv, const void* L1_in, const void* L2_
                               void* L3_grad_out, const void* rows, const void* cols, uint64_t nnz,
                               uint64_t node_count, void* workspace, const void* transpose_perm, void* stream);
 
+/* The same with call flags, as oeq_conv_backward_ex: OEQ_CALL_PREPARED promises that the workspace still holds both graph
+ * preparations an earlier double backward of exactly this graph left there, and nothing else has written it since. */
+int  oeq_conv_double_backward_ex(oeq_conv* conv, const void* L1_in, const void* L2_in, const void* weights,
+                                 const void* L3_grad, const void* L1_grad_cot, const void* L2_grad_cot,
+                                 const void* weights_grad_cot, void* L1_out, void* L2_out, void* weights_out,
+                                 void* L3_grad_out, const void* rows, const void* cols, uint64_t nnz,
+                                 uint64_t node_count, void* workspace, const void* transpose_perm, void* stream,
+                                 uint32_t call_flags);
+
 /* Workspace bytes the forward steps use when every node is walked by one wavefront (no pieces):
  * fixed_bytes + bytes_per_node * node_count + bytes_per_edge * nnz.  The host sets it from the plan it
  * built the operator with; oeq_conv_forward_noalloc checks graphs against it.  (The reference sizes

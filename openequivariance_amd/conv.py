@@ -208,8 +208,8 @@ class TensorProductConv:
         self.graph_cache = tunables.current.graph_cache if graph_cache is None else bool(graph_cache)
         self._internal_unaligned = None
         # Kernels of the double backward and its workspace function.  The operator torch differentiates has them from the
-        # start, so that the first call does not wait for the compiler; the first call makes them `_double` and lets the
-        # workspace, until then sized for the first-order kernels, grow for them.
+        # start, so that the first call does not wait for the compiler; the first call makes them `_double` and takes the
+        # workspace they need.
         self._double = None
         self._double_built = self._double_kernels() if torch_op else None
         self._reorder = WeightReorder(config)
@@ -249,12 +249,12 @@ class TensorProductConv:
         return self._bwd_variants[name]
 
     def _double_usable(self) -> bool:
-        """Not under stream capture before its first use, which lets the workspace grow: the first-order kernels have
-        theirs, and the second derivatives are composed from them there."""
+        """Not under stream capture before its first use, which takes its workspace: the first-order kernels have theirs,
+        and the second derivatives are composed from them there."""
         return self._double is not None or not torch.cuda.is_current_stream_capturing()
 
     def _double_kernels(self):
-        """(kernel set, workspace function) of the fused double backward; its steps share the operator's workspace."""
+        """(kernel set, workspace function) of the fused double backward."""
         idx = "i64" if self.idx_dtype == np.int64 else "int"
 
         def build():
@@ -266,11 +266,14 @@ class TensorProductConv:
                                    lambda code, plan: rt.ConvImpl(code, [], _make_steps(plan[0], need)))
         return impl, ws
 
+    def _double_ws_bytes(self, nnz: int, node_count: int) -> int:
+        self._double_impl()
+        return self._double_built[1](nnz, node_count)
+
     def _double_impl(self) -> "rt.ConvImpl":
         if self._double is None:
-            impl, ws = self._double_built = self._double_built or self._double_kernels()
-            self._ws_fns.append(ws)
-            self._double = impl
+            self._double_built = self._double_built or self._double_kernels()
+            self._double = self._double_built[0]
         return self._double
 
     @staticmethod
@@ -278,18 +281,21 @@ class TensorProductConv:
         return "LoopUnrollConv"
 
     # ------------------------------------------------------------------ helpers
-    def _workspace_record(self, nnz: int, node_count: int, stream: typing.Optional[int] = None) -> _StreamWorkspace:
+    def _workspace_record(self, nnz: int, node_count: int, stream: typing.Optional[int] = None, need: int = 0,
+                          own: str = "") -> _StreamWorkspace:
         """The operator's scratch for ``stream`` (torch's current one by default), grown on demand.  Every
         stream gets its own, so two streams using one operator do not share CSR pointers or position
         lists.  A buffer that has been outgrown is freed unless a HIP graph capture has used it: a captured
         graph has the address baked in, so such buffers stay alive as long as the operator (the reference
-        allocates its workspace once at a fixed size: ConvolutionBase.py:93-100)."""
+        allocates its workspace once at a fixed size: ConvolutionBase.py:93-100).  ``need``: bytes beyond those of
+        the first-order kernels; ``own``: another scratch than theirs, of ``need`` bytes."""
         dev = torch.cuda.current_device()
-        sid = (dev, self._stream(dev) if stream is None else int(stream))
+        sid = (dev, self._stream(dev) if stream is None else int(stream), own)
         rec = self._workspaces.get(sid)
         if rec is None:
             rec = self._workspaces[sid] = _StreamWorkspace()
-        need = self._ws_bytes(nnz, node_count)
+        if not own:
+            need = max(need, self._ws_bytes(nnz, node_count))
         if need > rec.size:
             if rec.captured and rec.buffer is not None:
                 rec.retired.append(rec.buffer)
@@ -409,23 +415,27 @@ class TensorProductConv:
                               self._stream() if stream is None else stream, prepared, counters_zero)
 
     def double_backward_rawptrs(self, L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot, L1_out, L2_out,
-                                weights_out, L3_grad_out, rows, cols, nnz, node_count, transpose_perm=0, stream=None):
+                                weights_out, L3_grad_out, rows, cols, nnz, node_count, transpose_perm=0, stream=None, workspace=0,
+                                prepared=False, counters_zero=False):
         """Gradients of the backward's inputs (x, y, w, dz) for cotangents of its outputs, in two passes over the edges
-        (codegen/uvu_conv_double.py).  Builds both graph preparations anew in the operator's scratch for the stream, so
-        neither the forward's nor the backward's cached one is valid afterwards."""
+        (codegen/uvu_conv_double.py).  Without ``workspace`` both graph preparations are built in the operator's scratch for
+        the stream, so neither the forward's nor the backward's cached one is valid afterwards.  ``prepared`` and
+        ``counters_zero`` promise about ``workspace`` what they do in exec_conv_rawptrs, for both preparations."""
         nnz, node_count = int(nnz), int(node_count)
         if self.deterministic and nnz > 0 and not transpose_perm:
             raise ValueError("the deterministic double backward needs transpose_perm (a device pointer), got 0")
         if any(int(p) % 16 for p in (L1_out, L3_grad_out)):
             raise ValueError("the double backward writes 16-byte vectors: its node outputs must be 16-byte aligned")
         impl = self._double_impl()
-        rec = self._workspace_record(nnz, node_count, stream)
-        if torch.cuda.is_current_stream_capturing():
-            rec.captured = True
-        rec.fwd_key = rec.bwd_key = rec.zero_fwd = rec.zero_bwd = None
+        if not workspace:
+            rec = self._workspace_record(nnz, node_count, stream, need=self._double_ws_bytes(nnz, node_count))
+            if torch.cuda.is_current_stream_capturing():
+                rec.captured = True
+            rec.fwd_key = rec.bwd_key = rec.zero_fwd = rec.zero_bwd = None
+            workspace, prepared, counters_zero = rec.buffer.data_ptr(), False, False
         impl.double_backward(L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot, L1_out, L2_out,
-                             weights_out, L3_grad_out, rows, cols, nnz, node_count, rec.buffer.data_ptr(), transpose_perm,
-                             self._stream() if stream is None else stream)
+                             weights_out, L3_grad_out, rows, cols, nnz, node_count, workspace, transpose_perm,
+                             self._stream() if stream is None else stream, prepared, counters_zero)
 
     def _time_backward_variants(self, run, names=("atomic", "grouped"), repeats: int = 3) -> str:
         """Fastest of the backward variants on the caller's own tensors: one untimed call each (compilation,
@@ -446,17 +456,21 @@ class TensorProductConv:
         return min(best, key=best.get)
 
     def _cached_call(self, which: str, rows, cols, tperm, E: int, N: int, launch, tag: str = "",
-                     stream: typing.Optional[int] = None) -> None:
+                     stream: typing.Optional[int] = None, double: bool = False) -> None:
         """Run ``launch(workspace pointer, prepared, counters_zero)`` for the torch operators.  The graph preparation a
         call leaves in the stream's workspace is reused by the next call of the same direction when it
         names the same graph: same index tensors (address and in-place version counter), same sizes.  The
         tensors are kept referenced while their key is cached, so the addresses cannot be handed to other
         tensors meanwhile.  Under HIP graph capture, and on a workspace that a capture has used, the
-        preparation always runs: a replay may rewrite the workspace behind the cache's back."""
-        if self._ws_bytes(E, N) == 0:
+        preparation always runs: a replay may rewrite the workspace behind the cache's back.  ``double``: a call of the
+        double backward, in a scratch of its own so that the three directions keep their preparations."""
+        if double:
+            rec = self._workspace_record(E, N, stream, need=self._double_ws_bytes(E, N), own="double")
+        elif self._ws_bytes(E, N) == 0:
             launch(0, False, False)
             return
-        rec = self._workspace_record(E, N, stream)
+        else:
+            rec = self._workspace_record(E, N, stream)
         if torch.cuda.is_current_stream_capturing():
             rec.captured = True
         key = None
@@ -550,10 +564,17 @@ class TensorProductConv:
             if a.shape != x.shape or a.device != x.device:
                 raise ValueError("the cotangents must match the operands' nodes and device")
             out = [torch.empty_like(t) for t in (x, y, w, g)]
+            E, N = rows.shape[0], x.shape[0]
             with _on_device(x.device):
-                self.double_backward_rawptrs(*(t.data_ptr() for t in (x, y, w, g, a, b, v, *out, rows, cols)), rows.shape[0],
-                                             x.shape[0], tperm.data_ptr() if tperm is not None else 0,
-                                             stream=self._stream(x.device.index))
+                stream = self._stream(x.device.index)
+
+                def launch(ws=0, prepared=False, zero=False):
+                    self.double_backward_rawptrs(*(t.data_ptr() for t in (x, y, w, g, a, b, v, *out, rows, cols)), E, N,
+                                                 tperm.data_ptr() if tperm is not None else 0, stream, ws, prepared, zero)
+                if self.graph_cache:
+                    self._cached_call("fwd", rows, cols, tperm, E, N, launch, stream=stream, double=True)
+                else:                # (scratch shared with the first-order kernels: there is nothing to keep)
+                    launch()
             return out
 
         fused = define_operator(

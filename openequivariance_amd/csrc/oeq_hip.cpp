@@ -388,19 +388,30 @@ int oeq_conv_backward_ex(oeq_conv* c, const void* L1, void* L1g, const void* L2,
     return conv_backward(c, L1, L1g, L2, L2g, W, Wg, L3g, rows, cols, nnz, node_count, workspace, tperm, stream, call_flags);
 }
 
-int oeq_conv_double_backward(oeq_conv* c, const void* L1, const void* L2, const void* W, const void* L3g, const void* L1c,
-                             const void* L2c, const void* Wc, void* L1o, void* L2o, void* Wo, void* L3o, const void* rows,
-                             const void* cols, uint64_t nnz, uint64_t node_count, void* workspace, const void* tperm,
-                             void* stream) {
+int oeq_conv_double_backward_ex(oeq_conv* c, const void* L1, const void* L2, const void* W, const void* L3g, const void* L1c,
+                                const void* L2c, const void* Wc, void* L1o, void* L2o, void* Wo, void* L3o, const void* rows,
+                                const void* cols, uint64_t nnz, uint64_t node_count, void* workspace, const void* tperm,
+                                void* stream, uint32_t call_flags) {
     if (!c) return fail("null handle");
     if (c->bwd.empty()) return fail("this operator was built without a double backward plan");
     if (nnz > 0 && node_count == 0) return fail("convolution called with %llu edges but no nodes", (unsigned long long)nnz);
     if (nnz > 0 && (!rows || !cols)) return fail("double backward: rows / cols are NULL");
     if ((nnz > 0 || node_count > 0) && check_pointers(c->bwd, workspace, nnz > 0 ? tperm : (const void*)1, "double backward")) return 1;
+    if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("double backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3g, &L1c, &L2c, &Wc, &L1o, &L2o, &Wo, &L3o, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
-    for (auto& s : c->bwd)
+    for (auto& s : c->bwd) {
+        if (skipped(s.desc, call_flags)) continue;
         if (launch(s, nnz, node_count, args, stream)) return 1;
+    }
     return 0;
+}
+
+int oeq_conv_double_backward(oeq_conv* c, const void* L1, const void* L2, const void* W, const void* L3g, const void* L1c,
+                             const void* L2c, const void* Wc, void* L1o, void* L2o, void* Wo, void* L3o, const void* rows,
+                             const void* cols, uint64_t nnz, uint64_t node_count, void* workspace, const void* tperm,
+                             void* stream) {
+    return oeq_conv_double_backward_ex(c, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, rows, cols, nnz, node_count, workspace,
+                                       tperm, stream, 0);
 }
 
 int oeq_conv_set_forward_workspace(oeq_conv* c, uint64_t fixed_bytes, uint64_t bytes_per_node, uint64_t bytes_per_edge) {

@@ -99,6 +99,7 @@ def lib() -> C.CDLL:
             "oeq_conv_forward_ex": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, u64, u64, vp, vp, vp, C.c_uint32]),
             "oeq_conv_backward_ex": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, u64, u64, vp, vp, vp, C.c_uint32]),
             "oeq_conv_double_backward": (C.c_int, [vp] * 14 + [u64, u64, vp, vp, vp]),
+            "oeq_conv_double_backward_ex": (C.c_int, [vp] * 14 + [u64, u64, vp, vp, vp, C.c_uint32]),
             "oeq_conv_set_forward_workspace": (C.c_int, [vp, u64, u64, u64]),
             "oeq_conv_forward_noalloc": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, u64, u64, vp, vp]),
             "oeq_module_load": (C.c_int, [vp, sz, C.POINTER(vp)]),
@@ -127,7 +128,8 @@ EXPORTED_SYMBOLS = [
     "oeq_last_error", "oeq_device_props", "oeq_device_count", "oeq_compile", "oeq_free", "oeq_hiprtc_version",
     "oeq_tp_create", "oeq_tp_destroy", "oeq_tp_forward", "oeq_tp_backward", "oeq_tp_double_backward",
     "oeq_conv_create", "oeq_conv_destroy", "oeq_conv_forward", "oeq_conv_backward",
-    "oeq_conv_forward_ex", "oeq_conv_backward_ex", "oeq_conv_double_backward", "oeq_conv_set_forward_workspace", "oeq_conv_forward_noalloc",
+    "oeq_conv_forward_ex", "oeq_conv_backward_ex", "oeq_conv_double_backward", "oeq_conv_double_backward_ex",
+    "oeq_conv_set_forward_workspace", "oeq_conv_forward_noalloc",
     "oeq_module_load", "oeq_module_unload", "oeq_module_launch",
     "oeq_timer_create", "oeq_timer_destroy", "oeq_timer_start", "oeq_timer_stop", "oeq_timer_clear_cache",
     "oeq_buffer_alloc", "oeq_buffer_free", "oeq_buffer_h2d", "oeq_buffer_d2h", "oeq_buffer_zero",
@@ -321,10 +323,11 @@ class ConvImpl:
                                           tperm, stream, flags))
 
     def double_backward(self, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, rows, cols, nnz, node_count, workspace=0,
-                        tperm=0, stream=0):
+                        tperm=0, stream=0, prepared=False, counters_zero=False):
         """Of a handle created from a double backward's code object with its plan as the backward steps."""
-        _check(lib().oeq_conv_double_backward(self._h, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, rows, cols, nnz,
-                                              node_count, workspace, tperm, stream))
+        flags = (CALL_PREPARED if prepared else 0) | (CALL_COUNTERS_ZERO if counters_zero else 0)
+        _check(lib().oeq_conv_double_backward_ex(self._h, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, rows, cols, nnz,
+                                                 node_count, workspace, tperm, stream, flags))
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None

@@ -176,6 +176,38 @@ def test_operator(cuda, case, deterministic, dtype, monkeypatch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("deterministic", [False, True])
+def test_graph_cache_keeps_the_preparations_of_all_three_directions(cuda, deterministic, monkeypatch):
+    """With ``graph_cache`` a training step on forces over an unchanged edge list prepares nothing anew; a change of the
+    edge list, seen by the version counter, rebuilds."""
+    import torch
+    from openequivariance_amd import runtime as rt
+    irreps, nodes, nnz, _, _ = CASES["hubs"]
+    prob, oprob = common.channelwise(irreps)
+    conv = oeq.TensorProductConv(prob, torch_op=True, deterministic=deterministic, graph_cache=True)
+    calls, plain = [], rt.ConvImpl.double_backward
+    monkeypatch.setattr(rt.ConvImpl, "double_backward", lambda self, *a: calls.append(a[-2:]) or plain(self, *a))
+    args = _inputs(prob, nodes, nnz, 41, np.float32)
+    x, y, w, g = (t.requires_grad_() for t in _device(cuda, args[:4]))
+    cots = _device(cuda, args[4:])
+    graphs = [_graph("hubs", deterministic, seed)[:3 if deterministic else 2] for seed in (42, 43)]
+    index = _device(cuda, graphs[0])
+    for k, graph in enumerate((graphs[0], graphs[0], graphs[0], graphs[1], graphs[1])):
+        if k == 3:
+            for dst, src in zip(index, _device(cuda, graphs[1])):
+                dst.copy_(src)
+        first = torch.autograd.grad(conv(x, y, w, *index), (x, y, w), g, create_graph=True)
+        rec = conv._workspace_record(nnz, nodes)
+        keys = rec.fwd_key, rec.bwd_key
+        assert k == 0 or None not in keys     # (the first backward of the unsorted operator lets the workspace grow)
+        second = torch.autograd.grad(first, (x, y, w, g), cots)
+        assert conv._workspace_record(nnz, nodes) is rec and (rec.fwd_key, rec.bwd_key) == keys
+        for a, b in zip(second, _reference(oprob, graph[0], graph[1], *args)):
+            assert rel_err(a.cpu().numpy(), b) <= 2e-5
+    assert [prepared for prepared, _ in calls] == [False, True, True, False, True]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("deterministic", [False, True])
 def test_empty_edge_list_and_other_graph_sizes(cuda, deterministic):
     """No edges: node gradients are zeros.  A larger graph afterwards grows the workspace, a smaller one reuses it."""
     import torch
