@@ -108,8 +108,8 @@ class UVWGenerator:
             raise NotImplementedError("this generator handles shared weights; see uvw_batched.py for per-row weights")
         # forward K loop: steps fetched per batch of loads, and unroll factor of the batch loop.  Measured on MI355X, 100 000
         # rows, fp32 4 / 1 against 4 / 2: 64 channels 304 / 297 us, 20 channels 102 / 95, 100 -> 30 channels 142 / 142; with
-        # one path per block (50 channels) 259 / 265, hence the exception below.  fp64 1 / 3 against 2 / 2 and 1 / 4: 540 /
-        # 623 / 641.  (A loop written out on alternating register sets, so that nothing is
+        # one path per block (50 channels) 259 / 265, hence the exception below; an odd number of batches leaves an exit in the
+        # middle of an unrolled body, see k_unroll.  fp64 1 / 3 against 2 / 2 and 1 / 4: 540 / 623 / 641.  (A loop written out on alternating register sets, so that nothing is
         # copied between sets, has 0.9 instead of 2.1 vector-ALU instructions per MFMA and measured 0.341
         # against 0.331 ms; larger groups for the cheap work items 0.361 - 0.422 against 0.359 ms.)
         self.fwd_group, self.fwd_unroll = self.FWD_PIPELINE[self.itemsize]
@@ -352,6 +352,12 @@ class UVWGenerator:
         return _ceil(self.WA_END, 256)
 
     # =============================================================== forward
+    def k_unroll(self, batches: int) -> int:
+        """Unroll factor of a forward K loop.  fp32: 1 where the factor does not divide the batches of four steps; 100 000
+        rows, l <= 1, unrolled twice against not: 68 channels (5 batches) 168 / 147 us, 100 (7) 306 / 252, 112 (7) 266 /
+        234; 48 channels, l <= 2 (3) 208 / 195; with an even number 64 (4) 90 / 94, 96 (6) 188 / 199, 128 (8) 272 / 277."""
+        return self.fwd_unroll if self.itemsize == 8 or batches % self.fwd_unroll == 0 else 1
+
     def forward_body(self) -> str:
         E = Emitter()
         NO = len(self.fwd_items)
@@ -460,7 +466,7 @@ class UVWGenerator:
                 E.level += 1
                 # the CG tensor is contracted with the row's Y once per path; the small matrix is applied per channel
                 self.emit_cg_matrix(E, p, "y", "m")
-                E(f"#pragma unroll {self.fwd_unroll}")
+                E(f"#pragma unroll {self.k_unroll(NG)}")
                 E(f"for (int sg = 0; sg < {NG}; ++sg) {{")
                 E.level += 1
                 E("const T " + ", ".join(f"c{r} = {r}" for r in regs(p)) + ";")

@@ -78,6 +78,18 @@ def test_source_that_nearly_fills_lds_builds():
     assert rt.kernel_metadata(rt.compile_source(g.render()))["backward"][".group_segment_fixed_size"] == g.lds_bytes()
 
 
+@pytest.mark.parametrize("generator", [UVWGenerator, UVWSmallGenerator])
+def test_fp32_forward_loops_are_unrolled_where_the_factor_divides_them(generator):
+    """Several paths per block: 1 to 9 batches of four steps."""
+    import re
+    for batches in range(1, 10):
+        irreps = natural(16 * batches - 3, 1)
+        g = generator(common.fully_connected((irreps, natural(1, 1), irreps), shared=True, dtype=np.float32)[0])
+        body = g.forward_body()
+        assert set(re.findall(r"sg < (\d+);", body)) == {str(batches)}
+        assert set(re.findall(r"#pragma unroll (\d)\n *for \(int sg", body)) == {"1" if batches % 2 else "2"}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ["16_words", "copies_f64"])
 def test_wide_second_operands_on_the_gpu(cuda, case):
