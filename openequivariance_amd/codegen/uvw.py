@@ -60,6 +60,7 @@ class WPath:
     mv: int = 1                     # ... out of this many (the instruction's weights are [u][v][w])
     poff: int = 0                   # offset of this path's [u][w] slice in the dense dW partial rows
     gs: int = 4                     # forward K steps fetched at a time
+    no_multiple: int = 0            # forward K steps not to be a multiple of this where one step more avoids it (0: no matter)
 
     @property
     def mu(self) -> int:
@@ -71,7 +72,8 @@ class WPath:
 
     @property
     def SU(self) -> int:            # K steps over u (forward): blocks of 16 channels, 4 steps each (step s: channels 4 g + s)
-        return 4 * (self.mu // 16) + self.gs * _ceil(min(4, self.mu % 16), self.gs)
+        s = 4 * (self.mu // 16) + self.gs * _ceil(min(4, self.mu % 16), self.gs)
+        return s + 1 if self.no_multiple and s % self.no_multiple == 0 and s < 4 * _ceil(self.mu, 16) else s
 
     @property
     def SW(self) -> int:            # K steps over w (backward dX)
@@ -96,6 +98,10 @@ class UVWGenerator:
     # 0.329 -> 0.376 ms, fp64 0.566 -> 0.694 ms - the CG part of a tile is then computed once per range.)
     FWD_ACC_LIMIT = 80
     FWD_PIPELINE = {4: (4, 2), 8: (1, 3)}
+    # Steps of an fp64 path (one a batch, unrolled three times) that are a multiple of three cost more than another one: per
+    # step and 100 000 rows 13 us with 20 or 19 of them, 18 us with 18.  66 channels l <= 1, 18 / 20 / 19 steps 316 / 267 /
+    # 259 us; 114 channels l <= 2, 30 / 32 / 31 steps 1067 / 910 / 891; 33 channels l <= 2, 9 / 12 / 10 steps 354 / 429 / 305
+    FWD_NO_MULTIPLE = {4: 0, 8: 3}
     BWD_LDS_LIMIT = 80 * 1024    # dZ tile of the backward: two workgroups per compute unit (gfx950: 160 KB)
 
     def __init__(self, problem: TPProblem):
@@ -142,7 +148,7 @@ class UVWGenerator:
             for v in range(b.mul):
                 bv = Block(b.idx, 1, b.l, b.off + v * b.D)
                 p = WPath(len(self.paths), a, bv, o, ins.path_weight, woff, v=v, mv=b.mul, poff=woff + v * a.mul * o.mul,
-                          gs=self.fwd_group)
+                          gs=self.fwd_group, no_multiple=self.FWD_NO_MULTIPLE[self.itemsize])
                 for i, j, k in np.argwhere(np.abs(c) > 1e-14):
                     p.pairs.setdefault((int(i), int(j)), []).append((int(k), float(c[i, j, k])))
                 self.paths.append(p)

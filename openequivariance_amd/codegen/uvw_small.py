@@ -30,6 +30,7 @@ class UVWSmallGenerator(UVWGenerator):
     BWD_LDS_LIMIT = 144 * 1024   # the dZ tile may fill a compute unit: there is one workgroup for each at most
     LDS_BYTES = 160 * 1024       # of a compute unit: what a kernel's arrays together may take (see lds_bytes)
     FWD_PIPELINE = {4: (4, 2), 8: (1, 4)}
+    FWD_NO_MULTIPLE = {4: 0, 8: 0}
     DW_WAVES = 16
     DW_REGISTERS = 88            # of 128 a lane has with 16 wavefronts: accumulators, operands and one T of a dW unit
 

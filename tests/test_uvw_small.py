@@ -90,6 +90,30 @@ def test_fp32_forward_loops_are_unrolled_where_the_factor_divides_them(generator
         assert set(re.findall(r"#pragma unroll (\d)\n *for \(int sg", body)) == {"1" if batches % 2 else "2"}
 
 
+def test_fp64_forward_steps():
+    """Every channel has a step, none is a whole block beyond the last, and three divides their number only where no step
+    past the last channel is left to take."""
+    for mu in range(1, 130):
+        ir = f"{mu}x0e"
+        p = UVWGenerator(common.fully_connected((ir, "1x0e", "20x0e"), shared=True, dtype=np.float64)[0]).paths[0]
+        full = 4 * -(-mu // 16)
+        need = 4 * (mu // 16) + min(4, mu % 16)
+        assert p.SU == (need + 1 if need % 3 == 0 and need < full else need) <= full
+        assert p.SU % 3 or p.SU == full
+        s = UVWSmallGenerator(common.fully_connected((ir, "1x0e", "20x0e"), shared=True, dtype=np.float64)[0]).paths[0]
+        assert s.SU == need
+
+
+def test_emulated_step_past_the_last_channel():
+    prob, oprob = common.fully_connected(("18x0e+33x1o", "1x0e+1x1o", "5x0e+3x1o"), shared=True, dtype=np.float64)
+    g = UVWGenerator(prob)
+    assert {p.SU for p in g.paths} == {7, 10}
+    X, Y, We, _ = common.tp_inputs(prob, 19, 9, np.float64, w_scale=0.3)
+    fwd, _, ws = g.plan()
+    out = emu.run_tp(g, fwd, X, Y, ow.e3nn_to_oeq(oprob, We), ws_bytes=ws())
+    assert rel(out["Z"], otp.forward(oprob, X, Y, We)) < TOL[np.float64]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ["16_words", "copies_f64"])
 def test_wide_second_operands_on_the_gpu(cuda, case):
