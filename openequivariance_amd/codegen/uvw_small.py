@@ -69,16 +69,31 @@ class UVWSmallGenerator(UVWGenerator):
             pos += ch * p.mu * self._width(p, lo, hi)
         assert pos <= self.ws_elems, "the partial rows of few workgroups per path outgrow those of all paths"
 
-    @staticmethod
-    def row_limits(g: UVWGenerator):
-        """Largest batch (forward, backward) these kernels take from ``g``'s.  Forward, 64 channels: fp32 8192 rows 50 -> 42
-        us, 65 536 rows 194 -> 234; fp64 2000 rows 47 -> 34, 4097 rows 50 -> 53.  Backward, where a block is read by several
-        paths, each of which fetches it here (64 channels, 3.9 times): 4097 rows 73 -> 60 us in fp32 and 118 -> 104 in fp64, 8192
-        rows 81 -> 84 and 131 -> 149; where every block has one path (50 channels) 65 536 rows still gain, 512 -> 459
-        and 803 -> 619."""
+    @classmethod
+    def row_limits(cls, g: UVWGenerator):
+        """Largest batch (forward, backward) these kernels take from ``g``'s.
+
+        Forward: none where the longest work item is not cut here (fp64, 500 rows: 97 -> 13 channels l <= 2 25 against 32 us, 100
+        -> 30 channels 43 / 48, 32 channels 15 / 17).  fp64 otherwise 64 channels 2000 rows 47 -> 34, 4097 rows 50 -> 53.  fp32
+        where that item is halved: 64 channels 8192 rows 50 -> 42 us, 65 536 rows 194 -> 234; where it loses less, the further
+        wavefronts cost as much from the size on at which they no longer have a SIMD each: 4096 / 5120 rows, 100 channels l <=
+        1 21 -> 19 / 22 -> 26, 128 channels l <= 2 48 -> 42 / 50 -> 59.  Up to 16 channels likewise, a path is one batch of K
+        steps with as much work around it, which every cut item repeats: 16 -> 100 channels 4096 / 8192 rows 19 -> 18 / 27 -> 29.
+
+        Backward, where a block is read by several paths, each of which fetches it here (64 channels, 3.9 times): 4097 rows 73
+        -> 60 us in fp32 and 118 -> 104 in fp64, 8192 rows 81 -> 84 and 131 -> 149; where every block has one path (50
+        channels) 65 536 rows still gain, 512 -> 459 and 803 -> 619."""
+        own = cls(g.problem)
+        longest = lambda h: max((hi - lo) * sum(p.o.D * p.SU for p in h.paths_into(o.idx)) for o, lo, hi in h.fwd_order)
+        if g.fwd_order[0] in own.fwd_order:
+            forward = 0
+        elif g.itemsize == 8:
+            forward = 2048
+        else:
+            forward = 8192 if longest(own) <= 0.6 * longest(g) and max(p.mu for p in g.paths) > 16 else 4096
         fetched = sum(p.a.dim + p.o.dim for p in g.paths)
         once = sum(g.in1[a].dim for a in g.used_in1) + sum(g.out[o].dim for o in g.used_out)
-        return (8192 if g.itemsize == 4 else 2048), (65536 if fetched <= 1.25 * once else 5120)
+        return forward, (65536 if fetched <= 1.25 * once else 5120)
 
     @staticmethod
     def _width(p, lo, hi) -> int:

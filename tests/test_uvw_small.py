@@ -90,6 +90,20 @@ def test_fp32_forward_loops_are_unrolled_where_the_factor_divides_them(generator
         assert set(re.findall(r"#pragma unroll (\d)\n *for \(int sg", body)) == {"1" if batches % 2 else "2"}
 
 
+def test_largest_batches():
+    """The forward is left to the kernels for large batches where the longest work item stays whole, and earlier where it
+    is not halved."""
+    def limits(a, b, dtype, in2=natural(1, 2)):
+        return UVWSmallGenerator.row_limits(UVWGenerator(common.fully_connected((natural(a, 2), in2, natural(b, 2)), shared=True, dtype=dtype)[0]))
+    for dtype, most in ((np.float32, 8192), (np.float64, 2048)):
+        assert limits(64, 64, dtype) == limits(50, 50, dtype) == (most, 5120)
+        assert limits(50, 50, dtype, "1x0e") == (most, 65536)
+        for a, b in ((97, 13), (32, 32), (100, 30)):
+            assert limits(a, b, dtype) == (0, 5120)
+        assert limits(32, 100, dtype) == limits(68, 68, dtype, natural(1, 1)) == (most, 5120)
+        assert limits(16, 100, dtype) == limits(36, 36, dtype) == limits(128, 128, dtype, natural(1, 1)) == (min(most, 4096), 5120)
+
+
 def test_fp64_forward_steps():
     """Every channel has a step, none is a whole block beyond the last, and three divides their number only where no step
     past the last channel is left to take."""
