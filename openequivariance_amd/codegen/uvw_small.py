@@ -45,6 +45,8 @@ class UVWSmallGenerator(UVWGenerator):
             for a in sorted(cost, key=lambda k: -cost[k]):
                 min(groups, key=lambda m: sum(cost[k] for k in m)).append(a)
             self.bwd_groups = [sorted(m) for m in groups]
+            loads = [sum(cost[a] for a in m) for m in self.bwd_groups]
+            self.balance = sum(loads) / len(loads) / max(loads)
         # dW units: (path, first w tile, end w tile, wavefronts along u)
         self.units = []
         for p in self.paths:
@@ -81,8 +83,21 @@ class UVWSmallGenerator(UVWGenerator):
         steps with as much work around it, which every cut item repeats: 16 -> 100 channels 4096 / 8192 rows 19 -> 18 / 27 -> 29.
 
         Backward, where a block is read by several paths, each of which fetches it here (64 channels, 3.9 times): 4097 rows 73
-        -> 60 us in fp32 and 118 -> 104 in fp64, 8192 rows 81 -> 84 and 131 -> 149; where every block has one path (50
-        channels) 65 536 rows still gain, 512 -> 459 and 803 -> 619."""
+        -> 60 us in fp32 and 118 -> 104 in fp64, 8192 rows 81 -> 84 and 131 -> 149.  Where every block has one path it depends
+        on how evenly the blocks load the groups of wavefronts (their balance: mean over largest load), for a full chip waits
+        for the slowest.  fp32, second operand 1x0e, general / these kernels, us:
+
+            channels, blocks            balance     8192      20 480      65 536 rows
+            64, l <= 1                    0.67     34 / 32    52 / 49    108 / 95
+            50, both parities, l <= 2     0.85     76 / 65   147 / 129   512 / 458
+            20 -> 64, l <= 2              0.60     41 / 33    64 / 54    153 / 127     (general: two wavefronts of four)
+            64, l <= 2                    0.60     48 / 46    79 / 84    223 / 261
+            80, l <= 2                    0.60     66 / 62   113 / 124   327 / 385
+            64, l <= 3                    0.57     67 / 71   122 / 139   371 / 453     (5120 rows 59 / 58)
+
+        fp64, where the general kernel holds one wavefront per SIMD: 50 channels of both parities 65 536 rows 802 / 620, 80
+        channels l <= 2 960 / 685; only where that kernel's four wavefronts have whole tiles and these are uneven 64 channels
+        l <= 2 (0.90) 16 384 rows 109 / 111, 65 536 rows 433 / 464, against 64 channels l <= 3 (1.00) 964 / 810."""
         own = cls(g.problem)
         longest = lambda h: max((hi - lo) * sum(p.o.D * p.SU for p in h.paths_into(o.idx)) for o, lo, hi in h.fwd_order)
         if g.fwd_order[0] in own.fwd_order:
@@ -93,7 +108,14 @@ class UVWSmallGenerator(UVWGenerator):
             forward = 8192 if longest(own) <= 0.6 * longest(g) and max(p.mu for p in g.paths) > 16 else 4096
         fetched = sum(p.a.dim + p.o.dim for p in g.paths)
         once = sum(g.in1[a].dim for a in g.used_in1) + sum(g.out[o].dim for o in g.used_out)
-        return forward, (65536 if fetched <= 1.25 * once else 5120)
+        muls = [g.in1[a].mul for a in g.used_in1]
+        if fetched > 1.25 * once or not own.bwd_lds:
+            backward = 5120
+        elif g.itemsize == 8:
+            backward = 16384 if own.balance < 1 and all(m % 64 == 0 for m in muls) else 65536
+        else:
+            backward = 65536 if own.balance >= 0.65 or max(muls) <= 48 else 8192 if own.balance >= 0.595 else 5120
+        return forward, backward
 
     @staticmethod
     def _width(p, lo, hi) -> int:

@@ -92,16 +92,25 @@ def test_fp32_forward_loops_are_unrolled_where_the_factor_divides_them(generator
 
 def test_largest_batches():
     """The forward is left to the kernels for large batches where the longest work item stays whole, and earlier where it
-    is not halved."""
+    is not halved; the backward where several wavefronts of a large batch would wait for one."""
     def limits(a, b, dtype, in2=natural(1, 2)):
         return UVWSmallGenerator.row_limits(UVWGenerator(common.fully_connected((natural(a, 2), in2, natural(b, 2)), shared=True, dtype=dtype)[0]))
     for dtype, most in ((np.float32, 8192), (np.float64, 2048)):
         assert limits(64, 64, dtype) == limits(50, 50, dtype) == (most, 5120)
-        assert limits(50, 50, dtype, "1x0e") == (most, 65536)
+        assert limits(50, 50, dtype, "1x0e") == (most, 8192 if dtype == np.float32 else 65536)
         for a, b in ((97, 13), (32, 32), (100, 30)):
             assert limits(a, b, dtype) == (0, 5120)
         assert limits(32, 100, dtype) == limits(68, 68, dtype, natural(1, 1)) == (most, 5120)
         assert limits(16, 100, dtype) == limits(36, 36, dtype) == limits(128, 128, dtype, natural(1, 1)) == (min(most, 4096), 5120)
+
+
+@pytest.mark.parametrize("irreps,fp32,fp64", [
+    (natural(64, 1), 65536, 16384), (BOTH[0], 65536, 65536), (natural(33, 2), 65536, 65536), (natural(80, 2), 8192, 65536),
+    (natural(64, 2), 8192, 16384), (natural(64, 3), 5120, 65536)])
+def test_largest_batches_of_one_path_per_block(irreps, fp32, fp64):
+    for dtype, limit in ((np.float32, fp32), (np.float64, fp64)):
+        prob, _ = common.fully_connected((irreps, "1x0e", irreps), shared=True, dtype=dtype)
+        assert UVWSmallGenerator.row_limits(UVWGenerator(prob))[1] == limit
 
 
 def test_fp64_forward_steps():
