@@ -232,7 +232,7 @@ def test_empty_edge_list_and_other_graph_sizes(cuda, deterministic):
 
 @pytest.mark.gpu
 def test_capture_before_first_use_composes(cuda):
-    """A stream capture does not load code objects: the second derivatives recorded before the fused kernels exist come
+    """The first use takes its workspace, which a stream capture does not: the second derivatives recorded before it come
     from the first-order ones, recorded afterwards from the fused ones; every replay gives the eager numbers."""
     import torch
     prob, _ = common.channelwise(common.NEQUIP)

@@ -65,12 +65,17 @@ def _reference(oprob, X, Y, We, G, A, B, Ve):
     return [t.numpy() for t in torch.autograd.grad(first, (x, y, w, g), [torch.tensor(a.astype(np.float64)) for a in (A, B, Ve)])]
 
 
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_generated_source_without_vector_stores(case, monkeypatch):
+    test_generated_source(case, None, monkeypatch, vector_stores=False)
+
+
 @pytest.mark.parametrize("ahead", [False, True])
 @pytest.mark.parametrize("case", sorted(CASES))
-def test_generated_source(case, ahead, monkeypatch):
+def test_generated_source(case, ahead, monkeypatch, vector_stores=True):
     prob, oprob = _problems(case)
     monkeypatch.setattr(UVUDoubleGenerator, "ONE_BLOCK_AHEAD", ahead)
-    g = UVUDoubleGenerator(prob)
+    g = UVUDoubleGenerator(prob, vector_stores=vector_stores)
     exe = emu.build(g.render(prelude=emu.emu_prelude(g.T)), MAIN)
     for n in CASES[case][1]:
         X, Y, We, G, A, B, Ve = _inputs(prob, n, 5, np.float32)
@@ -118,8 +123,8 @@ def test_operator(cuda, case, dtype):
 
 @pytest.mark.gpu
 def test_loss_on_one_of_the_gradients_and_misaligned_operands(cuda):
-    """Forces usually come from dY alone: the other two cotangents do not exist.  A dZ at an odd storage offset takes
-    the kernels without 16-byte stores only where its own gradient needs it."""
+    """Forces usually come from dY alone: the other two cotangents do not exist.  A dZ at an odd storage offset changes
+    nothing: the operator's outputs, which 16-byte stores go to, are its own."""
     import torch
     prob, oprob = common.channelwise(common.NEQUIP)
     tp = oeq.TensorProduct(prob, torch_op=True)
@@ -132,3 +137,24 @@ def test_loss_on_one_of_the_gradients_and_misaligned_operands(cuda):
     for a, b in zip(got, ref):
         if a is not None and np.abs(b).max() > 0:
             assert rel_err(a.cpu().numpy(), b) <= 2e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_misaligned_outputs(cuda, dtype):
+    """Raw outputs that are not 16-byte aligned take the kernels without 16-byte stores; nothing beside them is written."""
+    import torch
+    prob, oprob = common.channelwise(common.NEQUIP, dtype)
+    tp = oeq.TensorProduct(prob, torch_op=False)
+    X, Y, W, G, A, B, V = _inputs(prob, 41, 8, dtype)
+    ops = [torch.tensor(a, device=cuda) for a in (X, Y, W, G, A, B, V)]
+    for offset in (0, 1):
+        pads = [torch.full((t.numel() + 8,), 7.0, dtype=t.dtype, device=cuda) for t in ops[:4]]
+        outs = [p[offset:offset + t.numel()].view(t.shape) for p, t in zip(pads, ops)]
+        tp.double_backward_raw(41, *(t.data_ptr() for t in (*ops, *outs)))
+        torch.cuda.synchronize()
+        assert (offset == 0) in tp._double
+        for p, t in zip(pads, ops):
+            assert bool((p[:offset] == 7).all()) and bool((p[offset + t.numel():] == 7).all())
+        for a, b in zip(outs, _reference(oprob, X, Y, W, G, A, B, V)):
+            assert rel_err(a.cpu().numpy(), b) <= (2e-5 if dtype == np.float32 else 2e-12)

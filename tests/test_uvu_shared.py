@@ -51,6 +51,20 @@ def test_generated_source(case, monkeypatch):
             assert rel_err(got, ref) < 2e-6      # fp32 sums of at most 130 rows x 7 words against fp64
 
 
+@pytest.mark.parametrize("case", ["sixteen_rows", "two_ragged_chunks"])
+def test_generated_source_without_vector_stores(case):
+    prob, oprob = _problems(case)
+    g = UVUSharedGenerator(prob, vector_stores=False)
+    fwd, bwd, ws = g.plan()
+    n = CASES[case][3][-1]
+    X, Y, We, G = common.tp_inputs(prob, n, 19)
+    W = ow.e3nn_to_oeq(oprob, We)
+    assert rel_err(emu.run_tp(g, fwd, X, Y, W, ws_bytes=ws())["Z"], otp.forward(oprob, X, Y, We)) < 2e-6
+    out = emu.run_tp(g, bwd, X, Y, W, G, ws_bytes=ws())
+    for got, ref in zip((out["Xg"], out["Yg"], ow.oeq_to_e3nn(oprob, out["Wg"])), otp.backward(oprob, X, Y, We, G)):
+        assert rel_err(got, ref) < 2e-6
+
+
 # wide second operands beside the sixteen or eight wavefronts of a row: (dtype, in1 = out, in2, taken)
 WIDE = {
     "144_words": (np.float64, "1024x0e+1024x1o", "+".join(f"1x{l}e" for l in range(12)), True),
@@ -93,3 +107,23 @@ def test_operator(cuda, case, dtype):
         for got, ref in ((z.detach(), otp.forward(oprob, X, Y, We)), (x.grad, dX), (y.grad, dY)):
             assert rel_err(got.cpu().numpy(), ref) <= tol
         assert rel_err(ow.oeq_to_e3nn(oprob, w.grad.cpu().numpy()), dW) <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_misaligned_operands(cuda, dtype):
+    """Operands at an odd storage offset take the kernels without 16-byte stores."""
+    import torch
+    prob, oprob = _problems("two_ragged_chunks", dtype)
+    tol = FP32_TOL if dtype == np.float32 else FP64_TOL
+    tp = oeq.TensorProduct(prob, torch_op=True)
+    X, Y, We, G = common.tp_inputs(prob, 301, 20, dtype)
+    odd = lambda a: torch.zeros(a.size + 1, dtype=torch.tensor(a).dtype, device=cuda)[1:].view(a.shape).copy_(torch.tensor(a))
+    x, y, w, g = (odd(a) for a in (X, Y, ow.e3nn_to_oeq(oprob, We), G))
+    got = [tp.forward(x, y, w), *tp.backward_helper(x, y, w, g)]
+    torch.cuda.synchronize()
+    assert tp._internal_unaligned is not None
+    got = [t.cpu().numpy() for t in got]
+    got[3] = ow.oeq_to_e3nn(oprob, got[3])
+    for a, b in zip(got, (otp.forward(oprob, X, Y, We), *otp.backward(oprob, X, Y, We, G))):
+        assert rel_err(a, b) <= tol
