@@ -12,7 +12,10 @@ threads each added 1024 partial rows one after the other, + 71 us forward); this
 
 Multiplicities above 64 take one wavefront per 64-channel chunk of a row, all in one workgroup, which adds the chunks'
 dY through LDS once per tile of rows.  Problems with a run-time loop over the copies of the second operand (more than 8)
-keep the schedule of ``uvu.py``: their dW sums do not fit registers.
+keep the schedule of ``uvu.py``: their dW sums do not fit registers.  The row's own X, dZ and dX come on top of what the
+rule counts, so long rows spill: 128 channels l <= 4, 42 paths, 2.7 KB per lane, 256 channels l <= 3 in fp64 1.4 KB.  The
+staged schedule spills more there and is slower at every size tried: backward of 19 531 rows 15.5 -> 4.5 ms, of 15 258
+rows 14.8 -> 3.3 ms.
 """
 from __future__ import annotations
 
@@ -32,7 +35,8 @@ class UVUSharedGenerator(UVUDirectGenerator):
 
     @classmethod
     def suits(cls, problem: TPProblem) -> bool:
-        """dW sums and weights of a channel fit the registers, and a row's chunks one workgroup and its LDS."""
+        """A channel's dW sums and weights leave room in the registers (a long row may spill beside them, which still is the
+        faster schedule), and a row's chunks fit one workgroup and its LDS."""
         muls = [problem.irreps_in2[i.i_in2].mul for i in problem.instructions]
         words = 2 * sum(muls) * (2 if problem.irrep_dtype().itemsize == 8 else 1)
         widest = max(mul for mul, _ in list(problem.irreps_in1) + list(problem.irreps_out))

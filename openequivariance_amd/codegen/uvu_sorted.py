@@ -62,10 +62,11 @@ class UVUSortedGenerator:
             if recv_backward is not False and (recv_backward or self.fwd.D3 >= self.RECV_ORDER_MIN_RATIO * self.fwd.D1):
                 # long dZ rows: the two-pass backward in receiver order (pass 1 over the receiver grouping, which the
                 # backward then builds as well; pass 2 over the sender grouping), where pass 1 can stage its operands
-                # (fp32).  In fp64 pass 1, one launch per in1 block, runs over the position list as well and is taken on
-                # request only: it keeps a dX row per edge in the workspace (2.8 GB), which the sender order does not.
-                # The MACE problem, 10 000 nodes / 300 000 edges, forward + backward, both staged: 6.86 ms in sender
-                # order, 6.12 ms in receiver order; 32 channels, 5000 nodes / 150 000 edges 1.10 / 1.04 ms
+                # (fp32).  In fp64 pass 1, one launch per in1 block, runs over the position list as well but is taken on
+                # request only.  That default dates from register loads, when the second counting sort cost what the order
+                # gains (backward 5.16 / 5.32 ms); with both orders staged the receiver order is the faster one, for a dX row
+                # per edge in the workspace (2.8 GB): the MACE problem, 10 000 nodes / 300 000 edges, forward + backward
+                # 6.86 ms in sender order, 6.12 ms in receiver order; 32 channels, 5000 nodes / 150 000 edges 1.10 / 1.04 ms
                 recv = UVURecvGenerator(problem, vector_stores=vector_stores, idx_ctype=idx_ctype, backward_perm=True)
                 if recv_backward is True or recv.staged_edges:
                     self.bwd, self.recv_backward = recv, True

@@ -188,7 +188,7 @@ class TensorProductConv:
         self.backward_needs_tperm = deterministic
         self.jit_kernel = self.generator.render()
         self._ws_fns = []
-        self._ws_last = (None, 0)          # (sizes, bytes) of the last workspace query
+        self._ws_last = self._double_ws_last = (None, 0)          # (sizes, bytes) of the last workspace query
         self.internal = self._build(self.generator, self.jit_kernel)
         self._workspaces: typing.Dict[tuple, _StreamWorkspace] = {}      # (device, stream) -> scratch
         # Unsorted edge lists: whether the backward scatters dX with float atomics or groups the edges by
@@ -267,8 +267,11 @@ class TensorProductConv:
         return impl, ws
 
     def _double_ws_bytes(self, nnz: int, node_count: int) -> int:
-        self._double_impl()
-        return self._double_built[1](nnz, node_count)
+        last = self._double_ws_last
+        if last[0] != (nnz, node_count):
+            self._double_impl()
+            last = self._double_ws_last = ((nnz, node_count), self._double_built[1](nnz, node_count))
+        return last[1]
 
     def _double_impl(self) -> "rt.ConvImpl":
         if self._double is None:

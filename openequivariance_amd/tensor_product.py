@@ -202,11 +202,11 @@ class TensorProduct(TensorProductBase):
 
         def build():
             g = UVWSmallGenerator.create(self.config)
-            return (None, None) if g is None else (g.render(), g.plan()[:2])
-        impl, _ = rt.variant(("uvw few rows", self.config.signature()), torch.cuda.current_device(), build,
-                             lambda code, plan: rt.TPImpl(code, *(_make_steps(steps, self._step_flags) for steps in plan)))
+            return (None, None) if g is None else (g.render(), (*g.plan()[:2], UVWSmallGenerator.row_limits(self.generator)))
+        impl, plan = rt.variant(("uvw few rows", self.config.signature()), torch.cuda.current_device(), build,
+                                lambda code, plan: rt.TPImpl(code, *(_make_steps(steps, self._step_flags) for steps in plan[:2])))
         # (None: a problem whose units do not fit their registers or LDS)
-        return none if impl is None else (impl, UVWSmallGenerator.row_limits(self.generator))
+        return none if impl is None else (impl, plan[2])
 
     def _double_kernels(self, aligned: bool) -> "rt.TPImpl":
         def build():
