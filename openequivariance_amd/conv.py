@@ -232,10 +232,10 @@ class TensorProductConv:
         return impl
 
     def _ws_bytes(self, nnz: int, node_count: int) -> int:
-        key = (nnz, node_count, len(self._ws_fns))
-        if key != self._ws_last[0]:
-            self._ws_last = (key, max(f(nnz, node_count) for f in self._ws_fns))
-        return self._ws_last[1]
+        key, last = (nnz, node_count, len(self._ws_fns)), self._ws_last       # (read once: other threads ask for other sizes)
+        if key != last[0]:
+            last = self._ws_last = (key, max(f(nnz, node_count) for f in self._ws_fns))
+        return last[1]
 
     def _backward_variant(self, name: str):
         """(kernel set, whether its backward overwrites dX) of a backward variant of the unsorted operator,

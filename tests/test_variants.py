@@ -77,3 +77,22 @@ def test_no_call_waits_for_the_compiler(case, monkeypatch):
         before = op._ws_bytes(5000, 300)
         assert op._double_usable() and op._double_impl().code and op._double_impl() is op._double
         assert op._double_ws_bytes(5000, 300) > 0 and op._ws_bytes(5000, 300) == before
+
+
+def test_workspace_sizes_asked_for_by_several_threads(monkeypatch):
+    """Another thread's question in the middle of one does not change its answer."""
+    class Conv(oeq.TensorProductConv):
+        """Every read of the last answer comes after another thread has asked for a small graph."""
+        def __init__(self):
+            self._ws_fns, self._double_built = [lambda nnz, nodes: 8 * nnz], (None, lambda nnz, nodes: 16 * nnz)
+
+        def _double_impl(self):
+            pass
+    for name, factor in (("_ws_last", 8), ("_double_ws_last", 16)):
+        def get(self, name=name, factor=factor):
+            return ((1, 1) if name == "_double_ws_last" else (1, 1, 1)), factor
+        setattr(Conv, name, property(get, lambda self, v: None))
+    conv = Conv()
+    for nnz in (1000, 1000, 7):
+        assert conv._ws_bytes(nnz, 5) == 8 * nnz
+        assert conv._double_ws_bytes(nnz, 5) == 16 * nnz
