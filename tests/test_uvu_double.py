@@ -158,3 +158,35 @@ def test_misaligned_outputs(cuda, dtype):
             assert bool((p[:offset] == 7).all()) and bool((p[offset + t.numel():] == 7).all())
         for a, b in zip(outs, _reference(oprob, X, Y, W, G, A, B, V)):
             assert rel_err(a.cpu().numpy(), b) <= (2e-5 if dtype == np.float32 else 2e-12)
+
+
+@pytest.mark.gpu
+def test_capture_before_the_first_call(cuda):
+    """The kernels are loaded with the operator: a stream capture records them without an eager call before it."""
+    import torch
+    prob, oprob = common.channelwise(common.NEQUIP)
+    X, Y, W, G, A, B, V = _inputs(prob, 70, 9, np.float32)
+    x, y, w, g = (torch.tensor(a, device=cuda, requires_grad=True) for a in (X, Y, W, G))
+    cots = [torch.tensor(a, device=cuda) for a in (A, B, V)]
+
+    def step(tp):
+        first = torch.autograd.grad(tp(x, y, w), (x, y, w), g, create_graph=True)
+        return torch.autograd.grad(first, (x, y, w, g), cots)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        eager = step(oeq.TensorProduct(prob, torch_op=True))             # (torch's own first use, by another operator)
+    side.synchronize()
+    tp = oeq.TensorProduct(prob, torch_op=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = step(tp)
+    for _ in range(3):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, eager))
+        assert all(torch.equal(a, b) for a, b in zip(step(tp), eager))
+    for a, b in zip(out, _reference(oprob, X, Y, W, G, A, B, V)):
+        assert rel_err(a.cpu().numpy(), b) <= 2e-5
