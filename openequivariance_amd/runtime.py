@@ -207,16 +207,19 @@ def variant(key: tuple, device: int, build, load):
     ``key`` is everything they depend on.  A source of None: there is no such kernel set, and no handle."""
     with _variants_lock:
         got = _VARIANTS.get(key)
-        if got is None:
-            source, plan = build()
-            got = _VARIANTS[key] = (None if source is None else compile_source(source), plan)
+        if got is not None:
+            _VARIANTS.move_to_end(key)
+    if got is None:                  # (without the lock: other problems' operators need not wait for this compilation)
+        source, plan = build()
+        code = None if source is None else compile_source(source)
+        with _variants_lock:
+            got = _VARIANTS.setdefault(key, (code, plan))
             if len(_VARIANTS) > _VARIANTS_MAX:
                 _VARIANTS.popitem(last=False)
-        else:
-            _VARIANTS.move_to_end(key)
-        code, plan = got
-        if code is None:
-            return None, plan
+    code, plan = got
+    if code is None:
+        return None, plan
+    with _variants_lock:
         handle = _LOADED.get((key, device))
         if handle is None:
             handle = _LOADED[(key, device)] = load(code, plan)

@@ -37,6 +37,31 @@ def test_shared_while_held(monkeypatch):
         del rt._VARIANTS[key]
 
 
+def test_no_thread_waits_for_another_problems_compilation(monkeypatch):
+    import threading
+    entered, release, got = threading.Event(), threading.Event(), []
+
+    def compile_source(source):
+        if source == "slow":
+            entered.set()
+            assert release.wait(30)
+        return source.encode()
+    monkeypatch.setattr(rt, "compile_source", compile_source)
+    monkeypatch.setattr(rt, "_VARIANTS", type(rt._VARIANTS)())
+    get = lambda source: got.append(rt.variant((source,), 0, lambda: (source, None), Handle)[0])
+    slow = threading.Thread(target=get, args=("slow",))
+    slow.start()
+    assert entered.wait(30)
+    quick = threading.Thread(target=get, args=("quick",))
+    quick.start()
+    quick.join(10)
+    waited = quick.is_alive()
+    release.set()
+    slow.join(30)
+    quick.join(30)
+    assert not waited and [h.code for h in got] == [b"quick", b"slow"]
+
+
 class Impl:
     def __init__(self, code, *steps):
         self.code = code
