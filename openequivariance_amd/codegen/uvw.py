@@ -336,28 +336,39 @@ class UVWGenerator:
         E("const int q = blockIdx.x * 256 + threadIdx.x;")
         E("T* __restrict__ wsT = (T*)ws;")
         for p in self.paths:
-            nb = p.SU * 64 * p.NTW
-            E(f"if (q >= {p.wb} && q < {p.wb + nb}) {{   // forward copy of path {p.t}: [s][lane][nt]")
-            E(f"    const int e = q - {p.wb};")
-            E(f"    const int nt = e % {p.NTW}; const int ln = (e / {p.NTW}) & 63; const int s = e / {64 * p.NTW};")
-            E(f"    const int u = 16 * (s >> 2) + 4 * (ln >> 4) + (s & 3); const int w = {p.NTW} * (ln & 15) + nt;   // K order of forward_body")
-            E(f"    wsT[q] = (u < {p.mu} && w < {p.mw}) ? W[{self.oeq_index(p, 'u', 'w')}] : (T)0;")
-            E("}")
-            VW, SQ = self.VW, _ceil(p.SW, self.VW)
-            na = p.NTU * SQ * 64 * VW
-            E(f"if (q >= {p.wa} && q < {p.wa + na}) {{   // backward copy of path {p.t}: [mt][s / {VW}][lane][s % {VW}]")
-            E(f"    const int e = q - {p.wa};")
-            E(f"    const int ln = (e / {VW}) & 63; const int s = {VW} * ((e / {64 * VW}) % {SQ}) + e % {VW}; const int mt = e / {64 * VW * SQ};")
-            E(f"    const int u = 16 * mt + (ln & 15); const int w = 4 * s + (ln >> 4);")
-            E(f"    wsT[q] = (u < {p.mu} && w < {p.mw}) ? W[{self.oeq_index(p, 'u', 'w')}] : (T)0;")
-            E("}")
+            self._pack_forward_copy(E, p)
+            self._pack_backward_copy(E, p)
         return E.text()
+
+    def _pack_forward_copy(self, E: Emitter, p: WPath) -> None:
+        nb = p.SU * 64 * p.NTW
+        E(f"if (q >= {p.wb} && q < {p.wb + nb}) {{   // forward copy of path {p.t}: [s][lane][nt]")
+        E(f"    const int e = q - {p.wb};")
+        E(f"    const int nt = e % {p.NTW}; const int ln = (e / {p.NTW}) & 63; const int s = e / {64 * p.NTW};")
+        E(f"    const int u = 16 * (s >> 2) + 4 * (ln >> 4) + (s & 3); const int w = {p.NTW} * (ln & 15) + nt;   // K order of forward_body")
+        E(f"    wsT[q] = (u < {p.mu} && w < {p.mw}) ? W[{self.oeq_index(p, 'u', 'w')}] : (T)0;")
+        E("}")
+
+    def _pack_backward_copy(self, E: Emitter, p: WPath) -> None:
+        VW, SQ = self.VW, _ceil(p.SW, self.VW)
+        na = p.NTU * SQ * 64 * VW
+        E(f"if (q >= {p.wa} && q < {p.wa + na}) {{   // backward copy of path {p.t}: [mt][s / {VW}][lane][s % {VW}]")
+        E(f"    const int e = q - {p.wa};")
+        E(f"    const int ln = (e / {VW}) & 63; const int s = {VW} * ((e / {64 * VW}) % {SQ}) + e % {VW}; const int mt = e / {64 * VW * SQ};")
+        E(f"    const int u = 16 * mt + (ln & 15); const int w = 4 * s + (ln >> 4);")
+        E(f"    wsT[q] = (u < {p.mu} && w < {p.mw}) ? W[{self.oeq_index(p, 'u', 'w')}] : (T)0;")
+        E("}")
+
+    def prep_backward_body(self) -> str:
+        return self.prep_body()
 
     @property
     def prep_blocks(self) -> int:
         return _ceil(self.WA_END, 256)
 
     # =============================================================== forward
+    forward_threads = 64
+
     def k_unroll(self, batches: int) -> int:
         """Unroll factor of a forward K loop.  fp32: 1 where the factor does not divide the batches of four steps; 100 000
         rows, l <= 1, unrolled twice against not: 68 channels (5 batches) 168 / 147 us, 100 (7) 306 / 252, 112 (7) 266 /
@@ -783,6 +794,9 @@ class UVWGenerator:
             if cur:
                 passes.append((grp, cur))
         return passes
+
+    def dw_globals(self) -> str:
+        return ""
 
     def backward_dw_body(self) -> str:
         E = Emitter()

@@ -15,6 +15,7 @@ from .codegen.uvu_conv_double import conv_double_generator
 from .codegen.uvu_double import UVUDoubleGenerator
 from .codegen.uvw import UVWGenerator
 from .codegen.uvw_small import UVWSmallGenerator
+from .codegen.uvw_split import UVWSplitGenerator
 from .conv import select_conv_generator
 from .problem import ChannelwiseTPP, FullyConnectedTPProblem, TPProblem
 from .tensor_product import select_generator
@@ -31,7 +32,7 @@ def benchmark_generators():
     def tp(label, problem):
         g = select_generator(problem)
         gens.append((label, g))
-        if type(g) is UVWGenerator:
+        if type(g) in (UVWGenerator, UVWSplitGenerator):
             few = UVWSmallGenerator.create(problem)
             if few is not None:
                 gens.append((label + " few rows", few))

@@ -22,6 +22,7 @@ from .codegen.uvu_direct import UVUDirectGenerator
 from .codegen.uvu_double import UVUDoubleGenerator
 from .codegen.uvw import UVWGenerator
 from .codegen.uvw_small import UVWSmallGenerator
+from .codegen.uvw_split import UVWSplitGenerator
 from .codegen.uvw_batched import UVWBatchedGenerator
 from .problem import TPProblem
 from .weight_order import WeightReorder
@@ -60,8 +61,9 @@ def _on_device(device):
 
 
 def select_generator(config: TPProblem):
-    """The kernel generator of a batch tensor product: MFMA kernels for uvw with shared weights (vector-ALU
-    kernels with a row per lane when the weights are few and the multiplicities small),
+    """The kernel generator of a batch tensor product: matrix-core kernels for uvw with shared weights (in fp32 on
+    operands split into three bf16 numbers, in the directions where that is the faster way; vector-ALU kernels with a row
+    per lane when the weights are few and the multiplicities small),
     streaming vector-ALU kernels for uvw with per-row weights, register-direct streaming kernels for uvu, with
     dW sums held in registers across rows when the weights are shared (dW partial rows in memory and LDS-staged
     loads where those sums do not fit)."""
@@ -69,7 +71,7 @@ def select_generator(config: TPProblem):
     if mode == "uvw" and config.shared_weights:
         from .codegen.uvw_rows import UVWRowsGenerator
         # a few hundred weights on multiplicities far below a 16 x 16 tile: one row per lane on the vector ALU
-        return UVWRowsGenerator(config) if UVWRowsGenerator.suits(config) else UVWGenerator(config)
+        return UVWRowsGenerator(config) if UVWRowsGenerator.suits(config) else UVWSplitGenerator.create(config) or UVWGenerator(config)
     if mode == "uvw":
         from .codegen.uvw_batched import UVWBatchedGenerator
         return UVWBatchedGenerator(config)
@@ -133,6 +135,8 @@ class TensorProduct(TensorProductBase):
         # dense uvw: kernels for few rows and their largest batch (forward, backward).  Built here like the double backward's,
         # not by the call that first needs them: that call would wait for the compiler, and a stream capture cannot
         self._few_rows, self._few_rows_limits = self._few_row_kernels()
+        # ... and what they keep of it where the generator's kernels on split operands are the faster ones on few rows too
+        self._few_rows_kept = getattr(self.generator, "few_rows", tuple)(self._few_rows_limits)
         # double backward in one launch: kernels by alignment of the outputs (misaligned ones are compiled on first need)
         self._double_generator = UVUDoubleGenerator if mode == "uvu" and UVUDoubleGenerator.suits(config) else None
         self._double = {}
@@ -191,13 +195,15 @@ class TensorProduct(TensorProductBase):
         return self.internal
 
     def _pick_rows(self, batch: int, backward: bool):
-        """The kernels for few rows where ``batch`` is one, else None."""
-        return self._few_rows if 0 < batch <= self._few_rows_limits[backward] else None
+        """The kernels for a batch of few rows, None where ``batch`` is not one."""
+        if not 0 < batch <= self._few_rows_limits[backward]:
+            return None
+        return self._few_rows if batch <= self._few_rows_kept[backward] else self.internal
 
     def _few_row_kernels(self):
         """(kernel set, limits) of the kernels for few rows of a dense uvw product."""
         none = None, (0, 0)
-        if type(self.generator) is not UVWGenerator:
+        if type(self.generator) not in (UVWGenerator, UVWSplitGenerator):
             return none
 
         def build():

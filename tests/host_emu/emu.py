@@ -57,13 +57,14 @@ static inline void oeq_sync() { pthread_barrier_wait(&g_wbar[threadIdx.x >> 6]);
 static inline T oeq_fma(T a, T b, T c) { return std::fma(a, b, c); }
 static inline void oeq_atomic_add(T* p, T v) { std::lock_guard<std::mutex> g(g_atomic_mutex); *p += v; }
 static inline T oeq_shfl_xor(T v, int mask) { g_xT[threadIdx.x] = v; oeq_sync(); T r = g_xT[threadIdx.x ^ mask]; oeq_sync(); return r; }
-static inline int oeq_shfl_i32(int v, int src) { g_xi[threadIdx.x] = v; oeq_sync(); int r = g_xi[src & 63]; oeq_sync(); return r; }
+static inline int oeq_shfl_i32(int v, int src) { g_xi[threadIdx.x] = v; oeq_sync(); int r = g_xi[(threadIdx.x & ~63) + (src & 63)]; oeq_sync(); return r; }
 static i64 g_xl[1024];
 static inline i64 oeq_shfl_up_i64(i64 v, int delta) { g_xl[threadIdx.x] = v; oeq_sync(); const int l = threadIdx.x & 63; i64 r = l >= delta ? g_xl[threadIdx.x - delta] : v; oeq_sync(); return r; }
 static inline int oeq_shfl_xor_i32(int v, int mask) { g_xi[threadIdx.x] = v; oeq_sync(); int r = g_xi[threadIdx.x ^ mask]; oeq_sync(); return r; }
 #define __builtin_amdgcn_readfirstlane(x) oeq_shfl_i32((x), 0)
 static inline u64 oeq_uniform_u64(u64 v) { return v; }
 struct VT { T v[16 / sizeof(T)]; T& operator[](int i) { return v[i]; } const T& operator[](int i) const { return v[i]; } };
+static inline VT operator*(VT a, T b) { for (T& x : a.v) x *= b; return a; }
 typedef VT VTU;
 #define __builtin_nontemporal_store(v, p) (*(p) = (v))
 #define __builtin_nontemporal_load(p) (*(p))
@@ -111,6 +112,62 @@ static inline V4 oeq_mfma(T a, T b, V4 c) {
     pthread_barrier_wait(&g_wbar[wv]);
     return d;
 }
+// fp32 numbers split into three bf16 numbers, and matrix-core steps on them
+struct U4 { unsigned v[4]; unsigned& operator[](int i) { return v[i]; } const unsigned& operator[](int i) const { return v[i]; } };
+static inline unsigned emu_bf16(float x) {
+    unsigned u; memcpy(&u, &x, 4);
+    if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0u;
+    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+static inline float emu_f32(unsigned h) { h <<= 16; float x; memcpy(&x, &h, 4); return x; }
+static inline void oeq_split2(T a, T b, unsigned& h, unsigned& m, unsigned& l) {
+    const float x[2] = {(float)a, (float)b};
+    h = m = l = 0;
+    for (int q = 0; q < 2; ++q) {
+        const unsigned u = emu_bf16(x[q]); const float r = x[q] - emu_f32(u);
+        const unsigned v = emu_bf16(r);
+        h |= u << (16 * q); m |= v << (16 * q); l |= emu_bf16(r - emu_f32(v)) << (16 * q);
+    }
+}
+static inline void oeq_split8(const T* e, U4& h, U4& m, U4& l) {
+    for (int q = 0; q < 4; ++q) oeq_split2(e[2 * q], e[2 * q + 1], h[q], m[q], l[q]);
+}
+static inline float emu_elem(const U4& v, int j) { return emu_f32((v[j / 2] >> (16 * (j & 1))) & 0xffffu); }
+static U4 g_bA[16][64], g_bB[16][64];
+static inline V4 oeq_mfma_bf16(U4 a, U4 b, V4 c) {
+    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
+    g_bA[wv][l] = a; g_bB[wv][l] = b;
+    pthread_barrier_wait(&g_wbar[wv]);
+    V4 d = c;
+    for (int r = 0; r < 4; ++r) {
+        const int i = 4 * (l >> 4) + r, j = l & 15;
+        double acc = 0;
+        for (int k = 0; k < 32; ++k) acc += (double)emu_elem(g_bA[wv][16 * (k / 8) + i], k % 8) * emu_elem(g_bB[wv][16 * (k / 8) + j], k % 8);
+        d[r] = (T)(c[r] + acc);
+    }
+    pthread_barrier_wait(&g_wbar[wv]);
+    return d;
+}
+struct V16 { T v[16]; T& operator[](int i) { return v[i]; } const T& operator[](int i) const { return v[i]; } };
+static inline V16 oeq_mfma32_bf16(U4 a, U4 b, V16 c) {
+    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
+    g_bA[wv][l] = a; g_bB[wv][l] = b;
+    pthread_barrier_wait(&g_wbar[wv]);
+    V16 d = c;
+    for (int r = 0; r < 16; ++r) {
+        const int i = 8 * (r / 4) + 4 * (l >> 5) + r % 4, j = l & 31;
+        double acc = 0;
+        for (int k = 0; k < 16; ++k) acc += (double)emu_elem(g_bA[wv][32 * (k / 8) + i], k % 8) * emu_elem(g_bB[wv][32 * (k / 8) + j], k % 8);
+        d[r] = (T)(c[r] + acc);
+    }
+    pthread_barrier_wait(&g_wbar[wv]);
+    return d;
+}
+#define OEQ_PIN(x) ((void)0)
+#define __constant__ static const
+#define oeq_priority(p) ((void)0)
+static int g_any[1024];
+static inline bool oeq_any(bool v) { g_any[threadIdx.x] = v; oeq_sync(); int r = 0; for (int i = 0; i < 64; ++i) r |= g_any[(threadIdx.x & ~63) + i]; oeq_sync(); return r; }
 
 static void emu_run(unsigned gx, unsigned gy, unsigned block, const std::function<void()>& kernel) {
     gridDim = {gx, gy, 1}; blockDim = {block, 1, 1};

@@ -1,0 +1,126 @@
+"""Dense uvw products on operands split into three bf16 numbers: generated source on the host, choice of kernels, and (on the
+GPU) both against the fp64 oracle, with infinities and NaN among the operands too."""
+import re
+
+import numpy as np
+import pytest
+
+import common
+import openequivariance_amd as oeq
+from host_emu import emu
+from openequivariance_amd.codegen.uvw import UVWGenerator
+from openequivariance_amd.codegen.uvw_split import UVWSplitGenerator
+from oracle import tp as otp
+from oracle import weights as ow
+
+
+def natural(mul, lmax):
+    return "+".join(f"{mul}x{l}{'eo'[l % 2]}" for l in range(lmax + 1))
+
+
+def worst(got, ref):
+    """Largest error among the rows whose reference is finite, and whether finite values are where the reference has them."""
+    rows = np.isfinite(ref).reshape(ref.shape[0], -1).all(1)
+    return float(np.abs(got[rows] - ref[rows]).max() / np.abs(ref[rows]).max()), bool((np.isfinite(got) == np.isfinite(ref)).all())
+
+
+EMULATED = {
+    "whole rows through LDS, two tiles a workgroup": ("20x0e+24x1o", "1x0e+1x1o+1x2e", "36x0e+12x1o+5x1e+8x2e", 3, 37),
+    "records stored directly, odd channels": ("5x0e+21x1o", "1x0e+1x1o+1x2e", "18x0e+7x1o+3x2e", 3, 37),
+    "second operand in another order, a block no path reads, an output no path writes": ("33x0e+2x3o", "1x2e+1x0e", "34x0e+33x2e+4x1o", 2, 19),
+    "several tiles for a dW workgroup, two of its kinds": ("70x0e+20x1o", "1x0e+1x1o", "68x0e+16x1o", 2, 150),
+}
+
+
+@pytest.mark.parametrize("name", EMULATED)
+def test_generated_source(name, monkeypatch):
+    """Every direction forced onto the split kernels.  37, 19 and 150 rows: whole tiles and a ragged one.  The tolerance is that
+    of the fp32 kernels' emulation; the split itself holds 24 bits, the products left out are 2^-26 of the largest."""
+    a1, a2, a3, groups, n = EMULATED[name]
+    monkeypatch.setattr(UVWSplitGenerator, "DW_WORKGROUPS", groups)
+    monkeypatch.setattr(UVWSplitGenerator, "_pays", lambda *args: True)
+    prob, oprob = common.fully_connected((a1, a2, a3), shared=True, dtype=np.float32)
+    g = UVWSplitGenerator(prob)
+    assert g.split_forward and g.split_dx and g.dw_kinds and len(g.dw_kinds) <= groups
+    X, Y, We, G = common.tp_inputs(prob, n, 9, np.float32, w_scale=0.3)
+    W = ow.e3nn_to_oeq(oprob, We)
+    fwd, bwd, ws = g.plan()
+    for special in (False, True):
+        if special:                                          # the part of a wavefront that meets them is computed in fp32
+            X[3, 1], G[n - 2, 2] = np.inf, np.nan
+        with np.errstate(invalid="ignore"):
+            refs = (otp.forward(oprob, X, Y, We), *otp.backward(oprob, X, Y, We, G))
+        out = emu.run_tp(g, fwd, X, Y, W, ws_bytes=ws())
+        back = emu.run_tp(g, bwd, X, Y, W, G, ws_bytes=ws())
+        got = (out["Z"], back["Xg"], back["Yg"], ow.oeq_to_e3nn(oprob, back["Wg"])[:, None])
+        for value, ref in zip(got, (*refs[:3], refs[3][:, None])):
+            error, finite = worst(value, ref)
+            assert error < 2e-6 and finite
+
+
+def test_directions_and_rows():
+    """Which kernels serve a problem: padding and wavefronts without a tile decide per direction, other types take the fp32 or
+    fp64 kernels altogether, and the kernels for few rows keep only the backward's smallest batches."""
+    def made(a, b, in2=natural(1, 2), dtype=np.float32):
+        return UVWSplitGenerator.create(common.fully_connected((natural(a, 2), in2, natural(b, 2)), shared=True, dtype=dtype)[0])
+    g = made(64, 64)
+    assert g.split_forward and g.split_dx and len(g.dw_kinds) == 1 and g.few_rows((8192, 5120)) == (0, 2048)
+    g = made(20, 72)
+    assert g.split_forward and not g.split_dx and g.few_rows((8192, 5120)) == (0, 5120)
+    g = made(96, 9)
+    assert not g.split_forward and not g.split_dx
+    assert made(64, 64, dtype=np.float64) is None
+    for a, b in ((64, 64), (100, 100), (8, 100), (100, 8), (33, 50)):
+        g = made(a, b)
+        assert g.ws_elems >= UVWGenerator(g.problem).ws_elems
+        for kernel in g.render().split("__global__")[1:]:
+            arrays = re.findall(r"__shared__ (\w+) \w+\[([\d* +]+)\]", kernel)
+            assert sum({"T": 4, "VT": 16, "U4": 16}[t] * eval(size) for t, size in arrays) <= UVWSplitGenerator.LDS_BYTES
+
+
+GPU = {"64": (natural(64, 2), natural(1, 2), natural(64, 2)), "100": (natural(100, 2), natural(1, 1), natural(100, 1)),
+       "20 -> 72": (natural(20, 2), natural(1, 2), natural(72, 2)), "50, both parities": ("50x0e+50x1o+50x1e", "1x0e", "50x0e+50x1o+50x1e"),
+       "33 -> 47": (natural(33, 1), natural(1, 1), natural(47, 2)), "132": (natural(132, 1), "1x0e", natural(132, 1))}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", GPU)
+@pytest.mark.parametrize("n", [1, 16, 2049, 6001])
+def test_gpu_against_oracle(name, n):
+    import torch
+    prob, _ = common.fully_connected(GPU[name], shared=True, dtype=np.float32)
+    p64, _ = common.fully_connected(GPU[name], shared=True, dtype=np.float64)
+    op, ref = oeq.TensorProduct(prob), oeq.TensorProduct(p64)
+    assert type(op.generator) is UVWSplitGenerator
+    X, Y, W, G = (torch.tensor(t, device="cuda") for t in common.tp_inputs(prob, n, 5, np.float32))
+    refs = (ref.forward(X.double(), Y.double(), W.double()), *ref.backward_helper(X.double(), Y.double(), W.double(), G.double()))
+    got = (op.forward(X, Y, W), *op.backward_helper(X, Y, W, G))
+    # fp32 sums of at most 11 x 132 products, dW of 6001 rows: 2-norm errors of a few 1e-7 (fp32 matrix instructions: 1 to 4e-7)
+    for a, b in zip(got, refs):
+        assert float((a.double() - b).norm() / b.norm()) < 1e-6
+
+
+@pytest.mark.gpu
+def test_gpu_infinities_and_large_values():
+    """Rows with an infinity, a NaN and values whose bf16 rounding is infinite; the other rows keep their accuracy."""
+    import torch
+    prob, oprob = common.fully_connected((natural(64, 1), natural(1, 1), natural(64, 1)), shared=True, dtype=np.float32)
+    op = oeq.TensorProduct(prob)
+    assert op.generator.split_forward and op.generator.split_dx and op.generator.dw_kinds
+    n = 4100
+    X, Y, We, G = common.tp_inputs(prob, n, 6, np.float32, w_scale=1e-3)
+    X[5, 3], G[40, 7], X[70, 9], G[n - 1, 0] = np.inf, np.nan, 3.4e38, -np.inf
+    x, y, w, g = (torch.tensor(t, device="cuda") for t in (X, Y, ow.e3nn_to_oeq(oprob, We), G))
+    z = op.forward(x, y, w)
+    dx, dy, dw = op.backward_helper(x, y, w, g)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = (otp.forward(oprob, X, Y, We), *otp.backward(oprob, X, Y, We, G))
+    big = np.arange(n) == 70                                 # (fp32 may overflow there where the oracle does not)
+    for value, r in zip((z, dx, dy), ref):
+        error, _ = worst(value.cpu().numpy()[~big], r[~big])
+        assert error < 2e-6
+        assert (np.isfinite(value.cpu().numpy()[~big]) == np.isfinite(r[~big])).all()
+    zb, rb = z.cpu().numpy()[big], ref[0][big]
+    assert np.isfinite(zb).all() and np.abs(zb - rb).max() <= 2e-6 * np.abs(rb).max()
+    got = ow.oeq_to_e3nn(oprob, dw.cpu().numpy())
+    assert (~np.isfinite(got))[~np.isfinite(ref[3])].all()
