@@ -29,7 +29,7 @@ computes its part again with fp32 multiply-adds from the original operands.
 Measured, 64x0e+64x1o+64x2e with 1x0e+1x1o+1x2e, fp32 kernels / these: 100 000 rows forward 291 / 175 us, backward 575 / 440 us;
 4097 rows 31 / 15 and 61 / 52; 100 channels, 50 000 rows 455 / 294 and 2048 / 690 (the fp32 dW walks the batch once per pass of
 accumulators there).  Relative errors against fp64 (2-norm; Z, dX, dY, dW) at 100 000 rows: 2.9e-7 1.6e-7 2.0e-7 7.7e-7 / 1.1e-7
-1.1e-7 1.6e-7 2.1e-7, and smaller than those of the fp32 kernels on every problem of ``_pays`` and batch from 500 rows on.
+1.1e-7 1.6e-7 2.1e-7, and smaller than those of the kernels they replace on every problem of ``_pays``, 4097 and 50 000 rows.
 
 What bounds them: forward and dX/dY keep the matrix cores busy for 46 % of the time (bf16 steps at the clock under this load:
 84 of 175 us); the rest is weight fragments through L1 (270 KB per tile: 70 us when every one hits it, as measured with all
@@ -198,9 +198,10 @@ class UVWSplitGenerator(UVWGenerator):
         tile a workgroup whose wavefronts share its output channels, so the forward leaves them nothing; the backward's dW
         workgroups are later to start.  Backward with l <= 2, few rows / split, 1000 and 4097 rows, kernels in us: 64 channels
         33 / 38 and 69 / 57, 32 channels 24 / 25 and 37 / 33, 48 channels 27 / 35 and 59 / 55, 100 channels 65 / 64 and
-        144 / 111."""
+        144 / 111; up to 16 channels, where half of a matrix step is padding, 17 / 22 and 26 / 29."""
         forward, backward = limits
-        return 0 if self.split_forward else forward, min(self.FEW_ROWS, backward) if self.split_dx and self.dw_kinds else backward
+        kept = min(self.FEW_ROWS, backward) if self.split_dx and self.dw_kinds and max(p.mw for p in self.paths) > 16 else backward
+        return 0 if self.split_forward else forward, kept
 
     def _chunks(self, paths: List[WPath], comps, tiles) -> List[List[WPath]]:
         """Paths that read the same rows (one in1 block forward, one output block backward), as many together as
