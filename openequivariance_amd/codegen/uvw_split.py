@@ -185,10 +185,13 @@ class UVWSplitGenerator(UVWGenerator):
 
     @classmethod
     def create(cls, problem: TPProblem):
-        """The generator, or None where the fp32 kernels serve every direction."""
+        """The generator, or None where the fp32 kernels serve every direction: also where no multiplicity exceeds 16 and half of
+        every matrix step is padding (16 channels, l <= 2, 4097 rows: 26 / 29 us backward; 40 000 rows 108 / 76)."""
         if problem.irrep_dtype != np.float32 or not problem.shared_weights:
             return None
         g = cls(problem)
+        if max(max(p.mu, p.mw) for p in g.paths) <= 16:
+            return None
         return g if g.split_forward or g.split_dx or g.dw_kinds else None
 
     FEW_ROWS = 2048

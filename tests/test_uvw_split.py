@@ -69,7 +69,7 @@ def test_directions_and_rows():
     assert g.split_forward and not g.split_dx and g.few_rows((8192, 5120)) == (0, 5120)
     g = made(96, 9)
     assert not g.split_forward and not g.split_dx
-    assert made(64, 64, dtype=np.float64) is None
+    assert made(64, 64, dtype=np.float64) is None and made(16, 16) is None and made(17, 16) is not None
     for a, b in ((64, 64), (100, 100), (8, 100), (100, 8), (33, 50)):
         g = made(a, b)
         assert g.ws_elems >= UVWGenerator(g.problem).ws_elems
