@@ -778,14 +778,18 @@ class UVWSplitGenerator(UVWGenerator):
                     return None
                 jobs = sorted(((b, u) for b, m in enumerate(bins) for u in range(_ceil(m[0][0].mu, 32))),
                               key=lambda j: (-base.cost(bins[j[0]]), j))
-                count = _ceil(len(jobs), 8)
-                for q in range(count):
-                    mine = jobs[q::count]
+                count, per = _ceil(len(jobs), 8), max(1, 8 // len(bins))
+                # all bins of ``per`` tiles of u each, whose kinds share their code, where that takes no more kinds
+                ranged = [[j for j in jobs if j[1] // per == q] for q in range(_ceil(1 + max(u for _, u in jobs), per))]
+                dealt = ranged if len(bins) <= 8 and len(ranged) <= count else [jobs[q::count] for q in range(count)]
+                for mine in dealt:
                     # wavefronts w and w + 4 share a SIMD: the most expensive jobs beside the cheapest
                     head, tail = mine[:4], mine[4:]
                     waves = head + [None] * (4 - len(head)) + ([None] * (4 - len(tail)) + tail[::-1])
                     kinds.append(DWKind(self, some, bins, waves))
-        return kinds if len(kinds) <= 16 else None
+        # (code and compile time grow with the column ranges: 64 channels 4 s where the fp32 kernels take 2, 100 channels 9 and 5,
+        # 200 channels with four ranges 43 and 13)
+        return kinds if len(kinds) <= 16 and len({tuple(k.blocks) for k in kinds}) <= 4 else None
 
     def _dw_bins(self, kind: "DWKind"):
         """The kind's paths in bins of one in1 block each, within DW_REGISTERS and of about an eighth of the work per bin."""
@@ -822,7 +826,7 @@ class UVWSplitGenerator(UVWGenerator):
         if not self.dw_kinds:
             return ""
         out = []
-        for q, kind in enumerate(self.dw_kinds):
+        for q, kind in ((m[0], self.dw_kinds[m[0]]) for m in self._dw_programs()):
             coeff, first = [], []
             for _, y, c in sorted(kind.entries.values()):
                 at = min(y, self.D2 - kind.width)            # every entry reads ``width`` values of Y, within the row
@@ -854,24 +858,34 @@ class UVWSplitGenerator(UVWGenerator):
         E(f"    const u64 row = ((u64)first + (q >= {16 * D2} ? step : 0)) * 16 + (q % {16 * D2}) / {D2};")
         E(f"    yl[q] = row < n ? Y[row * {D2} + q % {D2}] : (T)0;      // rows past the end: M = 0, T = 0")
         E("}")
-        for q, kind in enumerate(kinds):
-            E(f"if (kind == {q}) {{   // output blocks (w tiles) {kind.blocks}")
+        for members in self._dw_programs():
+            kind, q = kinds[members[0]], members[0]
+            E(f"if ({' || '.join(f'kind == {m}' for m in members)}) {{   // output blocks (w tiles) {kind.blocks}")
             E.level += 1
             code = {}
             for w, job in enumerate(kind.waves):
-                code.setdefault(job[0] if job else None, []).append((w, job[1] if job else 0))
+                code.setdefault(job[0] if job else None, []).append(w)
             stage = self._dw_stage(kind, code)
-            for at, (b, members) in enumerate(code.items()):
-                E(f"{'else ' if at else ''}if ({' || '.join(f'wv == {w}' for w, _ in members)}) {{")
+            for at, (b, waves) in enumerate(code.items()):
+                E(f"{'else ' if at else ''}if ({' || '.join(f'wv == {w}' for w in waves)}) {{")
                 E.level += 1
-                E("const int ut = " + "".join(f"wv == {w} ? {u} : " for w, u in members[:-1]) + f"{members[-1][1]};")
-                E("const int turn = " + "".join(f"wv == {w} ? {t} : " for t, (w, _) in enumerate(members[:-1])) + f"{len(members) - 1};")
-                self._dw_bin(E, kind, q, kind.bins[b] if b is not None else [], stage[b], len(members))
+                cases = [(m, w, kinds[m].waves[w][1] if kinds[m].waves[w] else 0) for m in members for w in waves]
+                E("const int ut = " + "".join(f"kind == {m} && wv == {w} ? {u} : " for m, w, u in cases[:-1]) + f"{cases[-1][2]};")
+                E("const int turn = " + "".join(f"wv == {w} ? {t} : " for t, w in enumerate(waves[:-1])) + f"{len(waves) - 1};")
+                self._dw_bin(E, kind, q, kind.bins[b] if b is not None else [], stage[b], len(waves))
                 E.level -= 1
                 E("}")
             E.level -= 1
             E("}")
         return E.text()
+
+    def _dw_programs(self):
+        """Kinds (by number) that differ only in the 32-channel tiles of u of their wavefronts."""
+        programs = {}
+        for q, kind in enumerate(self.dw_kinds):
+            key = tuple(kind.blocks), tuple(job and job[0] for job in kind.waves)
+            programs.setdefault(key, []).append(q)
+        return list(programs.values())
 
     def _dw_matrix(self, kind: "DWKind", q: int, buf: str, sign: str):
         """M of the tile whose Y is in yl[buf], times ``sign`` -> mt[buf]: a thread takes four rows of an entry."""
@@ -1049,29 +1063,33 @@ class UVWSplitGenerator(UVWGenerator):
                 E(f"fin = oeq_fma(acc{p.t}_{wt}_{r}, (T)0, fin);")
             E("if (oeq_any(!(fin == (T)0))) {   // infinities or NaN: again with fp32 multiply-adds")
             E.level += 1
-            E("T sum[16]; for (int r = 0; r < 16; ++r) sum[r] = (T)0;")
+            E("#pragma unroll 1")
+            E("for (int r = 0; r < 16; ++r) {")
+            E.level += 1
+            E(f"const int u = 32 * ut + 8 * (r >> 2) + 4 * h + (r & 3), w = {32 * wt} + c;")
+            E("T sum = (T)0;")
             E("for (u64 tile = first; tile < ntiles; tile += step)")
             E("#pragma unroll 1")
             E("for (u64 row = tile * 16; row < min(n, tile * 16 + 16); ++row) {")
             E.level += 1
             for f in sorted({p.b.off + j for (_, j) in p.pairs}):
                 E(f"const T y{f} = Y[row * {self.D2} + {f}];")
-            E(f"const T* __restrict__ gp = G + row * {self.D3} + {p.o.off} + min({32 * wt} + c, {p.mw - 1}) * {p.o.D};")
-            E("const T " + ", ".join(f"gz{k} = gp[{k}]" for k in range(p.o.D)) + ";")
-            E("for (int r = 0; r < 16; ++r) {")
-            E(f"const T* __restrict__ xp = X + row * {self.D1} + {p.a.off} + min(32 * ut + 8 * (r / 4) + 4 * h + r % 4, {p.mu - 1}) * {p.a.D};")
+            E(f"const T* __restrict__ gp = G + row * {self.D3} + {p.o.off} + min(w, {p.mw - 1}) * {p.o.D};")
+            E(f"const T* __restrict__ xp = X + row * {self.D1} + {p.a.off} + min(u, {p.mu - 1}) * {p.a.D};")
             E("const T " + ", ".join(f"x{i} = xp[{i}]" for i in range(p.a.D)) + ";")
             self.emit_cg_forward(E, p, "x", "y", "t")
             for k in range(p.o.D):
-                E(f"sum[r] = oeq_fma(t{k}, gz{k}, sum[r]);")
-            E("}")
+                E(f"sum = oeq_fma(t{k}, gp[{k}], sum);")
             E.level -= 1
             E("}")
-            E(" ".join(f"acc{p.t}_{wt}_{r} = sum[{r}];" for r in range(16)))
+            E(f"if (u < {p.mu} && w < {p.mw}) part[{p.poff} + u * {p.mw} + w] = sum;")
             E.level -= 1
             E("}")
+            E.level -= 1
+            E("} else {")
             for r in range(16):
-                E(f"{{ const int u = 32 * ut + {8 * (r // 4) + r % 4} + 4 * h, w = {32 * wt} + c; if (u < {p.mu} && w < {p.mw}) part[{p.poff} + u * {p.mw} + w] = acc{p.t}_{wt}_{r}; }}")
+                E(f"    {{ const int u = 32 * ut + {8 * (r // 4) + r % 4} + 4 * h, w = {32 * wt} + c; if (u < {p.mu} && w < {p.mw}) part[{p.poff} + u * {p.mw} + w] = acc{p.t}_{wt}_{r}; }}")
+            E("}")
             E.level -= 1
             E("}")
 
