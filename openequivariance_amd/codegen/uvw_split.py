@@ -97,8 +97,13 @@ class DWKind:
     def cost(segs) -> int:
         return sum(p.o.D * (hi - lo) for p, lo, hi in segs)
 
+    @property
+    def lds_units(self) -> int:
+        """LDS in units of 16 bytes: Y, split dZ and M of two tiles each, one behind the other."""
+        return 2 * (4 * self.g.D2 + self.units + 4 * len(self.entries))
+
     def lds_bytes(self) -> int:
-        return 2 * (16 * self.units + 64 * len(self.entries) + 64 * max(1, self.g.D2))
+        return 16 * self.lds_units
 
 
 class UVWSplitGenerator(UVWGenerator):
@@ -849,9 +854,9 @@ class UVWSplitGenerator(UVWGenerator):
         E(f"const int kind = blockIdx.x / {share}, first = blockIdx.x % {share};")
         E(f"const u64 step = {share};")
         E(f"if (kind >= {len(kinds)} || (u64)first >= ntiles) return;")
-        E(f"__shared__ U4 gs[{2 * max(k.units for k in kinds)}];                 // dZ of a tile, split: two buffers")
-        E(f"__shared__ VT mt[{8 * max(len(k.entries) for k in kinds)}];             // M of a tile, [entry][row]: two buffers")
-        E(f"__shared__ T yl[{2 * 16 * D2}];")
+        # (one array, divided by each kind: the kind that stages most of dZ need not be the one with most entries of M)
+        E(f"__shared__ U4 lds[{max(k.lds_units for k in kinds)}];")
+        E("T* __restrict__ yl = (T*)lds;                                // Y of a tile: two buffers")
         E(f"T* __restrict__ part = (T*)ws + {self.PART_OFF} + (u64)first * {self.WN};")
         # Y of the first two tiles
         E(f"for (int q = threadIdx.x; q < {32 * D2}; q += 512) {{")
@@ -862,6 +867,8 @@ class UVWSplitGenerator(UVWGenerator):
             kind, q = kinds[members[0]], members[0]
             E(f"if ({' || '.join(f'kind == {m}' for m in members)}) {{   // output blocks (w tiles) {kind.blocks}")
             E.level += 1
+            E(f"U4* __restrict__ gs = lds + {8 * D2};                      // dZ of a tile, split: two buffers")
+            E(f"VT* __restrict__ mt = (VT*)(gs + {2 * kind.units});        // M of a tile, [entry][row]: two buffers")
             code = {}
             for w, job in enumerate(kind.waves):
                 code.setdefault(job[0] if job else None, []).append(w)

@@ -117,10 +117,10 @@ def conv_reference_on_valid_edges(otp, oprob, X, Y, W, G, rows, cols, valid):
 def lds_bytes(source, itemsize):
     """{kernel: bytes} of the LDS arrays that a generated source declares."""
     import re
-    size = {"T": itemsize, "float": 4, "double": 8, "int": 4, "i64": 8, "u64": 8}
+    size = {"T": itemsize, "float": 4, "double": 8, "int": 4, "i64": 8, "u64": 8, "VT": 16, "U4": 16}
     out = {}
     for body in re.split(r'extern "C" __global__', source)[1:]:
-        arrays = re.findall(r"__shared__ (?:__attribute__\(\(aligned\(16\)\)\) )?(\w+) \w+\[([\d *]+)\];", body)
+        arrays = re.findall(r"__shared__ (?:__attribute__\(\(aligned\(16\)\)\) )?(\w+) \w+\[([\d *+]+)\];", body)
         assert len(arrays) == body.count("__shared__")
         out[re.search(r"void (\w+)\s*\(", body).group(1)] = sum(size[t] * eval(n) for t, n in arrays)
     return out

@@ -18,6 +18,10 @@ def natural(mul, lmax):
     return "+".join(f"{mul}x{l}{'eo'[l % 2]}" for l in range(lmax + 1))
 
 
+def both(mul, lmax):
+    return "+".join(f"{mul}x{l}{p}" for l in range(lmax + 1) for p in "eo")
+
+
 def worst(got, ref):
     """Largest error among the rows whose reference is finite, and whether finite values are where the reference has them."""
     rows = np.isfinite(ref).reshape(ref.shape[0], -1).all(1)
@@ -78,9 +82,42 @@ def test_directions_and_rows():
             assert sum({"T": 4, "VT": 16, "U4": 16}[t] * eval(size) for t, size in arrays) <= UVWSplitGenerator.LDS_BYTES
 
 
+# dW workgroups of several kinds: the one that stages most of dZ is not the one with most entries of the M table, and the two
+# together would exceed a compute unit; both parities, degrees up to 5, uneven multiplicities
+KINDS = {
+    "64 -> 96, both parities": (natural(64, 2), natural(1, 2), "96x0e+96x0o+96x1e+96x1o+96x2e+96x2o"),
+    "64x4e": ("64x4e", natural(1, 4), "100x5o+32x5o+20x4e"),
+    "scalars": ("109x0o+79x0e", natural(1, 3), "68x0e+86x0o+75x1e+96x1o+68x2e+90x2o"),
+    "17 and 38 -> 94": ("17x0e+38x1o+17x2e", natural(1, 2), "94x0e+94x0o+94x1e+94x1o+94x2e+94x2o"),
+    "92 and 40 -> 98": ("92x0e+40x1o", natural(1, 4), "98x0e+98x0o+77x1e+4x1o+98x2e+98x2o"),
+    "127 and 40 -> 72": ("127x0e+40x1o+40x2e+40x3o", natural(1, 4), "72x0e+72x1o+72x2e+72x3o+17x4e"),
+    "85 -> 10, 4 and 76": ("85x0e+85x0o+85x1e+85x1o", natural(1, 4), "10x2e+4x0e+76x4e+76x1o+76x3o"),
+    **{f"{mul}, both parities": (both(mul, 2), natural(1, 2), both(mul, 2)) for mul in (20, 33, 72, 128)},
+    **{f"{mul}, l <= {lmax}": (natural(mul, lmax), natural(1, lmax), natural(mul, lmax)) for mul in (24, 65, 128) for lmax in (1, 3, 4)},
+}
+
+
+@pytest.mark.parametrize("name", KINDS)
+def test_arrays_fit_lds_together(name):
+    """A kernel's arrays as emitted, not one kind of workgroup or one array at a time: what exceeds 160 KB does not compile."""
+    g = UVWSplitGenerator.create(common.fully_connected(KINDS[name], shared=True, dtype=np.float32)[0])
+    used = common.lds_bytes(g.render(), 4) if g is not None else {}
+    assert all(size <= 160 * 1024 for size in used.values()), used
+    if g is not None and g.dw_kinds:
+        assert used["backward_dw"] == max(kind.lds_bytes() for kind in g.dw_kinds)
+
+
+def test_source_whose_dw_kinds_nearly_fill_lds_builds():
+    from openequivariance_amd import runtime as rt
+    g = UVWSplitGenerator.create(common.fully_connected(KINDS["scalars"], shared=True, dtype=np.float32)[0])
+    used = rt.kernel_metadata(rt.compile_source(g.render()))["backward_dw"][".group_segment_fixed_size"]
+    assert 150 * 1024 < used <= 160 * 1024
+
+
 GPU = {"64": (natural(64, 2), natural(1, 2), natural(64, 2)), "100": (natural(100, 2), natural(1, 1), natural(100, 1)),
        "20 -> 72": (natural(20, 2), natural(1, 2), natural(72, 2)), "50, both parities": ("50x0e+50x1o+50x1e", "1x0e", "50x0e+50x1o+50x1e"),
-       "33 -> 47": (natural(33, 1), natural(1, 1), natural(47, 2)), "132": (natural(132, 1), "1x0e", natural(132, 1))}
+       "33 -> 47": (natural(33, 1), natural(1, 1), natural(47, 2)), "132": (natural(132, 1), "1x0e", natural(132, 1)),
+       "three kinds of dW workgroups that nearly fill LDS": KINDS["scalars"]}
 
 
 @pytest.mark.gpu
