@@ -2,8 +2,8 @@
 :mod:`.uvw`; reference: the register-tiled CUDA-core matmul of openequivariance/templates/wmm.cuh:1-88).
 
 Every fp32 operand of a contraction is split into three bf16 numbers, ``x = h + m + l``, each the rounding of what the ones
-before it leave: together they hold all 24 bits of ``x``, and of the nine products of two such numbers the three below
-2^-26 of the largest (m l, l m, l l) are left out.  The other six are v_mfma_f32_16x16x32_bf16 steps into one fp32
+before it leave: together they hold all 24 bits of ``x``, denormal numbers included (``SCALE``), and of the nine products of
+two such numbers the three below 2^-26 of the largest (m l, l m, l l) are left out.  The other six are v_mfma_f32_16x16x32_bf16 steps into one fp32
 accumulator: 6 x 16 cycles per 16 x 16 x 32 block where v_mfma_f32_16x16x4_f32 takes 8 x 32, and a block of 32 channels
 meets the accumulator with 6 roundings where the fp32 instruction has 8 to 32.
 
@@ -23,7 +23,7 @@ dW_t[u, w] = sum_bk T_t[b, u, k] dz[b, w, k] runs over the batch, in steps of 16
 is split into LDS once per workgroup (two buffers), T is formed in the registers of the wavefront that multiplies it, from M
 in LDS, split and used for all w, beside the matrix steps of the component before.
 
-An infinity or a NaN among the operands makes the residuals of its split NaN.  A wavefront whose results are not all finite
+An infinity, a NaN or a number whose multiple overflows among the operands makes the residuals of its split NaN.  A wavefront whose results are not all finite
 computes its part again with fp32 multiply-adds from the original operands.
 
 Measured, 64x0e+64x1o+64x2e with 1x0e+1x1o+1x2e, fp32 kernels / these: 100 000 rows forward 291 / 175 us, backward 575 / 440 us;
@@ -49,6 +49,11 @@ from ..problem import TPProblem
 from .common import Emitter
 from .uvw import UVWGenerator, WPath, _ceil
 
+# Operands are split times 2^24, which is exact, and results taken back by 2^-48: the last bit of the smallest fp32 number,
+# 2^-149, is then a normal bf16 number, and no part of a split falls below what bf16 (or a matrix step) holds.  Operands from 2^103
+# on, and sums from 2^79, overflow on the way and are computed with fp32 multiply-adds like infinities and NaN.  (Without the
+# factor: operands of 1e-36 lost 8 of their 24 bits, 2.7e-5 relative error of a result.)
+SCALE, BACK = 2.0 ** 24, 2.0 ** -48
 PRODUCTS = ((2, 0), (0, 2), (1, 1), (1, 0), (0, 1), (0, 0))     # (split of A, split of B), smallest products first
 
 
@@ -245,7 +250,7 @@ class UVWSplitGenerator(UVWGenerator):
             E.level += 1
             E(f"const int e = q - {first}, ln = e & 63, kb = (e >> 6) % {kb}, {row} = 16 * (e / {64 * kb}) + (ln & 15), k0 = 32 * kb + 8 * (ln >> 4);")
             E("T v[8];")
-            E(f"for (int j = 0; j < 8; ++j) {{ const int {k} = k0 + j; v[j] = (u < {p.mu} && w < {p.mw}) ? W[{self.oeq_index(p, 'u', 'w')}] : (T)0; }}")
+            E(f"for (int j = 0; j < 8; ++j) {{ const int {k} = k0 + j; v[j] = (u < {p.mu} && w < {p.mw}) ? {self.lit(SCALE)} * W[{self.oeq_index(p, 'u', 'w')}] : (T)0; }}")
             E("U4 h, m, l;")
             E("oeq_split8(v, h, m, l);")
             E(f"U4* __restrict__ d = wsp + {base} + (e >> 6) * 192 + ln;")
@@ -380,7 +385,7 @@ class UVWSplitGenerator(UVWGenerator):
             o, noct, tag = blocks[b], 4 * self.kblocks(blocks[b].mul), f"{b}_{q}"
             E(f"{guard}{{ U4* __restrict__ d = xs + (r{tag} >> 4) * {units} + {offs[b]} + o{tag} * 16 + ((r{tag} ^ (2 * o{tag})) & 15);")
             for i in range(o.D):
-                E(f"    {{ const T e[8] = {{{', '.join(f'v{tag}[{j * o.D + i}]' for j in range(8))}}}; U4 h, m, l;")
+                E(f"    {{ const T e[8] = {{{', '.join(f'{self.lit(SCALE)} * v{tag}[{j * o.D + i}]' for j in range(8))}}}; U4 h, m, l;")
                 E("      oeq_split8(e, h, m, l);")
                 E("      " + " ".join(f"d[{(s * o.D + i) * noct * 16}] = {nm};" for s, nm in enumerate("hml")) + " }")
             E("}")
@@ -541,8 +546,10 @@ class UVWSplitGenerator(UVWGenerator):
         E("T fin = (T)0;")
         for nm in names:
             E(" ".join(f"fin = oeq_fma({nm}[{r}], (T)0, fin);" for r in range(4)))
+        E(f"T back = {self.lit(BACK)};")
         E("if (oeq_any(!(fin == (T)0))) {   // infinities or NaN: again with fp32 multiply-adds")
         E.level += 1
+        E("back = (T)1;")
         E(f"const T* __restrict__ Xr = X + rowB * {self.D1};")
         for nm in names:
             E(f"{nm} = V4{{0, 0, 0, 0}};")
@@ -565,6 +572,8 @@ class UVWSplitGenerator(UVWGenerator):
                 E("}")
         E.level -= 1
         E("}")
+        for nm in names:
+            E(" ".join(f"{nm}[{r}] *= back;" for r in range(4)))
 
     def _zero_blocks(self, E: Emitter, dst: str, d: int, blocks, used) -> None:
         for o in blocks:
@@ -709,8 +718,9 @@ class UVWSplitGenerator(UVWGenerator):
                 E("T " + ", ".join(names) + ";")
                 self._records_in(E, "Xr", a, names, "VTU")
             E("T " + ", ".join(f"d{nm} = (T)0" for nm in names) + ";")
-        before = [f"dy{f}" for f in self.used_y]
-        E("const T " + ", ".join(f"was_{nm} = {nm}" for nm in before) + ";")
+        sums = [f"dy{f}" for f in self.used_y]
+        E("const T " + ", ".join(f"was_{nm} = {nm}" for nm in sums) + ";")
+        E(" ".join(f"{nm} = (T)0;" for nm in sums))
 
         def apply(p):
             lines = []
@@ -734,15 +744,15 @@ class UVWSplitGenerator(UVWGenerator):
             E("}")
         names = [f"dx{ai}_{r}_{i}" for ai in ins for r in range(4) for i in range(self.in1[ai].D)]
         E("T fin = (T)0;")
-        for nm in names + before:
+        for nm in names + sums:
             E(f"fin = oeq_fma({nm}, (T)0, fin);")
+        E(f"T back = {self.lit(BACK)};")
         E("if (oeq_any(!(fin == (T)0))) {   // infinities or NaN: again with fp32 multiply-adds")
         E.level += 1
+        E("back = (T)1;")
         E(f"const T* __restrict__ Gr = G + rowB * {self.D3};")
-        for nm in names:
+        for nm in names + sums:
             E(f"{nm} = (T)0;")
-        for nm in before:
-            E(f"{nm} = was_{nm};")
         for ai in ins:
             for p in self.paths_from(ai):
                 for r in range(4):
@@ -757,6 +767,10 @@ class UVWSplitGenerator(UVWGenerator):
                     E("}")
         E.level -= 1
         E("}")
+        for nm in names:
+            E(f"{nm} *= back;")
+        for nm in sums:
+            E(f"{nm} = oeq_fma({nm}, back, was_{nm});")
 
     # ============================================================ backward: dW
     DW_REGISTERS = 160           # accumulators and X records of a wavefront
@@ -963,7 +977,7 @@ class UVWSplitGenerator(UVWGenerator):
                 E("{ " + find)
                 E(f"if (hh < 2) {{ U4* __restrict__ d = gs + ({buf}) * {kind.units} + {kind.offs[o.idx]} + hh * {np_} + w;")
                 for k in range(o.D):
-                    E(f"  {{ const T e[8] = {{{', '.join(f'g{o.idx}_{q}_{j}_{k}' for j in range(8))}}}; U4 a_, b_, c_; oeq_split8(e, a_, b_, c_); "
+                    E(f"  {{ const T e[8] = {{{', '.join(f'{self.lit(SCALE)} * g{o.idx}_{q}_{j}_{k}' for j in range(8))}}}; U4 a_, b_, c_; oeq_split8(e, a_, b_, c_); "
                       + " ".join(f"d[{(s * o.D + k) * 2 * np_}] = {nm};" for s, nm in enumerate(("a_", "b_", "c_"))) + " }")
                 E("} }")
 
@@ -973,17 +987,18 @@ class UVWSplitGenerator(UVWGenerator):
         if a:
             E.extend(x_loads())
         E("oeq_block_sync();                               // yl")
-        E.extend(self._dw_matrix(kind, at_kind, "0", "first & 1 ? (T)-1 : (T)1"))
+        E.extend(self._dw_matrix(kind, at_kind, "0", f"first & 1 ? {self.lit(-SCALE)} : {self.lit(SCALE)}"))
         split_g("0")
         E("}")
         E("oeq_block_sync();")
         E("int buf = 0;")
-        E("T sign = first & 1 ? (T)-1 : (T)1;")
+        E(f"T sign = first & 1 ? {self.lit(-SCALE)} : {self.lit(SCALE)};")
         E("for (u64 tile = first; tile < ntiles; tile += step) {")
         E.level += 1
         E(f"const U4* __restrict__ gb = gs + buf * {kind.units} + h * 32 + c;")
         E(f"const VT* __restrict__ mb = mt + buf * {4 * entries} + 2 * h;")
         E("const u64 next = tile + step, after = next + step;")
+        E(f"const T back = sign * {self.lit(BACK / SCALE)};")
         # (the last tile fetches itself again rather than branch around the requests)
         rows("next < ntiles ? next : tile")
         load_g()
@@ -1045,7 +1060,7 @@ class UVWSplitGenerator(UVWGenerator):
                 if reads:
                     E(reads.pop(0))
                 E("oeq_sched_fence();")
-            adds = [f"acc{p.t}_{wt}_{r} = oeq_fma(sign, s{at % sums}[{r}], acc{p.t}_{wt}_{r}); OEQ_PIN(acc{p.t}_{wt}_{r});" for r in range(16)]
+            adds = [f"acc{p.t}_{wt}_{r} = oeq_fma(back, s{at % sums}[{r}], acc{p.t}_{wt}_{r}); OEQ_PIN(acc{p.t}_{wt}_{r});" for r in range(16)]
             if sums == 1 or at + 1 == len(steps):
                 E.extend(adds)
                 adds = []

@@ -62,6 +62,27 @@ def test_generated_source(name, monkeypatch):
             assert error < 2e-6 and finite
 
 
+# X, W and dZ times these: what bf16 holds of a small number ends at 2^-133, 16 bits above the last bit of fp32
+SCALES = {"small rows": (1e-36, 1, 1), "small gradients": (1, 1, 1e-36), "small weights": (1, 1e-36, 1), "denormal rows": (1e-41, 1e8, 1e8),
+          "large rows": (1e30, 1, 1), "largest rows": (3e36, 1e-3, 1e-3)}      # (M x of 4100 rows: up to 40 times 3e36, finite in fp32)
+
+
+@pytest.mark.parametrize("name", SCALES)
+def test_small_and_large_operands(name, monkeypatch):
+    """No direction loses bits of operands that fp32 holds (tolerance as above)."""
+    monkeypatch.setattr(UVWSplitGenerator, "DW_WORKGROUPS", 2)
+    monkeypatch.setattr(UVWSplitGenerator, "_pays", lambda *args: True)
+    prob, oprob = common.fully_connected(("5x0e+21x1o", "1x0e+1x1o", "18x0e+7x1o"), shared=True, dtype=np.float32)
+    g = UVWSplitGenerator(prob)
+    X, Y, We, G = (t * np.float32(f) for t, f in zip(common.tp_inputs(prob, 37, 9, np.float32, w_scale=0.3), np.insert(SCALES[name], 1, 1.0)))
+    fwd, bwd, ws = g.plan()
+    W = ow.e3nn_to_oeq(oprob, We)
+    out, back = emu.run_tp(g, fwd, X, Y, W, ws_bytes=ws()), emu.run_tp(g, bwd, X, Y, W, G, ws_bytes=ws())
+    refs = (otp.forward(oprob, X, Y, We), *otp.backward(oprob, X, Y, We, G))
+    for value, ref in zip((out["Z"], back["Xg"], back["Yg"], ow.oeq_to_e3nn(oprob, back["Wg"])), refs):
+        assert np.isfinite(value).all() and np.abs(value - ref).max() < 2e-6 * np.abs(ref).max()
+
+
 def test_directions_and_rows():
     """Which kernels serve a problem: padding and wavefronts without a tile decide per direction, other types take the fp32 or
     fp64 kernels altogether, and the kernels for few rows keep only the backward's smallest batches."""
@@ -135,6 +156,23 @@ def test_gpu_against_oracle(name, n):
     # fp32 sums of at most 11 x 132 products, dW of 6001 rows: 2-norm errors of a few 1e-7 (fp32 matrix instructions: 1 to 4e-7)
     for a, b in zip(got, refs):
         assert float((a.double() - b).norm() / b.norm()) < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", SCALES)
+def test_gpu_small_and_large_operands(name):
+    import torch
+    prob, _ = common.fully_connected(GPU["64"], shared=True, dtype=np.float32)
+    p64, _ = common.fully_connected(GPU["64"], shared=True, dtype=np.float64)
+    op, ref = oeq.TensorProduct(prob), oeq.TensorProduct(p64)
+    assert op.generator.split_forward and op.generator.split_dx and op.generator.dw_kinds
+    X, Y, W, G = (torch.tensor(t * np.float32(f), device="cuda")
+                  for t, f in zip(common.tp_inputs(prob, 4100, 5, np.float32), np.insert(SCALES[name], 1, 1.0)))
+    refs = (ref.forward(X.double(), Y.double(), W.double()), *ref.backward_helper(X.double(), Y.double(), W.double(), G.double()))
+    for a, b in zip((op.forward(X, Y, W), *op.backward_helper(X, Y, W, G)), refs):
+        # (dW: a denormal T = M x of 1e-41 is rounded at 2^-149 in fp32 arithmetic of any kind, here at 2^-150; measured 2.5e-6)
+        tol = 2.0 ** -149 / 1e-41 if b.ndim == 1 and name == "denormal rows" else 1e-6
+        assert float((a.double() - b).norm() / b.norm()) < tol
 
 
 @pytest.mark.gpu
