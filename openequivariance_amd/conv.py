@@ -329,6 +329,8 @@ class TensorProductConv:
         d1, d2, d3, wn = self._dims
         if N >= 2 ** 31:
             raise ValueError("node count must be below 2^31")
+        if E >= 2 ** 32 and isinstance(self.generator, UVUSortedGenerator):
+            raise ValueError("edge count of an unsorted edge list must be below 2^32")
         if x.ndim != 2 or x.shape[1] != d1:
             raise ValueError(f"L1_in must have shape [nodes, {d1}], got {tuple(x.shape)}")
         if y.shape != (E, d2):

@@ -133,6 +133,16 @@ int check_pointers(const std::vector<Step>& steps, const void* workspace, const 
     return 0;
 }
 
+// Rejects an edge list whose positions do not fit the 32 bits that the grouping kernels (the per-edge steps of a graph
+// preparation) keep them in, before anything is launched.
+int check_edges(const std::vector<Step>& steps, uint64_t nnz, const char* what) {
+    if (nnz >> 32)
+        for (auto& s : steps)
+            if ((s.desc.flags & OEQ_STEP_GRAPH_PREP) && s.desc.grid_kind == OEQ_GRID_PER_ROW)
+                return fail("%s: %llu edges, but an unsorted edge list must have fewer than 2^32", what, (unsigned long long)nnz);
+    return 0;
+}
+
 }  // namespace
 
 struct oeq_tp {
@@ -337,6 +347,7 @@ static int conv_forward(oeq_conv* c, const void* L1, const void* L2, const void*
     if (nnz > 0 && (!rows || !cols)) return fail("forward: rows / cols are NULL");
     // (an empty edge list has no transpose permutation to read: a NULL pointer is what an empty tensor gives)
     if ((nnz > 0 || node_count > 0) && check_pointers(c->fwd, workspace, nnz > 0 ? tperm : (const void*)1, "forward")) return 1;
+    if (check_edges(c->fwd, nnz, "forward")) return 1;
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("forward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     for (auto& s : c->fwd) {
@@ -355,6 +366,7 @@ static int conv_backward(oeq_conv* c, const void* L1, void* L1g, const void* L2,
     if (nnz > 0 && (!rows || !cols)) return fail("backward: rows / cols are NULL");
     // (an empty edge list has no transpose permutation to read: a NULL pointer is what an empty tensor gives)
     if ((nnz > 0 || node_count > 0) && check_pointers(c->bwd, workspace, nnz > 0 ? tperm : (const void*)1, "backward")) return 1;
+    if (check_edges(c->bwd, nnz, "backward")) return 1;
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L1g, &L2, &L2g, &W, &Wg, &L3g, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     for (auto& s : c->bwd) {
@@ -397,6 +409,7 @@ int oeq_conv_double_backward_ex(oeq_conv* c, const void* L1, const void* L2, con
     if (nnz > 0 && node_count == 0) return fail("convolution called with %llu edges but no nodes", (unsigned long long)nnz);
     if (nnz > 0 && (!rows || !cols)) return fail("double backward: rows / cols are NULL");
     if ((nnz > 0 || node_count > 0) && check_pointers(c->bwd, workspace, nnz > 0 ? tperm : (const void*)1, "double backward")) return 1;
+    if (check_edges(c->bwd, nnz, "double backward")) return 1;
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("double backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3g, &L1c, &L2c, &Wc, &L1o, &L2o, &Wo, &L3o, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     for (auto& s : c->bwd) {

@@ -1,8 +1,10 @@
 """The counting sort that groups an unsorted edge list: ranges of nodes, the scan in LDS and in memory, several workgroups."""
 import numpy as np
 import pytest
+import torch
 
 import common
+import openequivariance_amd as oeq
 from host_emu import emu
 from openequivariance_amd.codegen.uvu_sorted import UVUSortedGenerator
 from oracle import tp as otp
@@ -31,3 +33,18 @@ def test_groups_of_several_ranges_and_workgroups(range_nodes, nodes, monkeypatch
     out = emu.run_conv(g, bwd + again[1], X, Y, W, rows, cols, G=G, ws_bytes=ws(nnz, nodes))
     for got, ref in zip((out["Xg"], out["Yg"], out["Wg"]), (dX, dY, dW)):
         assert common.rel_err(got, ref) < 2e-6
+
+
+def test_edge_positions_hold_32_bits():
+    """The grouping kernels keep positions in 32 bits: longer edge lists are refused before anything is launched (tensors
+    without storage)."""
+    class Conv(oeq.TensorProductConv):
+        def __init__(self, generator):
+            self.generator, self.deterministic, self._dims = generator, False, (8, 4, 8, 4)
+            self._torch_dtype, self._torch_idx = torch.float32, torch.int64
+    conv = Conv(UVUSortedGenerator(common.channelwise(("2x0e+2x1o", "1x0e+1x1o", "2x0e+2x1o"))[0]))
+    for edges, message in ((2 ** 32, "edge count"), (2 ** 32 - 1, "must be on the GPU")):
+        x, y, w = (torch.empty(n, d, device="meta") for n, d in ((10, 8), (edges, 4), (edges, 4)))
+        rows, cols = (torch.empty(edges, dtype=torch.int64, device="meta") for _ in range(2))
+        with pytest.raises(ValueError, match=message):
+            conv._check(x, y, w, rows, cols)
