@@ -34,8 +34,11 @@ from .uvu_recv import UVURecvGenerator
 class UVUSortedGenerator:
     kind = "conv_atomic"
     SCAN_THREADS = 1024              # of the grouping kernels' workgroups,
-    GROUP_EDGES = 4                  # ... edges each of these takes,
-    GROUP_NODES = 16384              # ... nodes counted in LDS at a time (64 KB)
+    GROUP_WORKGROUPS = 128           # ... how many of these there are at most,
+    GROUP_FEW_EDGES = 32768          # ... lists of which a thread takes one edge,
+    GROUP_EDGES = 4                  # ... edges it takes at a time otherwise,
+    GROUP_NODES = 16384              # ... nodes counted in LDS at a time (64 KB),
+    GROUP_RANGES = 4                 # ... and such ranges that a workgroup walks at most
     SEGMENTED = UVUDetGenerator      # what walks the groups
 
     # dX values per edge from which the grouped backward is the starting choice.  Measured with the grouping
@@ -102,8 +105,8 @@ class UVUSortedGenerator:
         def grouping(sfx):
             return [dict(kernel="group_clear" + sfx, num_threads=256, grid_kind=NODE, work_per_block=256,
                          prep=True, counter_clear=True),
-                    dict(kernel="group_count" + sfx, num_threads=S, grid_kind=ROW, work_per_block=S * self.GROUP_EDGES, prep=True),
-                    dict(kernel="group_fill" + sfx, num_threads=S, grid_kind=ROW, work_per_block=S * self.GROUP_EDGES, prep=True)]
+                    dict(kernel="group_count" + sfx, num_threads=S, grid_kind=ROW, work_per_block=S, num_blocks=self.GROUP_WORKGROUPS, prep=True),
+                    dict(kernel="group_fill" + sfx, num_threads=S, grid_kind=ROW, work_per_block=S, num_blocks=self.GROUP_WORKGROUPS, prep=True)]
         fwd = grouping("") + f.forward_steps(dict(kernel="forward", num_threads=64, grid_kind=3, work_per_block=1,
                                                   num_blocks=f.LONG, grid_y=f.NCH))
         G = f.group_bytes

@@ -69,8 +69,6 @@ typedef VT VTU;
 #define __builtin_nontemporal_store(v, p) (*(p) = (v))
 #define __builtin_nontemporal_load(p) (*(p))
 #define OEQ_DMA(BYTES, POLICY, g, lds_base) memcpy((char*)(lds_base) + ((BYTES) == 12 ? 16 : (BYTES)) * (threadIdx.x & 63), (g), (BYTES))
-static inline void oeq_release_agent() {}
-static inline void oeq_acquire_agent() {}
 static inline int oeq_ticket_add(int* p) { std::lock_guard<std::mutex> g(g_atomic_mutex); return (*p)++; }
 static inline void oeq_st_agent(T* p, T v) { *p = v; }
 static inline T oeq_ld_agent(const T* p) { return *p; }
@@ -94,8 +92,8 @@ static inline void __syncthreads() { pthread_barrier_wait(&g_bar); }
 #define __HIP_MEMORY_SCOPE_AGENT 0
 #define __HIP_MEMORY_SCOPE_WORKGROUP 0
 template <class V> static inline V __hip_atomic_fetch_add(V* p, V v, int, int) { std::lock_guard<std::mutex> g(g_atomic_mutex); V o = *p; *p += v; return o; }
-static inline i64 oeq_read_count(i64* p) { std::lock_guard<std::mutex> g(g_atomic_mutex); return *p; }
 static inline i64 oeq_take_count(i64* p) { std::lock_guard<std::mutex> g(g_atomic_mutex); const i64 o = *p; *p = 0; return o; }
+static inline i64 oeq_lds_claim(i64* slot, i64 key) { std::lock_guard<std::mutex> g(g_atomic_mutex); const i64 old = *slot; if (old == -1) *slot = key; return old; }
 // matrix-core step of one wavefront, emulated collectively by its 64 threads
 struct V4 { T v[4]; T& operator[](int i) { return v[i]; } const T& operator[](int i) const { return v[i]; } };
 static T g_mA[16][16][4], g_mB[16][4][16];

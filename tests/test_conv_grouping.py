@@ -35,6 +35,35 @@ def test_groups_of_several_ranges_and_workgroups(range_nodes, nodes, monkeypatch
         assert common.rel_err(got, ref) < 2e-6
 
 
+SHAPES = {"keys over more ranges than a workgroup walks": dict(GROUP_RANGES=1, GROUP_NODES=16, GROUP_EDGES=1),
+          "... with runs of equal keys": dict(GROUP_RANGES=1, GROUP_NODES=16, GROUP_FEW_EDGES=0),
+          "one workgroup, several turns of its threads": dict(GROUP_WORKGROUPS=1, GROUP_FEW_EDGES=0, GROUP_EDGES=1),
+          "ranges from the first node named, runs": dict(GROUP_NODES=16, GROUP_FEW_EDGES=0)}
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("order", ["random", "by receiver"])
+def test_shares_and_spans_of_workgroups(shape, order, monkeypatch):
+    """275 edges in workgroups of 128 threads, a hub, edges naming no node among them."""
+    for name, value in dict(SHAPES[shape], SCAN_THREADS=128).items():
+        monkeypatch.setattr(UVUSortedGenerator, name, value)
+    prob, oprob = common.channelwise(("2x0e+2x1o", "1x0e+1x1o", "2x0e+2x1o"))
+    g = UVUSortedGenerator(prob, grouped_backward=False)
+    nnz, nodes = 275, 60
+    rng = np.random.default_rng(7)
+    rows, cols = rng.integers(5, nodes, nnz), rng.integers(0, nodes, nnz)
+    rows[50:150] = 50
+    if order == "by receiver":
+        rows.sort()
+    rows[200:203], cols[205:207] = (-1, nodes, 2 ** 40), (nodes, -7)
+    valid = (rows >= 0) & (rows < nodes) & (cols >= 0) & (cols < nodes)
+    X, Y, W, G = common.conv_inputs(prob, nodes, nnz, 3)
+    Z = common.conv_reference_on_valid_edges(otp, oprob, X, Y, W, G, rows, cols, valid)[0]
+    fwd, _, ws = g.plan()
+    out = emu.run_conv(g, fwd, X, Y, W, rows, cols, ws_bytes=ws(nnz, nodes))
+    assert common.rel_err(out["Z"], Z) < 2e-6
+
+
 def test_edge_positions_hold_32_bits():
     """The grouping kernels keep positions in 32 bits: longer edge lists are refused before anything is launched (tensors
     without storage)."""
@@ -48,3 +77,33 @@ def test_edge_positions_hold_32_bits():
         rows, cols = (torch.empty(edges, dtype=torch.int64, device="meta") for _ in range(2))
         with pytest.raises(ValueError, match=message):
             conv._check(x, y, w, rows, cols)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nodes", [1023, 16383, 16384, 16385, 100_001])
+@pytest.mark.parametrize("order", ["random", "by receiver", "hub"])
+def test_gpu_against_sorted_edges(nodes, order):
+    """Edges of the ranges in LDS, of keys over more nodes than a workgroup walks, and of lists long enough for four per thread;
+    the deterministic operator on the sorted list sums the same edges of a node in its own order."""
+    prob, _ = common.channelwise(("4x0e+4x1o", "1x0e+1x1o", "4x0e+4x1o"))
+    free, fixed = oeq.TensorProductConv(prob, torch_op=True), oeq.TensorProductConv(prob, torch_op=True, deterministic=True)
+    nnz = 150_001
+    gen = torch.Generator(device="cuda").manual_seed(nodes)
+    rows, cols = (torch.randint(0, nodes, (nnz,), device="cuda", generator=gen) for _ in range(2))
+    if order == "hub":
+        rows[torch.randperm(nnz, device="cuda", generator=gen)[:nnz // 2]] = nodes - 1
+    if order == "by receiver":
+        rows = rows.sort().values
+    x, y, w = (torch.randn(n, d, device="cuda", generator=gen)
+               for n, d in ((nodes, prob.irreps_in1.dim), (nnz, prob.irreps_in2.dim), (nnz, prob.weight_numel)))
+    g = torch.randn(nodes, prob.irreps_out.dim, device="cuda", generator=gen)
+    r, c, perm, tperm = oeq.sort_by_receiver(rows, cols, nodes)
+    want = [fixed.forward(x, y[perm], w[perm], r, c, tperm)]
+    dx, dy, dw = fixed.backward_helper(x, y[perm], w[perm], g, r, c, tperm)
+    back = torch.empty_like(perm)
+    back[perm] = torch.arange(nnz, device="cuda")
+    want += [dx, dy[back], dw[back]]
+    for _ in range(2):
+        got = (free.forward(x, y, w, rows, cols), *free.backward_helper(x, y, w, g, rows, cols))
+        for a, b in zip(got, want):
+            assert float((a - b).norm() / b.norm()) < 2e-6     # (a hub's 75 000 edges summed in another order)
