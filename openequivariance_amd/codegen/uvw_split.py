@@ -130,8 +130,8 @@ class UVWSplitGenerator(UVWGenerator):
         # cycles of the fp32 instruction over those of the split one
         forward = sum(p.o.D * p.SU * p.NTW * 32 for p in self.paths) / sum(p.a.D * self.kblocks(p.mu) * p.NTW * 96 for p in self.paths)
         backward = sum(p.o.D * p.SW * p.NTU * 32 for p in self.paths) / sum(p.o.D * self.kblocks(p.mw) * p.NTU * 96 for p in self.paths)
-        self.split_forward = self._pays(self.fwd_shape, forward, 1.5, 0)
-        self.split_dx = self._pays(self.bwd_shape, backward, 1.3, 64 * max(1, self.D2))
+        self.split_forward = self._pays(self.fwd_shape, forward, 1.5, 0, 7 if self._single(self.used_in1) else 5)
+        self.split_dx = self._pays(self.bwd_shape, backward, 1.3, 64 * max(1, self.D2), 5)
         # packed copies, in words: forward, then backward
         self.FWD_WORDS = self._place("wb", 0, self.split_forward, lambda p: p.NTW * self.kblocks(p.mu) * 192, lambda p: p.SU * 64 * p.NTW)
         self.WA_END = self._place("wa", self.FWD_WORDS, self.split_dx, lambda p: p.NTU * self.kblocks(p.mw) * 192,
@@ -176,7 +176,11 @@ class UVWSplitGenerator(UVWGenerator):
         a wavefront writes at the same column fall on different banks."""
         return d + (4 - d) % 64
 
-    def _pays(self, shape: Shape, gain: float, least: float, extra: int) -> bool:
+    def _single(self, blocks) -> bool:
+        """Whether at most one path reads each block on average: its split rows serve one contraction only."""
+        return len(self.paths) <= len(blocks)
+
+    def _pays(self, shape: Shape, gain: float, least: float, extra: int, resident: int) -> bool:
         """Whether the split kernel of a direction is the faster one: its tiles fit LDS, three wavefronts or more of a workgroup
         have a tile of output channels, and the padding to 32 (K) leaves enough of the 2.67 times shorter matrix steps.
         40 000 rows, l <= 2 with second operand l <= 2, gain, fp32 / split kernel in us:
@@ -189,9 +193,26 @@ class UVWSplitGenerator(UVWGenerator):
             20 -> 72     2.67  116.5 /  80.0    2.00  115.8 / 261.6   (two wavefronts)
             16           1.33   18.8 /  21.3    1.33   38.5 /  28.7
             9 -> 95      1.33   91.0 /  91.7    2.67  227.4 / 257.2   (one wavefront)
-            96 -> 9      2.67   83.1 / 245.0    1.00  185.8 / 120.1   (one wavefront forward)"""
+            96 -> 9      2.67   83.1 / 245.0    1.00  185.8 / 120.1   (one wavefront forward)
+
+        And as many wavefronts as ``resident`` in the workgroups that LDS lets a compute unit hold, for they wait for one another at
+        both ends of a tile: five, of the forward seven where split rows serve one path each.  40 000 rows, wavefronts, whole
+        forward and backward calls (the dX of both on the same dW), fp32 / split, us:
+
+            64, l <= 3, in2 l <= 1            4   175 / 256    316 / 408
+            50, l <= 3, in2 l <= 2            4   299 / 393    408 / 649
+            50, both parities, l <= 2, 1x0e   4   108 / 175    248 / 325
+            33, both parities, in2 l <= 2     3   219 / 476    494 / 840
+            65, l <= 2, in2 l <= 2            5   244 / 178    472 / 462
+            96, l <= 2, in2 l <= 1            6   236 / 136    375 / 341
+            65, l <= 2, 1x0e                  5    81 /  99    221 / 224   (72, l <= 3, 1x0e: 193 / 166, 369 / 360)
+            33 | 48, l <= 2, 1x0e (65 536)    6    45 /  54     50 /  56   (forward of each)
+            100, l <= 2, 1x0e                 7   151 / 121    278 / 270
+            64, l <= 2, 1x0e (65 536)         8   100 /  74
+            150 | 200, l <= 1, in2 l <= 1     8   197 / 132, 423 / 218;  422 / 345, 590 / 485"""
         lds = 16 * self._lds_units(shape, self.D1, self.D3) + extra * shape.waves * shape.tiles
-        return lds <= self.LDS_BYTES and shape.waves * shape.tiles >= 3 and gain >= least
+        waves = shape.waves * shape.tiles
+        return waves >= 3 and gain >= least and self.LDS_BYTES // lds * waves >= resident
 
     @classmethod
     def create(cls, problem: TPProblem):

@@ -103,6 +103,27 @@ def test_directions_and_rows():
             assert sum({"T": 4, "VT": 16, "U4": 16}[t] * eval(size) for t, size in arrays) <= UVWSplitGenerator.LDS_BYTES
 
 
+# Few wavefronts on a compute unit beside long rows: what was slower than the fp32 kernels (40 000 rows, both sides with the rules);
+# forward, dX / dY, dW on split operands
+DIRECTIONS = {
+    "four wavefronts": (natural(64, 3), natural(1, 1), natural(64, 3), False, False, True),
+    "four wavefronts, both parities": (both(50, 2), "1x0e", both(50, 2), False, False, True),
+    "three wavefronts, both parities": (both(33, 2), natural(1, 2), both(33, 2), False, False, True),
+    "two workgroups of four": (both(50, 1), "1x0e", both(50, 1), True, True, True),
+    "five, several paths a block": (natural(65, 2), natural(1, 2), natural(65, 2), True, True, True),
+    "five, one path a block": (natural(65, 2), "1x0e", natural(65, 2), False, True, True),
+    "six, one path a block": (natural(48, 2), "1x0e", natural(48, 2), False, True, True),
+    "seven, one path a block": (natural(100, 2), "1x0e", natural(100, 2), True, True, True),
+}
+
+
+@pytest.mark.parametrize("name", DIRECTIONS)
+def test_directions_that_pay(name):
+    *irreps, forward, dx, dw = DIRECTIONS[name]
+    g = UVWSplitGenerator.create(common.fully_connected(irreps, shared=True, dtype=np.float32)[0])
+    assert (g.split_forward, g.split_dx, bool(g.dw_kinds)) == (forward, dx, dw)
+
+
 # dW workgroups of several kinds: the one that stages most of dZ is not the one with most entries of the M table, and the two
 # together would exceed a compute unit; both parities, degrees up to 5, uneven multiplicities
 KINDS = {
