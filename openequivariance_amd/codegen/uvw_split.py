@@ -801,8 +801,29 @@ class UVWSplitGenerator(UVWGenerator):
     def dw_kinds(self):
         """Workgroup kinds of the dW kernel, a list of DWKind, or None where the fp32 kernel serves the problem.  A kind stages at
         most 64 channels of its output blocks; its jobs are bins of paths (with a range of w tiles) from one in1 block times
-        32-channel tiles of u, one per wavefront."""
+        32-channel tiles of u, one per wavefront.
+
+        Not where T, split for a single w tile that is half padding, is most of the work (from three u tiles on within
+        2 % of the fp32 kernel), nor where each kind of workgroup, which
+        fetches and splits rows for itself, has one path for each and pads to 32 besides.  40 000 rows, backward on the fp32 dX
+        with the fp32 / split dW kernel, us (gain as in ``_pays``):
+
+            in1 -> out, l <= 2            in2 l <= 2                1x0e
+            64 -> 8                   1.33   125 /  132
+            96 -> 9                   1.33   268 /  274
+            100 -> 12                 1.17   335 /  334      (100 -> 8)  1.17   149 /  142
+            32 -> 16                  1.33   123 /   99      (64 -> 16)  1.33    94 /   91
+            8 -> 100                  1.17   440 /  236
+            9 -> 33                   1.00   178 /  126
+            64 | 65, 4 kinds of 65    2.67   268 /  238                  1.85   206 /  221
+            100, 4 kinds              2.04  1590 /  640                  2.04   311 /  278
+            40 | 64 both, 3 kinds                                 1.50 201 / 208, 2.67 279 / 280
+            33 | 96 both, 4 | 6 kinds 1.50   708 /  494                  2.67  1105 /  630
+            128, 4 kinds              2.67  2449 /  757
+            200, 15 kinds             2.30  8036 / 3136"""
         tiles = lambda o: _ceil(self.out[o].mul, 32)
+        if max(p.mw for p in self.paths) <= 16 and 32 < max(p.mu for p in self.paths) <= 64 and len(self.paths) > 2 * len(self.used_in1):
+            return None
         kinds: List[DWKind] = []
         for lo in range(0, max(tiles(o) for o in self.used_out), 2):
             blocks = [(o, lo, min(lo + 2, tiles(o))) for o in self.used_out if tiles(o) > lo]
@@ -827,6 +848,11 @@ class UVWSplitGenerator(UVWGenerator):
                     head, tail = mine[:4], mine[4:]
                     waves = head + [None] * (4 - len(head)) + ([None] * (4 - len(tail)) + tail[::-1])
                     kinds.append(DWKind(self, some, bins, waves))
+        # cycles of the fp32 instruction over those of the split one
+        gain = (sum(128 * p.NTU * p.NTW * p.o.D for p in self.paths)
+                / sum(192 * _ceil(p.mu, 32) * _ceil(p.mw, 32) * p.o.D for p in self.paths))
+        if len(kinds) >= 3 and self._single(self.used_out) and gain < 2:
+            return None
         # (code and compile time grow with the column ranges: 64 channels 4 s where the fp32 kernels take 2, 100 channels 9 and 5,
         # 200 channels with four ranges 43 and 13)
         return kinds if len(kinds) <= 16 and len({tuple(k.blocks) for k in kinds}) <= 4 else None

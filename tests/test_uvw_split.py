@@ -111,9 +111,11 @@ DIRECTIONS = {
     "three wavefronts, both parities": (both(33, 2), natural(1, 2), both(33, 2), False, False, True),
     "two workgroups of four": (both(50, 1), "1x0e", both(50, 1), True, True, True),
     "five, several paths a block": (natural(65, 2), natural(1, 2), natural(65, 2), True, True, True),
-    "five, one path a block": (natural(65, 2), "1x0e", natural(65, 2), False, True, True),
+    "five, one path a block": (natural(65, 2), "1x0e", natural(65, 2), False, True, False),
     "six, one path a block": (natural(48, 2), "1x0e", natural(48, 2), False, True, True),
     "seven, one path a block": (natural(100, 2), "1x0e", natural(100, 2), True, True, True),
+    "narrow outputs": (natural(64, 2), natural(1, 2), natural(16, 2), False, True, False),
+    "narrow outputs of few paths": (natural(64, 2), "1x0e", natural(16, 2), False, True, True),
 }
 
 
