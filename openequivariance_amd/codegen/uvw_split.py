@@ -225,17 +225,46 @@ class UVWSplitGenerator(UVWGenerator):
             return None
         return g if g.split_forward or g.split_dx or g.dw_kinds else None
 
-    FEW_ROWS = 2048
-
     def few_rows(self, limits):
-        """Largest batches of the kernels for few rows (``limits``: beside the fp32 kernels).  The split kernels give every 16-row
-        tile a workgroup whose wavefronts share its output channels, so the forward leaves them nothing; the backward's dW
-        workgroups are later to start.  Backward with l <= 2, few rows / split, 1000 and 4097 rows, kernels in us: 64 channels
-        33 / 38 and 69 / 57, 32 channels 24 / 25 and 37 / 33, 48 channels 27 / 35 and 59 / 55, 100 channels 65 / 64 and
-        144 / 111; up to 16 channels, where half of a matrix step is padding, 17 / 22 and 26 / 29."""
+        """Largest batches of the kernels for few rows (``limits``: beside the fp32 kernels) that these leave them.
+
+        Forward: every 16-row tile has a workgroup whose wavefronts share its output channels, so next to nothing.  Only rows that
+        serve one path each and whose channels are no multiple of eight, which are split number by number: few rows / split, 500
+        and 2048 rows, us: 50 channels of both parities, l <= 1, 8.6 / 9.9 and 9.6 / 10.2, 20 -> 64 l <= 2 7.3 / 8.9 and 8.6 / 9.3,
+        100 12.1 / 14.0 and 15.8 / 14.8 (1000 rows 13.4 / 14.9); 64 9.0 / 8.7 and 10.3 / 9.1, 128 l <= 1 11.8 / 8.8.
+
+        Backward: the dW workgroups are later to start, with a chain of 32 channels and more for each path.  us:
+
+            channels                       500 rows      2048          4096          4097
+            64, l <= 2                  29.5 / 32.0   37.7 / 42.2   51.3 / 49.2   60.5 / 54.3
+            32, l <= 2                  20.2 / 22.5   23.8 / 25.9   29.4 / 33.8   35.6 / 34.0
+            48, l <= 2                                            42.0 / 48.2   49.4 / 52.3
+            25, l <= 1                  14.5 / 16.7   18.7 / 19.5   19.8 / 24.2   20.9 / 24.2
+            64, both parities, l <= 1   23.4 / 25.6   28.0 / 35.8   34.3 / 41.0   40.8 / 43.0
+            65, l <= 2                  45.2 / 40.0   63.5 / 54.7   84.0 / 67.8
+            128, l <= 1                 31.0 / 25.4   37.8 / 36.7   46.8 / 39.3
+            one path a block:
+            64, l <= 1                  15.2 / 15.2   22.6 / 18.7   27.9 / 24.2   (1000 rows 18.1 / 18.0)
+            64, l <= 2                  19.2 / 19.8   28.1 / 24.1   34.2 / 31.8   (22.4 / 22.9)
+            50, both parities, l <= 1   17.4 / 20.5   23.6 / 25.0   26.7 / 32.5   (8192 rows 36.5 / 37.1, 20 480 64.0 / 60.9)
+
+        Up to 16 channels half of a matrix step is padding: 17 / 22 at 1000 and 26 / 29 at 4097 rows."""
         forward, backward = limits
-        kept = min(self.FEW_ROWS, backward) if self.split_dx and self.dw_kinds and max(p.mw for p in self.paths) > 16 else backward
-        return 0 if self.split_forward else forward, kept
+        widest = max(max(p.mu, p.mw) for p in self.paths)
+        if self.split_forward:
+            odd = self._single(self.used_in1) and any(self.in1[a].mul % 8 for a in self.used_in1)
+            forward = min(forward, 0 if not odd else 2048 if widest <= 64 else 1024)
+        if self.split_dx and self.dw_kinds and max(p.mw for p in self.paths) > 16:
+            if max(p.mw for p in self.paths) > 64:
+                most = 0
+            elif self._single(self.used_out):
+                most = 8192 if len(self.used_in1) >= 4 else 1024
+            elif max(self.in1[a].D for a in self.used_in1) <= 3:
+                most = 5120
+            else:
+                most = 4096 if widest < 64 else 2048
+            backward = min(backward, most)
+        return forward, backward
 
     def _chunks(self, paths: List[WPath], comps, tiles) -> List[List[WPath]]:
         """Paths that read the same rows (one in1 block forward, one output block backward), as many together as

@@ -126,6 +126,16 @@ def test_directions_that_pay(name):
     assert (g.split_forward, g.split_dx, bool(g.dw_kinds)) == (forward, dx, dw)
 
 
+@pytest.mark.parametrize("irreps,kept", [
+    ((natural(48, 2), natural(1, 2), natural(48, 2)), (0, 4096)), ((natural(25, 1), natural(1, 2), natural(25, 1)), (0, 5120)),
+    ((natural(65, 2), natural(1, 2), natural(65, 2)), (0, 0)), ((natural(64, 2), "1x0e", natural(64, 2)), (0, 1024)),
+    ((both(50, 1), "1x0e", both(50, 1)), (2048, 8192)), ((natural(100, 2), "1x0e", natural(100, 2)), (1024, 0)),
+    ((natural(20, 2), "1x0e", natural(64, 2)), (2048, 65536)), ((both(50, 2), "1x0e", both(50, 2)), (8192, 65536))])
+def test_rows_left_to_the_kernels_for_few(irreps, kept):
+    g = UVWSplitGenerator.create(common.fully_connected(irreps, shared=True, dtype=np.float32)[0])
+    assert g.few_rows((8192, 65536)) == kept and g.few_rows((0, 0)) == (0, 0)
+
+
 # dW workgroups of several kinds: the one that stages most of dZ is not the one with most entries of the M table, and the two
 # together would exceed a compute unit; both parities, degrees up to 5, uneven multiplicities
 KINDS = {
