@@ -368,6 +368,7 @@ class UVWGenerator:
 
     # =============================================================== forward
     forward_threads = 64
+    has_forward = True           # (False: backward kernels alone)
 
     def k_unroll(self, batches: int) -> int:
         """Unroll factor of a forward K loop.  fp32: 1 where the factor does not divide the batches of four steps; 100 000
@@ -1015,4 +1016,4 @@ class UVWGenerator:
                dict(kernel="backward_dw", num_threads=self.dw_threads, grid_kind=FIXED,
                     num_blocks=self.DW_WORKGROUPS),
                dict(kernel="backward_reduce", num_threads=256, grid_kind=FIXED, num_blocks=_ceil(self.WN, 256))]
-        return fwd, bwd, (lambda nnz=0, nodes=0: self.ws_elems * self.itemsize)
+        return fwd if self.has_forward else [], bwd, (lambda nnz=0, nodes=0: self.ws_elems * self.itemsize)

@@ -14,11 +14,10 @@ from . import runtime as rt
 from .codegen.uvu_conv_double import conv_double_generator
 from .codegen.uvu_double import UVUDoubleGenerator
 from .codegen.uvw import UVWGenerator
-from .codegen.uvw_small import UVWSmallGenerator
 from .codegen.uvw_split import UVWSplitGenerator
 from .conv import select_conv_generator
 from .problem import ChannelwiseTPP, FullyConnectedTPProblem, TPProblem
-from .tensor_product import select_generator
+from .tensor_product import few_rows_generator, select_generator
 from .workloads import get as get_workload
 from .workloads import DENSE, DIFFDOCK_L2, LARGE, MACE, MACE_ALL, NEQUIP, TETRIS_POLY
 
@@ -33,7 +32,7 @@ def benchmark_generators():
         g = select_generator(problem)
         gens.append((label, g))
         if type(g) in (UVWGenerator, UVWSplitGenerator):
-            few = UVWSmallGenerator.create(problem)
+            few, _ = few_rows_generator(problem, g)
             if few is not None:
                 gens.append((label + " few rows", few))
         elif problem.instructions[0].connection_mode == "uvu" and UVUDoubleGenerator.suits(problem):

@@ -113,6 +113,17 @@ class TensorProductBase:
         return self.forward(L1_in, L2_in, weights)
 
 
+def few_rows_generator(config: TPProblem, generator: UVWGenerator):
+    """(generator, largest batches forward and backward) of the kernels for few rows beside a dense uvw product's
+    ``generator``: without a forward where they leave it none, (None, (0, 0)) where they have no batch at all."""
+    small = UVWSmallGenerator.create(config)
+    if small is None:
+        return None, (0, 0)
+    limits = getattr(generator, "few_rows", tuple)(UVWSmallGenerator.row_limits(generator))
+    small.has_forward = limits[0] > 0
+    return (small, limits) if any(limits) else (None, (0, 0))
+
+
 class TensorProduct(TensorProductBase):
     """Drop-in for ``oeq.TensorProduct(problem, torch_op=True)``."""
 
@@ -135,8 +146,6 @@ class TensorProduct(TensorProductBase):
         # dense uvw: kernels for few rows and their largest batch (forward, backward).  Built here like the double backward's,
         # not by the call that first needs them: that call would wait for the compiler, and a stream capture cannot
         self._few_rows, self._few_rows_limits = self._few_row_kernels()
-        # ... and what they keep of it where the generator's kernels on split operands are the faster ones on few rows too
-        self._few_rows_kept = getattr(self.generator, "few_rows", tuple)(self._few_rows_limits)
         # double backward in one launch: kernels by alignment of the outputs (misaligned ones are compiled on first need)
         self._double_generator = UVUDoubleGenerator if mode == "uvu" and UVUDoubleGenerator.suits(config) else None
         self._double = {}
@@ -195,23 +204,20 @@ class TensorProduct(TensorProductBase):
         return self.internal
 
     def _pick_rows(self, batch: int, backward: bool):
-        """The kernels for a batch of few rows, None where ``batch`` is not one."""
-        if not 0 < batch <= self._few_rows_limits[backward]:
-            return None
-        return self._few_rows if batch <= self._few_rows_kept[backward] else self.internal
+        """The kernels for few rows where ``batch`` is one, else None."""
+        return self._few_rows if 0 < batch <= self._few_rows_limits[backward] else None
 
     def _few_row_kernels(self):
         """(kernel set, limits) of the kernels for few rows of a dense uvw product."""
+        def build():
+            g, limits = few_rows_generator(self.config, self.generator)
+            return (None, None) if g is None else (g.render(), (*g.plan()[:2], limits))
         none = None, (0, 0)
         if type(self.generator) not in (UVWGenerator, UVWSplitGenerator):
             return none
-
-        def build():
-            g = UVWSmallGenerator.create(self.config)
-            return (None, None) if g is None else (g.render(), (*g.plan()[:2], UVWSmallGenerator.row_limits(self.generator)))
         impl, plan = rt.variant(("uvw few rows", self.config.signature()), torch.cuda.current_device(), build,
                                 lambda code, plan: rt.TPImpl(code, *(_make_steps(steps, self._step_flags) for steps in plan[:2])))
-        # (None: a problem whose units do not fit their registers or LDS)
+        # (None: a problem whose units do not fit their registers or LDS, or none of whose batches they are for)
         return none if impl is None else (impl, plan[2])
 
     def _double_kernels(self, aligned: bool) -> "rt.TPImpl":

@@ -161,24 +161,37 @@ def test_wide_second_operands_on_the_gpu(cuda, case):
 def test_on_the_gpu(cuda, irreps, dtype):
     import torch
     import openequivariance_amd as oeq
+    from openequivariance_amd import runtime as rt
+    from openequivariance_amd.tensor_product import _make_steps
     prob, oprob = common.fully_connected(irreps, shared=True, dtype=dtype)
     tp = oeq.TensorProduct(prob, torch_op=True)
-    limits = tp._few_rows_limits
+    limits = UVWSmallGenerator.row_limits(UVWGenerator(prob))
     assert limits[1] == (65536 if irreps is BOTH else 5120)
+    # fp32 kernels on split operands leave these fewer rows, and no forward where they leave it none: here both sides are built
+    # whole, without them
+    kept = tp._few_rows_limits
+    assert all(k <= most for k, most in zip(kept, limits)) and (dtype == np.float32 or kept == limits)
+    def build(generator):
+        return rt.TPImpl(rt.compile_source(generator.render()), *(_make_steps(steps, tp._step_flags) for steps in generator.plan()[:2]))
+    few, large = build(UVWSmallGenerator.create(prob)), build(UVWGenerator(prob))
     for n in (1, 16, 37, 2049, 4097, 5120, 5121):
         X, Y, We, G = common.tp_inputs(prob, n, n, dtype, w_scale=0.3)
         x, y, w, g = (torch.tensor(a, device=cuda) for a in (X, Y, ow.e3nn_to_oeq(oprob, We), G))
-        assert [tp._pick_rows(n, back) is None for back in (False, True)] == [n > limit for limit in limits]
-        got = [tp.forward(x, y, w), *tp.backward_helper(x, y, w, g)]
+        assert [tp._pick_rows(n, back) is None for back in (False, True)] == [n > limit for limit in kept]
+        def run():
+            return [tp.forward(x, y, w), *tp.backward_helper(x, y, w, g)]
+        as_built = run()
+        tp._few_rows, tp._few_rows_limits, own = few, (n, n), tp._few_rows
+        got, again = run(), run()
         if n <= 37:
             ref = [otp.forward(oprob, X, Y, We), *otp.backward(oprob, X, Y, We, G)]
             ref[3] = ow.e3nn_to_oeq(oprob, ref[3])
             tol = TOL[dtype]
         else:
             # the kernels for large batches; a weight gradient is a sum over the batch in another order
-            tp._few_rows_limits = (0, 0)
-            ref = [t.cpu().numpy() for t in (tp.forward(x, y, w), *tp.backward_helper(x, y, w, g))]
-            tp._few_rows_limits, tol = limits, 4 * TOL[dtype]
-        for a, b in zip(got, ref):
-            assert rel(a.cpu().numpy(), b) < tol
-        assert all(torch.equal(a, b) for a, b in zip(got[1:], tp.backward_helper(x, y, w, g)))
+            tp._few_rows = large
+            ref, tol = [t.cpu().numpy() for t in run()], 4 * TOL[dtype]
+        tp._few_rows, tp._few_rows_limits = own, kept
+        for a, c, b in zip(got, as_built, ref):
+            assert rel(a.cpu().numpy(), b) < tol and rel(c.cpu().numpy(), b) < tol
+        assert all(torch.equal(a, b) for a, b in zip(got[1:], again[1:]))

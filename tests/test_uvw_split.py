@@ -10,6 +10,7 @@ import openequivariance_amd as oeq
 from host_emu import emu
 from openequivariance_amd.codegen.uvw import UVWGenerator
 from openequivariance_amd.codegen.uvw_split import UVWSplitGenerator
+from openequivariance_amd.tensor_product import few_rows_generator
 from oracle import tp as otp
 from oracle import weights as ow
 
@@ -134,6 +135,10 @@ def test_directions_that_pay(name):
 def test_rows_left_to_the_kernels_for_few(irreps, kept):
     g = UVWSplitGenerator.create(common.fully_connected(irreps, shared=True, dtype=np.float32)[0])
     assert g.few_rows((8192, 65536)) == kept and g.few_rows((0, 0)) == (0, 0)
+    few, limits = few_rows_generator(g.problem, g)
+    assert (few is None) == (not any(limits)) and all(a <= b for a, b in zip(limits, kept))
+    if few is not None:
+        assert ("void forward(" in few.render()) == bool(few.plan()[0]) == (limits[0] > 0)
 
 
 # dW workgroups of several kinds: the one that stages most of dZ is not the one with most entries of the M table, and the two
