@@ -1,4 +1,6 @@
 """The counting sort that groups an unsorted edge list: ranges of nodes, the scan in LDS and in memory, several workgroups."""
+import subprocess
+
 import numpy as np
 import pytest
 import torch
@@ -77,6 +79,17 @@ def test_edge_positions_hold_32_bits():
         rows, cols = (torch.empty(edges, dtype=torch.int64, device="meta") for _ in range(2))
         with pytest.raises(ValueError, match=message):
             conv._check(x, y, w, rows, cols)
+
+
+def test_shares_cover_every_edge_list():
+    """A workgroup's share of the edges times the workgroups launched, up to the longest list that is taken."""
+    g = UVUSortedGenerator(common.channelwise(("2x0e+2x1o", "1x0e+1x1o", "2x0e+2x1o"))[0])
+    edges = [1, 1024, 1025, 32768, 32769, 4096 * 128, 4096 * 128 + 1, 2 ** 31, 2 ** 32 - 128, 2 ** 32 - 127, 2 ** 32 - 1]
+    main = "int main() { for (u64 n : {" + ", ".join(f"{n}ull" for n in edges) + '}) printf("%llu\\n", (unsigned long long)oeq_group_share(n)); }'
+    shares = subprocess.run([emu.build(g.render(prelude=emu.emu_prelude("float")), main)], capture_output=True, text=True, check=True).stdout.split()
+    step = next(s for s in g.plan()[0] if s["kernel"] == "group_count")
+    for n, share in zip(edges, map(int, shares)):
+        assert share % step["num_threads"] == 0 and share * emu.grid_of(step, n, 1) >= n
 
 
 @pytest.mark.gpu
