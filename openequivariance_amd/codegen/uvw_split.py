@@ -460,10 +460,11 @@ class UVWSplitGenerator(UVWGenerator):
         E(f"    if (idx < {pieces} && base0 + r_ < n) *(VTU*)({dst} + (base0 + r_) * {d} + 4 * col) = *(const VT*)(raw + r_ * {pitch} + 4 * col);")
         E("}")
 
-    def _products(self, E: Emitter, chunks, offs, blocks, row_block, tile: str, base, tiles_of, apply) -> None:
+    def _products(self, E: Emitter, chunks, offs, blocks, row_block, tile: str, base, tiles_of, apply, apart=lambda p: False) -> None:
         """The contractions of ``chunks``, one after the other, as slots of one product (a matrix step per path) with the
         loads of later slots and the Clebsch-Gordan part of finished paths (``apply``: a list of statements) spread
-        between them: a wavefront issues in order, and a burst of loads or vector instructions is time its matrix core idles."""
+        between them: a wavefront issues in order, and a burst of loads or vector instructions is time its matrix core idles.
+        ``apart``: paths whose five smaller products have an accumulator of their own."""
         KB = lambda ch: self.kblocks(blocks[row_block(ch[0])].mul)
         D = lambda ch: blocks[row_block(ch[0])].D
         steps = [(ci, kb) for ci, ch in enumerate(chunks) for kb in range(KB(ch))]
@@ -502,9 +503,10 @@ class UVWSplitGenerator(UVWGenerator):
             if kb == 0 and i == 0:
                 E(f"// paths {[p.t for p in ch]}")
                 for p in ch:
-                    E("V4 " + ", ".join(f"u{p.t}_{q} = {{0, 0, 0, 0}}" for q in range(D(ch))) + ";")
+                    E("V4 " + ", ".join(f"{nm}{p.t}_{q} = {{0, 0, 0, 0}}" for nm in ("us" if apart(p) else "u") for q in range(D(ch))) + ";")
             for sa, sb in PRODUCTS:
-                E(" ".join(f"u{p.t}_{i} = oeq_mfma_bf16(a{n}_{p.t}_{sa}, b{n}_{i}_{sb}, u{p.t}_{i}); OEQ_PIN(u{p.t}_{i});" for p in ch))
+                acc = [f"{'s' if sa + sb and apart(p) else 'u'}{p.t}_{i}" for p in ch]
+                E(" ".join(f"{u} = oeq_mfma_bf16(a{n}_{p.t}_{sa}, b{n}_{i}_{sb}, {u}); OEQ_PIN({u});" for p, u in zip(ch, acc)))
                 for _ in range(per):
                     if loads:
                         E(loads.pop(0))
@@ -516,6 +518,8 @@ class UVWSplitGenerator(UVWGenerator):
                 E("oeq_sched_fence();")
             if kb + 1 == KB(ch) and i + 1 == D(ch):
                 for p in ch:
+                    if apart(p):
+                        after += [f"u{p.t}_{q}[{r}] += s{p.t}_{q}[{r}];" for q in range(D(ch)) for r in range(4)]
                     after += apply(p)
         E.extend(after)
 
@@ -655,6 +659,15 @@ class UVWSplitGenerator(UVWGenerator):
         E("}")
 
     # ====================================================== backward: dX, dY
+    def _apart(self, p) -> bool:
+        """Whether V of a path sums its five smaller products apart from the largest.  An accumulator is a multiple of its last bit,
+        so what a small addend loses to it is a matter of the addend alone, and of operands of one sign that is much the same for
+all channels of a row: dY adds it up.  All operands in 0.5 .. 1.5, 4100 rows, relative error of dY against fp64, fp32
+        kernel / together / apart: 200 channels (l <= 1) 4.9e-8 / 4.3e-8, 256 scalars 4.7 / 5.6 / 4.3, 384 5.5 / 6.9 / 4.7, 512
+        5.4 / 8.2 / 4.2 (operands of mean zero 4.2e-7 / 3.4e-7 / 1.6e-7, dX 4.1e-7 / 3.4e-7 / 1.3e-7).  In time no difference: 256
+        scalars, 40 000 rows, backward 117 / 116 us, 256 channels, l <= 1, 20 000 rows 195 / 195."""
+        return self.kblocks(p.mw) >= 8
+
     @property
     def backward_threads(self) -> int:
         return self.bwd_shape.threads if self.split_dx else 256
@@ -738,7 +751,9 @@ class UVWSplitGenerator(UVWGenerator):
         else:
             self._zero_blocks(E, "Xg", self.D1, self.in1, self.used_in1)
         waves, tiles = shape.waves, shape.tiles
-        # ---- dY: sum over the 4 lane groups (channels), then over the tile's wavefronts, fixed order
+        # ---- dY: sum over the 4 lane groups (channels), then over the tile's wavefronts, in pairs: eight sums of one sign one
+        # after the other round at the size of the whole four times and more (512 channels, all operands positive: relative error
+        # against fp64 9.0e-8, in pairs 8.2e-8; 128 channels, l <= 1, 5.8e-8 and 4.4e-8, the fp32 kernel's four 5.3e-8)
         for f in self.used_y:
             E(f"dy{f} += oeq_shfl_xor(dy{f}, 16);")
             E(f"dy{f} += oeq_shfl_xor(dy{f}, 32);")
@@ -750,9 +765,10 @@ class UVWSplitGenerator(UVWGenerator):
         E(f"for (int q = threadIdx.x; q < {16 * tiles * self.D2}; q += {self.backward_threads}) {{")
         E(f"    const int r_ = q / {self.D2}, f = q - r_ * {self.D2};")
         E(f"    const T* __restrict__ s_ = dyl + ((r_ >> 4) * {16 * waves} + (r_ & 15)) * {self.D2} + f;")
-        E("    T sum = s_[0];")
-        E(f"    for (int w_ = 1; w_ < {waves}; ++w_) sum += s_[w_ * {16 * self.D2}];")
-        E(f"    if (base0 + r_ < n) Yg[(base0 + r_) * {self.D2} + f] = sum;")
+        terms = [f"s_[{w * 16 * self.D2}]" for w in range(waves)]
+        while len(terms) > 1:
+            terms = [f"({' + '.join(terms[q:q + 2])})" for q in range(0, len(terms), 2)]
+        E(f"    if (base0 + r_ < n) Yg[(base0 + r_) * {self.D2} + f] = {terms[0]};")
         E("}")
         return E.text()
 
@@ -789,10 +805,10 @@ class UVWSplitGenerator(UVWGenerator):
         for nt in sorted({p.NTU for p in self.paths if p.a.idx in ins}):
             paths = [p for p in self.paths if p.a.idx in ins and p.NTU == nt]
             chunks = [ch for o in sorted(self.used_out, key=lambda o: -self.out[o].D)
-                      for ch in self._chunks([p for p in paths if p.o.idx == o], lambda p: p.o.D, lambda p: p.NTU)]
+                      for ch in self._chunks([p for p in paths if p.o.idx == o], lambda p: p.o.D * (2 if self._apart(p) else 1), lambda p: p.NTU)]
             E(f"if (ut < {nt}) {{" if nt < NTU else "{")
             E.level += 1
-            self._products(E, chunks, offs, self.out, lambda p: p.o.idx, "ut", lambda p: p.wa, lambda p: p.NTU, apply)
+            self._products(E, chunks, offs, self.out, lambda p: p.o.idx, "ut", lambda p: p.wa, lambda p: p.NTU, apply, self._apart)
             E.level -= 1
             E("}")
         names = [f"dx{ai}_{r}_{i}" for ai in ins for r in range(4) for i in range(self.in1[ai].D)]

@@ -34,6 +34,7 @@ EMULATED = {
     "records stored directly, odd channels": ("5x0e+21x1o", "1x0e+1x1o+1x2e", "18x0e+7x1o+3x2e", 3, 37),
     "second operand in another order, a block no path reads, an output no path writes": ("33x0e+2x3o", "1x2e+1x0e", "34x0e+33x2e+4x1o", 2, 19),
     "several tiles for a dW workgroup, two of its kinds": ("70x0e+20x1o", "1x0e+1x1o", "68x0e+16x1o", 2, 150),
+    "eight K blocks: the smaller products of dX summed apart, and not": ("18x0e+17x1o", "1x0e+1x1o", "226x0e+18x1o", 4, 37),
 }
 
 
@@ -210,6 +211,28 @@ def test_gpu_small_and_large_operands(name):
     for a, b in zip((op.forward(X, Y, W), *op.backward_helper(X, Y, W, G)), refs):
         # (dW: a denormal T = M x of 1e-41 is rounded at 2^-149 in fp32 arithmetic of any kind, here at 2^-150; measured 2.5e-6)
         tol = 2.0 ** -149 / 1e-41 if b.ndim == 1 and name == "denormal rows" else 1e-6
+        assert float((a.double() - b).norm() / b.norm()) < tol
+
+
+# operands of one sign: all channels of a row meet the same roundings, and dY adds them up
+ONE_SIGN = {"64": (GPU["64"], True), "200, l <= 1": ((natural(200, 1), natural(1, 1), natural(200, 1)), True),
+            "256 scalars": (("256x0e", "1x0e", "256x0e"), True), "512 scalars": (("512x0e", "1x0e", "512x0e"), False)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ONE_SIGN)
+def test_gpu_operands_of_one_sign(name):
+    import torch
+    irreps, dw_kinds = ONE_SIGN[name]
+    prob, p64 = (common.fully_connected(irreps, shared=True, dtype=t)[0] for t in (np.float32, np.float64))
+    op, ref = oeq.TensorProduct(prob), oeq.TensorProduct(p64)
+    assert op.generator.split_forward and op.generator.split_dx and bool(op.generator.dw_kinds) == dw_kinds
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    X, Y, W, G = (torch.rand(*s, device="cuda", generator=gen) + 0.5
+                  for s in ((4100, prob.irreps_in1.dim), (4100, prob.irreps_in2.dim), (prob.weight_numel,), (4100, prob.irreps_out.dim)))
+    refs = (ref.forward(X.double(), Y.double(), W.double()), *ref.backward_helper(X.double(), Y.double(), W.double(), G.double()))
+    # fp32 matrix instructions: Z, dX up to 3.2e-7, dW 2.5e-7; dY up to 6e-8 - one rounding of a result is 3.4e-8
+    for a, b, tol in zip((op.forward(X, Y, W), *op.backward_helper(X, Y, W, G)), refs, (3.2e-7, 3.2e-7, 2.0 ** -24, 2.5e-7)):
         assert float((a.double() - b).norm() / b.norm()) < tol
 
 
