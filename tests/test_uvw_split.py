@@ -237,6 +237,61 @@ def test_gpu_operands_of_one_sign(name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name", ["64", "33 -> 47", "50, both parities"])
+def test_gpu_misaligned_and_strided_rows(name):
+    """Views that start at any word and rows cut from wider ones, in every operand: as for contiguous copies, bit for bit."""
+    import torch
+    prob, _ = common.fully_connected(GPU[name], shared=True, dtype=np.float32)
+    op = oeq.TensorProduct(prob, torch_op=True)
+    op._few_rows_limits = (0, 0)
+    operands = [torch.tensor(t, device="cuda") for t in common.tp_inputs(prob, 4099, 5, np.float32)]
+    def run(x, y, w, g):
+        x, y, w = (t.detach().requires_grad_() for t in (x, y, w))
+        z = op(x, y, w)
+        return [z.detach(), *torch.autograd.grad(z, (x, y, w), g)]
+    want = run(*operands)
+    for off in (1, 2, 3):
+        def shifted(t):
+            out = torch.empty(t.numel() + off, device="cuda")[off:].view(t.shape)
+            return out.copy_(t)
+        def cut(t):
+            wide = torch.full((*t.shape[:-1], t.shape[-1] + off + 2), float("nan"), device="cuda")
+            return wide[..., off:off + t.shape[-1]].copy_(t)
+        for view in (shifted, cut):
+            assert all(torch.equal(a, b) for a, b in zip(run(*map(view, operands)), want))
+    # results at any word, through the raw entry points
+    n, off = operands[0].shape[0], 3
+    x, y, w, g = (torch.empty(t.numel() + off, device="cuda")[off:].copy_(t.reshape(-1)) for t in operands)
+    dx, dy, dw = (torch.empty(t.numel() + 1, device="cuda")[1:] for t in operands[:3])
+    z = torch.empty(operands[3].numel() + 1, device="cuda")[1:]
+    op.forward_raw(n, x.data_ptr(), y.data_ptr(), z.data_ptr(), w.data_ptr())
+    op.backward_raw(n, x.data_ptr(), dx.data_ptr(), y.data_ptr(), dy.data_ptr(), w.data_ptr(), dw.data_ptr(), g.data_ptr())
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b.reshape(-1)) for a, b in zip((z, dx, dy, dw), want))
+
+
+@pytest.mark.gpu
+def test_gpu_streams_of_one_operator():
+    """Packed weights and partial sums lie in a workspace per stream: calls with weights of their own on four streams at once."""
+    import torch
+    prob, _ = common.fully_connected(GPU["64"], shared=True, dtype=np.float32)
+    op = oeq.TensorProduct(prob)
+    sets = [[torch.tensor(t, device="cuda") for t in common.tp_inputs(prob, 6001, seed, np.float32)] for seed in range(4)]
+    want = [[op.forward(*s[:3]), *op.backward_helper(*s)] for s in sets]
+    streams = [torch.cuda.Stream() for _ in sets]
+    torch.cuda.synchronize()
+    got = [[] for _ in sets]
+    for _ in range(3):
+        for q, (stream, s) in enumerate(zip(streams, sets)):
+            with torch.cuda.stream(stream):
+                got[q].append([op.forward(*s[:3]), *op.backward_helper(*s)])
+    torch.cuda.synchronize()
+    for q in range(len(sets)):
+        for out in got[q]:
+            assert all(torch.equal(a, b) for a, b in zip(out, want[q]))
+
+
+@pytest.mark.gpu
 def test_gpu_infinities_and_large_values():
     """Rows with an infinity, a NaN and values whose bf16 rounding is infinite; the other rows keep their accuracy."""
     import torch
