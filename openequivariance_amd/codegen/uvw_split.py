@@ -42,6 +42,8 @@ workgroup per compute unit (55 KB of LDS and 200 - 256 registers each).  Measure
 """
 from __future__ import annotations
 
+import threading
+from collections import OrderedDict
 from dataclasses import dataclass
 from functools import cached_property
 from typing import List
@@ -1250,6 +1252,28 @@ all channels of a row: dY adds it up.  All operands in 0.5 .. 1.5, 4100 rows, re
         return E.text()
 
     # ---------------------------------------------------------------- rendering
+    # Sources by problem, as writing one takes longer than all else a built operator does (64 channels, 11 paths, 780 KB: 15 ms,
+    # the fp32 kernels' 7): the layers of a model share it.  Bounded: the least recently asked for goes.
+    _SOURCES: "OrderedDict[tuple, str]" = OrderedDict()
+    _SOURCES_MAX = 16
+    _sources_lock = threading.Lock()
+
+    def render(self, prelude: str = None) -> str:
+        if prelude is not None:
+            return super().render(prelude)
+        key = self.problem.signature()
+        with self._sources_lock:
+            source = self._SOURCES.get(key)
+            if source is not None:
+                self._SOURCES.move_to_end(key)
+                return source
+        source = super().render()
+        with self._sources_lock:
+            self._SOURCES[key] = source
+            while len(self._SOURCES) > self._SOURCES_MAX:
+                self._SOURCES.popitem(last=False)
+        return source
+
     def describe(self) -> str:
         return super().describe().replace("mfma=16x16x4", "mfma=16x16x32 bf16 split in three")
 

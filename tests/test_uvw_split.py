@@ -105,6 +105,18 @@ def test_directions_and_rows():
             assert sum({"T": 4, "VT": 16, "U4": 16}[t] * eval(size) for t, size in arrays) <= UVWSplitGenerator.LDS_BYTES
 
 
+def test_operators_of_one_problem_share_a_source(monkeypatch):
+    """Written once for equal problems, and for no more than a few of them kept."""
+    monkeypatch.setattr(UVWSplitGenerator, "_SOURCES", type(UVWSplitGenerator._SOURCES)())
+    monkeypatch.setattr(UVWSplitGenerator, "_SOURCES_MAX", 2)
+    def generator(mul):
+        return UVWSplitGenerator(common.fully_connected((f"{mul}x0e", "1x0e", f"{mul}x0e"), shared=True, dtype=np.float32)[0])
+    first = generator(64).render()
+    assert generator(64).render() is first and generator(72).render() != first
+    generator(80).render()
+    assert len(UVWSplitGenerator._SOURCES) == 2 and generator(64).render() == first
+
+
 # Few wavefronts on a compute unit beside long rows: what was slower than the fp32 kernels (40 000 rows, both sides with the rules);
 # forward, dX / dY, dW on split operands
 DIRECTIONS = {
