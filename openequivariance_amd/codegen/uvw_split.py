@@ -32,10 +32,11 @@ groups of four channels concerned and until all of their sums are NaN.  64 chann
 Measured, 64x0e+64x1o+64x2e with 1x0e+1x1o+1x2e, fp32 kernels / these: 100 000 rows forward 291 / 175 us, backward 575 / 440 us;
 4097 rows 31 / 15 and 61 / 52; 100 channels, 50 000 rows 455 / 294 and 2048 / 690 (the fp32 dW walks the batch once per pass of
 accumulators there).  Relative errors against fp64 (2-norm; Z, dX, dY, dW) at 100 000 rows: 2.9e-7 1.6e-7 2.0e-7 7.7e-7 / 1.1e-7
-1.1e-7 1.6e-7 2.1e-7, and smaller than those of the kernels they replace on every problem of ``_pays``, 4097 and 50 000 rows.
+1.1e-7 1.6e-7 2.1e-7, and smaller than those of the kernels they replace on every problem of ``_pays``, 4097 and 50 000 rows, and on
+64 to 512 channels with all operands of one sign (dY too, ``_apart``).
 
-What bounds them: forward and dX/dY keep the matrix cores busy for 46 % of the time (bf16 steps at the clock under this load:
-84 of 175 us); the rest is weight fragments through L1 (270 KB per tile: 70 us when every one hits it, as measured with all
+What bounds them: the matrix cores are busy for 47 % of the forward's time, 34 % of dX/dY's and 37 % of dW's (counters); the rest of
+the first two is weight fragments through L1 (270 KB per tile: 70 us when every one hits it, as measured with all
 loads at one address), and what a workgroup does before its first product - rows in, split, two barriers - beside one other
 workgroup per compute unit (55 KB of LDS and 200 - 256 registers each).  Measured without gain: eight wavefronts per tile at
 128 registers (206 / 201), two tiles a workgroup (241 / 233), three or four paths a chunk (216 / 217).
