@@ -196,6 +196,13 @@ class UVWGenerator:
         self.bwd_rs = self._pick_row_stride()
         self.bwd_groups = [list(self.used_in1)]          # in1 blocks by group of wavefronts (one group: four wavefronts a tile)
         self.bwd_lds = 16 * self.bwd_rs * self.itemsize <= self.BWD_LDS_LIMIT
+        # What does not fit LDS is held in registers, an output block's dZ beside its weight fragments, but read in the K loop where
+        # these alone take a wavefront's 512: with hundreds of spilled registers dX was wrong on the device for 320x3o -> 320x3o
+        # (2.4e-2) and 512x1o -> 512x1o (0.7), the same source right on the host.  8192 rows, whole backward, held / in the loop, us:
+        # 320x3o 565 / 511, 512x2e 1142 / 1166, 600x1o 1043 / 1443, 16x1o -> 900x1o 220 / 262; blocks that fit: 180 channels,
+        # l <= 3, 1097 / 1143, 150 of both parities, l <= 2, 593 / 739.  fp64 stays as it is: no wrong result on 22 such problems.
+        held = max((_ceil(self.out[o].mul, 4) * (self.out[o].D + 1) for o in self.used_out), default=0)
+        self.bwd_direct = not self.bwd_lds and self.itemsize == 4 and held >= 512
         # packed weight copies in the workspace
         pos = 0
         for p in self.paths:
@@ -613,7 +620,7 @@ class UVWGenerator:
                     E(f"      {guard}{{ T* __restrict__ xp = Xg + (row0 + c) * {self.D1} + {a.off} + u * {a.D}; "
                       + " ".join(f"xp[{i}] = dx{a.idx}_{q}_{r}_{i};" for i in range(a.D)) + " } }")
                 E("}")
-        by_in1 = self.bwd_lds
+        by_in1 = self.bwd_lds or self.bwd_direct
         if by_in1:
             load_x(E, in1[0])
         else:
@@ -653,7 +660,7 @@ class UVWGenerator:
             pass
         elif self.bwd_lds:
             E("oeq_block_sync();")
-        else:
+        elif not self.bwd_direct:
             for oi in self.used_out:
                 o = self.out[oi]
                 E("T " + ", ".join(f"gz{oi}_{s_}_{k}" for s_ in range(_ceil(o.mul, 4)) for k in range(o.D)) + ";")
@@ -680,26 +687,30 @@ class UVWGenerator:
                 E(f"V4 acc{k} = {{0, 0, 0, 0}};")
             E(f"if ({cond}) {{")
             E.level += 1
-            if self.bwd_lds:
-                E(f"const T* __restrict__ gb = gl + c * {self.bwd_rs} + {o.off} + g * {o.D};")
+            if by_in1:
+                tile = f"gl + c * {self.bwd_rs}"
+                if not self.bwd_lds:         # (opaque: what one item has read is not to be kept for the next)
+                    E("int at_ = 0; OEQ_OPAQUE(at_);")
+                    tile = "Gr + at_"
+                E(f"const T* __restrict__ gb = {tile} + {o.off} + g * {o.D};")
             for s_ in range(SW):
-                if self.bwd_lds:
+                if by_in1:
                     if o.mul % 4 == 0:
                         E("{ const T " + ", ".join(f"b{k} = gb[{4 * s_ * o.D + k}]" for k in range(o.D)) + ";")
                     else:
-                        E(f"{{ const bool in_ = {4 * s_} + g < {o.mul}; const T* __restrict__ gq = in_ ? gb + {4 * s_ * o.D} : gl;")
+                        E(f"{{ const bool in_ = {4 * s_} + g < {o.mul}; const T* __restrict__ gq = in_ ? gb + {4 * s_ * o.D} : {'gl' if self.bwd_lds else 'Gr'};")
                         E("  const T " + ", ".join(f"b{k} = in_ ? gq[{k}] : (T)0" for k in range(o.D)) + ";")
                     E("  " + " ".join(f"acc{k} = oeq_mfma(af{j % NSETS}_{s_}, b{k}, acc{k});" for k in range(o.D)) + " }")
                 else:
                     E(" ".join(f"acc{k} = oeq_mfma(af{j % NSETS}_{s_}, gz{oi}_{s_}_{k}, acc{k});" for k in range(o.D)))
             E.level -= 1
             E("}")
-            if j + 1 < len(items) and (NSETS == 1 or (last_of_block and not self.bwd_lds)):
+            if j + 1 < len(items) and (NSETS == 1 or (last_of_block and not by_in1)):
                 # the fragment registers (one set) and, at the end of a block, the dZ registers are free
                 # from here on: request the next ones now, the vector-ALU part below covers the latency
                 if NSETS == 1:
                     load_a(E, j + 1)
-                if last_of_block and not self.bwd_lds:
+                if last_of_block and not by_in1:
                     load_gz(E, items[j + 1][0])
             E(f"if ({cond}) {{")
             E.level += 1
