@@ -32,6 +32,10 @@ class _DoublePlan:
         fwd, bwd, _ = self.plan()
         return fwd + bwd
 
+    def steps_few(self):
+        fwd, bwd, _ = self.plan_few()
+        return fwd + bwd
+
     @staticmethod
     def variant():
         """What the source depends on beside the problem."""
@@ -59,6 +63,7 @@ class UVUDetDoubleGenerator(_DoublePlan, DoubleArithmetic, UVUDetGenerator):
     # per launch) against this: 127 words 128 channels fp32 433 / 418, fp64 654 / 503, 64 channels fp64 566 / 411;
     # 254 words 32 channels fp32 532 / 490 (in one launch 870), 64 channels fp32 566 / 488, fp64 900 / 625 (one: 1121)
     SPLIT_WORDS = 144
+    TEAM_WAVES_MANY_WORDS = UVUDetGenerator.TEAM_WAVES         # (fp64, 64 channels, 1000 nodes: 266 / 213)
     CALL_FWD_ARGS = CALL_BWD_ARGS = CALL_ARGS
 
     def __init__(self, problem, **kw):

@@ -27,6 +27,7 @@ kernel reads both at the unpermuted position: templates/loop_unroll_conv_det.cuh
 from __future__ import annotations
 
 import contextlib
+import copy
 
 from .. import tunables
 from ..problem import TPProblem
@@ -121,7 +122,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         # a node that does not exist (see emit_invalid_edge_rows)
         part = f" + {self.dy_slots}ull * nnz * {self.D2} * sizeof(T)" if self.dy_slots > 1 else ""
         self.flags_off = f"((({self.dypart_off}{part}) + 7ull) & ~7ull)"
-        words = max(words_of(g_) for g_ in self.out_groups)
+        words = self.sender_words = max(words_of(g_) for g_ in self.out_groups)
         # fetch the next edge's operands while the current edge is being computed; pays when the
         # per-edge register footprint is small enough to keep several wavefronts per SIMD
         if prefetch_backward is None:
@@ -264,15 +265,15 @@ class UVUDetGenerator(UVUDirectGenerator):
 
     def forward_kernel_sources(self):
         """The forward's compute kernels as the templates emit them: name and body."""
-        return [dict(name=name, body=self.conv_det_forward_body(h)) for name, h in self.forward_kernels()]
+        return [dict(name=name, threads=WAVE * self.team, body=self.conv_det_forward_body(h)) for name, h in self.forward_kernels()]
 
     def forward_steps(self, step: dict):
         """One launch like ``step`` per group of output blocks."""
-        return [dict(step, kernel=name) for name, _ in self.forward_kernels()]
+        return [dict(step, kernel=name, num_threads=WAVE * self.team) for name, _ in self.forward_kernels()]
 
     def backward_kernel_sources(self):
         """The backward's compute kernels as the templates emit them: name, workgroup size, attributes, body."""
-        return [dict(name=name, threads=64, attr=self.backward_attr(), body=self.conv_det_backward_body(h))
+        return [dict(name=name, threads=WAVE * self.team, attr=self.backward_attr(), body=self.conv_det_backward_body(h))
                 for name, h in self.backward_kernels()]
 
     def act(self, blk):
@@ -387,6 +388,9 @@ class UVUDetGenerator(UVUDirectGenerator):
         E("node = oeq_uniform_u64(node); beg = (i64)oeq_uniform_u64((u64)beg); end = (i64)oeq_uniform_u64((u64)end);")
         if self.pieces:
             E("qh = oeq_uniform_u64(qh); npieces = __builtin_amdgcn_readfirstlane(npieces);")
+        if self.team > 1:
+            E("// this wavefront's part of the list")
+            E(f"{{ const i64 n_ = end - beg, b_ = beg; beg = b_ + n_ * wave_ / {self.team}; end = b_ + n_ * (wave_ + 1) / {self.team}; }}")
         E("const bool nv = node < node_count;")
         E("const int len = (int)(end - beg);")
         E(f"const int maxlen = (len + {R - 1}) / {R};")
@@ -403,6 +407,8 @@ class UVUDetGenerator(UVUDirectGenerator):
         for blk in blocks:
             if blk.idx in used and blk.dim:
                 self.emit_sub_sum(E, regs_of(blk))
+        if self.team > 1:
+            self.emit_team_sum(E, [n for blk in blocks if blk.idx in used and blk.dim for n in regs_of(blk)])
 
         def store(E, base: str, row: str, existing: bool, zero: bool, agent: bool = False):
             for blk in blocks:
@@ -493,6 +499,106 @@ class UVUDetGenerator(UVUDirectGenerator):
         E.level -= 1
         E("}")
 
+    # ---- several wavefronts per node
+    # On a graph of few nodes a launch lasts as long as one wavefront's walk over a node's edges, and the chip is empty beside it
+    # (1000 nodes: one wavefront per SIMD).  There a node's list is cut into TEAM parts of equal length, a wavefront each,
+    # whose sums are added through LDS in the order of the list: fixed for a graph's size, so results repeat bit for bit.
+    # All nodes are in flight at once then and need no order (order_backward, 4 - 6 us, is not launched).  Receiver pass,
+    # sender pass with its preparation, and double backward, us, one wavefront / four:
+    #   32 channels, 11 paths   200 nodes, 24 edges each 16.5 / 10.6, 35 / 16, 70 / 32; 1000 nodes 22 / 17, 43 / 37, 83 / 73
+    #   64 channels, l <= 1     500 nodes 21.5 / 11.6, 33 / 15, 68 / 30; 2000 nodes 29 / 17, 47 / 35, 89 / 75
+    #   128 channels, 13 paths  200 nodes 36 / 18, 106 / 45, 180 / 80; 1000 nodes 57 / 52, 142 / 144, 265 / 240
+    # Four: with two wavefronts the small graphs keep half of the gain (200 nodes, 32 channels 35 -> 21 us for the sender pass),
+    # with eight LDS holds the stages of few nodes (1000 nodes, 32 channels: receiver pass 28 us).
+    TEAM = 4
+    TEAM_WAVES = 2048             # row groups (workgroups x lane groups) up to which a team walks a node (0: never)
+    TEAM_MANY_WORDS, TEAM_WAVES_MANY_WORDS = 40, 768         # ... in the sender pass with more operand words per edge than this
+    TEAM_LDS = 160 * 1024         # of a compute unit; problems whose teams would need more keep single wavefronts
+    team, team_lds = 1, 0         # wavefronts that walk one node's edges here; LDS they share, bytes (as emitted)
+    few_sources = {"forward": [], "backward": []}            # kernels for few nodes beside the others (add_few_nodes)
+
+    def team_twin(self, team: int = TEAM):
+        """This generator with teams of wavefronts, on the same workspace."""
+        twin = copy.copy(self)
+        twin.team, twin.ordered_backward = team, False
+        return twin
+
+    def add_few_nodes(self, which=("forward", "backward")):
+        """Adds the kernels for few nodes to what is rendered, and to the launch plans of ``plan_few``."""
+        twin = self.team_twin()
+        kernels = dict(forward=twin.forward_kernel_sources, backward=twin.backward_kernel_sources)
+        sources = {w: [dict(k, name=k["name"] + "_few") for k in kernels[w]() if k["threads"] > WAVE] for w in which}
+        if twin.team_lds <= self.TEAM_LDS:
+            self.few_sources = {"forward": [], "backward": [], **{w: sources[w] for w in which if self.few_limits(w)[0]}}
+        return self
+
+    def few_limits(self, which: str):
+        """(nodes, edges per node): a team walks the nodes of graphs of at most so many nodes and at least so many edges for
+        each: few enough workgroups, and two turns of the edge loop for each wavefront.  Both sides of the lines, one
+        wavefront / four: receiver pass, 24 edges a node: 64 channels (one row group), 2000 nodes 26 / 15 us, 4000 32 / 27; 32
+        channels (two) 1000 nodes 20.1 / 14.3, 2000 23.8 / 28.9; 16 channels (four) 500 nodes 10.6 / 8.7, 1000 11.3 / 14.8;
+        8 channels (eight) 200 nodes 7.8 / 7.5, 500 9.6 / 12.9; 8 edges a node there (one turn) 5.3 / 6.8.  Sender pass, more
+        words per edge: fp64, 64 channels, 11 paths, 500 nodes 96 / 75, 1000 nodes 129 / 135; fewer: 64 channels, l <= 1,
+        2000 nodes 47 / 35."""
+        many = which == "backward" and self.R == 1 and self.sender_words > self.TEAM_MANY_WORDS
+        return (min(self.TEAM_WAVES, self.TEAM_WAVES_MANY_WORDS) if many else self.TEAM_WAVES) // (self.NCH * self.R), 2 * self.R
+
+    def few_steps(self, which: str, steps):
+        """The launches ``steps`` with those for few nodes beside those that they replace there."""
+        names, out = {k["name"] for k in self.few_sources[which]}, []
+        for s in steps:
+            if s["kernel"] + "_few" in names:
+                out += [dict(s, many_nodes=self.few_limits(which)),
+                        dict(s, kernel=s["kernel"] + "_few", num_threads=WAVE * self.TEAM, few_nodes=self.few_limits(which))]
+            else:
+                out.append(dict(s, many_nodes=self.few_limits(which)) if names and s["kernel"] == "order_backward" else s)
+        return out
+
+    def plan_few(self):
+        fwd, bwd, ws = self.plan()
+        return self.few_steps("forward", fwd), self.few_steps("backward", bwd), ws
+
+    def emit_lane_direct(self, E: Emitter, lds: bool = False) -> None:
+        if self.team == 1:
+            super().emit_lane_direct(E, lds=lds)
+            return
+        E("const int wave_ = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;")
+        E(f"const int sub = lane >> {self.LOGP};")
+        E(f"const int ul = lane & {self.P - 1};")
+        if lds and self.lds_elems:
+            E(f"__shared__ __attribute__((aligned(16))) T lds[{self.lds_elems}];")
+
+    def emit_stage(self, E: Emitter, words: int, sums: int) -> None:
+        """The LDS stage of a wavefront (``words`` of 4 bytes; 0: none).  The wavefronts of a team have one each, and leave
+        their ``sums`` values per lane in the same memory when the loop is over."""
+        if self.team == 1:
+            if words:
+                E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{words}];")
+            return
+        area = max(4 * words * self.team, self.itemsize * WAVE * sums * (self.team - 1))
+        self.team_lds = max(self.team_lds, area + self.lds_elems * self.itemsize)
+        E(f"__shared__ __attribute__((aligned(16))) unsigned char team_[{area}];")
+        if words:
+            E(f"{self.stage_type()}* stage = ({self.stage_type()}*)team_ + wave_ * {words};")
+
+    @staticmethod
+    def _sums(blocks, used) -> int:
+        return sum(b.D for b in blocks if b.idx in used and b.dim)
+
+    def emit_team_sum(self, E: Emitter, names) -> None:
+        """The team's sums of the registers ``names`` in its first wavefront, in the order of the edge list; the others are
+        done."""
+        E("oeq_block_sync();")
+        E(f"T* __restrict__ part_ = (T*)team_ + lane;")
+        E("if (wave_ > 0) {")
+        E(f"    T* __restrict__ q_ = part_ + (wave_ - 1) * {len(names) * WAVE};")
+        E("    " + " ".join(f"q_[{i * WAVE}] = {n};" for i, n in enumerate(names)))
+        E("}")
+        E("oeq_block_sync();")
+        E("if (wave_ > 0) return;")
+        for t in range(self.team - 1):
+            E(" ".join(f"{n} += part_[{(t * len(names) + i) * WAVE}];" for i, n in enumerate(names)))
+
     def ld(self, ptr: str, idx) -> str:
         return f"oeq_ldnt({ptr} + {idx})" if self.nontemporal else f"{ptr}[{idx}]"
 
@@ -521,12 +627,12 @@ class UVUDetGenerator(UVUDirectGenerator):
         return dict(kernel="order_backward", num_threads=self.ORDER_THREADS, grid_kind=0, num_blocks=1, prep=True)
 
     def order_bytes(self, nodes: int) -> int:
-        return nodes * 8 if self.ordered_backward else 0
+        return nodes * 8              # (kept where no order is written: teams share the workspace of single wavefronts)
 
     def backward_steps(self):
         """Launches of the segmented backward behind the pointer / position-list preparation."""
         steps = [self.order_step()] if self.ordered_backward else []
-        steps += [dict(kernel=name, num_threads=64, grid_kind=3, work_per_block=1, num_blocks=self.LONG, grid_y=self.NCH)
+        steps += [dict(kernel=name, num_threads=WAVE * self.team, grid_kind=3, work_per_block=1, num_blocks=self.LONG, grid_y=self.NCH)
                   for name, _ in self.backward_kernels()]
         if self.dy_slots > 1:
             steps.append(dict(kernel="backward_dy_reduce", num_threads=256, grid_kind=1,
@@ -547,7 +653,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         preparation kernels leave one flag per 256 edges; the first workgroup of every (chunk, group)
         launch row ORs them and, only if some edge is flagged, walks the edge list and writes zeros into
         the rows of those edges: dW and dY (or this launch's dY partial slot)."""
-        E("if (bx_ == 0) {")
+        E("if (bx_ == 0" + (" && wave_ == 0) {" if self.team > 1 else ") {"))
         E.level += 1
         E("const int* __restrict__ bad_ = (const int*)((const char*)ws + FLAGS_OFF);")
         E("int any_ = 0;")
@@ -668,6 +774,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         if self.lds_forward:
             self._emit_staged_forward(E, compute)
         else:
+            self.emit_stage(E, 0, self._sums(self.out, self.used_out))
             self.emit_pingpong_loop(E, names, load_idx, load, compute)
         E("const bool rv = nv;")
         self.emit_node_output(E, self.out, self.used_out, lambda o: [f"z{o.idx}_{k}" for k in range(o.D)], self.NODE_OUT, self.D3,
@@ -972,6 +1079,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         if self.staged_backward:
             self._emit_staged_backward(E, compute, grp)
         else:
+            self.emit_stage(E, 0, self._sums(self.in1, self.used_in1))
             self.emit_pingpong_loop(E, names, load_idx, load, compute, prefetch_first=self.prefetch_backward)
         E("rv = nv;")
         self.emit_node_output(E, self.in1, self.used_in1, lambda a: [f"dx{a.idx}_{m}" for m in range(a.D)], "Xg", self.D1,
@@ -1056,7 +1164,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         nt = 2 if self.nontemporal else 0
         slabs, words = self._forward_slabs()
         y_off = words - WAVE * len(self.EDGE_Y)
-        E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{words}];")
+        self.emit_stage(E, words, self._sums(self.out, self.used_out))
 
         def dma(E, e, n):
             E("{")
@@ -1096,7 +1204,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         y_off = self._edge_slabs(slabs, off)
         off = y_off + WAVE * len(self.EDGE_Y)
         assert off <= self.stage_words
-        E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{off}];")
+        self.emit_stage(E, off, self._sums(self.in1, self.used_in1))
 
         def dma(E, e, n):
             E("{")

@@ -25,8 +25,9 @@ tiles: the dZ row of a receiver whose edges span two tiles is then re-read from 
 from __future__ import annotations
 
 from ..problem import TPProblem
-from .common import Emitter
+from .common import Emitter, WAVE
 from .uvu_det import UVUDetGenerator
+from .uvu_direct import UVUDirectGenerator
 
 
 class UVURecvGenerator(UVUDetGenerator):
@@ -64,6 +65,7 @@ class UVURecvGenerator(UVUDetGenerator):
         self.lds_backward = False
         self.waves_per_eu = 0
         self.ordered_backward = False
+        self.sender_words = 0                                     # (pass 2 holds a row of dX and nothing else)
         # words of dX one lane produces per edge (= spill words per lane)
         self.NW = sum(self.in1[i].D for i in self.used_in1)
         self.spill_row = self.NCH * self.NW * self.P              # words per edge
@@ -127,9 +129,9 @@ class UVURecvGenerator(UVUDetGenerator):
 
     # ------------------------------------------------------------------ plan
     def backward_steps(self):
-        steps = [dict(kernel=name, num_threads=64, grid_kind=1, work_per_block=self.MIN_TILE_ITERS * self.R,
+        steps = [dict(kernel=name, num_threads=WAVE, grid_kind=1, work_per_block=self.MIN_TILE_ITERS * self.R,
                       num_blocks=self.MAX_TILES, grid_y=self.NCH) for name, _ in self.backward_kernels()] \
-            + [dict(kernel="backward_dx", num_threads=64, grid_kind=3, work_per_block=1, num_blocks=self.LONG, grid_y=self.NCH)]
+            + [dict(kernel="backward_dx", num_threads=WAVE * self.team, grid_kind=3, work_per_block=1, num_blocks=self.LONG, grid_y=self.NCH)]
         if self.dy_slots > 1:
             steps.append(dict(kernel="backward_dy_reduce", num_threads=256, grid_kind=1,
                               work_per_block=self.dy_rows_per_block))
@@ -185,14 +187,14 @@ class UVURecvGenerator(UVUDetGenerator):
             with self._group(h, self.recv_groups):
                 w = self.group_waves_hint()
             return f" __attribute__((amdgpu_waves_per_eu({w}, {w})))" if w else ""
-        return [dict(name=name, threads=64, attr=attr(h), body=self._edges_body(h)) for name, h in self.backward_kernels()] \
-            + [dict(name="backward_dx", threads=64, attr="", body=self._dx_body())]
+        return [dict(name=name, threads=WAVE, attr=attr(h), body=self._edges_body(h)) for name, h in self.backward_kernels()] \
+            + [dict(name="backward_dx", threads=WAVE * self.team, attr="", body=self._dx_body())]
 
     # ---------------------------------------------------------------- pass 1
     def _edges_body(self, h: int = 0) -> str:
         E = Emitter()
         R, P, NCH = self.R, self.P, self.NCH
-        self.emit_lane_direct(E, lds=False)
+        UVUDirectGenerator.emit_lane_direct(self, E, lds=False)              # (a tile is one wavefront's)
         with self._group(h, self.recv_groups):
             return self._edges_body_staged(E, h) if self.uses_stage else self._edges_body_registers(E, h)
 
@@ -521,6 +523,7 @@ class UVURecvGenerator(UVUDetGenerator):
         def key(E, pos):
             E(f"{{ const i64 e0_ = (i64)elist[{pos}]; if (e0_ >= 0 && e0_ < (i64)nnz) kv_ = (i64)cols[e0_]; }}")
         self._node_setup(E, self.bwd_ptr_off, key=key)
+        self.emit_stage(E, 0, self.NW)
         E(f"const T* __restrict__ spill = (const T*)((const char*)ws + {self.spill_off});")
         E("T " + ", ".join(f"acc{w} = (T)0" for w in range(self.NW)) + ";")
         E(f"for (int it = 0; it < maxlen; it += {U}) {{")

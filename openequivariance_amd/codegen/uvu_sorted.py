@@ -126,6 +126,17 @@ class UVUSortedGenerator:
             return ((main + 255) & ~255) + b.piece_bytes(nnz, nodes)
         return fwd, bwd, ws
 
+    def add_few_nodes(self):
+        """See UVUDetGenerator.add_few_nodes (the per-edge backward has no nodes to share)."""
+        self.fwd.add_few_nodes(("forward",))
+        if self.grouped_backward:
+            self.bwd.add_few_nodes(("backward",))
+        return self
+
+    def plan_few(self):
+        fwd, bwd, ws = self.plan()
+        return self.fwd.few_steps("forward", fwd), self.bwd.few_steps("backward", bwd) if self.grouped_backward else bwd, ws
+
     def forward_workspace_model(self):
         """(fixed, per node, per edge) bytes the forward steps use when no node is cut into pieces."""
         return 32, 24, 8

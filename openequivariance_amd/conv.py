@@ -131,6 +131,11 @@ def select_conv_generator(config: TPProblem, deterministic: bool, vector_stores:
     return UVUSortedGenerator(config, vector_stores=vector_stores, idx_ctype=idx_ctype)
 
 
+def with_few_nodes(generator):
+    """``generator`` with the kernels for graphs of few nodes beside the others, as the operators build it."""
+    return generator.add_few_nodes() if hasattr(generator, "add_few_nodes") else generator
+
+
 class _StreamWorkspace:
     """Device scratch of one operator on one stream, and which graph its preparation areas
     (CSR pointers, position lists, node order) currently describe."""
@@ -179,7 +184,7 @@ class TensorProductConv:
         if mode != "uvu":
             raise NotImplementedError("TensorProductConv supports uvu problems")
 
-        self.generator = select_conv_generator(config, deterministic, idx_dtype=self.idx_dtype)
+        self.generator = with_few_nodes(select_conv_generator(config, deterministic, idx_dtype=self.idx_dtype))
         # True: the forward writes every row of Z itself; False: it accumulates into a zeroed Z
         self.forward_overwrites = not isinstance(self.generator, UVUDirectGenerator) or deterministic
         # likewise for dX in the backward (the per-edge backward accumulates with atomics)
@@ -219,9 +224,9 @@ class TensorProductConv:
             self._setup_torch_module()
 
     def _build(self, generator, source=None) -> "rt.ConvImpl":
-        """Compile one kernel set of this operator.  Every set shares the operator's workspace, which is
+        """Compile one kernel set of this operator (``with_few_nodes``).  Every set shares the operator's workspace, which is
         sized for the largest of them."""
-        fwd, bwd, ws = generator.plan()
+        fwd, bwd, ws = getattr(generator, "plan_few", generator.plan)()
         self._ws_fns.append(ws)
         need_ws = rt.STEP_NEEDS_WORKSPACE if ws(1, 1) > 0 else 0
         need_tp = rt.STEP_NEEDS_TPERM if self.backward_needs_tperm else 0
@@ -241,8 +246,8 @@ class TensorProductConv:
         """(kernel set, whether its backward overwrites dX) of a backward variant of the unsorted operator,
         compiled on first need."""
         if name not in self._bwd_variants:
-            g = UVUSortedGenerator(self.config, grouped_backward=(name == "grouped"),
-                                   idx_ctype="i64" if self.idx_dtype == np.int64 else "int")
+            g = with_few_nodes(UVUSortedGenerator(self.config, grouped_backward=(name == "grouped"),
+                                                  idx_ctype="i64" if self.idx_dtype == np.int64 else "int"))
             self._bwd_variants[name] = (self._build(g), name == "grouped")
             for rec in self._workspaces.values():            # the workspace may have to grow: sizes are re-checked per call
                 rec.bwd_key = None
@@ -258,8 +263,8 @@ class TensorProductConv:
         idx = "i64" if self.idx_dtype == np.int64 else "int"
 
         def build():
-            g = conv_double_generator(self.config, self.deterministic, idx)
-            return g.render(), (g.steps(), g.plan()[2])
+            g = with_few_nodes(conv_double_generator(self.config, self.deterministic, idx))
+            return g.render(), (g.steps_few(), g.plan()[2])
         need = rt.STEP_NEEDS_WORKSPACE | (rt.STEP_NEEDS_TPERM if self.deterministic else 0)
         impl, (_, ws) = rt.variant(("conv double", self.config.signature(), self.deterministic, idx,
                                     UVUDetDoubleGenerator.variant()), torch.cuda.current_device(), build,
@@ -372,7 +377,8 @@ class TensorProductConv:
             bits |= int(p)
         if bits % 16:
             if self._internal_unaligned is None:
-                g = select_conv_generator(self.config, self.deterministic, vector_stores=False, idx_dtype=self.idx_dtype)
+                g = with_few_nodes(select_conv_generator(self.config, self.deterministic, vector_stores=False,
+                                                         idx_dtype=self.idx_dtype))
                 self._internal_unaligned = self._build(g)
             return self._internal_unaligned
         return self.internal

@@ -68,6 +68,8 @@ int load_steps(Module& m, const void* code, size_t code_size, const oeq_step* st
             return fail("step %d (%s): bad workgroup size %u", i, s.desc.kernel, s.desc.num_threads);
         if (s.desc.grid_kind > OEQ_GRID_PER_NODE_AND_PIECE)
             return fail("step %d (%s): unknown grid rule %u", i, s.desc.kernel, s.desc.grid_kind);
+        if ((s.desc.flags & OEQ_STEP_FEW_NODES(0, 0)) && (s.desc.flags & OEQ_STEP_MANY_NODES(0, 0)))
+            return fail("step %d (%s): for few nodes and for many", i, s.desc.kernel);
         if (s.desc.grid_kind != OEQ_GRID_FIXED && s.desc.work_per_block == 0)
             return fail("step %d (%s): work_per_block must be > 0", i, s.desc.kernel);
         if (s.desc.grid_kind == OEQ_GRID_FIXED && s.desc.num_blocks == 0)
@@ -331,8 +333,14 @@ int oeq_conv_create(const void* code, size_t code_size, const oeq_step* fs, int 
 
 void oeq_conv_destroy(oeq_conv* c) { delete c; }
 
-// A step is skipped when the call says that the state it would build is already in the workspace.
-static bool skipped(const oeq_step& d, uint32_t call_flags) {
+// A step is skipped on graphs of another size than it is for, and when the call says that the state it would build is already
+// in the workspace.
+static bool skipped(const oeq_step& d, uint32_t call_flags, uint64_t nnz, uint64_t nodes) {
+    const uint32_t sizes = d.flags & (OEQ_STEP_FEW_NODES(0, 0) | OEQ_STEP_MANY_NODES(0, 0));
+    if (sizes) {
+        const bool few = nodes <= ((d.flags >> 8) & 0xfff) && nnz >= ((d.flags >> 20) & 0xff) * nodes;
+        if (few != (sizes == OEQ_STEP_FEW_NODES(0, 0))) return true;
+    }
     if ((call_flags & OEQ_CALL_PREPARED) && (d.flags & OEQ_STEP_GRAPH_PREP)) return true;
     if ((call_flags & OEQ_CALL_COUNTERS_ZERO) && (d.flags & OEQ_STEP_COUNTER_CLEAR)) return true;
     return false;
@@ -351,7 +359,7 @@ static int conv_forward(oeq_conv* c, const void* L1, const void* L2, const void*
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("forward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     for (auto& s : c->fwd) {
-        if (skipped(s.desc, call_flags)) continue;
+        if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream, pieces)) return 1;
     }
     return 0;
@@ -370,7 +378,7 @@ static int conv_backward(oeq_conv* c, const void* L1, void* L1g, const void* L2,
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L1g, &L2, &L2g, &W, &Wg, &L3g, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     for (auto& s : c->bwd) {
-        if (skipped(s.desc, call_flags)) continue;
+        if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream)) return 1;
     }
     return 0;
@@ -413,7 +421,7 @@ int oeq_conv_double_backward_ex(oeq_conv* c, const void* L1, const void* L2, con
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("double backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3g, &L1c, &L2c, &Wc, &L1o, &L2o, &Wo, &L3o, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     for (auto& s : c->bwd) {
-        if (skipped(s.desc, call_flags)) continue;
+        if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream)) return 1;
     }
     return 0;

@@ -15,7 +15,7 @@ from .codegen.uvu_conv_double import conv_double_generator
 from .codegen.uvu_double import UVUDoubleGenerator
 from .codegen.uvw import UVWGenerator
 from .codegen.uvw_split import UVWSplitGenerator
-from .conv import select_conv_generator
+from .conv import select_conv_generator, with_few_nodes
 from .problem import ChannelwiseTPP, FullyConnectedTPProblem, TPProblem
 from .tensor_product import few_rows_generator, select_generator
 from .workloads import get as get_workload
@@ -39,8 +39,8 @@ def benchmark_generators():
             gens.append((label + " double backward", UVUDoubleGenerator(problem)))
 
     def conv(label, problem, deterministic):
-        gens.append((label, select_conv_generator(problem, deterministic)))
-        gens.append((label + " double backward", conv_double_generator(problem, deterministic)))
+        gens.append((label, with_few_nodes(select_conv_generator(problem, deterministic))))
+        gens.append((label + " double backward", with_few_nodes(conv_double_generator(problem, deterministic))))
 
     tp("readme/tp", readme)
     tp("mace/tp", ChannelwiseTPP(*MACE))

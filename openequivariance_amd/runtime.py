@@ -25,6 +25,7 @@ TARGET_ARCH = "gfx950"
 
 GRID_FIXED, GRID_PER_ROW, GRID_PER_NODE, GRID_PER_NODE_AND_PIECE = 0, 1, 2, 3
 STEP_NEEDS_WORKSPACE, STEP_NEEDS_TPERM, STEP_GRAPH_PREP, STEP_COUNTER_CLEAR = 1, 2, 4, 8
+STEP_FEW_NODES, STEP_MANY_NODES = 16, 32
 CALL_PREPARED, CALL_COUNTERS_ZERO = 1, 2
 PIECE_MIN_EDGES = 32                     # OEQ_PIECE_MIN_EDGES
 NOALLOC_SCRATCH_BYTES = 16 << 20        # OEQ_NOALLOC_SCRATCH_BYTES
@@ -37,6 +38,18 @@ class DeviceProp(C.Structure):
                 ("maxSharedMemPerBlock", C.c_int64), ("totalGlobalMem", C.c_int64),
                 ("clockRateKHz", C.c_int32), ("memoryClockRateKHz", C.c_int32),
                 ("memoryBusWidth", C.c_int32), ("l2CacheSize", C.c_int32)]
+
+
+def step_few_nodes(nodes: int, edges_per_node: int) -> int:
+    """OEQ_STEP_FEW_NODES with its limits: the step runs on graphs of at most ``nodes`` nodes and at least ``edges_per_node`` times
+    as many edges."""
+    assert 0 < nodes < 4096 and 0 <= edges_per_node < 256
+    return STEP_FEW_NODES | nodes << 8 | edges_per_node << 20
+
+
+def step_many_nodes(nodes: int, edges_per_node: int) -> int:
+    """OEQ_STEP_MANY_NODES: the step runs on all other graphs."""
+    return step_few_nodes(nodes, edges_per_node) ^ STEP_FEW_NODES ^ STEP_MANY_NODES
 
 
 class Step(C.Structure):

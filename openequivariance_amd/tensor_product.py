@@ -32,11 +32,16 @@ from .wigner import wigner_3j
 def _make_steps(descs, flags: int = 0):
     """Plan dictionaries of a generator -> ``runtime.Step`` records.  ``flags`` (STEP_NEEDS_*) apply to
     every step of the plan; a step's own ``prep=True`` marks it as graph preparation, ``counter_clear=True``
-    as one that only zeroes counters which the operator's other steps leave zeroed again."""
+    as one that only zeroes counters which the operator's other steps leave zeroed again, ``few_nodes`` / ``many_nodes`` =
+    (nodes, edges per node) as one that runs only on / never on graphs of few nodes."""
+    def size_rule(d):
+        if "few_nodes" in d:
+            return rt.step_few_nodes(*d["few_nodes"])
+        return rt.step_many_nodes(*d["many_nodes"]) if "many_nodes" in d else 0
     return [rt.Step.make(d["kernel"], d["num_threads"], d.get("smem", 0), d.get("grid_kind", rt.GRID_PER_ROW),
                          d.get("work_per_block", 1), d.get("num_blocks", 0), d.get("grid_y", 1),
                          flags | (rt.STEP_GRAPH_PREP if d.get("prep") else 0)
-                         | (rt.STEP_COUNTER_CLEAR if d.get("counter_clear") else 0)) for d in descs]
+                         | (rt.STEP_COUNTER_CLEAR if d.get("counter_clear") else 0) | size_rule(d)) for d in descs]
 
 
 class _NoSwitch:
