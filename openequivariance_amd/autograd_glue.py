@@ -25,26 +25,62 @@ def _operators() -> "torch.library.Library":
         return _library
 
 
-def define_operator(name: str, arguments, returns: str, implementation, fake, device: str = "CUDA"):
-    """Operator ``name`` with tensor ``arguments``, its GPU implementation and its fake kernel.  Registered without the
+class Native:
+    """An operator's part in the C++ kernels (csrc/oeq_torch.cpp): what they run, and the scratch that they are lent.  None of it
+    is taken back: operators live as long as the process."""
+    KINDS = {"tp_forward": 0, "tp_backward": 1, "tp_double": 2, "conv_forward": 3, "conv_backward": 4, "conv_double": 5}
+
+    def __init__(self, id: int):
+        self.id, self.ops = id, getattr(torch.ops, NAMESPACE)
+
+    @classmethod
+    def create(cls, handles, dtype64, index64, dims, scratch=0, conv=False, shared=False, deterministic=False, tuned=False,
+               few_limits=(0, 0), first=(), second=()):
+        """``handles``: kernel sets (main, for few rows, of the double backward; None where there is none).  None where the
+        main one is not a handle of the C library."""
+        from . import runtime as rt
+        raw = [getattr(getattr(h, "_h", None), "value", None) or 0 for h in handles]
+        if not raw[0]:
+            return None
+        _operators()
+        ops = getattr(torch.ops, NAMESPACE)
+        ops.native_library(rt.entry_points())
+        return cls(ops.native_operator([int(dtype64), int(index64), *dims, int(scratch), int(conv), int(shared), int(deterministic),
+                                        int(tuned), *raw, *few_limits], [int(v) for t in first for v in t],
+                                       [int(v) for t in second for v in t]))
+
+
+def define_operator(name: str, arguments, returns: str, implementation, fake, device: str = "CUDA", native=None, kind: str = ""):
+    """Operator ``name`` with tensor ``arguments``, its GPU implementation and its fake kernel.  With ``native`` the C++ kernel
+    of ``kind`` is its implementation, and ``implementation`` that of the operator ``name``_general, which takes what the kernel
+    leaves.  Registered without the
     wrappers of torch.library.custom_op, which take as long per call as launching a small product does: a forward without
     a graph 14 -> 4.5 us of dispatch, a training step 104 -> 51 us (one CPU, kernels left out; 45 us of that is what
     torch's own product of three tensors takes)."""
     lib = _operators()
-    lib.define(f"{name}({', '.join('Tensor ' + a for a in arguments)}) -> {returns}", tags=(torch.Tag.pt2_compliant_tag,))
-    lib.impl(name, torch._disable_dynamo(implementation), device)
+    general = name if native is None else name + "_general"
+    for n in {name, general}:
+        lib.define(f"{n}({', '.join('Tensor ' + a for a in arguments)}) -> {returns}", tags=(torch.Tag.pt2_compliant_tag,))
+    lib.impl(general, torch._disable_dynamo(implementation), device)
+    if native is not None:
+        native.ops.native_kernel(NAMESPACE, name, general, native.id, native.KINDS[kind])
     torch.library.register_fake(f"{NAMESPACE}::{name}", fake, lib=lib)
     return getattr(getattr(torch.ops, NAMESPACE), name).default
 
 
-def define_derivatives(forward: str, backward: str, arguments, second_derivatives) -> None:
+def define_derivatives(forward: str, backward: str, arguments, second_derivatives, native=None, fused=None) -> None:
     """Makes operator ``backward`` (arguments: the first three, the output's gradient, the rest) the derivative of
-    ``forward``, and ``second_derivatives(x, y, w, dz, ddx, ddy, ddw, *index)`` that of ``backward``."""
+    ``forward``, and ``second_derivatives(x, y, w, dz, ddx, ddy, ddw, *index)`` that of ``backward``: with ``native`` and the name
+    of the ``fused`` operator, where that one cannot serve directly."""
     lib = _operators()
     name, index = backward + "_derivative", list(arguments[3:])
     names = [*arguments[:3], "L3_grad", "L1_cot", "L2_cot", "weights_cot", *index]
-    lib.define(f"{name}({', '.join('Tensor ' + a for a in names)}) -> Tensor[]")
-    lib.impl(name, second_derivatives, "CompositeImplicitAutograd")
+    general = name if native is None or fused is None else name + "_general"
+    for n in {name, general}:
+        lib.define(f"{n}({', '.join('Tensor ' + a for a in names)}) -> Tensor[]")
+    lib.impl(general, second_derivatives, "CompositeImplicitAutograd")
+    if general != name:
+        native.ops.native_derivative(NAMESPACE, name, fused, general, native.id)
     ops = getattr(torch.ops, NAMESPACE)
     ops.register_derivative(NAMESPACE, forward, backward, 3)
     ops.register_derivative(NAMESPACE, backward, name, 4)

@@ -55,7 +55,9 @@ def build_torch_ops(verbose: bool = True) -> pathlib.Path:
     root = pathlib.Path(torch.__file__).resolve().parent
     cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{root / 'include'}", f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
-           str(CSRC / "oeq_torch.cpp"), "-o", str(TORCH_LIB_PATH), f"-L{root / 'lib'}", "-ltorch", "-ltorch_cpu", "-lc10"]
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f"-I{ROCM / 'include'}",
+           str(CSRC / "oeq_torch.cpp"), "-o", str(TORCH_LIB_PATH), f"-L{root / 'lib'}", "-ltorch", "-ltorch_cpu", "-lc10",
+           "-lc10_hip", "-lamdhip64"]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)

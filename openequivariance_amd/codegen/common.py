@@ -22,6 +22,7 @@ def jinja_env() -> jinja2.Environment:
     return env
 
 
+@functools.lru_cache(maxsize=4096)
 def literal(value: float, ctype: str) -> str:
     """Exact hexadecimal floating literal of ``value`` rounded to the kernel's precision."""
     if ctype == "float":

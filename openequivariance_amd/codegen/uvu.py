@@ -28,6 +28,7 @@ schedule is new):
 """
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass, field
 from typing import Dict, List, Tuple
 
@@ -47,13 +48,9 @@ class Block:
     l: int
     off: int
 
-    @property
-    def D(self) -> int:
-        return 2 * self.l + 1
-
-    @property
-    def dim(self) -> int:
-        return self.mul * self.D
+    def __post_init__(self) -> None:             # (plain attributes: the generators read them ten thousands of times)
+        self.D = 2 * self.l + 1
+        self.dim = self.mul * self.D
 
 
 @dataclass
@@ -421,7 +418,9 @@ class UVUGenerator:
                 E("}")
             E("}")
 
-    def _cg_key(self, k: int, val: float):
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def _cg_key(k: int, val: float):
         return (k, float(np.float64(abs(val)).round(12)))
 
     def _emit_cg_products(self, E: Emitter, p: Path) -> None:

@@ -73,6 +73,7 @@ class UVUDetGenerator(UVUDirectGenerator):
                  allow_split: bool = True, lds=None, long_node=None, fwd_split=None):
         super().__init__(problem, "conv_det", vector_stores=vector_stores)
         self.idx_ctype = idx_ctype
+        self._lines = {}              # of the arithmetic, shared with the twin (_written_once)
         # True: the forward walks the receiver-grouped edge order listed in the workspace (built on
         # the fly from an unsorted edge list) instead of the edge list itself
         self.forward_perm = forward_perm
@@ -255,6 +256,18 @@ class UVUDetGenerator(UVUDirectGenerator):
         finally:
             self.paths, self.used_out, self.used_in1, self.used_y = saved
 
+    @contextlib.contextmanager
+    def _written_once(self, E: Emitter, what):
+        """An emitter for lines that this generator and its twin repeat; None, with the lines written, from the second time on."""
+        key = (what, E.level, self.regroup_pairs)
+        if key in self._lines:
+            yield None
+        else:
+            part = Emitter(E.level)
+            yield part
+            self._lines[key] = part.lines
+        E.lines.extend(self._lines[key])
+
     def backward_kernels(self):
         """(kernel name, group) of the backward launches, in launch order."""
         return [("backward" if h == 0 else f"backward_g{h}", h) for h in range(self.H)]
@@ -410,6 +423,13 @@ class UVUDetGenerator(UVUDirectGenerator):
         if self.team > 1:
             self.emit_team_sum(E, [n for blk in blocks if blk.idx in used and blk.dim for n in regs_of(blk)])
 
+        with self._written_once(E, ("output", ptr, tuple(used), add_existing, zero_unused, self.pieces)) as rest:
+            if rest:
+                self._emit_output_rows(rest, blocks, used, regs_of, ptr, rowdim, via_lds, zero_unused, add_existing, elsewhere)
+
+    def _emit_output_rows(self, E: Emitter, blocks, used, regs_of, ptr: str, rowdim: int, via_lds: bool, zero_unused: bool,
+                          add_existing: bool, elsewhere) -> None:
+        """The part of emit_node_output behind the sums."""
         def store(E, base: str, row: str, existing: bool, zero: bool, agent: bool = False):
             for blk in blocks:
                 if blk.dim == 0:
@@ -698,6 +718,14 @@ class UVUDetGenerator(UVUDirectGenerator):
         b = 2 * (nodes + 1) * 8 + self.order_bytes(nodes) + self.dy_partial_bytes(nnz) + self.flag_bytes(nnz)
         return (b + 255) & ~255
 
+    def workspace_terms(self):
+        """The workspace of ``plan`` as numbers: bytes fixed, per node and per edge, per edge behind a round-up to 256 (0: no such
+        part), whether flags follow; then the piece area: chunks, bytes of a partial row, long-node factor, least edges."""
+        return 16, 24, self.dy_partial_bytes(1), 0, 1, *self.piece_terms()
+
+    def piece_terms(self):
+        return self.NCH, self.piece_row_words * self.itemsize, self.LONG, self.PIECE_MIN_EDGES
+
     def forward_workspace_model(self):
         """(fixed, per node, per edge) bytes the forward steps use when no node is cut into pieces."""
         return 8, 8, 0
@@ -768,9 +796,10 @@ class UVUDetGenerator(UVUDirectGenerator):
             E.level -= 1
             E("}")
 
-        def compute(E, h):
-            for oi in self.used_out:
-                self.emit_receiver_block(E, self.out[oi], f"z{oi}_")
+        def compute(E, _):
+            with self._written_once(E, ("forward", h)) as E:
+                for oi in self.used_out if E else ():
+                    self.emit_receiver_block(E, self.out[oi], f"z{oi}_")
         if self.lds_forward:
             self._emit_staged_forward(E, compute)
         else:
@@ -1048,6 +1077,12 @@ class UVUDetGenerator(UVUDirectGenerator):
             E(f"T* __restrict__ Wgr = Wg + e * {self.WN};")
             for f in self.used_y:
                 E(f"T dy{f} = (T)0;")
+            with self._written_once(E, ("backward", grp)) as B:
+                if B:
+                    products(B)
+            finish(E)
+
+        def products(E):
             for oi in self.used_out:
                 o = self.out[oi]
                 E("{")
@@ -1063,6 +1098,8 @@ class UVUDetGenerator(UVUDirectGenerator):
                 self.emit_sender_block(E, o, sink)
                 E.level -= 1
                 E("}")
+
+        def finish(E):
             self.emit_dy_sum(E)
             if self.staged_backward:
                 E(" ".join(f"pdy{f} = dy{f};" for f in self.used_y) + " pe = e; pv = rv;")

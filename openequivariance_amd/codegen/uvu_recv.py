@@ -152,6 +152,10 @@ class UVURecvGenerator(UVUDetGenerator):
             + self.dy_partial_bytes(nnz)
         return ((((head + 255) & ~255) + self.spill_bytes(nnz) + self.flag_bytes(nnz)) + 255) & ~255
 
+    def workspace_terms(self):
+        head = (64, 56, 16) if self.backward_perm else (16, 24, 0)
+        return *head[:2], head[2] + self.dy_partial_bytes(1), self.spill_bytes(1), 1, *self.piece_terms()
+
     def _disjoint_groups(self, limit: int):
         """Groups of output blocks of at most ``limit`` words per channel (where the problem allows) such that no in1
         block is read by paths of two groups: the connected sets of (output block, in1 block) are packed in the

@@ -137,6 +137,14 @@ class UVUSortedGenerator:
         fwd, bwd, ws = self.plan()
         return self.fwd.few_steps("forward", fwd), self.bwd.few_steps("backward", bwd) if self.grouped_backward else bwd, ws
 
+    def workspace_terms(self):
+        """See UVUDetGenerator.workspace_terms."""
+        if not self.grouped_backward:
+            return 32, 24, 8, 0, 0, *self.fwd.piece_terms()
+        if self.recv_backward:
+            return self.bwd.workspace_terms()
+        return 64, 56, 16 + self.bwd.dy_partial_bytes(1), 0, 1, *self.bwd.piece_terms()
+
     def forward_workspace_model(self):
         """(fixed, per node, per edge) bytes the forward steps use when no node is cut into pieces."""
         return 32, 24, 8

@@ -15,6 +15,7 @@ assumption about the graph.
 """
 from __future__ import annotations
 
+import ctypes
 import typing
 
 import numpy as np
@@ -22,7 +23,7 @@ import torch
 
 from . import runtime as rt
 from . import tunables
-from .autograd_glue import define_derivatives, define_operator, double_backward_terms
+from .autograd_glue import Native, define_derivatives, define_operator, double_backward_terms
 from .codegen.uvu_conv_double import UVUDetDoubleGenerator, conv_double_generator
 from .codegen.uvu_det import UVUDetGenerator
 from .codegen.uvu_direct import UVUDirectGenerator
@@ -140,16 +141,30 @@ class _StreamWorkspace:
     """Device scratch of one operator on one stream, and which graph its preparation areas
     (CSR pointers, position lists, node order) currently describe."""
 
+    TAGS = ("", "atomic", "grouped")
+
     def __init__(self):
         self.buffer, self.size = None, 0
         self.retired = []            # outgrown buffers that a captured HIP graph may still name
-        self.captured = False        # a HIP graph capture has used this workspace
+        # three numbers each of zero_fwd and zero_bwd, and captured: the operators' C++ kernels read and write them too
+        self.state = (ctypes.c_int64 * 8)()
         self.fwd_key = self.bwd_key = None
         self.refs = {}               # index tensors of the cached keys, kept alive so that their addresses stay theirs
-        # (nnz, node_count) of the last completed call of each direction, while nothing else has written the
-        # workspace since: the counters of the on-the-fly grouping are then known to be zero where a call
-        # with the same sizes keeps them, and the step that clears them is skipped
-        self.zero_fwd = self.zero_bwd = None
+
+    def _zero(self, at):
+        nnz, nodes, tag = self.state[at:at + 3]
+        return (nnz, nodes, self.TAGS[tag - 1]) if tag else None
+
+    def _set_zero(self, at, value):
+        self.state[at:at + 3] = [0, 0, 0] if value is None else [value[0], value[1], self.TAGS.index(value[2]) + 1]
+
+    # (nnz, node_count, kind of backward) of the last completed call of each direction, while nothing else has written the
+    # workspace since: the counters of the on-the-fly grouping are then known to be zero where a call
+    # with the same sizes keeps them, and the step that clears them is skipped
+    zero_fwd = property(lambda self: self._zero(0), lambda self, value: self._set_zero(0, value))
+    zero_bwd = property(lambda self: self._zero(3), lambda self, value: self._set_zero(3, value))
+    # a HIP graph capture has used this workspace
+    captured = property(lambda self: bool(self.state[6]), lambda self, value: self.state.__setitem__(6, int(value)))
 
 
 class TensorProductConv:
@@ -192,6 +207,7 @@ class TensorProductConv:
         # the deterministic backward walks the caller's transpose permutation
         self.backward_needs_tperm = deterministic
         self.jit_kernel = self.generator.render()
+        self._native = None                       # the operator's part in the C++ kernels (torch_op=True)
         self._ws_fns = []
         self._ws_last = self._double_ws_last = (None, 0)          # (sizes, bytes) of the last workspace query
         self.internal = self._build(self.generator, self.jit_kernel)
@@ -204,7 +220,8 @@ class TensorProductConv:
         # deterministic operator never chooses by timing: which kernel runs must not depend on a stopwatch
         # if results are to repeat bit for bit from one process to the next.
         self._bwd_variants = {}
-        self._bwd_choice: typing.Dict[tuple, str] = {}
+        self._double = None
+        self._choices: typing.Dict[tuple, str] = {}               # (through _bwd_choice)
         if isinstance(self.generator, UVUSortedGenerator):
             self._bwd_default = "grouped" if self.generator.grouped_backward else "atomic"
             self._bwd_variants[self._bwd_default] = (self.internal, self.backward_overwrites)
@@ -215,7 +232,6 @@ class TensorProductConv:
         # Kernels of the double backward and its workspace function.  The operator torch differentiates has them from the
         # start, so that the first call does not wait for the compiler; the first call makes them `_double` and takes the
         # workspace they need.
-        self._double = None
         self._double_built = self._double_kernels() if torch_op else None
         self._reorder = WeightReorder(config)
         self.reorder_weights_e3nn_to_oeq = self._reorder.e3nn_to_oeq
@@ -228,6 +244,8 @@ class TensorProductConv:
         sized for the largest of them."""
         fwd, bwd, ws = getattr(generator, "plan_few", generator.plan)()
         self._ws_fns.append(ws)
+        if self._native is not None:
+            self._native.ops.native_bytes(self._native.id, generator.workspace_terms())
         need_ws = rt.STEP_NEEDS_WORKSPACE if ws(1, 1) > 0 else 0
         need_tp = rt.STEP_NEEDS_TPERM if self.backward_needs_tperm else 0
         code = rt.compile_source(source if source is not None else generator.render())
@@ -259,17 +277,17 @@ class TensorProductConv:
         return self._double is not None or not torch.cuda.is_current_stream_capturing()
 
     def _double_kernels(self):
-        """(kernel set, workspace function) of the fused double backward."""
+        """(kernel set, workspace function and its numbers) of the fused double backward."""
         idx = "i64" if self.idx_dtype == np.int64 else "int"
 
         def build():
             g = with_few_nodes(conv_double_generator(self.config, self.deterministic, idx))
-            return g.render(), (g.steps_few(), g.plan()[2])
+            return g.render(), (g.steps_few(), g.plan()[2], g.workspace_terms())
         need = rt.STEP_NEEDS_WORKSPACE | (rt.STEP_NEEDS_TPERM if self.deterministic else 0)
-        impl, (_, ws) = rt.variant(("conv double", self.config.signature(), self.deterministic, idx,
+        impl, (_, ws, terms) = rt.variant(("conv double", self.config.signature(), self.deterministic, idx,
                                     UVUDetDoubleGenerator.variant()), torch.cuda.current_device(), build,
                                    lambda code, plan: rt.ConvImpl(code, [], _make_steps(plan[0], need)))
-        return impl, ws
+        return impl, ws, terms
 
     def _double_ws_bytes(self, nnz: int, node_count: int) -> int:
         last = self._double_ws_last
@@ -282,11 +300,57 @@ class TensorProductConv:
         if self._double is None:
             self._double_built = self._double_built or self._double_kernels()
             self._double = self._double_built[0]
+            self._native_enable()
         return self._double
 
     @staticmethod
     def name():
         return "LoopUnrollConv"
+
+    # ------------------------------------------------------------------ what the C++ kernels have to know of
+    def _native_enable(self) -> None:
+        if self._native is not None:
+            self._native.ops.native_enable(self._native.id, not self._graph_cache, self._double is not None)
+
+    @property
+    def graph_cache(self) -> bool:
+        return self._graph_cache
+
+    @graph_cache.setter
+    def graph_cache(self, value: bool) -> None:
+        self._graph_cache = bool(value)
+        for rec in self._workspaces.values():       # (the C++ kernels, which prepare every call, kept no keys meanwhile)
+            rec.fwd_key = rec.bwd_key = None
+        self._native_enable()
+
+    @property
+    def autotune(self) -> bool:
+        return self._autotune
+
+    @autotune.setter
+    def autotune(self, value: bool) -> None:
+        self._autotune = bool(value)
+        self._forget_native_variants()
+
+    @property
+    def _bwd_choice(self):
+        return self._choices
+
+    @_bwd_choice.setter
+    def _bwd_choice(self, choices) -> None:
+        self._choices = choices
+        self._forget_native_variants()
+
+    def _forget_native_variants(self) -> None:
+        if self._native is not None:
+            self._native.ops.native_variant(self._native.id, 0, 0, 0, False, 0)
+
+    def _lend_variant(self, size_class) -> None:
+        """Tells the C++ kernels which backward a size class takes."""
+        if self._native is not None and self._autotune:
+            name = self._choices[size_class]
+            impl, overwrites = self._backward_variant(name)
+            self._native.ops.native_variant(self._native.id, *size_class, impl._h.value, overwrites, _StreamWorkspace.TAGS.index(name) + 1)
 
     # ------------------------------------------------------------------ helpers
     def _workspace_record(self, nnz: int, node_count: int, stream: typing.Optional[int] = None, need: int = 0,
@@ -311,6 +375,8 @@ class TensorProductConv:
             rec.buffer = torch.empty(rec.size, dtype=torch.uint8, device=f"cuda:{dev}")
             rec.fwd_key = rec.bwd_key = rec.zero_fwd = rec.zero_bwd = None
             rec.refs.clear()
+            if self._native is not None and not own:
+                self._native.ops.native_lease(self._native.id, rec.buffer, *sid[:2], ctypes.addressof(rec.state))
         return rec
 
     def workspace_ptr(self, nnz: int, node_count: int, stream: typing.Optional[int] = None) -> int:
@@ -549,6 +615,7 @@ class TensorProductConv:
                         return bwd_run(x, y, w, g, rows, cols, tperm, E, N)
                     self._bwd_choice[size_class] = self._time_backward_variants(
                         lambda name: bwd_run(x, y, w, g, rows, cols, tperm, E, N, name))
+                    self._lend_variant(size_class)
                 return bwd_run(x, y, w, g, rows, cols, tperm, E, N, self._bwd_choice[size_class])
 
         # the two variants differ only in the trailing transpose_perm argument, which the operators' schemas spell out
@@ -559,13 +626,22 @@ class TensorProductConv:
         def like(*tensors):
             return [t.new_empty(*t.shape) for t in tensors]
 
+        native = None
+        if self.forward_overwrites and hasattr(self.generator, "workspace_terms"):
+            native = Native.create(
+                (self.internal, None, self._double_built[0]), self.config.irrep_dtype == np.float64, self.idx_dtype == np.int64, self._dims,
+                conv=True, deterministic=det, tuned=not self.backward_overwrites or self.autotune,
+                first=[self.generator.workspace_terms()], second=[t for t in self._double_built[2:] if t])
+        self._native = native
+        self._native_enable()
+
         forward = define_operator(
             f"conv_forward{cid}", operands + index, "Tensor", lambda x, y, w, *index: fwd_impl(x, y, w, *tperm_of(index)),
-            lambda L1_in, L2_in, weights, *index: L1_in.new_empty(L1_in.shape[0], L3_dim))
+            lambda L1_in, L2_in, weights, *index: L1_in.new_empty(L1_in.shape[0], L3_dim), native=native, kind="conv_forward")
         backward_helper = define_operator(
             f"conv_backward{cid}", (*operands, "L3_grad", *index), "Tensor[]",
             lambda x, y, w, g, *index: bwd_impl(x, y, w, g, *tperm_of(index)),
-            lambda L1_in, L2_in, weights, L3_grad, *index: like(L1_in, L2_in, weights))
+            lambda L1_in, L2_in, weights, L3_grad, *index: like(L1_in, L2_in, weights), native=native, kind="conv_backward")
 
         def double_impl(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, rows, cols, tperm):
             x, y, w, g, a, b, v, rows, cols, tperm = _contiguous(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot,
@@ -591,13 +667,15 @@ class TensorProductConv:
         fused = define_operator(
             f"conv_double_backward{cid}", (*operands, "L3_grad", "L1_cot", "L2_cot", "weights_cot", *index), "Tensor[]",
             lambda x, y, w, g, a, b, v, *index: double_impl(x, y, w, g, a, b, v, *tperm_of(index)),
-            lambda L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, *index: like(L1_in, L2_in, weights, L3_grad))
+            lambda L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot, *index: like(L1_in, L2_in, weights, L3_grad),
+            native=native, kind="conv_double")
 
         def double_backward(x, y, w, g, a, b, v, *index):
             return list(double_backward_terms(forward, backward_helper, x, y, w, g, a, b, v, index,
                                               fused=fused if self._double_usable() else None))
 
-        define_derivatives(f"conv_forward{cid}", f"conv_backward{cid}", operands + index, double_backward)
+        define_derivatives(f"conv_forward{cid}", f"conv_backward{cid}", operands + index, double_backward, native,
+                           f"conv_double_backward{cid}")
         self.forward = forward
         self.backward_helper = backward_helper
 

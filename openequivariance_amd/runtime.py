@@ -155,6 +155,13 @@ def _check(status: int) -> None:
         raise RuntimeError(lib().oeq_last_error().decode(errors="replace"))
 
 
+def entry_points() -> List[int]:
+    """Addresses of the calls that the torch operators' C++ kernels make."""
+    return [C.cast(getattr(lib(), name), C.c_void_p).value for name in
+            ("oeq_tp_forward", "oeq_tp_backward", "oeq_tp_double_backward", "oeq_conv_forward_ex", "oeq_conv_backward_ex",
+             "oeq_conv_double_backward_ex", "oeq_last_error")]
+
+
 # --------------------------------------------------------------------------- device
 def device_count() -> int:
     n = C.c_int(0)

@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from . import runtime as rt
-from .autograd_glue import define_derivatives, define_operator, double_backward_terms
+from .autograd_glue import Native, define_derivatives, define_operator, double_backward_terms
 from .codegen.uvu import UVUGenerator
 from .codegen.uvu_direct import UVUDirectGenerator
 from .codegen.uvu_double import UVUDoubleGenerator
@@ -146,6 +146,7 @@ class TensorProduct(TensorProductBase):
         self.internal = rt.TPImpl(code, _make_steps(fwd, self._step_flags), _make_steps(bwd, self._step_flags))
         self._torch_dtype = {np.float32: torch.float32, np.float64: torch.float64}[self.irrep_dtype]
         self._dims = (self.L1.dim, self.L2.dim, self.L3.dim, config.weight_numel)
+        self._native = None                   # the operator's part in the C++ kernels (torch_op=True)
         self._workspaces = {}                 # (device, stream) -> scratch tensor (fixed size, never regrown)
         self._internal_unaligned = None       # kernels without 16-byte vector stores, compiled on first need
         # dense uvw: kernels for few rows and their largest batch (forward, backward).  Built here like the double backward's,
@@ -179,6 +180,8 @@ class TensorProduct(TensorProductBase):
         buf = self._workspaces.get(key)
         if buf is None:
             buf = self._workspaces[key] = torch.empty(self.workspace_bytes, dtype=torch.uint8, device=f"cuda:{dev}")
+            if self._native is not None:
+                self._native.ops.native_lease(self._native.id, buf, *key, 0)
         return buf.data_ptr()
 
     @staticmethod
@@ -292,6 +295,9 @@ class TensorProduct(TensorProductBase):
 
         operands = ("L1_in", "L2_in", "weights")
         tp_id = self.tp_id
+        native = self._native = Native.create(
+            (self.internal, self._few_rows, self._double.get(True)), self.irrep_dtype == np.float64, True, self._dims, self.workspace_bytes,
+            shared=self.config.shared_weights, few_limits=self._few_rows_limits)
 
         def forward_impl(L1_in, L2_in, weights):
             x, y, w = _contiguous(L1_in, L2_in, weights)
@@ -305,7 +311,8 @@ class TensorProduct(TensorProductBase):
         def forward_fake(L1_in, L2_in, weights):
             return L1_in.new_empty(L1_in.shape[0], L3_dim)
 
-        forward = self.forward = define_operator(f"tp_forward{tp_id}", operands, "Tensor", forward_impl, forward_fake)
+        forward = self.forward = define_operator(f"tp_forward{tp_id}", operands, "Tensor", forward_impl, forward_fake,
+                                                 native=native, kind="tp_forward")
 
         def backward_impl(L1_in, L2_in, weights, L3_grad):
             x, y, w, g = _contiguous(L1_in, L2_in, weights, L3_grad)
@@ -321,7 +328,7 @@ class TensorProduct(TensorProductBase):
 
         backward_helper = self.backward_helper = define_operator(
             f"tp_grad_helper{tp_id}", (*operands, "L3_grad"), "Tensor[]", backward_impl,
-            lambda L1_in, L2_in, weights, L3_grad: like(L1_in, L2_in, weights))
+            lambda L1_in, L2_in, weights, L3_grad: like(L1_in, L2_in, weights), native=native, kind="tp_backward")
 
         fused = None
         if self._double_generator is not None:
@@ -339,13 +346,15 @@ class TensorProduct(TensorProductBase):
 
             fused = define_operator(
                 f"tp_double_backward{tp_id}", (*operands, "L3_grad", "L1_cot", "L2_cot", "weights_cot"), "Tensor[]", double_impl,
-                lambda L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot: like(L1_in, L2_in, weights, L3_grad))
+                lambda L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot: like(L1_in, L2_in, weights, L3_grad),
+                native=native, kind="tp_double")
 
         def double_backward(L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot):
             return list(double_backward_terms(forward, backward_helper, L1_in, L2_in, weights, L3_grad, L1_cot, L2_cot, weights_cot,
                                               fused=fused))
 
-        define_derivatives(f"tp_forward{tp_id}", f"tp_grad_helper{tp_id}", operands, double_backward)
+        define_derivatives(f"tp_forward{tp_id}", f"tp_grad_helper{tp_id}", operands, double_backward, native,
+                           fused and f"tp_double_backward{tp_id}")
 
     def _check_inputs(self, x, y, w, g=None) -> None:
         """Shapes, dtypes and devices, before anything is launched (the kernels dereference every
