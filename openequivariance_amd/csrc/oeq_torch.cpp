@@ -24,7 +24,7 @@
 #include "../../include/oeq_hip.h"
 
 #include <algorithm>
-#include <array>
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -212,8 +212,9 @@ struct Native {
     at::ScalarType dtype, index;
     int64_t d1, d2, d3, wn, scratch;
     bool conv, shared, deterministic, tuned;         // tuned: the backward's variant is measured per size class
-    void *main, *few, *twice;                        // kernel sets: general, for few rows, of the double backward
-    int64_t few_forward, few_backward;
+    std::atomic<void*> main, few;                    // kernel sets: general, for few rows,
+    void* twice;                                     // ... of the double backward
+    std::atomic<int64_t> few_forward, few_backward;  // largest batches of the kernels for few rows
     std::vector<Bytes> first_order, second_order;
 
     std::mutex mutex;                                // of everything below, and of a convolution's launches
@@ -330,11 +331,11 @@ struct NativeKernel final : c10::OperatorKernel {
         const at::Tensor &x = *t[0], &y = *t[1], &w = *t[2];
         if (kind == TP_FORWARD) {
             out.push_back(at::empty({rows, n.d3}, x.options()));
-            auto* h = static_cast<oeq_tp*>(rows <= n.few_forward ? n.few : n.main);
+            auto* h = static_cast<oeq_tp*>(rows <= n.few_forward ? n.few.load() : n.main.load());
             done(g_lib.tp_forward(h, rows, in(&x), in(&y), to(out[0]), in(&w), scratch, stream));
         } else if (kind == TP_BACKWARD) {
             for (const at::Tensor* a : {&x, &y, &w}) out.push_back(at::empty_like(*a));
-            auto* h = static_cast<oeq_tp*>(rows <= n.few_backward ? n.few : n.main);
+            auto* h = static_cast<oeq_tp*>(rows <= n.few_backward ? n.few.load() : n.main.load());
             done(g_lib.tp_backward(h, rows, in(&x), to(out[0]), in(&y), to(out[1]), in(&w), to(out[2]), in(t[3]), scratch, stream));
         } else {
             for (size_t i = 0; i < 4; ++i) out.push_back(at::empty_like(*t[i]));
@@ -367,7 +368,7 @@ struct NativeKernel final : c10::OperatorKernel {
         if (kind == CONV_FORWARD) {
             out.push_back(at::empty({nodes, n.d3}, x.options()));
             call(forward_state, backward_state, 1, [&](uint32_t flags) {
-                return g_lib.conv_forward(static_cast<oeq_conv*>(n.main), in(&x), in(&y), in(&w), to(out[0]), rows, cols, edges, nodes,
+                return g_lib.conv_forward(static_cast<oeq_conv*>(n.main.load()), in(&x), in(&y), in(&w), to(out[0]), rows, cols, edges, nodes,
                                           to(buffer), perm, stream, flags);
             });
         } else if (kind == CONV_BACKWARD) {
@@ -440,7 +441,8 @@ int64_t native_operator(at::IntArrayRef v, at::IntArrayRef first, at::IntArrayRe
     n->d1 = v[2]; n->d2 = v[3]; n->d3 = v[4]; n->wn = v[5]; n->scratch = v[6];
     n->conv = v[7]; n->shared = v[8]; n->deterministic = v[9]; n->tuned = v[10];
     n->main = reinterpret_cast<void*>(v[11]); n->few = reinterpret_cast<void*>(v[12]); n->twice = reinterpret_cast<void*>(v[13]);
-    n->few_forward = n->few ? v[14] : 0; n->few_backward = n->few ? v[15] : 0;
+    n->few_forward = n->few ? v[14] : 0;
+    n->few_backward = n->few ? v[15] : 0;
     for (auto [from, into] : {std::make_pair(first, &n->first_order), std::make_pair(second, &n->second_order)})
         for (size_t i = 0; i < from.size(); i += 9)
             into->push_back({from[i], from[i + 1], from[i + 2], from[i + 3], from[i + 4], from[i + 5], from[i + 6], from[i + 7], from[i + 8]});
@@ -491,6 +493,16 @@ void native_enable(int64_t id, bool enabled, bool double_ready) {
     n.enabled = enabled;
     n.double_ready = n.double_ready || double_ready;
 }
+void native_kernels(int64_t id, int64_t main, int64_t few, int64_t forward, int64_t backward) {
+    Native& n = native(id);
+    n.main = reinterpret_cast<void*>(main);
+    n.few_forward = n.few_backward = 0;
+    n.few = reinterpret_cast<void*>(few);
+    if (few) {
+        n.few_forward = forward;
+        n.few_backward = backward;
+    }
+}
 int64_t native_workspace_bytes(int64_t id, bool second, int64_t edges, int64_t nodes) {
     Native& n = native(id);
     std::lock_guard<std::mutex> lock(n.mutex);
@@ -509,5 +521,6 @@ TORCH_LIBRARY_FRAGMENT(openequivariance_amd, m) {
     m.def("native_variant(int id, int edge_bits, int node_bits, int handle, bool overwrites, int kind) -> ()", native_variant);
     m.def("native_bytes(int id, int[] more) -> ()", native_bytes);
     m.def("native_enable(int id, bool enabled, bool double_ready) -> ()", native_enable);
+    m.def("native_kernels(int id, int main, int few, int forward, int backward) -> ()", native_kernels);
     m.def("native_workspace_bytes(int id, bool second, int edges, int nodes) -> int", native_workspace_bytes);
 }

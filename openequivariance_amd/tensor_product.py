@@ -129,6 +129,13 @@ def few_rows_generator(config: TPProblem, generator: UVWGenerator):
     return (small, limits) if any(limits) else (None, (0, 0))
 
 
+def _kernel_set(name: str) -> property:
+    def put(self, value) -> None:
+        self._sets[name] = value
+        self._tell_native()
+    return property(lambda self: self._sets[name], put)
+
+
 class TensorProduct(TensorProductBase):
     """Drop-in for ``oeq.TensorProduct(problem, torch_op=True)``."""
 
@@ -143,10 +150,11 @@ class TensorProduct(TensorProductBase):
         fwd, bwd, ws = self.generator.plan()
         self.workspace_bytes = ws()
         self._step_flags = rt.STEP_NEEDS_WORKSPACE if self.workspace_bytes else 0
+        self._native = None                   # the operator's part in the C++ kernels (torch_op=True)
+        self._sets = {"_few_rows": None, "_few_rows_limits": (0, 0)}
         self.internal = rt.TPImpl(code, _make_steps(fwd, self._step_flags), _make_steps(bwd, self._step_flags))
         self._torch_dtype = {np.float32: torch.float32, np.float64: torch.float64}[self.irrep_dtype]
         self._dims = (self.L1.dim, self.L2.dim, self.L3.dim, config.weight_numel)
-        self._native = None                   # the operator's part in the C++ kernels (torch_op=True)
         self._workspaces = {}                 # (device, stream) -> scratch tensor (fixed size, never regrown)
         self._internal_unaligned = None       # kernels without 16-byte vector stores, compiled on first need
         # dense uvw: kernels for few rows and their largest batch (forward, backward).  Built here like the double backward's,
@@ -214,6 +222,14 @@ class TensorProduct(TensorProductBase):
     def _pick_rows(self, batch: int, backward: bool):
         """The kernels for few rows where ``batch`` is one, else None."""
         return self._few_rows if 0 < batch <= self._few_rows_limits[backward] else None
+
+    def _tell_native(self) -> None:
+        """The C++ kernels launch these kernel sets (attributes, so that they can be exchanged)."""
+        if self._native is not None:
+            raw = [getattr(getattr(h, "_h", None), "value", None) or 0 for h in (self._sets["internal"], self._sets["_few_rows"])]
+            self._native.ops.native_kernels(self._native.id, *raw, *self._sets["_few_rows_limits"])
+
+    internal, _few_rows, _few_rows_limits = _kernel_set("internal"), _kernel_set("_few_rows"), _kernel_set("_few_rows_limits")
 
     def _few_row_kernels(self):
         """(kernel set, limits) of the kernels for few rows of a dense uvw product."""
