@@ -324,12 +324,6 @@ class UVUDetGenerator(UVUDirectGenerator):
     def emit_piece_helpers(self) -> str:
         """Device functions shared by the kernels of one code object (rendered once by the templates)."""
         return "\n".join([
-            "// s_waitcnt vmcnt(n): all vector-memory accesses but the n issued last have completed (they retire in order)",
-            "#ifdef __AMDGCN__",
-            "#define OEQ_WAIT_VM_BUT(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | ((n) >> 4 << 14))",
-            "#else",
-            "#define OEQ_WAIT_VM_BUT(n) ((void)0)",
-            "#endif",
             "// edges per piece of a long node's list, and tiles of that length in the whole list",
             "static __device__ __forceinline__ u64 oeq_piece_edges(u64 nnz, u64 node_count) {",
             f"    const u64 t_ = {self.LONG}ull * (node_count ? (nnz + node_count - 1) / node_count : 0);",
@@ -1018,81 +1012,6 @@ class UVUDetGenerator(UVUDirectGenerator):
             flush(E)
             E.level -= 1
             E("}")
-
-    def emit_staged_loop_deep(self, E: Emitter, pos_of, pos_list, nbr_list: str, words: int, transfers: int, dma, readback, compute,
-                              flush, pre, request) -> None:
-        """emit_staged_loop with the operands of two edges in flight, into two stages of ``words``: the wait at the top leaves the
-        ``transfers`` of the younger edge outstanding, so those of an iteration are its last vector-memory requests, behind the
-        index chain (one iteration longer) and what ``request(E, e)`` loads for the next iteration's edge."""
-        def pos(it):
-            return f"(({pos_of(it)}) < len ? (u64)(beg + {pos_of(it)}) : (u64)(nnz - 1))"
-
-        def fetch(it):
-            return f"{pos_list}[{pos(it)}]" if pos_list else f"(i64){pos(it)}"
-
-        def edge_ok(raw, it):
-            return f"(({pos_of(it)}) < len && {raw} >= 0 && {raw} < (i64)nnz)"
-
-        def nbr_ok(raw):
-            return f"({raw} >= 0 && {raw} < (i64)node_count)"
-        E("u64 e0 = 0, e1 = 0, e2 = 0, e3 = 0, n2 = 0; bool v0 = false, v1 = false, v2 = false, v3 = false; i64 rawE = 0, rawN = 0;")
-        E("// prologue: dependent loads, paid once per tile")
-        E("if (maxlen > 0) {")
-        E.level += 1
-        E(f"const i64 t0_ = {fetch('0')}, t1_ = {fetch('1')}, t2_ = {fetch('2')};")
-        for q in range(3):
-            E(f"v{q} = {edge_ok(f't{q}_', str(q))}; e{q} = v{q} ? (u64)t{q}_ : 0;")
-        E(f"const i64 r0_ = {nbr_list}[e0], r1_ = {nbr_list}[e1];")
-        E(f"rawN = {nbr_list}[e2]; rawE = {fetch('3')};")
-        request(E, "e0")
-        E(f"v0 = v0 && {nbr_ok('r0_')}; v1 = v1 && {nbr_ok('r1_')};")
-        for q in range(2):
-            E("{" if q == 0 else "if (maxlen > 1) {")
-            E.level += 1
-            E(f"{self.stage_type()}* stage = stages + {q * words};")
-            dma(E, f"e{q}", f"(v{q} ? (u64)r{q}_ : 0)")
-            E.level -= 1
-            E("}")
-        E.level -= 1
-        E("}")
-        E("for (int it = 0; it < maxlen; ++it) {")
-        E.level += 1
-        E("const u64 cur_e = e0; const bool cur_rv = v0; (void)cur_e; (void)cur_rv;")
-        E(f"{self.stage_type()}* stage = stages + (it & 1) * {words};")
-        E(f"if (it + 1 < maxlen) OEQ_WAIT_VM_BUT({transfers}); else oeq_wait_vm();")
-        E("oeq_sync();")
-        readback(E)
-        E("oeq_wait_lds();")
-        E("oeq_sync();")
-        E("if (it > 0) {")
-        E.level += 1
-        flush(E)
-        E.level -= 1
-        E("}")
-        E(f"v2 = v2 && {nbr_ok('rawN')}; n2 = v2 ? (u64)rawN : 0;")
-        E(f"v3 = {edge_ok('rawE', 'it + 3')}; e3 = v3 ? (u64)rawE : 0;")
-        pre(E)
-        E("if (it + 1 < maxlen) {")
-        E.level += 1
-        request(E, "e1")
-        E.level -= 1
-        E("}")
-        E(f"if (it + 3 < maxlen) rawN = {nbr_list}[e3];")
-        E(f"if (it + 4 < maxlen) rawE = {fetch('it + 4')};")
-        E("if (it + 2 < maxlen) {")
-        E.level += 1
-        dma(E, "e2", "n2")
-        E.level -= 1
-        E("}")
-        compute(E, 0)
-        E("e0 = e1; v0 = v1; e1 = e2; v1 = v2; e2 = e3; v2 = v3;")
-        E.level -= 1
-        E("}")
-        E("if (maxlen > 0) {")
-        E.level += 1
-        flush(E)
-        E.level -= 1
-        E("}")
 
     # ================================================================ backward
     def conv_det_backward_body(self, grp: int = 0) -> str:
