@@ -63,7 +63,6 @@ class UVUDetDoubleGenerator(_DoublePlan, DoubleArithmetic, UVUDetGenerator):
     # per launch) against this: 127 words 128 channels fp32 433 / 418, fp64 654 / 503, 64 channels fp64 566 / 411;
     # 254 words 32 channels fp32 532 / 490 (in one launch 870), 64 channels fp32 566 / 488, fp64 900 / 625 (one: 1121)
     SPLIT_WORDS = 144
-    TEAM_WAVES_MANY_WORDS = UVUDetGenerator.TEAM_WAVES         # (fp64, 64 channels, 1000 nodes: 266 / 213)
     CALL_FWD_ARGS = CALL_BWD_ARGS = CALL_ARGS
 
     def __init__(self, problem, **kw):

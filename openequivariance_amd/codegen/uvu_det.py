@@ -123,7 +123,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         # a node that does not exist (see emit_invalid_edge_rows)
         part = f" + {self.dy_slots}ull * nnz * {self.D2} * sizeof(T)" if self.dy_slots > 1 else ""
         self.flags_off = f"((({self.dypart_off}{part}) + 7ull) & ~7ull)"
-        words = self.sender_words = max(words_of(g_) for g_ in self.out_groups)
+        words = max(words_of(g_) for g_ in self.out_groups)
         # fetch the next edge's operands while the current edge is being computed; pays when the
         # per-edge register footprint is small enough to keep several wavefronts per SIMD
         if prefetch_backward is None:
@@ -278,7 +278,8 @@ class UVUDetGenerator(UVUDirectGenerator):
 
     def forward_kernel_sources(self):
         """The forward's compute kernels as the templates emit them: name and body."""
-        return [dict(name=name, threads=WAVE * self.team, body=self.conv_det_forward_body(h)) for name, h in self.forward_kernels()]
+        return [self.with_team(dict(name=name, threads=WAVE * self.team, body=self.conv_det_forward_body(h)))
+                for name, h in self.forward_kernels()]
 
     def forward_steps(self, step: dict):
         """One launch like ``step`` per group of output blocks."""
@@ -286,7 +287,7 @@ class UVUDetGenerator(UVUDirectGenerator):
 
     def backward_kernel_sources(self):
         """The backward's compute kernels as the templates emit them: name, workgroup size, attributes, body."""
-        return [dict(name=name, threads=WAVE * self.team, attr=self.backward_attr(), body=self.conv_det_backward_body(h))
+        return [self.with_team(dict(name=name, threads=WAVE * self.team, attr=self.backward_attr(), body=self.conv_det_backward_body(h)))
                 for name, h in self.backward_kernels()]
 
     def act(self, blk):
@@ -324,6 +325,12 @@ class UVUDetGenerator(UVUDirectGenerator):
     def emit_piece_helpers(self) -> str:
         """Device functions shared by the kernels of one code object (rendered once by the templates)."""
         return "\n".join([
+            "// LDS of a team of wavefronts: as much as its size needs; the whole where there is no dynamic LDS (the tests' host build)",
+            "#ifdef __AMDGCN__",
+            "#define OEQ_TEAM_LDS(most) extern __shared__ __attribute__((aligned(16))) unsigned char team_[]",
+            "#else",
+            "#define OEQ_TEAM_LDS(most) __shared__ __attribute__((aligned(16))) unsigned char team_[most]",
+            "#endif",
             "// edges per piece of a long node's list, and tiles of that length in the whole list",
             "static __device__ __forceinline__ u64 oeq_piece_edges(u64 nnz, u64 node_count) {",
             f"    const u64 t_ = {self.LONG}ull * (node_count ? (nnz + node_count - 1) / node_count : 0);",
@@ -403,7 +410,7 @@ class UVUDetGenerator(UVUDirectGenerator):
             E("qh = oeq_uniform_u64(qh); npieces = __builtin_amdgcn_readfirstlane(npieces);")
         if self.team > 1:
             E("// this wavefront's part of the list")
-            E(f"{{ const i64 n_ = end - beg, b_ = beg; beg = b_ + n_ * wave_ / {self.team}; end = b_ + n_ * (wave_ + 1) / {self.team}; }}")
+            E("{ const i64 n_ = end - beg, b_ = beg; beg = b_ + n_ * wave_ / team_size_; end = b_ + n_ * (wave_ + 1) / team_size_; }")
         E("const bool nv = node < node_count;")
         E("const int len = (int)(end - beg);")
         E(f"const int maxlen = (len + {R - 1}) / {R};")
@@ -521,57 +528,82 @@ class UVUDetGenerator(UVUDirectGenerator):
 
     # ---- several wavefronts per node
     # On a graph of few nodes a launch lasts as long as one wavefront's walk over a node's edges, and the chip is empty beside it
-    # (1000 nodes: one wavefront per SIMD).  There a node's list is cut into TEAM parts of equal length, a wavefront each,
+    # (1000 nodes: one wavefront per SIMD).  There a node's list is cut into four or two parts of equal length, a wavefront each,
     # whose sums are added through LDS in the order of the list: fixed for a graph's size, so results repeat bit for bit.
     # All nodes are in flight at once then and need no order (order_backward, 4 - 6 us, is not launched).  Receiver pass,
-    # sender pass with its preparation, and double backward, us, one wavefront / four:
-    #   32 channels, 11 paths   200 nodes, 24 edges each 16.5 / 10.6, 35 / 16, 70 / 32; 1000 nodes 22 / 17, 43 / 37, 83 / 73
+    # sender pass with its preparation, and double backward, us, one wavefront / the team that the rule gives:
+    #   32 channels, 11 paths   200 nodes, 24 edges each 16.6 / 10.7, 35 / 16, 70 / 33; 1001 nodes, 30 edges 24 / 18, 47 / 39, 90 / 75
     #   64 channels, l <= 1     500 nodes 21.5 / 11.6, 33 / 15, 68 / 30; 2000 nodes 29 / 17, 47 / 35, 89 / 75
-    #   128 channels, 13 paths  200 nodes 36 / 18, 106 / 45, 180 / 80; 1000 nodes 57 / 52, 142 / 144, 265 / 240
-    # Four: with two wavefronts the small graphs keep half of the gain (200 nodes, 32 channels 35 -> 21 us for the sender pass),
-    # with eight LDS holds the stages of few nodes (1000 nodes, 32 channels: receiver pass 28 us).
-    TEAM = 4
-    TEAM_WAVES = 2048             # row groups (workgroups x lane groups) up to which a team walks a node (0: never)
-    TEAM_MANY_WORDS, TEAM_WAVES_MANY_WORDS = 40, 768         # ... in the sender pass with more operand words per edge than this
-    TEAM_LDS = 160 * 1024         # of a compute unit; problems whose teams would need more keep single wavefronts
-    team, team_lds = 1, 0         # wavefronts that walk one node's edges here; LDS they share, bytes (as emitted)
+    #   128 channels, 13 paths  200 nodes 36 / 18, 106 / 45, 180 / 80; 500 nodes 49 / 33, 111 / 90, 211 / 150
+    # With eight wavefronts LDS holds the stages of few nodes (32 channels, 1000 nodes: receiver pass 28 us).
+    TEAM = 4                      # wavefronts of the largest team
+    TEAMS = ((4, 2048), (2, 4096))         # wavefronts, and row groups (nodes x chunks x lane groups) up to which they walk a node
+    TEAM_LDS, TEAM_CUS = 160 * 1024, 256   # LDS of a compute unit, compute units
+    TEAM_STEP = 128               # a team's least number of nodes is kept in these (OEQ_STEP_FEW_NODES)
+    team, team_need = 1, (0, 0, 0)         # wavefronts that walk one node's edges here; what a kernel of theirs needs (emit_stage)
     few_sources = {"forward": [], "backward": []}            # kernels for few nodes beside the others (add_few_nodes)
 
     def team_twin(self, team: int = TEAM):
-        """This generator with teams of wavefronts, on the same workspace."""
+        """This generator with teams of (at most) so many wavefronts, on the same workspace."""
         twin = copy.copy(self)
         twin.team, twin.ordered_backward = team, False
         return twin
+
+    def with_team(self, kernel: dict) -> dict:
+        """A kernel's source with what its teams need, when they walk the nodes."""
+        return kernel if kernel["threads"] == WAVE else dict(kernel, need=self.team_need)
 
     def add_few_nodes(self, which=("forward", "backward")):
         """Adds the kernels for few nodes to what is rendered, and to the launch plans of ``plan_few``."""
         twin = self.team_twin()
         kernels = dict(forward=twin.forward_kernel_sources, backward=twin.backward_kernel_sources)
         sources = {w: [dict(k, name=k["name"] + "_few") for k in kernels[w]() if k["threads"] > WAVE] for w in which}
-        if twin.team_lds <= self.TEAM_LDS:
-            self.few_sources = {"forward": [], "backward": [], **{w: sources[w] for w in which if self.few_limits(w)[0]}}
+        self.few_sources = {"forward": [], "backward": [], **sources}
+        self.few_sources.update({w: [] for w in which if not self.few_teams(w)})
         return self
 
-    def few_limits(self, which: str):
-        """(nodes, edges per node): a team walks the nodes of graphs of at most so many nodes and at least so many edges for
-        each: few enough workgroups, and two turns of the edge loop for each wavefront.  Both sides of the lines, one
-        wavefront / four: receiver pass, 24 edges a node: 64 channels (one row group), 2000 nodes 26 / 15 us, 4000 32 / 27; 32
-        channels (two) 1000 nodes 20.1 / 14.3, 2000 23.8 / 28.9; 16 channels (four) 500 nodes 10.6 / 8.7, 1000 11.3 / 14.8;
-        8 channels (eight) 200 nodes 7.8 / 7.5, 500 9.6 / 12.9; 8 edges a node there (one turn) 5.3 / 6.8.  Sender pass, more
-        words per edge: fp64, 64 channels, 11 paths, 500 nodes 96 / 75, 1000 nodes 129 / 135; fewer: 64 channels, l <= 1,
-        2000 nodes 47 / 35."""
-        many = which == "backward" and self.R == 1 and self.sender_words > self.TEAM_MANY_WORDS
-        return (min(self.TEAM_WAVES, self.TEAM_WAVES_MANY_WORDS) if many else self.TEAM_WAVES) // (self.NCH * self.R), 2 * self.R
+    def team_bytes(self, team: int, need) -> int:
+        """LDS of a team, dynamic: its wavefronts' stages, in which they leave their sums when the loop is over."""
+        stage, sums, _ = need
+        return max(4 * stage * team, self.itemsize * WAVE * sums * (team - 1))
+
+    def few_teams(self, which: str):
+        """[(wavefronts, nodes beyond which, nodes up to which)] of the teams of a pass, largest first: each up to the nodes that
+        are in flight at once - by LDS, and by the registers that the words a lane holds suggest - and to TEAMS' row groups, so
+        that a wavefront has a few turns of its loop.
+        us, one / two / four wavefronts: receiver pass, 32 channels, 24 edges a node: 760 nodes 16.7 / 12.1 / 11.3, 1500 20.7 /
+        17.6 / 20.3, 2000 21.9 / 20.2 / 26.4; outputs to l = 3 (LDS of two teams of four) 760 nodes 26 / 18 / 25, 1500 31.5 / 31.5 /
+        45; 16 channels (four lane groups) 500 nodes 10.7 / 8.3 / 8.6, 1001 11.9 / 10.3 / 15.6, 1500 12.6 / 13.3 / 20.8; 64, l <= 1,
+        2000 nodes 26 / 17 / 15, 4000 32 / 29 / 27; 128 channels, 1000 nodes 55 / 50 / 50.  Sender pass, 32 channels: 760 nodes 31 / 25 / 24, 1500 42 / 41 / 43; fp64, 64
+        channels, 760 nodes 100 / 95 / 101, 1001 143 / 162 / 156.  Double backward, 32 channels: 500 nodes 66 / 48 / 37, 1001
+        81 / 69 / 77, 1500 87 / 90 / 94."""
+        needs = [k["need"] for k in self.few_sources[which]]
+        out, beyond = [], 0
+        for team, groups in self.TEAMS:
+            if not needs or any(self.team_bytes(team, n) + self.lds_elems * self.itemsize > self.TEAM_LDS for n in needs):
+                continue
+            waves = 4 * min(8, 512 // (max(words for _, _, words in needs) * self.itemsize // 4 + 24))
+            per_cu = min([waves // team] + [self.TEAM_LDS // (self.team_bytes(team, n) + self.lds_elems * self.itemsize + 1) for n in needs])
+            upto = min(max(1, per_cu) * self.TEAM_CUS, groups // self.R) // self.NCH
+            upto = min(upto, 15 * self.TEAM_STEP) // self.TEAM_STEP * self.TEAM_STEP if team != self.TEAMS[-1][0] else min(upto, 4095)
+            if upto > beyond:
+                out.append((team, beyond, upto))
+                beyond = upto
+        return out
 
     def few_steps(self, which: str, steps):
-        """The launches ``steps`` with those for few nodes beside those that they replace there."""
-        names, out = {k["name"] for k in self.few_sources[which]}, []
+        """The launches ``steps`` with those of teams beside those that they replace on few nodes (and at least two edges a lane
+        group and node)."""
+        sources, teams, out = {k["name"]: k for k in self.few_sources[which]}, self.few_teams(which), []
         for s in steps:
-            if s["kernel"] + "_few" in names:
-                out += [dict(s, many_nodes=self.few_limits(which)),
-                        dict(s, kernel=s["kernel"] + "_few", num_threads=WAVE * self.TEAM, few_nodes=self.few_limits(which))]
+            few = sources.get(s["kernel"] + "_few")
+            if few or (teams and s["kernel"] == "order_backward"):
+                out.append(dict(s, many_nodes=(teams[-1][2], 2 * self.R)))
             else:
-                out.append(dict(s, many_nodes=self.few_limits(which)) if names and s["kernel"] == "order_backward" else s)
+                out.append(s)
+            for team, beyond, upto in reversed(teams) if few else ():
+                out.append(dict(s, kernel=few["name"], num_threads=WAVE * team, smem=self.team_bytes(team, few["need"]),
+                                few_nodes=(upto, 2 * self.R, beyond)))
         return out
 
     def plan_few(self):
@@ -582,24 +614,34 @@ class UVUDetGenerator(UVUDirectGenerator):
         if self.team == 1:
             super().emit_lane_direct(E, lds=lds)
             return
-        E("const int wave_ = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;")
+        E("const int wave_ = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63, team_size_ = blockDim.x >> 6;")
         E(f"const int sub = lane >> {self.LOGP};")
         E(f"const int ul = lane & {self.P - 1};")
         if lds and self.lds_elems:
             E(f"__shared__ __attribute__((aligned(16))) T lds[{self.lds_elems}];")
 
-    def emit_stage(self, E: Emitter, words: int, sums: int) -> None:
+    def emit_stage(self, E: Emitter, words: int, sums: int, held: int) -> None:
         """The LDS stage of a wavefront (``words`` of 4 bytes; 0: none).  The wavefronts of a team have one each, and leave
-        their ``sums`` values per lane in the same memory when the loop is over."""
+        their ``sums`` values per lane in the same memory when the loop is over.  ``held``: values a lane holds."""
         if self.team == 1:
             if words:
                 E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{words}];")
             return
-        area = max(4 * words * self.team, self.itemsize * WAVE * sums * (self.team - 1))
-        self.team_lds = max(self.team_lds, area + self.lds_elems * self.itemsize)
-        E(f"__shared__ __attribute__((aligned(16))) unsigned char team_[{area}];")
+        self.team_need = words, sums, held
+        E(f"OEQ_TEAM_LDS({self.team_bytes(self.team, self.team_need)});")
         if words:
             E(f"{self.stage_type()}* stage = ({self.stage_type()}*)team_ + wave_ * {words};")
+
+    def _edge_words(self) -> int:
+        return len(self.EDGE_W) * sum(p.mv for p in self.paths) + len(self.EDGE_Y) * len(self.used_y)
+
+    def _held_receiver(self, sets: int) -> int:
+        return (self._sums(self.out, self.used_out)
+                + sets * (len(self.NODE_X) * self._sums(self.in1, self.used_in1) + self._edge_words()))
+
+    def _held_sender(self, sets: int) -> int:
+        return ((1 + len(self.NODE_X)) * self._sums(self.in1, self.used_in1)
+                + sets * (self._sums(self.out, self.used_out) + self._edge_words()))
 
     @staticmethod
     def _sums(blocks, used) -> int:
@@ -609,15 +651,16 @@ class UVUDetGenerator(UVUDirectGenerator):
         """The team's sums of the registers ``names`` in its first wavefront, in the order of the edge list; the others are
         done."""
         E("oeq_block_sync();")
-        E(f"T* __restrict__ part_ = (T*)team_ + lane;")
+        E("T* part_ = (T*)team_ + lane;")
         E("if (wave_ > 0) {")
-        E(f"    T* __restrict__ q_ = part_ + (wave_ - 1) * {len(names) * WAVE};")
+        E(f"    T* q_ = part_ + (wave_ - 1) * {len(names) * WAVE};")
         E("    " + " ".join(f"q_[{i * WAVE}] = {n};" for i, n in enumerate(names)))
         E("}")
         E("oeq_block_sync();")
         E("if (wave_ > 0) return;")
-        for t in range(self.team - 1):
-            E(" ".join(f"{n} += part_[{(t * len(names) + i) * WAVE}];" for i, n in enumerate(names)))
+        E(f"for (int t_ = 1; t_ < team_size_; ++t_, part_ += {len(names) * WAVE}) {{")
+        E("    " + " ".join(f"{n} += part_[{i * WAVE}];" for i, n in enumerate(names)))
+        E("}")
 
     def ld(self, ptr: str, idx) -> str:
         return f"oeq_ldnt({ptr} + {idx})" if self.nontemporal else f"{ptr}[{idx}]"
@@ -803,7 +846,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         if self.lds_forward:
             self._emit_staged_forward(E, compute)
         else:
-            self.emit_stage(E, 0, self._sums(self.out, self.used_out))
+            self.emit_stage(E, 0, self._sums(self.out, self.used_out), self._held_receiver(2))
             self.emit_pingpong_loop(E, names, load_idx, load, compute)
         E("const bool rv = nv;")
         self.emit_node_output(E, self.out, self.used_out, lambda o: [f"z{o.idx}_{k}" for k in range(o.D)], self.NODE_OUT, self.D3,
@@ -1116,7 +1159,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         if self.staged_backward:
             self._emit_staged_backward(E, compute, grp)
         else:
-            self.emit_stage(E, 0, self._sums(self.in1, self.used_in1))
+            self.emit_stage(E, 0, self._sums(self.in1, self.used_in1), self._held_sender(2 if self.prefetch_backward else 1))
             self.emit_pingpong_loop(E, names, load_idx, load, compute, prefetch_first=self.prefetch_backward)
         E("rv = nv;")
         self.emit_node_output(E, self.in1, self.used_in1, lambda a: [f"dx{a.idx}_{m}" for m in range(a.D)], "Xg", self.D1,
@@ -1201,7 +1244,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         nt = 2 if self.nontemporal else 0
         slabs, words = self._forward_slabs()
         y_off = words - WAVE * len(self.EDGE_Y)
-        self.emit_stage(E, words, self._sums(self.out, self.used_out))
+        self.emit_stage(E, words, self._sums(self.out, self.used_out), self._held_receiver(1))
 
         def dma(E, e, n):
             E("{")
@@ -1241,7 +1284,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         y_off = self._edge_slabs(slabs, off)
         off = y_off + WAVE * len(self.EDGE_Y)
         assert off <= self.stage_words
-        self.emit_stage(E, off, self._sums(self.in1, self.used_in1))
+        self.emit_stage(E, off, self._sums(self.in1, self.used_in1), self._held_sender(1))
 
         def dma(E, e, n):
             E("{")

@@ -65,7 +65,6 @@ class UVURecvGenerator(UVUDetGenerator):
         self.lds_backward = False
         self.waves_per_eu = 0
         self.ordered_backward = False
-        self.sender_words = 0                                     # (pass 2 holds a row of dX and nothing else)
         # words of dX one lane produces per edge (= spill words per lane)
         self.NW = sum(self.in1[i].D for i in self.used_in1)
         self.spill_row = self.NCH * self.NW * self.P              # words per edge
@@ -192,7 +191,7 @@ class UVURecvGenerator(UVUDetGenerator):
                 w = self.group_waves_hint()
             return f" __attribute__((amdgpu_waves_per_eu({w}, {w})))" if w else ""
         return [dict(name=name, threads=WAVE, attr=attr(h), body=self._edges_body(h)) for name, h in self.backward_kernels()] \
-            + [dict(name="backward_dx", threads=WAVE * self.team, attr="", body=self._dx_body())]
+            + [self.with_team(dict(name="backward_dx", threads=WAVE * self.team, attr="", body=self._dx_body()))]
 
     # ---------------------------------------------------------------- pass 1
     def _edges_body(self, h: int = 0) -> str:
@@ -532,7 +531,7 @@ class UVURecvGenerator(UVUDetGenerator):
         def key(E, pos):
             E(f"{{ const i64 e0_ = (i64)elist[{pos}]; if (e0_ >= 0 && e0_ < (i64)nnz) kv_ = (i64)cols[e0_]; }}")
         self._node_setup(E, self.bwd_ptr_off, key=key)
-        self.emit_stage(E, 0, self.NW)
+        self.emit_stage(E, 0, self.NW, self.NW * (1 + self.DX_UNROLL))
         E(f"const T* __restrict__ spill = (const T*)((const char*)ws + {self.spill_off});")
         E("T " + ", ".join(f"acc{w} = (T)0" for w in range(self.NW)) + ";")
         E(f"for (int it = 0; it < maxlen; it += {U}) {{")

@@ -216,9 +216,14 @@ class UVWBatchedGenerator(UVWGenerator):
         return E.text()
 
     # ---------------------------------------------------------------- backward
-    PREFETCH = 2          # weight chunks whose loads are in flight ahead of the one being worked on
-
-    COMPUTE_UNROLL = 4    # steps of a chunk's row loop in flight; all 16 at once would take 100 more registers
+    # Weight chunks whose loads are in flight ahead of the one being worked on, and steps of a chunk's row loop in flight (all 16 at
+    # once would take 100 more registers).  Many chunks are short - 100 words between two 10-channel blocks - and two of them
+    # ahead cover less than a memory latency.  2 and 4 steps / 4 and 8: DiffDock's layer, 50 000 rows 617 / 592 us; 30 channels,
+    # 15 000 rows 161 / 154; 42, 10 000 rows 155 / 150; 8, 20 000 rows 41.6 / 40.6.  More wavefronts per SIMD instead (96 registers)
+    # spill: 656.  fp64, where a word is two registers, gains nothing (465 / 463) and keeps two and 4 (48 channels, l <= 2: 248
+    # registers, 324 with the others).
+    PREFETCH = {"float": 4, "double": 2}
+    COMPUTE_UNROLL = {"float": 8, "double": 4}
     NONTEMPORAL = True    # the weights and their gradient are touched once
     def backward_body(self) -> str:
         E = Emitter()
@@ -245,7 +250,8 @@ class UVWBatchedGenerator(UVWGenerator):
 
         def regs(job):
             return width(job) * _ceil(job[3], 64 * width(job))
-        nbuf = self.PREFETCH + 1
+        ahead = self.PREFETCH[self.T]
+        nbuf = ahead + 1
         for b in range(min(nbuf, len(jobs))):
             E(f"T r{b}_[{max(regs(job) for job in jobs[b::nbuf])}];")
 
@@ -262,7 +268,7 @@ class UVWBatchedGenerator(UVWGenerator):
                     else:
                         E(f"{guard}r{n % nbuf}_[{i}] = {self.ld(f'Wr + {base + 64 * i} + lane')};")
 
-        for n in range(self.PREFETCH):
+        for n in range(ahead):
             request(n)
         E(f"for (int q = lane; q < {self.D3}; q += 64) gl[q] = G[row * {self.D3} + q];")
         E("oeq_sync();")
@@ -305,7 +311,7 @@ class UVWBatchedGenerator(UVWGenerator):
                             E(f"{guard}{{ " + " ".join(f"tile[{pos(f'{64 * V * i + h} + {V} * lane')}] = r{n % nbuf}_[{V * i + h}];"
                                                         for h in range(V)) + " }")
                         E("oeq_sync();")
-                        request(n + self.PREFETCH)
+                        request(n + ahead)
                         full, tail = divmod(wl, ns)
 
                         def step(wq):
@@ -317,7 +323,7 @@ class UVWBatchedGenerator(UVWGenerator):
                             E(("  if (act) " if lp != ul else "  ") + f"tile[ur * {S} + {wq}] = "
                               + " + ".join(f"t{k} * g{k}" for k in range(o.D)) + ";")
                         if full:
-                            E(f"#pragma unroll {self.COMPUTE_UNROLL}")
+                            E(f"#pragma unroll {self.COMPUTE_UNROLL[self.T]}")
                             E(f"for (int j = 0; j < {full}; ++j) {{")
                             step(f"ws + {ns} * j")
                             E("}")

@@ -68,7 +68,7 @@ int load_steps(Module& m, const void* code, size_t code_size, const oeq_step* st
             return fail("step %d (%s): bad workgroup size %u", i, s.desc.kernel, s.desc.num_threads);
         if (s.desc.grid_kind > OEQ_GRID_PER_NODE_AND_PIECE)
             return fail("step %d (%s): unknown grid rule %u", i, s.desc.kernel, s.desc.grid_kind);
-        if ((s.desc.flags & OEQ_STEP_FEW_NODES(0, 0)) && (s.desc.flags & OEQ_STEP_MANY_NODES(0, 0)))
+        if ((s.desc.flags & OEQ_STEP_FEW_NODES(0, 0, 0)) && (s.desc.flags & OEQ_STEP_MANY_NODES(0, 0)))
             return fail("step %d (%s): for few nodes and for many", i, s.desc.kernel);
         if (s.desc.grid_kind != OEQ_GRID_FIXED && s.desc.work_per_block == 0)
             return fail("step %d (%s): work_per_block must be > 0", i, s.desc.kernel);
@@ -336,10 +336,10 @@ void oeq_conv_destroy(oeq_conv* c) { delete c; }
 // A step is skipped on graphs of another size than it is for, and when the call says that the state it would build is already
 // in the workspace.
 static bool skipped(const oeq_step& d, uint32_t call_flags, uint64_t nnz, uint64_t nodes) {
-    const uint32_t sizes = d.flags & (OEQ_STEP_FEW_NODES(0, 0) | OEQ_STEP_MANY_NODES(0, 0));
-    if (sizes) {
+    const bool for_few = d.flags & OEQ_STEP_FEW_NODES(0, 0, 0), for_many = d.flags & OEQ_STEP_MANY_NODES(0, 0);
+    if (for_few || for_many) {
         const bool few = nodes <= ((d.flags >> 8) & 0xfff) && nnz >= ((d.flags >> 20) & 0xff) * nodes;
-        if (few != (sizes == OEQ_STEP_FEW_NODES(0, 0))) return true;
+        if (few == for_many || (for_few && nodes <= (uint64_t)(d.flags >> 28) * 128)) return true;
     }
     if ((call_flags & OEQ_CALL_PREPARED) && (d.flags & OEQ_STEP_GRAPH_PREP)) return true;
     if ((call_flags & OEQ_CALL_COUNTERS_ZERO) && (d.flags & OEQ_STEP_COUNTER_CLEAR)) return true;

@@ -40,15 +40,15 @@ class DeviceProp(C.Structure):
                 ("memoryBusWidth", C.c_int32), ("l2CacheSize", C.c_int32)]
 
 
-def step_few_nodes(nodes: int, edges_per_node: int) -> int:
-    """OEQ_STEP_FEW_NODES with its limits: the step runs on graphs of at most ``nodes`` nodes and at least ``edges_per_node`` times
-    as many edges."""
-    assert 0 < nodes < 4096 and 0 <= edges_per_node < 256
-    return STEP_FEW_NODES | nodes << 8 | edges_per_node << 20
+def step_few_nodes(nodes: int, edges_per_node: int, beyond: int = 0) -> int:
+    """OEQ_STEP_FEW_NODES with its limits: the step runs on graphs of at most ``nodes`` nodes, more than ``beyond`` (a multiple of
+    128), and at least ``edges_per_node`` times as many edges."""
+    assert 0 < nodes < 4096 and 0 <= edges_per_node < 256 and beyond % 128 == 0 and 0 <= beyond < 2048
+    return STEP_FEW_NODES | nodes << 8 | edges_per_node << 20 | beyond // 128 << 28
 
 
 def step_many_nodes(nodes: int, edges_per_node: int) -> int:
-    """OEQ_STEP_MANY_NODES: the step runs on all other graphs."""
+    """OEQ_STEP_MANY_NODES: the step runs on graphs of more nodes, or of fewer edges for each."""
     return step_few_nodes(nodes, edges_per_node) ^ STEP_FEW_NODES ^ STEP_MANY_NODES
 
 

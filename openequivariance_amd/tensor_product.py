@@ -32,8 +32,8 @@ from .wigner import wigner_3j
 def _make_steps(descs, flags: int = 0):
     """Plan dictionaries of a generator -> ``runtime.Step`` records.  ``flags`` (STEP_NEEDS_*) apply to
     every step of the plan; a step's own ``prep=True`` marks it as graph preparation, ``counter_clear=True``
-    as one that only zeroes counters which the operator's other steps leave zeroed again, ``few_nodes`` / ``many_nodes`` =
-    (nodes, edges per node) as one that runs only on / never on graphs of few nodes."""
+    as one that only zeroes counters which the operator's other steps leave zeroed again, ``few_nodes`` / ``many_nodes``
+    (arguments of runtime.step_few_nodes / step_many_nodes) as one for graphs of few or many nodes."""
     def size_rule(d):
         if "few_nodes" in d:
             return rt.step_few_nodes(*d["few_nodes"])

@@ -79,16 +79,20 @@ def test_on_the_gpu(cuda, irreps, dtype, deterministic, monkeypatch):
     import openequivariance_amd as oeq
     prob, _ = common.channelwise(irreps, dtype=dtype)
     conv = oeq.TensorProductConv(prob, torch_op=True, deterministic=deterministic)
-    monkeypatch.setattr(UVUDetGenerator, "TEAM_WAVES", 0)
+    monkeypatch.setattr(UVUDetGenerator, "TEAMS", ())
     single = oeq.TensorProductConv(prob, torch_op=True, deterministic=deterministic)
     assert "forward_few" in conv.jit_kernel and "forward_few" not in single.jit_kernel
     for c in (conv, single):
         if not deterministic:
             c._bwd_choice = type("Grouped", (dict,), dict(__contains__=lambda s, k: True, __getitem__=lambda s, k: "grouped"))()
     monkeypatch.undo()
-    nodes, each = getattr(conv.generator, "fwd", conv.generator).few_limits("forward")
-    for n, nnz, graph in ((nodes, nodes * each, common.random_graph), (nodes, nodes * each - 1, common.random_graph),
-                          (nodes + 1, 5 * nodes, common.random_graph), (1, 3, lambda n, nnz, seed: (np.zeros(3, np.int64),) * 2),
+    g = getattr(conv.generator, "fwd", conv.generator)
+    (_, _, four), (_, beyond, two) = g.few_teams("forward")
+    each = 2 * g.R
+    assert beyond == four < two
+    for n, nnz, graph in ((four, four * each, common.random_graph), (four + 1, 5 * four, common.random_graph),
+                          (two, two * each, common.random_graph), (two, two * each - 1, common.random_graph),
+                          (two + 1, 5 * two, common.random_graph), (1, 2 * each, lambda n, nnz, seed: (np.zeros(nnz, np.int64),) * 2),
                           (40, 900, lambda n, nnz, seed: common.hub_graph(n, nnz, seed, 3, 5, 300, 200))):
         print(n, nnz, flush=True)
         rows, cols, tperm, _ = otp.coord_graph(*graph(n, nnz, 7))
