@@ -14,14 +14,16 @@ path contiguous - so that a wavefront's access is one 256- or 512-byte run:
   park it in LDS; then lanes <-> (output channel w, a slice of u) walk the chunks with the loads a
   fixed number of steps ahead of the multiplies, branch-free, T read from LDS; the slices are
   summed with lane exchanges at the end of an output block;
-* backward: a chunk goes global -> registers (two chunks ahead) -> LDS, padded to an odd row length;
-  lanes <-> (u, a slice of w) then read their row of it, form dT (-> dX, dY through the CG
-  transpose) against dZ in LDS and put dW = T (x) dZ back into the same LDS words, which leave in
-  memory order again.
+* backward: the weights go global -> registers -> LDS, lanes <-> (u, a slice of w) then read their row of a
+  chunk, form dT (-> dX, dY through the CG transpose) against dZ in LDS and put dW = T (x) dZ back into
+  the same LDS words, which leave in memory order again.  A row's weights pass in batches of whole chunks, 16 bytes
+  per lane (backward_stream_body), or, where they do not divide into such, chunk by chunk.
 
 The external (oeq) weight order is addressed in place by index arithmetic.
 """
 from __future__ import annotations
+
+import math
 
 from ..problem import TPProblem
 from .common import Emitter, jinja_env
@@ -31,9 +33,11 @@ from .uvw import UVWGenerator, _ceil
 class UVWBatchedGenerator(UVWGenerator):
     _allow_batched = True
 
-    def __init__(self, problem: TPProblem, pairs: bool = True):
+    def __init__(self, problem: TPProblem, pairs: bool = True, stream: bool = True):
         """``pairs``: fp32 weights move two words per lane where a chunk's offset and width are even (an 8-byte
-        access sustains more of the HBM rate than a 4-byte one); needs W and dW at 8-byte aligned addresses."""
+        access sustains more of the HBM rate than a 4-byte one); needs W and dW at 8-byte aligned addresses.
+        ``stream``: the backward's weights move in batches of 16 bytes per lane where a row divides into such; needs
+        W and dW at 16-byte aligned addresses."""
         super().__init__(problem)
         self.pairs = bool(pairs) and self.T == "float" and self.WN % 2 == 0
         if self.shared:
@@ -41,6 +45,38 @@ class UVWBatchedGenerator(UVWGenerator):
         self.kind = "uvw_batched"
         self.t_lds = max([sum(p.mu * o.D for o in ph for p in self.paths_into(o.idx)) for ph in self.forward_phases()] + [0])
         self.ws_elems = 0
+        self.batches = self._batches() if stream else None
+        self.stream = self.batches is not None
+
+    STREAM_BYTES = 4096           # of a batch at most (a chunk of 32 x 32 words; 8192 in fp64)
+
+    def _batches(self):
+        """The row's weight chunks in the order they lie in memory, as batches of whole chunks that begin and end at multiples of
+        16 bytes: [[(path, uc, ul, wc, wl, offset), ..], ..]; None where the row does not divide into such."""
+        vw, most = 16 // self.itemsize, max(self.STREAM_BYTES, 1024 * self.itemsize) // self.itemsize
+        jobs = sorted(((p, uc, ul, wc, wl, self.chunk_base(p, uc, wc)) for p in self.paths for uc, ul in self.chunks(p.mu)
+                       for wc, wl in self.chunks(p.mw)), key=lambda job: job[-1])
+        batches, begin, end = [], 0, 0
+        todo = []                                    # chunks since the last multiple of 16 bytes
+        for job in jobs:
+            if job[-1] != end:
+                return None
+            end += job[2] * job[4]
+            todo.append(job)
+            if end % vw == 0:
+                if not batches or end - begin > most:
+                    begin = todo[0][-1]
+                    batches.append([])
+                batches[-1] += todo
+                todo = []
+                if end - begin > most:
+                    return None
+        if todo or end != self.WN or not batches:
+            return None
+        # whole lines and long chunks stay as they are: 32 channels, 20 000 rows 112 us against 116.5, 48 channels 160 against 163
+        # (16 channels, chunks of 256 words: 81.9 / 79.8)
+        whole = all(ul * wl * self.itemsize % 128 == 0 for _, _, ul, _, wl, _ in jobs)
+        return None if whole and self.WN * 4 >= 1600 * len(jobs) else batches
 
     def describe(self) -> str:
         return (f"uvw per-row weights T={self.T} paths={len(self.paths)} d1={self.D1} d2={self.D2} d3={self.D3} "
@@ -226,6 +262,8 @@ class UVWBatchedGenerator(UVWGenerator):
     COMPUTE_UNROLL = {"float": 8, "double": 4}
     NONTEMPORAL = True    # the weights and their gradient are touched once
     def backward_body(self) -> str:
+        if self.stream:
+            return self.backward_stream_body()
         E = Emitter()
         E("const int lane = threadIdx.x;")
         E("const u64 row = blockIdx.x;")
@@ -356,6 +394,131 @@ class UVWBatchedGenerator(UVWGenerator):
                 E.level -= 1
                 E("}")
         assert n == len(jobs)
+        for f in self.used_y:
+            E(f"dy{f} = oeq_wave_sum63(dy{f});")
+        E("if (lane == 63) {")
+        for f in range(self.D2):
+            E(f"    Yg[row * {self.D2} + {f}] = " + (f"dy{f};" if f in self.used_y else "(T)0;"))
+        E("}")
+        return E.text()
+
+    def backward_stream_body(self) -> str:
+        """The row's weights as batches of whole chunks, in memory order: a batch moves 16 bytes per lane and instruction, whole cache
+        lines, and the next one is in flight in registers while this one is worked on in LDS.  Chunk by chunk, an access
+        is as long as a chunk (400 bytes between two 10-channel blocks) and begins and ends inside a cache line.  All
+        of the row's dX are live at once, as memory order takes the input blocks in turns.  DiffDock's layer, 50 000 rows
+        595 -> 551 us (fp64, 20 000 rows, 465 -> 431); 8 channels, 20 000 rows 40.6 -> 38, 12, 61 -> 53, 42, 10 000 rows 150 -> 141, 36, 6000 rows
+        144 -> 141.  Batches of 6 KB: 561; two or four steps of a row at a time: 568."""
+        E = Emitter()
+        VW = 16 // self.itemsize
+        batches = self.batches
+        words = [sum(ul * wl for _, _, ul, _, wl, _ in b) for b in batches]
+        E("const int lane = threadIdx.x;")
+        E("const u64 row = blockIdx.x;")
+        E("if (row >= n) return;")
+        E(f"__shared__ __attribute__((aligned(16))) T tile[{max(words)}];")
+        E(f"__shared__ T gl[{max(1, self.D3)}];")
+        E(f"const T* __restrict__ Xr = X + row * {self.D1};")
+        E(f"const T* __restrict__ Wr = W + row * {self.WN};")
+        E(f"T* __restrict__ Wgr = Wg + row * {self.WN};")
+
+        def vectors(b):
+            """Positions of this lane's 16-byte pieces of batch b: lanes past its end repeat its last piece."""
+            return [f"{64 * VW * i} + {VW} * lane" if 64 * VW * (i + 1) <= words[b] else f"min({64 * VW * i} + {VW} * lane, {words[b] - VW})"
+                    for i in range(_ceil(words[b], 64 * VW))]
+
+        def request(b):
+            if b < len(batches):
+                E(f"// batch {b}: {words[b]} words at {batches[b][0][-1]}")
+                for i, at in enumerate(vectors(b)):
+                    E(f"const VT b{b}_{i} = oeq_ldnt16(Wr + {batches[b][0][-1]} + {at});")
+        request(0)
+        E(f"for (int q = lane; q < {self.D3}; q += 64) gl[q] = G[row * {self.D3} + q];")
+        for f in self.used_y:
+            E(f"const T y{f} = Y[row * {self.D2} + {f}];")
+            E(f"T dy{f} = (T)0;")
+        # lanes <-> (channel of a chunk, slice of its row), by the chunk's channels
+        for ul in sorted({ul for a in self.in1 for _, ul in self.chunks(a.mul)}):
+            lp, lg, _ = self._split(ul)
+            E(f"const int uq{ul} = lane & {lp - 1}, ws{ul} = lane >> {lg}, ur{ul} = min(uq{ul}, {ul - 1}); const bool act{ul} = uq{ul} < {ul};")
+        held = [(a, uc, ul) for a in self.in1 if a.dim for uc, ul in self.chunks(a.mul)]
+        for a, uc, ul in held:
+            E(f"const T* __restrict__ xp{a.idx}_{uc} = Xr + {a.off} + ({32 * uc} + ur{ul}) * {a.D};")
+            E("const T " + ", ".join(f"x{a.idx}_{uc}_{i} = xp{a.idx}_{uc}[{i}]" for i in range(a.D)) + ";")
+            E("T " + ", ".join(f"dx{a.idx}_{uc}_{i} = (T)0" for i in range(a.D)) + ";")
+        banks = 128 // self.itemsize               # values side by side in LDS that lanes read without conflict
+
+        def chunk(job, at):
+            p, uc, ul, wc, wl, _ = job
+            o = p.o
+            lp, _, ns = self._split(ul)
+            g = math.gcd(wl, banks)
+            turn = banks // g <= banks // 4        # rows of four and more lanes would begin in one bank
+            E(f"{{ // weights [{ul}][{wl}] of path {p.t}")
+            E.level += 1
+            if turn:
+                E(f"const int turn_ = ur{ul} * {g} / {banks} % {wl};     // rows that begin in one bank are walked from another column each")
+            full, tail = divmod(wl, ns)
+
+            def step(wq):
+                if turn:
+                    E(f"  int c_ = {wq} + turn_; c_ -= c_ < {wl} ? 0 : {wl};")
+                else:
+                    E(f"  const int c_ = {wq};")
+                E(f"  const T wv = tile[{at} + ur{ul} * {wl} + c_];")
+                E("  const T " + ", ".join(f"g{k} = gl[{o.off + 32 * wc * o.D + k} + c_ * {o.D}]" for k in range(o.D)) + ";")
+                for k in range(o.D):
+                    E(f"  dt{k} = oeq_fma(wv, g{k}, dt{k});")
+                E(("  if (act%d) " % ul if lp != ul else "  ") + f"tile[{at} + ur{ul} * {wl} + c_] = "
+                  + " + ".join(f"t{k} * g{k}" for k in range(o.D)) + ";")
+            if full:
+                E(f"#pragma unroll {self.COMPUTE_UNROLL[self.T]}")
+                E(f"for (int j = 0; j < {full}; ++j) {{")
+                step(f"ws{ul} + {ns} * j")
+                E("}")
+            if tail:
+                E(f"if (ws{ul} < {tail}) {{")
+                step(f"ws{ul} + {ns * full}")
+                E("}")
+            E.level -= 1
+            E("}")
+
+        def finish(p, uc, ul):
+            """dT of the channels is complete for the chunks worked on: slices summed, into dX and dY."""
+            lp, _, _ = self._split(ul)
+            s = lp
+            while s < 64:
+                E(" ".join(f"dt{k} += oeq_shfl_xor(dt{k}, {s});" for k in range(p.o.D)))
+                s *= 2
+            E(f"if (!act{ul} || ws{ul} != 0) {{ " + " ".join(f"dt{k} = (T)0;" for k in range(p.o.D)) + " }")
+            self.emit_cg_backward(E, p, "dt", f"x{p.a.idx}_{uc}_", "y", f"dx{p.a.idx}_{uc}_", "dy")
+        names = max(p.o.D for p in self.paths)
+        E("T " + ", ".join(f"{v}{k} = (T)0" for v in ("t", "dt") for k in range(names)) + ";")
+        now = None                                   # (path, uc, ul) whose t and dt the registers hold
+        for b, batch in enumerate(batches):
+            for i, at in enumerate(vectors(b)):
+                E(f"*(VT*)(tile + {at}) = b{b}_{i};")
+            E("oeq_sync();")
+            request(b + 1)
+            for job in batch:
+                p, uc, ul = job[:3]
+                if now is None or (p.t, uc) != (now[0].t, now[1]):
+                    if now:
+                        finish(*now)
+                    now = p, uc, ul
+                    E("{")
+                    self.emit_cg_forward(E, p, f"x{p.a.idx}_{uc}_", "y", "s")
+                    E(" ".join(f"t{k} = s{k}; dt{k} = (T)0;" for k in range(p.o.D)))
+                    E("}")
+                chunk(job, job[-1] - batch[0][-1])
+            E("oeq_sync();")
+            for i, at in enumerate(vectors(b)):
+                E(f"oeq_stnt16(Wgr + {batch[0][-1]} + {at}, *(const VT*)(tile + {at}));")
+            E("oeq_sync();")
+        finish(*now)
+        for a, uc, ul in held:
+            E(f"if (act{ul} && ws{ul} == 0) {{ T* __restrict__ dp = Xg + row * {self.D1} + {a.off} + ({32 * uc} + uq{ul}) * {a.D}; "
+              + " ".join(f"dp[{i}] = dx{a.idx}_{uc}_{i};" for i in range(a.D)) + " }")
         for f in self.used_y:
             E(f"dy{f} = oeq_wave_sum63(dy{f});")
         E("if (lane == 63) {")

@@ -157,6 +157,7 @@ class TensorProduct(TensorProductBase):
         self._dims = (self.L1.dim, self.L2.dim, self.L3.dim, config.weight_numel)
         self._workspaces = {}                 # (device, stream) -> scratch tensor (fixed size, never regrown)
         self._internal_unaligned = None       # kernels without 16-byte vector stores, compiled on first need
+        self._unaligned_batched = {}          # those of per-row uvw weights for tensors aligned to 8 bytes (True) or not
         # dense uvw: kernels for few rows and their largest batch (forward, backward).  Built here like the double backward's,
         # not by the call that first needs them: that call would wait for the compiler, and a stream capture cannot
         self._few_rows, self._few_rows_limits = self._few_row_kernels()
@@ -209,14 +210,15 @@ class TensorProduct(TensorProductBase):
                 self._internal_unaligned = rt.TPImpl(rt.compile_source(g.render()), _make_steps(fwd, self._step_flags),
                                                      _make_steps(bwd, self._step_flags))
             return self._internal_unaligned
-        if isinstance(self.generator, UVWBatchedGenerator) and self.generator.pairs and bits % 8:
-            # the same for the per-row-weights uvw kernels, which move fp32 weights two words at a time
-            if self._internal_unaligned is None:
-                g = UVWBatchedGenerator(self.config, pairs=False)
+        if isinstance(self.generator, UVWBatchedGenerator) and ((self.generator.pairs and bits % 8) or (self.generator.stream and bits % 16)):
+            # the same for the per-row-weights uvw kernels, which move weights 16 bytes at a time, or two fp32 words
+            pairs = bits % 8 == 0
+            if pairs not in self._unaligned_batched:
+                g = UVWBatchedGenerator(self.config, pairs=pairs, stream=False)
                 fwd, bwd, _ = g.plan()
-                self._internal_unaligned = rt.TPImpl(rt.compile_source(g.render()), _make_steps(fwd, self._step_flags),
-                                                     _make_steps(bwd, self._step_flags))
-            return self._internal_unaligned
+                self._unaligned_batched[pairs] = rt.TPImpl(rt.compile_source(g.render()), _make_steps(fwd, self._step_flags),
+                                                           _make_steps(bwd, self._step_flags))
+            return self._unaligned_batched[pairs]
         return self.internal
 
     def _pick_rows(self, batch: int, backward: bool):

@@ -1,0 +1,70 @@
+"""Backward of uvw products with per-row weights whose weights pass in batches of 16-byte pieces: chunks of every width that divides
+into such, rows of a chunk that would meet in one LDS bank (walked from other columns), several copies of the second operand,
+batches of one and of many chunks, both types; rows that do not divide keep the other schedule."""
+import numpy as np
+import pytest
+
+import common
+from common import rel_err
+from host_emu import emu
+from openequivariance_amd.codegen.uvw_batched import UVWBatchedGenerator
+from oracle import tp as otp
+from oracle import weights as ow
+
+CASES = {
+    "short_chunks": ("10x1o+10x1e+20x0e", "1x0e+1x1o", "10x1o+10x1e+20x0e"),
+    "rows_of_32_16_8_4_words": ("34x0e+6x1o", "1x0e+1x1o", "32x0e+48x1o+8x0o+4x2e"),
+    "copies": ("10x0e+40x1o", "3x0e+2x1o", "36x0e+10x1o"),
+    "odd_paths_even_row": ("3x0e+5x1o", "1x0e+1x1o", "4x0e+1x1o"),
+}
+TOL = {np.float32: 4e-6, np.float64: 1e-13}       # a few hundred roundings a value
+
+
+def generator(case, dtype):
+    prob, oprob = common.fully_connected(CASES[case], shared=False, dtype=dtype)
+    return UVWBatchedGenerator(prob), prob, oprob
+
+
+def test_which_rows_stream():
+    for case in CASES:
+        for dtype in TOL:
+            g, prob, _ = generator(case, dtype)
+            assert g.stream and sum(len(b) for b in g.batches) == sum(len(g.chunks(p.mu)) * len(g.chunks(p.mw)) for p in g.paths)
+            assert all(b[0][-1] * g.itemsize % 16 == 0 for b in g.batches) and len(g.batches) > (case != "odd_paths_even_row")
+            assert not UVWBatchedGenerator(prob, stream=False).stream
+    for irreps in (("5x0e+21x1o", "1x0e+1x1o+1x2e", "18x0e+7x1o+3x2e"), ("32x0e+32x1o", "1x0e+1x1o", "32x0e+32x1o")):
+        assert not UVWBatchedGenerator(common.fully_connected(irreps, shared=False)[0]).stream     # ragged; whole lines
+
+
+@pytest.mark.parametrize("dtype", list(TOL))
+@pytest.mark.parametrize("case", list(CASES))
+def test_emulated(case, dtype):
+    g, prob, oprob = generator(case, dtype)
+    X, Y, We, G = common.tp_inputs(prob, 3, 10, dtype=dtype, w_scale=0.3)
+    _, bwd, _ = g.plan()
+    out = emu.run_tp(g, bwd, X, Y, ow.e3nn_to_oeq(oprob, We), G)
+    dX, dY, dW = otp.backward(oprob, X, Y, We, G)
+    assert rel_err(out["Xg"], dX) < TOL[dtype] and rel_err(out["Yg"], dY) < TOL[dtype]
+    assert rel_err(ow.oeq_to_e3nn(oprob, out["Wg"]), dW) < TOL[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(TOL))
+@pytest.mark.parametrize("case", [*CASES, "diffdock"])
+def test_on_the_gpu(cuda, case, dtype, monkeypatch):
+    """Against the oracle, also with weights off 16 and off 8 bytes."""
+    import torch
+    import openequivariance_amd as oeq
+    monkeypatch.setitem(CASES, "diffdock", ("10x1o+10x1e+48x0e+48x0o", "1x0e+1x1o+1x2e", "10x1o+10x1e+48x0e+48x0o"))
+    g, prob, oprob = generator(case, dtype)
+    tp = oeq.TensorProduct(prob, torch_op=True)
+    assert tp.generator.stream
+    for n in (1, 37, 1025):
+        X, Y, We, G = common.tp_inputs(prob, n, n, dtype=dtype, w_scale=0.3)
+        x, y, w, dz = (torch.tensor(a, device=cuda) for a in (X, Y, ow.e3nn_to_oeq(oprob, We), G))
+        dX, dY, dW = otp.backward(oprob, X, Y, We, G)
+        for off in (0, 1, 2):
+            v = torch.cat([w.new_zeros(off), w.reshape(-1)])[off:].view(w.shape)
+            got = [t.cpu().numpy() for t in tp.backward_helper(x, y, v, dz)]
+            for a, b in zip((*got[:2], ow.oeq_to_e3nn(oprob, got[2])), (dX, dY, dW)):
+                assert rel_err(a, b) < TOL[dtype]
