@@ -10,7 +10,8 @@ the same weights through shared memory into a CUDA-core matmul).  Both kernels r
 weights in the order they lie in memory - the external order keeps each 32 x 32 chunk [u][w] of a
 path contiguous - so that a wavefront's access is one 256- or 512-byte run:
 
-* forward: lanes <-> channel u compute T_t[u, :] of every path into a group of output blocks and
+* forward: as for the backward, the weights pass through LDS in batches of 16-byte pieces where a row divides into such
+  (forward_stream_body).  Otherwise lanes <-> channel u compute T_t[u, :] of every path into a group of output blocks and
   park it in LDS; then lanes <-> (output channel w, a slice of u) walk the chunks with the loads a
   fixed number of steps ahead of the multiplies, branch-free, T read from LDS; the slices are
   summed with lane exchanges at the end of an output block;
@@ -47,7 +48,12 @@ class UVWBatchedGenerator(UVWGenerator):
         self.ws_elems = 0
         self.batches = self._batches() if stream else None
         self.stream = self.batches is not None
+        # the backward keeps its other walk where chunks are long and whole lines: 32 channels, 20 000 rows 112 us against 116.5, 48
+        # channels 160 against 163, fp64, 24 channels, 6000 rows 117 against 120 (16 channels, chunks of 256 words: 81.9 / 79.8)
+        self.stream_backward = self.stream and not (self.WN >= 400 * sum(map(len, self.batches)) and all(
+            ul * wl * self.itemsize % 128 == 0 for b in self.batches for _, _, ul, _, wl, _ in b))
 
+    STREAM_UNROLL = 4             # steps of a chunk's loop in flight in the forward
     STREAM_BYTES = 4096           # of a batch at most (a chunk of 32 x 32 words; 8192 in fp64)
 
     def _batches(self):
@@ -73,10 +79,7 @@ class UVWBatchedGenerator(UVWGenerator):
                     return None
         if todo or end != self.WN or not batches:
             return None
-        # whole lines and long chunks stay as they are: 32 channels, 20 000 rows 112 us against 116.5, 48 channels 160 against 163
-        # (16 channels, chunks of 256 words: 81.9 / 79.8)
-        whole = all(ul * wl * self.itemsize % 128 == 0 for _, _, ul, _, wl, _ in jobs)
-        return None if whole and self.WN * 4 >= 1600 * len(jobs) else batches
+        return batches
 
     def describe(self) -> str:
         return (f"uvw per-row weights T={self.T} paths={len(self.paths)} d1={self.D1} d2={self.D2} d3={self.D3} "
@@ -141,6 +144,8 @@ class UVWBatchedGenerator(UVWGenerator):
         return [ph for ph in phases if ph]
 
     def forward_body(self) -> str:
+        if self.stream:
+            return self.forward_stream_body()
         E = Emitter()
         E("const int lane = threadIdx.x;")
         E("const u64 row = blockIdx.x;")
@@ -251,6 +256,112 @@ class UVWBatchedGenerator(UVWGenerator):
             E("}")
         return E.text()
 
+    def _stream_header(self, E: Emitter, words) -> None:
+        E("const int lane = threadIdx.x;")
+        E("const u64 row = blockIdx.x;")
+        E("if (row >= n) return;")
+        E(f"__shared__ __attribute__((aligned(16))) T tile[{max(words)}];")
+        E(f"const T* __restrict__ Xr = X + row * {self.D1};")
+        E(f"const T* __restrict__ Wr = W + row * {self.WN};")
+
+    def _vectors(self, words: int):
+        """Positions of a lane's 16-byte pieces of a batch: lanes past its end repeat its last piece."""
+        VW = 16 // self.itemsize
+        return [f"{64 * VW * i} + {VW} * lane" if 64 * VW * (i + 1) <= words else f"min({64 * VW * i} + {VW} * lane, {words - VW})"
+                for i in range(_ceil(words, 64 * VW))]
+
+    def _stream(self, E: Emitter, words, work, store=None) -> None:
+        """The row's batches through LDS, the next one in flight in registers while ``work(job, offset in the tile)`` is
+        done on the chunks of one; ``store`` takes the tile back to memory."""
+        def request(b):
+            if b < len(words):
+                E(f"// batch {b}: {words[b]} words at {self.batches[b][0][-1]}")
+                for i, at in enumerate(self._vectors(words[b])):
+                    E(f"const VT b{b}_{i} = oeq_ldnt16(Wr + {self.batches[b][0][-1]} + {at});")
+        for b, batch in enumerate(self.batches):
+            if b == 0:
+                request(0)
+                yield
+            for i, at in enumerate(self._vectors(words[b])):
+                E(f"*(VT*)(tile + {at}) = b{b}_{i};")
+            E("oeq_sync();")
+            request(b + 1)
+            for job in batch:
+                work(job, job[-1] - batch[0][-1])
+            E("oeq_sync();")
+            if store:
+                for i, at in enumerate(self._vectors(words[b])):
+                    E(f"oeq_stnt16({store} + {batch[0][-1]} + {at}, *(const VT*)(tile + {at}));")
+                E("oeq_sync();")
+
+    def forward_stream_body(self) -> str:
+        """The forward over the same batches as backward_stream_body: T of a path goes to LDS when its weights come up (lanes <-> u),
+        then lanes <-> (output channel, slice of u).  Against lanes that read the weights from memory chunk by chunk: DiffDock's
+        layer, 50 000 rows 275 -> 252 us (5.9 TB/s), fp64, 20 000 rows 210 -> 197; 6 channels, 20 000 rows 26.5 -> 17.8, 12 31.7 ->
+        26.4, 42, 10 000 rows 67.6 -> 60.2, 48, 4000 rows 65.8 -> 64.0 (eight steps at a time: 70.8), fp64, 2500 rows 141 -> 80
+        (that walk spilled); 32 channels, 20 000 rows 53.8 and 54.0."""
+        E = Emitter()
+        words = [sum(ul * wl for _, _, ul, _, wl, _ in b) for b in self.batches]
+        self._stream_header(E, words)
+        E(f"__shared__ T tl[{max(p.mu * p.o.D for p in self.paths)}];")
+        for wl in sorted({wl for o in self.out for _, wl in self.chunks(o.mul)}):
+            lp, lg, _ = self._split(wl)
+            E(f"const int wq{wl} = min(lane & {lp - 1}, {wl - 1}), us{wl} = lane >> {lg};")
+        outs = [(o, wc, wl) for o in self.out if o.dim for wc, wl in self.chunks(o.mul)]
+        for o, wc, _ in outs:
+            E("T " + ", ".join(f"z{o.idx}_{wc}_{k} = (T)0" for k in range(o.D)) + ";")
+        held = [(a, h) for a in self.in1 if a.dim for h in range(_ceil(a.mul, 64))]
+        now = [None]
+
+        def work(job, at):
+            p, uc, ul, wc, wl, _ = job
+            o = p.o
+            if now[0] != p.t:
+                now[0] = p.t
+                E("oeq_sync();")
+                for h in range(_ceil(p.mu, 64)):
+                    E(f"{{ const int u = {64 * h} + lane;   // T of path {p.t}")
+                    E.level += 1
+                    self.emit_cg_forward(E, p, f"x{p.a.idx}_{h}_", "y", "t")
+                    E(f"if (u < {p.mu}) {{ " + " ".join(f"tl[u * {o.D} + {k}] = t{k};" for k in range(o.D)) + " }")
+                    E.level -= 1
+                    E("}")
+                E("oeq_sync();")
+            _, _, ns = self._split(wl)
+            full, tail = divmod(ul, ns)
+            E(f"{{ // weights [{ul}][{wl}] of path {p.t}")
+
+            def step(u):
+                E(f"  const int u_ = {u};")
+                E(f"  const T wv = tile[{at} + u_ * {wl} + wq{wl}];")
+                for k in range(o.D):
+                    E(f"  z{o.idx}_{wc}_{k} = oeq_fma(wv, tl[({32 * uc} + u_) * {o.D} + {k}], z{o.idx}_{wc}_{k});")
+            if full:
+                E(f"#pragma unroll {self.STREAM_UNROLL}")
+                E(f"for (int j = 0; j < {full}; ++j) {{")
+                step(f"us{wl} + {ns} * j")
+                E("}")
+            if tail:
+                E(f"if (us{wl} < {tail}) {{")
+                step(f"us{wl} + {ns * full}")
+                E("}")
+            E("}")
+        for _ in self._stream(E, words, work):           # (the first batch is on its way)
+            for f in self.used_y:
+                E(f"const T y{f} = Y[row * {self.D2} + {f}];")
+            for a, h in held:
+                E(f"const T* __restrict__ xp{a.idx}_{h} = Xr + {a.off} + min({64 * h} + lane, {a.mul - 1}) * {a.D};")
+                E("const T " + ", ".join(f"x{a.idx}_{h}_{i} = xp{a.idx}_{h}[{i}]" for i in range(a.D)) + ";")
+        for o, wc, wl in outs:
+            lp, _, _ = self._split(wl)
+            s = lp
+            while s < 64:
+                E(" ".join(f"z{o.idx}_{wc}_{k} += oeq_shfl_xor(z{o.idx}_{wc}_{k}, {s});" for k in range(o.D)))
+                s *= 2
+            E(f"if (lane < {wl}) {{ T* __restrict__ zp = Z + row * {self.D3} + {o.off} + ({32 * wc} + lane) * {o.D}; "
+              + " ".join(f"zp[{k}] = z{o.idx}_{wc}_{k};" for k in range(o.D)) + " }")
+        return E.text()
+
     # ---------------------------------------------------------------- backward
     # Weight chunks whose loads are in flight ahead of the one being worked on, and steps of a chunk's row loop in flight (all 16 at
     # once would take 100 more registers).  Many chunks are short - 100 words between two 10-channel blocks - and two of them
@@ -262,7 +373,7 @@ class UVWBatchedGenerator(UVWGenerator):
     COMPUTE_UNROLL = {"float": 8, "double": 4}
     NONTEMPORAL = True    # the weights and their gradient are touched once
     def backward_body(self) -> str:
-        if self.stream:
+        if self.stream_backward:
             return self.backward_stream_body()
         E = Emitter()
         E("const int lane = threadIdx.x;")
@@ -410,29 +521,25 @@ class UVWBatchedGenerator(UVWGenerator):
         595 -> 551 us (fp64, 20 000 rows, 465 -> 431); 8 channels, 20 000 rows 40.6 -> 38, 12, 61 -> 53, 42, 10 000 rows 150 -> 141, 36, 6000 rows
         144 -> 141.  Batches of 6 KB: 561; two or four steps of a row at a time: 568."""
         E = Emitter()
-        VW = 16 // self.itemsize
-        batches = self.batches
-        words = [sum(ul * wl for _, _, ul, _, wl, _ in b) for b in batches]
-        E("const int lane = threadIdx.x;")
-        E("const u64 row = blockIdx.x;")
-        E("if (row >= n) return;")
-        E(f"__shared__ __attribute__((aligned(16))) T tile[{max(words)}];")
+        words = [sum(ul * wl for _, _, ul, _, wl, _ in b) for b in self.batches]
+        self._stream_header(E, words)
         E(f"__shared__ T gl[{max(1, self.D3)}];")
-        E(f"const T* __restrict__ Xr = X + row * {self.D1};")
-        E(f"const T* __restrict__ Wr = W + row * {self.WN};")
         E(f"T* __restrict__ Wgr = Wg + row * {self.WN};")
+        now = [None]                                 # (path, uc, ul) whose t and dt the registers hold
 
-        def vectors(b):
-            """Positions of this lane's 16-byte pieces of batch b: lanes past its end repeat its last piece."""
-            return [f"{64 * VW * i} + {VW} * lane" if 64 * VW * (i + 1) <= words[b] else f"min({64 * VW * i} + {VW} * lane, {words[b] - VW})"
-                    for i in range(_ceil(words[b], 64 * VW))]
-
-        def request(b):
-            if b < len(batches):
-                E(f"// batch {b}: {words[b]} words at {batches[b][0][-1]}")
-                for i, at in enumerate(vectors(b)):
-                    E(f"const VT b{b}_{i} = oeq_ldnt16(Wr + {batches[b][0][-1]} + {at});")
-        request(0)
+        def work(job, at):
+            p, uc, ul = job[:3]
+            if now[0] is None or (p.t, uc) != (now[0][0].t, now[0][1]):
+                if now[0]:
+                    finish(*now[0])
+                now[0] = p, uc, ul
+                E("{")
+                self.emit_cg_forward(E, p, f"x{p.a.idx}_{uc}_", "y", "s")
+                E(" ".join(f"t{k} = s{k}; dt{k} = (T)0;" for k in range(p.o.D)))
+                E("}")
+            chunk(job, at)
+        stream = self._stream(E, words, work, "Wgr")
+        next(stream)                                 # (the first batch is on its way)
         E(f"for (int q = lane; q < {self.D3}; q += 64) gl[q] = G[row * {self.D3} + q];")
         for f in self.used_y:
             E(f"const T y{f} = Y[row * {self.D2} + {f}];")
@@ -494,28 +601,9 @@ class UVWBatchedGenerator(UVWGenerator):
             self.emit_cg_backward(E, p, "dt", f"x{p.a.idx}_{uc}_", "y", f"dx{p.a.idx}_{uc}_", "dy")
         names = max(p.o.D for p in self.paths)
         E("T " + ", ".join(f"{v}{k} = (T)0" for v in ("t", "dt") for k in range(names)) + ";")
-        now = None                                   # (path, uc, ul) whose t and dt the registers hold
-        for b, batch in enumerate(batches):
-            for i, at in enumerate(vectors(b)):
-                E(f"*(VT*)(tile + {at}) = b{b}_{i};")
-            E("oeq_sync();")
-            request(b + 1)
-            for job in batch:
-                p, uc, ul = job[:3]
-                if now is None or (p.t, uc) != (now[0].t, now[1]):
-                    if now:
-                        finish(*now)
-                    now = p, uc, ul
-                    E("{")
-                    self.emit_cg_forward(E, p, f"x{p.a.idx}_{uc}_", "y", "s")
-                    E(" ".join(f"t{k} = s{k}; dt{k} = (T)0;" for k in range(p.o.D)))
-                    E("}")
-                chunk(job, job[-1] - batch[0][-1])
-            E("oeq_sync();")
-            for i, at in enumerate(vectors(b)):
-                E(f"oeq_stnt16(Wgr + {batch[0][-1]} + {at}, *(const VT*)(tile + {at}));")
-            E("oeq_sync();")
-        finish(*now)
+        for _ in stream:
+            pass
+        finish(*now[0])
         for a, uc, ul in held:
             E(f"if (act{ul} && ws{ul} == 0) {{ T* __restrict__ dp = Xg + row * {self.D1} + {a.off} + ({32 * uc} + uq{ul}) * {a.D}; "
               + " ".join(f"dp[{i}] = dx{a.idx}_{uc}_{i};" for i in range(a.D)) + " }")

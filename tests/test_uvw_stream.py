@@ -1,4 +1,4 @@
-"""Backward of uvw products with per-row weights whose weights pass in batches of 16-byte pieces: chunks of every width that divides
+"""uvw products with per-row weights whose weights pass in batches of 16-byte pieces: chunks of every width that divides
 into such, rows of a chunk that would meet in one LDS bank (walked from other columns), several copies of the second operand,
 batches of one and of many chunks, both types; rows that do not divide keep the other schedule."""
 import numpy as np
@@ -29,11 +29,12 @@ def test_which_rows_stream():
     for case in CASES:
         for dtype in TOL:
             g, prob, _ = generator(case, dtype)
-            assert g.stream and sum(len(b) for b in g.batches) == sum(len(g.chunks(p.mu)) * len(g.chunks(p.mw)) for p in g.paths)
+            assert g.stream and g.stream_backward and sum(len(b) for b in g.batches) == sum(len(g.chunks(p.mu)) * len(g.chunks(p.mw)) for p in g.paths)
             assert all(b[0][-1] * g.itemsize % 16 == 0 for b in g.batches) and len(g.batches) > (case != "odd_paths_even_row")
             assert not UVWBatchedGenerator(prob, stream=False).stream
-    for irreps in (("5x0e+21x1o", "1x0e+1x1o+1x2e", "18x0e+7x1o+3x2e"), ("32x0e+32x1o", "1x0e+1x1o", "32x0e+32x1o")):
-        assert not UVWBatchedGenerator(common.fully_connected(irreps, shared=False)[0]).stream     # ragged; whole lines
+    ragged, lines = (UVWBatchedGenerator(common.fully_connected(irreps, shared=False)[0]) for irreps in
+                     (("5x0e+21x1o", "1x0e+1x1o+1x2e", "18x0e+7x1o+3x2e"), ("32x0e+32x1o", "1x0e+1x1o", "32x0e+32x1o")))
+    assert not ragged.stream and not ragged.stream_backward and lines.stream and not lines.stream_backward
 
 
 @pytest.mark.parametrize("dtype", list(TOL))
@@ -41,7 +42,9 @@ def test_which_rows_stream():
 def test_emulated(case, dtype):
     g, prob, oprob = generator(case, dtype)
     X, Y, We, G = common.tp_inputs(prob, 3, 10, dtype=dtype, w_scale=0.3)
-    _, bwd, _ = g.plan()
+    fwd, bwd, _ = g.plan()
+    out = emu.run_tp(g, fwd, X, Y, ow.e3nn_to_oeq(oprob, We))
+    assert rel_err(out["Z"], otp.forward(oprob, X, Y, We)) < TOL[dtype]
     out = emu.run_tp(g, bwd, X, Y, ow.e3nn_to_oeq(oprob, We), G)
     dX, dY, dW = otp.backward(oprob, X, Y, We, G)
     assert rel_err(out["Xg"], dX) < TOL[dtype] and rel_err(out["Yg"], dY) < TOL[dtype]
@@ -65,6 +68,7 @@ def test_on_the_gpu(cuda, case, dtype, monkeypatch):
         dX, dY, dW = otp.backward(oprob, X, Y, We, G)
         for off in (0, 1, 2):
             v = torch.cat([w.new_zeros(off), w.reshape(-1)])[off:].view(w.shape)
+            assert rel_err(tp.forward(x, y, v).cpu().numpy(), otp.forward(oprob, X, Y, We)) < TOL[dtype]
             got = [t.cpu().numpy() for t in tp.backward_helper(x, y, v, dz)]
             for a, b in zip((*got[:2], ow.oeq_to_e3nn(oprob, got[2])), (dX, dY, dW)):
                 assert rel_err(a, b) < TOL[dtype]
