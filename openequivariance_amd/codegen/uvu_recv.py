@@ -101,15 +101,24 @@ class UVURecvGenerator(UVUDetGenerator):
             if recv_split is None else recv_split
         self.recv_groups = self._disjoint_groups(limit)
         self.HR = len(self.recv_groups)
+        held_by = [sum(self.out[i].D for i in g_) for g_ in self.recv_groups]
         # receiver order is worth choosing in fp64: every launch of pass 1 holds few enough dZ words to leave room for an
         # edge's operands and results
         self.register_loads_fit = (self.T == "double" and not self.staged_edges and
-                                   max(sum(self.out[i].D for i in g_) for g_ in self.recv_groups)
-                                   <= self.RECV_SPLIT_WORDS_REGISTER_LOADS["double"])
+                                   max(held_by) <= self.RECV_SPLIT_WORDS_REGISTER_LOADS["double"])
         # Such launches go through the stage as well, an edge's operands as 4-byte words: 334 registers and one wavefront per
         # SIMD become 210 and two (17 paths at 128 channels, 10 000 nodes / 300 000 edges: forward + backward 6.56 -> 5.73 ms)
         self.staged_f64 = (self.register_loads_fit and self.P >= 2 * self.D2 and (True if staged is None else bool(staged)))
         self.uses_stage = self.staged_edges or self.staged_f64
+        # In fp64 the groups go in one launch, as neighbours in the order of dispatch: an edge's Y, its node indices and the X
+        # and dZ rows of its nodes are still in the cache of the XCD when the next group asks for them, and one ramp and one
+        # last wave are left instead of one per group.  Backward, a launch per group -> one (us): 64 channels, 3 groups,
+        # 10 000 nodes / 300 000 edges 4065 -> 3998, 4000 / 100 000 691 -> 664; 32 channels of either parity, 5 groups,
+        # 5000 / 100 000 650 -> 601, 400 / 8000 102 -> 63.  All groups then hold the registers of the longest, so the
+        # shortest has to hold half of the longest's words: two fp32 groups of 80 and 22 words of dZ take 281 apart and 314
+        # together (the short one runs two wavefronts per SIMD instead of five).  fp32 stays at a launch per group: most of
+        # its problems have one group (three of 110, 102 and 100 words: 753 apart, 700 together).
+        self.fused = self.staged_f64 and self.HR > 1 and 2 * min(held_by) >= max(held_by)
         self.regroup_pairs = bool(self.REGROUP_STAGED and self.uses_stage)
         if self.uses_stage:
             self.waves_hint = 0
@@ -129,7 +138,8 @@ class UVURecvGenerator(UVUDetGenerator):
     # ------------------------------------------------------------------ plan
     def backward_steps(self):
         steps = [dict(kernel=name, num_threads=WAVE, grid_kind=1, work_per_block=self.MIN_TILE_ITERS * self.R,
-                      num_blocks=self.MAX_TILES, grid_y=self.NCH) for name, _ in self.backward_kernels()] \
+                      num_blocks=self.MAX_TILES, grid_y=self.NCH * (self.HR if self.fused else 1))
+                 for name, _ in self.backward_kernels()] \
             + [dict(kernel="backward_dx", num_threads=WAVE * self.team, grid_kind=3, work_per_block=1, num_blocks=self.LONG, grid_y=self.NCH)]
         if self.dy_slots > 1:
             steps.append(dict(kernel="backward_dy_reduce", num_threads=256, grid_kind=1,
@@ -183,17 +193,44 @@ class UVURecvGenerator(UVUDetGenerator):
         return self.waves_hint if self.HR == 1 else 0
 
     def backward_kernels(self):
-        return [("backward" if h == 0 else f"backward_g{h}", h) for h in range(self.HR)]
+        return [("backward" if h == 0 else f"backward_g{h}", h) for h in range(1 if self.fused else self.HR)]
 
     def backward_kernel_sources(self):
         def attr(h):
             with self._group(h, self.recv_groups):
                 w = self.group_waves_hint()
             return f" __attribute__((amdgpu_waves_per_eu({w}, {w})))" if w else ""
-        return [dict(name=name, threads=WAVE, attr=attr(h), body=self._edges_body(h)) for name, h in self.backward_kernels()] \
+        return [dict(name=name, threads=WAVE, attr=attr(h), body=self._fused_body() if self.fused else self._edges_body(h))
+                for name, h in self.backward_kernels()] \
             + [self.with_team(dict(name="backward_dx", threads=WAVE * self.team, attr="", body=self._dx_body()))]
 
     # ---------------------------------------------------------------- pass 1
+    def _fused_body(self) -> str:
+        """All groups in one kernel: a workgroup takes the branch of its item's group; the branches share one stage."""
+        E = Emitter()
+        self._emit_item(E)
+        E(f"const int group_ = (int)(item % {self.HR});")
+        words = []
+        for h in range(self.HR):
+            with self._group(h, self.recv_groups):
+                words.append(self._forward_slabs()[1])
+        self._emit_stage(E, max(words))
+        for h in range(self.HR):
+            E(f"if (group_ == {h}) {{")
+            E.lines.append(self._edges_body(h))
+            E("}")
+        return E.text()
+
+    def _emit_stage(self, E: Emitter, words: int) -> None:
+        E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{words}];")
+
+    def _emit_item(self, E: Emitter) -> None:
+        E("// (tile, chunk) of this workgroup: ids are dealt to the 8 XCDs round robin, each XCD gets a contiguous run of items")
+        E(f"const u64 tiles = gridDim.x, items = tiles * {self.NCH * (self.HR if self.fused else 1)};")
+        E("const u64 bid = blockIdx.x + (u64)blockIdx.y * gridDim.x;")
+        E("const u64 xcd = bid & 7, turn = bid >> 3;")
+        E("const u64 item = xcd * (items >> 3) + min(xcd, items & 7) + turn;")
+
     def _edges_body(self, h: int = 0) -> str:
         E = Emitter()
         R, P, NCH = self.R, self.P, self.NCH
@@ -326,13 +363,13 @@ class UVURecvGenerator(UVUDetGenerator):
         """(tile, chunk) of the workgroup, the tile's range of list positions, and - over a position list built on
         the fly - the zero rows of the edges that are in no group."""
         R, P, NCH = self.R, self.P, self.NCH
-        E("// (tile, chunk) of this workgroup: ids are dealt to the 8 XCDs round robin, each XCD gets a contiguous run of items")
-        E(f"const u64 tiles = gridDim.x, items = tiles * {NCH};")
-        E("const u64 bid = blockIdx.x + (u64)blockIdx.y * gridDim.x;")
-        E("const u64 xcd = bid & 7, turn = bid >> 3;")
-        E("const u64 item = xcd * (items >> 3) + min(xcd, items & 7) + turn;")
-        E(f"const int c = (int)(item % {NCH}); (void)c;")
-        E(f"const u64 tile = item / {NCH};")
+        if self.fused:
+            E(f"const int c = (int)(item / {self.HR} % {NCH}); (void)c;")
+            E(f"const u64 tile = item / {NCH * self.HR};")
+        else:
+            self._emit_item(E)
+            E(f"const int c = (int)(item % {NCH}); (void)c;")
+            E(f"const u64 tile = item / {NCH};")
         E(f"const int u = c * {P} + ul;")
         E(f"const u64 per = ((nnz + tiles - 1) / tiles + {R - 1}) / {R} * {R};       // edges per tile")
         if self.backward_perm:
@@ -393,7 +430,8 @@ class UVURecvGenerator(UVUDetGenerator):
         E("i64 cur_rcv = -1, rawR = -1, rcv0 = -1;")
         slabs, words = self._forward_slabs()
         y_off = words - 64
-        E(f"__shared__ __attribute__((aligned(16))) {self.stage_type()} stage[{words}];")
+        if not self.fused:
+            self._emit_stage(E, words)
         res = [f"pw_{p.t}_{v}" for p in self.paths for v in range(p.mv)] + [f"pdy{f}" for f in self.used_y] \
             + [f"pdx{i}_{m}" for i in self.used_in1 for m in range(self.in1[i].D)]
         E("T " + ", ".join(f"{n} = (T)0" for n in res) + "; u64 pe = 0; bool pv = false, pev = false;")
