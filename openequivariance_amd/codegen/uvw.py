@@ -373,6 +373,8 @@ class UVWGenerator:
     def prep_blocks(self) -> int:
         return _ceil(self.WA_END, 256)
 
+    separate_prep = True         # (False: another backward kernel packs the weights)
+
     # =============================================================== forward
     forward_threads = 64
     has_forward = True           # (False: backward kernels alone)

@@ -9,7 +9,7 @@ the time of a launch.  Here the same work is cut finer:
 * backward dX/dY: the in1 blocks of a tile are dealt to two or four groups of four wavefronts, which share the dZ tile;
 * backward dW: a workgroup holds ONE path (or a range of its w tiles) and walks a share of the batch given by the path's
   cost; its 16 wavefronts are u-subtiles x phases of the batch, combined through LDS, so that the launch leaves 15 to 80
-  partial rows of a path instead of 256 of all paths.
+  partial rows of a path instead of 256 of all paths.  It comes first and packs the weights that dX reads.
 
 Bound: latency of the operand loads, four wavefronts per SIMD hide what one did not.  50x0e+50x1o+50x1e+50x2o+50x2e with
 one scalar, fp64, 4097 rows (kernel times, us): dX/dY 41 -> 30, dW 35 -> 19, reduction 16.7 -> 4.6; fp32 backward of that
@@ -156,6 +156,23 @@ class UVWSmallGenerator(UVWGenerator):
         return 64 * self.DW_WAVES
 
     # ============================================================ backward: dW
+    separate_prep = False
+
+    def _emit_packing(self, E: Emitter) -> None:
+        """The backward's packed weights, which dW does not read: 64 of every 16 384 elements a workgroup, one wavefront after
+        the other.  Whole backward with a launch for them / here, us: 50 channels of both parities, fp64, 500 rows 26.9 / 24.9,
+        4097 54.1 / 52.4; 64 channels l <= 2 of either operand, fp32, 500 rows 28.7 / 26.2, 4097 59.3 / 57.2; 20 -> 40 channels, 500
+        rows 17.2 / 15.0."""
+        waves, blocks = self.DW_WAVES, sum(self.chunks)
+        lo, hi = min(p.wa for p in self.paths), self.WA_END
+        E("T* __restrict__ wsT = (T*)ws;")
+        E(f"for (int q = {lo} + (wv * {blocks} + (int)blockIdx.x) * 64 + lane; q < {hi}; q += {64 * waves * blocks}) {{")
+        E.level += 1
+        for p in self.paths:
+            self._pack_backward_copy(E, p)
+        E.level -= 1
+        E("}")
+
     def _live_chunks(self, k: int) -> str:
         """Workgroups of unit k that have rows to walk (the rest leave no partial row)."""
         per = 4 * (self.DW_WAVES // self.units[k][3])
@@ -166,6 +183,7 @@ class UVWSmallGenerator(UVWGenerator):
         PH = lambda uw: self.DW_WAVES // uw
         E("const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;")
         E(f"__shared__ T comb[{max(1, self._phase_elems())}];")
+        self._emit_packing(E)
         first = 0
         for k, (p, lo, hi, uw) in enumerate(self.units):
             Q, ph, D = _ceil(p.NTU, uw), PH(uw), p.o.D
@@ -261,6 +279,7 @@ class UVWSmallGenerator(UVWGenerator):
 
     def plan(self):
         fwd, bwd, ws = super().plan()
-        bwd[2]["num_blocks"] = sum(self.chunks)
-        bwd[3]["num_blocks"] = _ceil(self.WN, 64)
-        return fwd, bwd, ws
+        _, dx, dw, reduce = bwd
+        dw["num_blocks"] = sum(self.chunks)
+        reduce["num_blocks"] = _ceil(self.WN, 64)
+        return fwd, [dw, dx, reduce], ws               # (dW packs the weights that dX reads)
