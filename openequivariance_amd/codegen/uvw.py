@@ -97,6 +97,18 @@ class UVWGenerator:
     # w tiles.  (48 instead of 80, for a third wavefront per SIMD, measured slower on 64x0e+64x1o+64x2e: fp32
     # 0.329 -> 0.376 ms, fp64 0.566 -> 0.694 ms - the CG part of a tile is then computed once per range.)
     FWD_ACC_LIMIT = 80
+    # fp64, outputs up to l = 1: a block of five or six w tiles (60 and 72 accumulators, 212 - 370 registers) is cut in two.  Whole /
+    # cut, us:
+    #     channels, second operand      500 rows     4097        20 000       50 000      100 000
+    #     70, 1x0e                     14.0 / 10.3  17.4 / 13.9   47 / 41      93 / 88    238 / 233
+    #     80, 1x0e                     13.6 / 10.0  17.8 / 14.3   48 / 40      94 / 90    226 / 231
+    #     96, 1x0e                     22.2 / 13.5  26.4 / 19.3   72 / 52     154 / 146   299 / 291
+    #     66, l <= 2                   30.8 / 21.4  34.8 / 25.1   97 / 65     192 / 143   366 / 310
+    #     80, l <= 1                   22.1 / 15.3  26.3 / 20.2   71 / 56     140 / 124   272 / 285
+    #     90, l <= 1                   37.3 / 23.7  41.7 / 29.4  115 / 78     233 / 189   460 / 396
+    # Beside outputs of l = 2, whose items are the longer ones, it goes either way (80 channels l <= 2 27 / 29 at 4097 rows, 253 / 263
+    # at 50 000; 70 with l <= 2 55 / 63, 542 / 503), and so does cutting those (64 channels 20 / 18, 142 / 182).
+    FWD_ACC_LIMIT_L1 = {4: 80, 8: 56}
     FWD_PIPELINE = {4: (4, 2), 8: (1, 3)}
     # Steps of an fp64 path (one a batch, unrolled three times) that are a multiple of three cost more than another one: per
     # step and 100 000 rows 13 us with 20 or 19 of them, 18 us with 18.  66 channels l <= 1, 18 / 20 / 19 steps 316 / 267 /
@@ -165,11 +177,11 @@ class UVWGenerator:
         # whose accumulator tile (D * tiles * 4 registers) exceeds FWD_ACC_LIMIT is cut into w ranges, each
         # a work item of its own: fewer accumulators per wavefront buy a third wavefront per SIMD, which
         # hides one wavefront's vector-ALU phases behind another's matrix-core phases
-        limit = self.FWD_ACC_LIMIT
+        limits = {3: min(self.FWD_ACC_LIMIT, self.FWD_ACC_LIMIT_L1[self.itemsize])} if max(self.out[o].D for o in self.used_out) == 3 else {}
         self.fwd_order = []
         for o in sorted([o for o in self.out if o.dim > 0], key=lambda o: -cost(o)):
             nt_all = _ceil(o.mul, 16)
-            parts = 1
+            parts, limit = 1, limits.get(o.D, self.FWD_ACC_LIMIT)
             if o.idx in self.used_out:
                 while 4 * o.D * _ceil(nt_all, parts) > limit and parts < nt_all:
                     parts += 1
