@@ -368,7 +368,7 @@ class UVUDetGenerator(UVUDirectGenerator):
             E("if (!piece) {")
             E.level += 1
         if order:
-            E(f"const i64 nd_ = bx_ < node_count ? {order}[bx_] : -1;")
+            E(f"const i64 nd_ = bx_ >= node_count ? -1 : nnz > 0 ? {order}[bx_] : (i64)bx_;      // (no edges: nothing has written an order)")
             E("if (nd_ >= 0 && (u64)nd_ < node_count) node = (u64)nd_;")
         else:
             E("if (bx_ < node_count) node = bx_;")

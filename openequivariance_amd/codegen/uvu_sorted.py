@@ -126,15 +126,22 @@ class UVUSortedGenerator:
             return ((main + 255) & ~255) + b.piece_bytes(nnz, nodes)
         return fwd, bwd, ws
 
+    # the launch order of the backward's nodes is made in the launch that writes the position list, by a workgroup of its own,
+    # instead of in one that follows it (in the plans of plan_few)
+    order_beside_fill = False
+
     def add_few_nodes(self):
         """See UVUDetGenerator.add_few_nodes (the per-edge backward has no nodes to share)."""
         self.fwd.add_few_nodes(("forward",))
         if self.grouped_backward:
             self.bwd.add_few_nodes(("backward",))
+            self.order_beside_fill = self.bwd.ordered_backward and self.bwd.ORDER_THREADS == self.SCAN_THREADS
         return self
 
     def plan_few(self):
         fwd, bwd, ws = self.plan()
+        if self.order_beside_fill:
+            bwd = [dict(s, grid_y=2) if s["kernel"] == "group_fill_backward" else s for s in bwd if s["kernel"] != "order_backward"]
         return self.fwd.few_steps("forward", fwd), self.bwd.few_steps("backward", bwd) if self.grouped_backward else bwd, ws
 
     def workspace_terms(self):
