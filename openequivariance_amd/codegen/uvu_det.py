@@ -540,6 +540,7 @@ class UVUDetGenerator(UVUDirectGenerator):
     TEAMS = ((4, 2048), (2, 4096))         # wavefronts, and row groups (nodes x chunks x lane groups) up to which they walk a node
     TEAM_LDS, TEAM_CUS = 160 * 1024, 256   # LDS of a compute unit, compute units
     TEAM_STEP = 128               # a team's least number of nodes is kept in these (OEQ_STEP_FEW_NODES)
+    both_prepared = False         # prep_backward fills the receivers' pointers as well, in a second row of workgroups
     team, team_need = 1, (0, 0, 0)         # wavefronts that walk one node's edges here; what a kernel of theirs needs (emit_stage)
     few_sources = {"forward": [], "backward": []}            # kernels for few nodes beside the others (add_few_nodes)
 
@@ -750,6 +751,8 @@ class UVUDetGenerator(UVUDirectGenerator):
                 s.update(work_per_block=1, grid_kind=3, num_blocks=self.LONG)
         fwd = [t for s in fwd for t in (self.forward_steps(s) if s["kernel"] == "forward" else [s])]
         bwd = [s for s in bwd if s["kernel"] == "prep_backward"] + self.backward_steps()
+        if self.both_prepared:
+            fwd, bwd = [s for s in fwd if s["kernel"] != "prep_forward"], [dict(bwd[0], grid_y=2)] + bwd[1:]
 
         def ws(nnz=0, nodes=0):
             return self.main_bytes(nnz, nodes) + self.piece_bytes(nnz, nodes)

@@ -118,6 +118,9 @@ class UVUSortedGenerator:
             return fwd, bwd, ws
         b = self.bwd
         bwd = (grouping("_recv") if self.recv_backward else []) + grouping("_backward") + b.backward_steps()
+        if self.both_prepared:
+            fwd = fwd[len(grouping("")):]
+            bwd = [dict(s, grid_y=2) if s["kernel"].startswith("group_") else s for s in bwd]
 
         def ws(nnz=0, nodes=0):
             if self.recv_backward:
@@ -129,6 +132,7 @@ class UVUSortedGenerator:
     # the launch order of the backward's nodes is made in the launch that writes the position list, by a workgroup of its own,
     # instead of in one that follows it (in the plans of plan_few)
     order_beside_fill = False
+    both_prepared = False            # the backward's grouping kernels make the forward's grouping as well, in a row of workgroups of its own
 
     def add_few_nodes(self):
         """See UVUDetGenerator.add_few_nodes (the per-edge backward has no nodes to share)."""
@@ -141,7 +145,8 @@ class UVUSortedGenerator:
     def plan_few(self):
         fwd, bwd, ws = self.plan()
         if self.order_beside_fill:
-            bwd = [dict(s, grid_y=2) if s["kernel"] == "group_fill_backward" else s for s in bwd if s["kernel"] != "order_backward"]
+            bwd = [dict(s, grid_y=s.get("grid_y", 1) + 1) if s["kernel"] == "group_fill_backward" else s for s in bwd
+                   if s["kernel"] != "order_backward"]
         return self.fwd.few_steps("forward", fwd), self.bwd.few_steps("backward", bwd) if self.grouped_backward else bwd, ws
 
     def workspace_terms(self):
