@@ -130,7 +130,8 @@ class UVUSortedGenerator:
         return fwd, bwd, ws
 
     # the launch order of the backward's nodes is made in the launch that writes the position list, by a workgroup of its own,
-    # instead of in one that follows it (in the plans of plan_few)
+    # instead of in one that follows it (in the plans of plan_few): 5000 nodes, 150 000 edges, 6.5 us of a step of 265 saved; the
+    # list takes 9 either way
     order_beside_fill = False
     both_prepared = False            # the backward's grouping kernels make the forward's grouping as well, in a row of workgroups of its own
 
