@@ -138,6 +138,8 @@ int  oeq_tp_double_backward(oeq_tp* tp, uint64_t num_products, const void* L1_in
  *   (const void* L1, void* L1g, const void* L2, void* L2g, const void* W, void* Wg,
  *    const void* L3g, const int64_t* rows, const int64_t* cols, uint64_t nnz,
  *    uint64_t node_count, void* workspace, const int64_t* transpose_perm).
+ * The launches of one call are issued without those of another call on the same workspace between them, here and in the batch
+ * product: threads may share a workspace on one stream.
  * A plan with per-edge preparation steps (the grouping of an unsorted edge list) takes fewer than 2^32 edges;
  * more are an error, reported before anything is launched.
  * The reference passes rows/cols/nnz/node_count as a by-value struct

@@ -124,6 +124,15 @@ int launch(const Step& s, uint64_t rows, uint64_t nodes, void** args, void* stre
     return 0;
 }
 
+// Held over the launches of a call on this workspace: what one step leaves there the next one reads, so two threads on one
+// stream must not mix theirs.  The workspace is what the kernel sets of an operator share, hence one lock for an address
+// (64 of them for all), whichever handle and entry point a call comes through.
+std::unique_lock<std::mutex> together(const void* workspace) {
+    static std::mutex locks[64];
+    if (!workspace) return {};
+    return std::unique_lock<std::mutex>(locks[(uint64_t)(uintptr_t)workspace * 0x9E3779B97F4A7C15ull >> 58]);
+}
+
 // Rejects a NULL workspace / transpose permutation that a step of the plan would dereference.
 int check_pointers(const std::vector<Step>& steps, const void* workspace, const void* tperm, const char* what) {
     for (auto& s : steps) {
@@ -282,6 +291,7 @@ int oeq_tp_forward(oeq_tp* tp, uint64_t n, const void* L1, const void* L2, void*
     if (!tp) return fail("null handle");
     if (tp->fwd.empty()) return fail("this operator was built without a forward plan");
     if (n > 0 && check_pointers(tp->fwd, workspace, (const void*)1, "forward")) return 1;
+    const auto lock = together(workspace);
     void* args[] = {&n, &L1, &L2, &L3, &W, &workspace};
     for (auto& s : tp->fwd)
         if (launch(s, n, 0, args, stream)) return 1;
@@ -293,6 +303,7 @@ int oeq_tp_backward(oeq_tp* tp, uint64_t n, const void* L1, void* L1g, const voi
     if (!tp) return fail("null handle");
     if (tp->bwd.empty()) return fail("this operator was built without a backward plan");
     if (n > 0 && check_pointers(tp->bwd, workspace, (const void*)1, "backward")) return 1;
+    const auto lock = together(workspace);
     void* args[] = {&n, &L1, &L1g, &L2, &L2g, &W, &Wg, &L3g, &workspace};
     for (auto& s : tp->bwd)
         if (launch(s, n, 0, args, stream)) return 1;
@@ -358,6 +369,7 @@ static int conv_forward(oeq_conv* c, const void* L1, const void* L2, const void*
     if (check_edges(c->fwd, nnz, "forward")) return 1;
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("forward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
+    const auto lock = together(workspace);
     for (auto& s : c->fwd) {
         if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream, pieces)) return 1;
@@ -377,6 +389,7 @@ static int conv_backward(oeq_conv* c, const void* L1, void* L1g, const void* L2,
     if (check_edges(c->bwd, nnz, "backward")) return 1;
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L1g, &L2, &L2g, &W, &Wg, &L3g, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
+    const auto lock = together(workspace);
     for (auto& s : c->bwd) {
         if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream)) return 1;
@@ -420,6 +433,7 @@ int oeq_conv_double_backward_ex(oeq_conv* c, const void* L1, const void* L2, con
     if (check_edges(c->bwd, nnz, "double backward")) return 1;
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("double backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3g, &L1c, &L2c, &Wc, &L1o, &L2o, &Wo, &L3o, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
+    const auto lock = together(workspace);
     for (auto& s : c->bwd) {
         if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream)) return 1;
