@@ -205,6 +205,32 @@ int  oeq_conv_double_backward_ex(oeq_conv* conv, const void* L1_in, const void* 
                                  uint64_t node_count, void* workspace, const void* transpose_perm, void* stream,
                                  uint32_t call_flags);
 
+/* The three calls with a record, kept by the caller beside the workspace and zero-initialised with it, of which completed calls
+ * left the counters in it zero: OEQ_CALL_COUNTERS_ZERO is then worked out and the record brought up to date while the launches are
+ * issued, under the lock that keeps those of a call together, so that threads may share workspace and record.  `kind` is the
+ * caller's number for the kernel set (kernel sets group differently); 0: nothing is known of the counters afterwards.  A record
+ * whose `captured` is set is not used: replays of a captured graph write the workspace unseen.  Whoever puts another buffer in
+ * the workspace's place zeroes the record.  The double backward uses `forward`; of kind 0 it voids both.  `counters` may be NULL. */
+typedef struct {
+    uint64_t forward[3], backward[3];   /* nnz, node_count and kind of the last completed call; kind 0: none */
+    uint64_t captured;
+} oeq_conv_counters;
+int  oeq_conv_forward_on(oeq_conv* conv, const void* L1_in, const void* L2_in, const void* weights,
+                         void* L3_out, const void* rows, const void* cols, uint64_t nnz,
+                         uint64_t node_count, void* workspace, const void* transpose_perm, void* stream,
+                         uint32_t call_flags, oeq_conv_counters* counters, uint64_t kind);
+int  oeq_conv_backward_on(oeq_conv* conv, const void* L1_in, void* L1_grad, const void* L2_in,
+                          void* L2_grad, const void* weights, void* weights_grad, const void* L3_grad,
+                          const void* rows, const void* cols, uint64_t nnz, uint64_t node_count,
+                          void* workspace, const void* transpose_perm, void* stream, uint32_t call_flags,
+                          oeq_conv_counters* counters, uint64_t kind);
+int  oeq_conv_double_backward_on(oeq_conv* conv, const void* L1_in, const void* L2_in, const void* weights,
+                                 const void* L3_grad, const void* L1_grad_cot, const void* L2_grad_cot,
+                                 const void* weights_grad_cot, void* L1_out, void* L2_out, void* weights_out,
+                                 void* L3_grad_out, const void* rows, const void* cols, uint64_t nnz,
+                                 uint64_t node_count, void* workspace, const void* transpose_perm, void* stream,
+                                 uint32_t call_flags, oeq_conv_counters* counters, uint64_t kind);
+
 /* Workspace bytes the forward steps use when every node is walked by one wavefront (no pieces):
  * fixed_bytes + bytes_per_node * node_count + bytes_per_edge * nnz.  The host sets it from the plan it
  * built the operator with; oeq_conv_forward_noalloc checks graphs against it.  (The reference sizes

@@ -15,7 +15,9 @@ assumption about the graph.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import threading
 import typing
 
 import numpy as np
@@ -146,25 +148,21 @@ class _StreamWorkspace:
     def __init__(self):
         self.buffer, self.size = None, 0
         self.retired = []            # outgrown buffers that a captured HIP graph may still name
-        # three numbers each of zero_fwd and zero_bwd, and captured: the operators' C++ kernels read and write them too
-        self.state = (ctypes.c_int64 * 8)()
+        # of which completed calls the counters in the buffer are known to be zero, and whether a HIP graph capture has used it:
+        # read and written by the C library, under the lock of a call's launches
+        self.counters = rt.ConvCounters()
         self.fwd_key = self.bwd_key = None
         self.refs = {}               # index tensors of the cached keys, kept alive so that their addresses stay theirs
 
     def _zero(self, at):
-        nnz, nodes, tag = self.state[at:at + 3]
-        return (nnz, nodes, self.TAGS[tag - 1]) if tag else None
-
-    def _set_zero(self, at, value):
-        self.state[at:at + 3] = [0, 0, 0] if value is None else [value[0], value[1], self.TAGS.index(value[2]) + 1]
+        nnz, nodes, kind = at
+        return (nnz, nodes, self.TAGS[kind - 1]) if kind else None
 
     # (nnz, node_count, kind of backward) of the last completed call of each direction, while nothing else has written the
-    # workspace since: the counters of the on-the-fly grouping are then known to be zero where a call
-    # with the same sizes keeps them, and the step that clears them is skipped
-    zero_fwd = property(lambda self: self._zero(0), lambda self, value: self._set_zero(0, value))
-    zero_bwd = property(lambda self: self._zero(3), lambda self, value: self._set_zero(3, value))
-    # a HIP graph capture has used this workspace
-    captured = property(lambda self: bool(self.state[6]), lambda self, value: self.state.__setitem__(6, int(value)))
+    # workspace since: a call with the same sizes skips the step that clears the counters of the on-the-fly grouping
+    zero_fwd = property(lambda self: self._zero(self.counters.forward))
+    zero_bwd = property(lambda self: self._zero(self.counters.backward))
+    captured = property(lambda self: bool(self.counters.captured), lambda self, value: setattr(self.counters, "captured", int(value)))
 
 
 class TensorProductConv:
@@ -207,6 +205,8 @@ class TensorProductConv:
         # the deterministic backward walks the caller's transpose permutation
         self.backward_needs_tperm = deterministic
         self.jit_kernel = self.generator.render()
+        # held from the look at a stream's workspace until the launches in it are issued: threads share it
+        self._lock = threading.RLock()
         self._native = None                       # the operator's part in the C++ kernels (torch_op=True)
         self._ws_fns = []
         self._ws_last = self._double_ws_last = (None, 0)          # (sizes, bytes) of the last workspace query
@@ -318,10 +318,11 @@ class TensorProductConv:
 
     @graph_cache.setter
     def graph_cache(self, value: bool) -> None:
-        self._graph_cache = bool(value)
-        for rec in self._workspaces.values():       # (the C++ kernels, which prepare every call, kept no keys meanwhile)
-            rec.fwd_key = rec.bwd_key = None
-        self._native_enable()
+        with self._lock:
+            self._graph_cache = bool(value)
+            for rec in self._workspaces.values():       # (the C++ kernels, which prepare every call, kept no keys meanwhile)
+                rec.fwd_key = rec.bwd_key = None
+            self._native_enable()
 
     @property
     def autotune(self) -> bool:
@@ -373,10 +374,12 @@ class TensorProductConv:
                 rec.retired.append(rec.buffer)
             rec.size = int(need * 1.25) + 256
             rec.buffer = torch.empty(rec.size, dtype=torch.uint8, device=f"cuda:{dev}")
-            rec.fwd_key = rec.bwd_key = rec.zero_fwd = rec.zero_bwd = None
+            rec.fwd_key = rec.bwd_key = None
             rec.refs.clear()
-            if self._native is not None and not own:
-                self._native.ops.native_lease(self._native.id, rec.buffer, *sid[:2], ctypes.addressof(rec.state))
+            if self._native is not None and not own:          # (voids the record of the counters where C++ calls cannot come between)
+                self._native.ops.native_lease(self._native.id, rec.buffer, *sid[:2], ctypes.addressof(rec.counters))
+            else:
+                rec.counters.forward[2] = rec.counters.backward[2] = 0
         return rec
 
     def workspace_ptr(self, nnz: int, node_count: int, stream: typing.Optional[int] = None) -> int:
@@ -385,7 +388,8 @@ class TensorProductConv:
         operator's own entry points is responsible for the ``prepared`` flag."""
         if self._ws_bytes(nnz, node_count) == 0:
             return 0
-        return self._workspace_record(nnz, node_count, stream).buffer.data_ptr()
+        with self._lock:
+            return self._workspace_record(nnz, node_count, stream).buffer.data_ptr()
 
     @staticmethod
     def _stream(device_index: typing.Optional[int] = None) -> int:
@@ -457,18 +461,19 @@ class TensorProductConv:
         preparation of exactly this graph (left by an earlier forward call): the preparation kernels are
         then skipped.  ``counters_zero=True`` promises that the counters the operator keeps in the workspace
         are zero (a zero-filled workspace, or one last written by a completed call of this operator with the
-        same sizes): the step that clears them is skipped."""
+        same sizes): the step that clears them is skipped.  A tuple: runtime.ConvImpl."""
         nnz, node_count = int(nnz), int(node_count)
         if nnz > 0 and not (rows and cols):
             raise ValueError("rows / cols must be device pointers")
         impl = self._pick(L1_in, L2_in, weights, L3_out)
-        if not workspace:
-            rec = self._workspace_record(nnz, node_count, stream)
-            rec.fwd_key = rec.zero_fwd = rec.zero_bwd = None    # the caller's graph is unknown to the cache
-            workspace = rec.buffer.data_ptr() if self._ws_bytes(nnz, node_count) else 0
-        impl.exec_conv_rawptrs(L1_in, L2_in, weights, L3_out, rows, cols, nnz, node_count,
-                               workspace, transpose_perm, self._stream() if stream is None else stream, prepared,
-                               counters_zero)
+        with self._lock if not workspace else contextlib.nullcontext():
+            if not workspace:
+                rec = self._workspace_record(nnz, node_count, stream)
+                rec.fwd_key = None                              # the caller's graph is unknown to the cache
+                workspace, counters_zero = rec.buffer.data_ptr() if self._ws_bytes(nnz, node_count) else 0, (rec.counters, 0, counters_zero)
+            impl.exec_conv_rawptrs(L1_in, L2_in, weights, L3_out, rows, cols, nnz, node_count,
+                                   workspace, transpose_perm, self._stream() if stream is None else stream, prepared,
+                                   counters_zero)
 
     def backward_rawptrs(self, L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad, rows, cols, nnz,
                          node_count, workspace=0, transpose_perm=0, stream=None, prepared=False, impl=None,
@@ -483,13 +488,14 @@ class TensorProductConv:
             raise ValueError("the deterministic backward needs transpose_perm (a device pointer), got 0")
         if impl is None:
             impl = self._pick(L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad)
-        if not workspace:
-            rec = self._workspace_record(nnz, node_count, stream)
-            rec.bwd_key = rec.zero_fwd = rec.zero_bwd = None
-            workspace = rec.buffer.data_ptr() if self._ws_bytes(nnz, node_count) else 0
-        impl.backward_rawptrs(L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad, rows, cols,
-                              nnz, node_count, workspace, transpose_perm,
-                              self._stream() if stream is None else stream, prepared, counters_zero)
+        with self._lock if not workspace else contextlib.nullcontext():
+            if not workspace:
+                rec = self._workspace_record(nnz, node_count, stream)
+                rec.bwd_key = None
+                workspace, counters_zero = rec.buffer.data_ptr() if self._ws_bytes(nnz, node_count) else 0, (rec.counters, 0, counters_zero)
+            impl.backward_rawptrs(L1_in, L1_grad, L2_in, L2_grad, weights, weights_grad, L3_grad, rows, cols,
+                                  nnz, node_count, workspace, transpose_perm,
+                                  self._stream() if stream is None else stream, prepared, counters_zero)
 
     def double_backward_rawptrs(self, L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot, L1_out, L2_out,
                                 weights_out, L3_grad_out, rows, cols, nnz, node_count, transpose_perm=0, stream=None, workspace=0,
@@ -504,15 +510,16 @@ class TensorProductConv:
         if any(int(p) % 16 for p in (L1_out, L3_grad_out)):
             raise ValueError("the double backward writes 16-byte vectors: its node outputs must be 16-byte aligned")
         impl = self._double_impl()
-        if not workspace:
-            rec = self._workspace_record(nnz, node_count, stream, need=self._double_ws_bytes(nnz, node_count))
-            if torch.cuda.is_current_stream_capturing():
-                rec.captured = True
-            rec.fwd_key = rec.bwd_key = rec.zero_fwd = rec.zero_bwd = None
-            workspace, prepared, counters_zero = rec.buffer.data_ptr(), False, False
-        impl.double_backward(L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot, L1_out, L2_out,
-                             weights_out, L3_grad_out, rows, cols, nnz, node_count, workspace, transpose_perm,
-                             self._stream() if stream is None else stream, prepared, counters_zero)
+        with self._lock if not workspace else contextlib.nullcontext():
+            if not workspace:
+                rec = self._workspace_record(nnz, node_count, stream, need=self._double_ws_bytes(nnz, node_count))
+                if torch.cuda.is_current_stream_capturing():
+                    rec.captured = True
+                rec.fwd_key = rec.bwd_key = None
+                workspace, prepared, counters_zero = rec.buffer.data_ptr(), False, (rec.counters, 0, False)
+            impl.double_backward(L1_in, L2_in, weights, L3_grad, L1_grad_cot, L2_grad_cot, weights_grad_cot, L1_out, L2_out,
+                                 weights_out, L3_grad_out, rows, cols, nnz, node_count, workspace, transpose_perm,
+                                 self._stream() if stream is None else stream, prepared, counters_zero)
 
     def _time_backward_variants(self, run, names=("atomic", "grouped"), repeats: int = 3) -> str:
         """Fastest of the backward variants on the caller's own tensors: one untimed call each (compilation,
@@ -540,32 +547,27 @@ class TensorProductConv:
         tensors are kept referenced while their key is cached, so the addresses cannot be handed to other
         tensors meanwhile.  Under HIP graph capture, and on a workspace that a capture has used, the
         preparation always runs: a replay may rewrite the workspace behind the cache's back.  ``double``: a call of the
-        double backward, in a scratch of its own so that the three directions keep their preparations."""
-        if double:
-            rec = self._workspace_record(E, N, stream, need=self._double_ws_bytes(E, N), own="double")
-        elif self._ws_bytes(E, N) == 0:
+        double backward, in a scratch of its own so that the three directions keep their preparations.  (Every call leaves the
+        grouping counters it used zeroed; the kernel sets of the backward variants differ in whether they group at all, hence
+        ``tag``, their kind.)"""
+        if not double and self._ws_bytes(E, N) == 0:
             launch(0, False, False)
             return
-        else:
-            rec = self._workspace_record(E, N, stream)
-        if torch.cuda.is_current_stream_capturing():
-            rec.captured = True
-        key = None
-        if self.graph_cache and not rec.captured:
-            key = (tag, E, N) + tuple((t.data_ptr(), t._version) for t in (rows, cols, tperm) if t is not None)
-        attr, zattr, other = which + "_key", "zero_" + which, "zero_" + ("bwd" if which == "fwd" else "fwd")
-        prepared = key is not None and getattr(rec, attr) == key
-        # every call leaves the grouping counters it used zeroed; a call with other sizes keeps them elsewhere
-        # (the kernel sets of the backward variants differ in whether they group at all, hence the tag)
-        counters_zero = not rec.captured and getattr(rec, zattr) == (E, N, tag)
-        if (getattr(rec, other) or (None,))[:2] != (E, N):
-            setattr(rec, other, None)
-        setattr(rec, attr, None)
-        setattr(rec, zattr, None)
-        launch(rec.buffer.data_ptr(), prepared, counters_zero)
-        setattr(rec, attr, key)
-        setattr(rec, zattr, None if rec.captured else (E, N, tag))
-        rec.refs[which] = (rows, cols, tperm) if key is not None else None
+        with self._lock:
+            if double:
+                rec = self._workspace_record(E, N, stream, need=self._double_ws_bytes(E, N), own="double")
+            else:
+                rec = self._workspace_record(E, N, stream)
+            if torch.cuda.is_current_stream_capturing():
+                rec.captured = True
+            key, attr = None, which + "_key"
+            if self.graph_cache and not rec.captured:
+                key = (tag, E, N) + tuple((t.data_ptr(), t._version) for t in (rows, cols, tperm) if t is not None)
+            prepared = key is not None and getattr(rec, attr) == key
+            setattr(rec, attr, None)
+            launch(rec.buffer.data_ptr(), prepared, (rec.counters, rec.TAGS.index(tag) + 1, False))
+            setattr(rec, attr, key)
+            rec.refs[which] = (rows, cols, tperm) if key is not None else None
 
     # ------------------------------------------------------------------ torch ops
     def _setup_torch_module(self) -> None:

@@ -357,9 +357,28 @@ static bool skipped(const oeq_step& d, uint32_t call_flags, uint64_t nnz, uint64
     return false;
 }
 
+// A caller's record of the counters over one call (made under the workspace's lock).
+struct Record {
+    oeq_conv_counters* c;
+    uint64_t* mine;
+    const uint64_t nnz, nodes, kind;
+    Record(oeq_conv_counters* c_, uint64_t* mine_, uint64_t* other, uint64_t nnz_, uint64_t nodes_, uint64_t kind_, uint32_t& call_flags)
+        : c(c_ && !c_->captured ? c_ : nullptr), mine(mine_), nnz(nnz_), nodes(nodes_), kind(kind_) {
+        if (c && kind && mine[2] == kind && mine[0] == nnz && mine[1] == nodes) call_flags |= OEQ_CALL_COUNTERS_ZERO;
+        // (a call of other sizes keeps its counters elsewhere, over those of the other direction)
+        if (c_ && (!c || !kind || other[0] != nnz || other[1] != nodes)) other[2] = 0;
+        if (c_) mine[2] = 0;
+    }
+    int completed() {
+        if (c && kind) { mine[0] = nnz; mine[1] = nodes; mine[2] = kind; }
+        return 0;
+    }
+};
+
 static int conv_forward(oeq_conv* c, const void* L1, const void* L2, const void* W, void* L3,
                         const void* rows, const void* cols, uint64_t nnz, uint64_t node_count,
-                        void* workspace, const void* tperm, void* stream, uint32_t call_flags, bool pieces = true) {
+                        void* workspace, const void* tperm, void* stream, uint32_t call_flags,
+                        oeq_conv_counters* counters = nullptr, uint64_t kind = 0, bool pieces = true) {
     if (!c) return fail("null handle");
     if (c->fwd.empty()) return fail("this operator was built without a forward plan");
     if (nnz > 0 && node_count == 0) return fail("convolution called with %llu edges but no nodes", (unsigned long long)nnz);
@@ -370,16 +389,18 @@ static int conv_forward(oeq_conv* c, const void* L1, const void* L2, const void*
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("forward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     const auto lock = together(workspace);
+    Record record(counters, counters ? counters->forward : nullptr, counters ? counters->backward : nullptr, nnz, node_count, kind, call_flags);
     for (auto& s : c->fwd) {
         if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream, pieces)) return 1;
     }
-    return 0;
+    return record.completed();
 }
 
 static int conv_backward(oeq_conv* c, const void* L1, void* L1g, const void* L2, void* L2g, const void* W,
                          void* Wg, const void* L3g, const void* rows, const void* cols, uint64_t nnz,
-                         uint64_t node_count, void* workspace, const void* tperm, void* stream, uint32_t call_flags) {
+                         uint64_t node_count, void* workspace, const void* tperm, void* stream, uint32_t call_flags,
+                         oeq_conv_counters* counters = nullptr, uint64_t kind = 0) {
     if (!c) return fail("null handle");
     if (c->bwd.empty()) return fail("this operator was built without a backward plan");
     if (nnz > 0 && node_count == 0) return fail("convolution called with %llu edges but no nodes", (unsigned long long)nnz);
@@ -390,11 +411,12 @@ static int conv_backward(oeq_conv* c, const void* L1, void* L1g, const void* L2,
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L1g, &L2, &L2g, &W, &Wg, &L3g, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     const auto lock = together(workspace);
+    Record record(counters, counters ? counters->backward : nullptr, counters ? counters->forward : nullptr, nnz, node_count, kind, call_flags);
     for (auto& s : c->bwd) {
         if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream)) return 1;
     }
-    return 0;
+    return record.completed();
 }
 
 int oeq_conv_forward(oeq_conv* c, const void* L1, const void* L2, const void* W, void* L3,
@@ -409,6 +431,13 @@ int oeq_conv_forward_ex(oeq_conv* c, const void* L1, const void* L2, const void*
     return conv_forward(c, L1, L2, W, L3, rows, cols, nnz, node_count, workspace, tperm, stream, call_flags);
 }
 
+int oeq_conv_forward_on(oeq_conv* c, const void* L1, const void* L2, const void* W, void* L3,
+                        const void* rows, const void* cols, uint64_t nnz, uint64_t node_count,
+                        void* workspace, const void* tperm, void* stream, uint32_t call_flags, oeq_conv_counters* counters,
+                        uint64_t kind) {
+    return conv_forward(c, L1, L2, W, L3, rows, cols, nnz, node_count, workspace, tperm, stream, call_flags, counters, kind);
+}
+
 int oeq_conv_backward(oeq_conv* c, const void* L1, void* L1g, const void* L2, void* L2g, const void* W,
                       void* Wg, const void* L3g, const void* rows, const void* cols, uint64_t nnz,
                       uint64_t node_count, void* workspace, const void* tperm, void* stream) {
@@ -421,10 +450,18 @@ int oeq_conv_backward_ex(oeq_conv* c, const void* L1, void* L1g, const void* L2,
     return conv_backward(c, L1, L1g, L2, L2g, W, Wg, L3g, rows, cols, nnz, node_count, workspace, tperm, stream, call_flags);
 }
 
-int oeq_conv_double_backward_ex(oeq_conv* c, const void* L1, const void* L2, const void* W, const void* L3g, const void* L1c,
+int oeq_conv_backward_on(oeq_conv* c, const void* L1, void* L1g, const void* L2, void* L2g, const void* W,
+                         void* Wg, const void* L3g, const void* rows, const void* cols, uint64_t nnz,
+                         uint64_t node_count, void* workspace, const void* tperm, void* stream, uint32_t call_flags,
+                         oeq_conv_counters* counters, uint64_t kind) {
+    return conv_backward(c, L1, L1g, L2, L2g, W, Wg, L3g, rows, cols, nnz, node_count, workspace, tperm, stream, call_flags, counters,
+                         kind);
+}
+
+int oeq_conv_double_backward_on(oeq_conv* c, const void* L1, const void* L2, const void* W, const void* L3g, const void* L1c,
                                 const void* L2c, const void* Wc, void* L1o, void* L2o, void* Wo, void* L3o, const void* rows,
                                 const void* cols, uint64_t nnz, uint64_t node_count, void* workspace, const void* tperm,
-                                void* stream, uint32_t call_flags) {
+                                void* stream, uint32_t call_flags, oeq_conv_counters* counters, uint64_t kind) {
     if (!c) return fail("null handle");
     if (c->bwd.empty()) return fail("this operator was built without a double backward plan");
     if (nnz > 0 && node_count == 0) return fail("convolution called with %llu edges but no nodes", (unsigned long long)nnz);
@@ -434,11 +471,20 @@ int oeq_conv_double_backward_ex(oeq_conv* c, const void* L1, const void* L2, con
     if (call_flags & ~(uint32_t)(OEQ_CALL_PREPARED | OEQ_CALL_COUNTERS_ZERO)) return fail("double backward: unknown call flags 0x%x", call_flags);
     void* args[] = {&L1, &L2, &W, &L3g, &L1c, &L2c, &Wc, &L1o, &L2o, &Wo, &L3o, &rows, &cols, &nnz, &node_count, &workspace, &tperm};
     const auto lock = together(workspace);
+    Record record(counters, counters ? counters->forward : nullptr, counters ? counters->backward : nullptr, nnz, node_count, kind, call_flags);
     for (auto& s : c->bwd) {
         if (skipped(s.desc, call_flags, nnz, node_count)) continue;
         if (launch(s, nnz, node_count, args, stream)) return 1;
     }
-    return 0;
+    return record.completed();
+}
+
+int oeq_conv_double_backward_ex(oeq_conv* c, const void* L1, const void* L2, const void* W, const void* L3g, const void* L1c,
+                                const void* L2c, const void* Wc, void* L1o, void* L2o, void* Wo, void* L3o, const void* rows,
+                                const void* cols, uint64_t nnz, uint64_t node_count, void* workspace, const void* tperm,
+                                void* stream, uint32_t call_flags) {
+    return oeq_conv_double_backward_on(c, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, rows, cols, nnz, node_count, workspace,
+                                       tperm, stream, call_flags, nullptr, 0);
 }
 
 int oeq_conv_double_backward(oeq_conv* c, const void* L1, const void* L2, const void* W, const void* L3g, const void* L1c,
@@ -494,7 +540,7 @@ int oeq_conv_forward_noalloc(oeq_conv* c, const void* L1, const void* L2, const 
                     (unsigned long long)OEQ_NOALLOC_SCRATCH_BYTES);
     void* scratch = nullptr;
     if (noalloc_scratch(&scratch)) return 1;
-    return conv_forward(c, L1, L2, W, L3, rows, cols, nnz, node_count, scratch, tperm, stream, 0, /*pieces=*/false);
+    return conv_forward(c, L1, L2, W, L3, rows, cols, nnz, node_count, scratch, tperm, stream, 0, nullptr, 0, /*pieces=*/false);
 }
 
 // ---------------------------------------------------------- generic module

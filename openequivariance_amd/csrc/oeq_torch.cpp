@@ -168,9 +168,9 @@ struct Library {
     decltype(&oeq_tp_forward) tp_forward;
     decltype(&oeq_tp_backward) tp_backward;
     decltype(&oeq_tp_double_backward) tp_double;
-    decltype(&oeq_conv_forward_ex) conv_forward;
-    decltype(&oeq_conv_backward_ex) conv_backward;
-    decltype(&oeq_conv_double_backward_ex) conv_double;
+    decltype(&oeq_conv_forward_on) conv_forward;
+    decltype(&oeq_conv_backward_on) conv_backward;
+    decltype(&oeq_conv_double_backward_on) conv_double;
     decltype(&oeq_last_error) last_error;
 } g_lib;
 
@@ -193,12 +193,11 @@ int64_t largest(const std::vector<Bytes>& all, int64_t e, int64_t n) {
     return b;
 }
 
-// Scratch that an operator in Python lends for one stream.  ``state``: sizes and kind of the last completed forward and
-// backward while their counters are known to be zero (kind 0: they are not), and whether a capture has used the scratch.
+// Scratch that an operator in Python lends for one stream, and a convolution's record of the counters in it.
 struct Lease {
     int64_t device, stream, size;
     at::Tensor buffer;
-    int64_t* state;
+    oeq_conv_counters* counters;
 };
 
 // A backward of the unsorted convolution: by float atomics into zeros, or over edges grouped by sender.
@@ -353,24 +352,13 @@ struct NativeKernel final : c10::OperatorKernel {
         if (!n.enabled) return false;
         Lease* l = n.lease(device.index(), at_stream);
         const int64_t first = largest(n.first_order, edges, nodes);
-        if (!l || l->state[6] || l->size < (kind == CONV_DOUBLE ? std::max(first, largest(n.second_order, edges, nodes)) : first))
+        if (!l || l->counters->captured || l->size < (kind == CONV_DOUBLE ? std::max(first, largest(n.second_order, edges, nodes)) : first))
             return false;
         const at::Tensor buffer = l->buffer;             // (held until the launches name it)
-        int64_t* const forward_state = l->state;
-        int64_t* const backward_state = l->state + 3;
-        const auto call = [&](int64_t* mine, int64_t* other, int64_t tag, auto&& launch) {
-            const uint32_t zero = mine[2] == tag && mine[0] == edges && mine[1] == nodes ? OEQ_CALL_COUNTERS_ZERO : 0;
-            if (other[0] != edges || other[1] != nodes) other[2] = 0;
-            mine[2] = 0;
-            done(launch(zero));
-            mine[0] = edges; mine[1] = nodes; mine[2] = tag;
-        };
         if (kind == CONV_FORWARD) {
             out.push_back(at::empty({nodes, n.d3}, x.options()));
-            call(forward_state, backward_state, 1, [&](uint32_t flags) {
-                return g_lib.conv_forward(static_cast<oeq_conv*>(n.main.load()), in(&x), in(&y), in(&w), to(out[0]), rows, cols, edges, nodes,
-                                          to(buffer), perm, stream, flags);
-            });
+            done(g_lib.conv_forward(static_cast<oeq_conv*>(n.main.load()), in(&x), in(&y), in(&w), to(out[0]), rows, cols, edges, nodes,
+                                    to(buffer), perm, stream, 0, l->counters, 1));
         } else if (kind == CONV_BACKWARD) {
             Variant v{n.main, true, 1};
             if (n.tuned) {
@@ -381,16 +369,14 @@ struct NativeKernel final : c10::OperatorKernel {
             out.push_back(v.overwrites ? at::empty_like(x) : at::zeros_like(x));
             out.push_back(at::empty_like(y));
             out.push_back(at::empty_like(w));
-            call(backward_state, forward_state, v.kind, [&](uint32_t flags) {
-                return g_lib.conv_backward(static_cast<oeq_conv*>(v.handle), in(&x), to(out[0]), in(&y), to(out[1]), in(&w), to(out[2]),
-                                           in(t[3]), rows, cols, edges, nodes, to(buffer), perm, stream, flags);
-            });
+            done(g_lib.conv_backward(static_cast<oeq_conv*>(v.handle), in(&x), to(out[0]), in(&y), to(out[1]), in(&w), to(out[2]),
+                                     in(t[3]), rows, cols, edges, nodes, to(buffer), perm, stream, 0, l->counters, v.kind));
         } else {
             if (!n.double_ready) return false;
             for (size_t i = 0; i < 4; ++i) out.push_back(at::empty_like(*t[i]));
-            forward_state[2] = backward_state[2] = 0;    // (both groupings are built in the scratch of the first-order kernels)
+            // (both groupings are built in the scratch of the first-order kernels: kind 0)
             done(g_lib.conv_double(static_cast<oeq_conv*>(n.twice), in(&x), in(&y), in(&w), in(t[3]), in(t[4]), in(t[5]), in(t[6]),
-                                   to(out[0]), to(out[1]), to(out[2]), to(out[3]), rows, cols, edges, nodes, to(buffer), perm, stream, 0));
+                                   to(out[0]), to(out[1]), to(out[2]), to(out[3]), rows, cols, edges, nodes, to(buffer), perm, stream, 0, l->counters, 0));
         }
         return true;
     }
@@ -462,11 +448,13 @@ void native_derivative(const std::string& ns, const std::string& name, const std
          torch::CppFunction::makeFromBoxedFunctor(std::make_unique<DerivativeKernel>(native(id), f, g)));
 }
 
-// Scratch for a stream, in place of what was lent for it before.
-void native_lease(int64_t id, const at::Tensor& buffer, int64_t device, int64_t stream, int64_t state) {
+// Scratch for a stream, in place of what was lent for it before.  Nothing is known of the counters in it, whatever a call in
+// what it replaces has left in the record until now.
+void native_lease(int64_t id, const at::Tensor& buffer, int64_t device, int64_t stream, int64_t counters) {
     Native& n = native(id);
     std::lock_guard<std::mutex> lock(n.mutex);
-    Lease l{device, stream, buffer.numel(), buffer, reinterpret_cast<int64_t*>(state)};
+    Lease l{device, stream, buffer.numel(), buffer, reinterpret_cast<oeq_conv_counters*>(counters)};
+    if (l.counters) l.counters->forward[2] = l.counters->backward[2] = 0;
     if (Lease* old = n.lease(device, stream))
         *old = l;
     else
@@ -517,7 +505,7 @@ TORCH_LIBRARY_FRAGMENT(openequivariance_amd, m) {
     m.def("native_operator(int[] v, int[] first, int[] second) -> int", native_operator);
     m.def("native_kernel(str ns, str name, str general, int id, int kind) -> ()", native_kernel);
     m.def("native_derivative(str ns, str name, str fused, str general, int id) -> ()", native_derivative);
-    m.def("native_lease(int id, Tensor buffer, int device, int stream, int state) -> ()", native_lease);
+    m.def("native_lease(int id, Tensor buffer, int device, int stream, int counters) -> ()", native_lease);
     m.def("native_variant(int id, int edge_bits, int node_bits, int handle, bool overwrites, int kind) -> ()", native_variant);
     m.def("native_bytes(int id, int[] more) -> ()", native_bytes);
     m.def("native_enable(int id, bool enabled, bool double_ready) -> ()", native_enable);

@@ -69,6 +69,11 @@ class Step(C.Structure):
         return s
 
 
+class ConvCounters(C.Structure):
+    """Mirror of ``oeq_conv_counters``: which completed calls left a workspace's counters zero."""
+    _fields_ = [("forward", C.c_uint64 * 3), ("backward", C.c_uint64 * 3), ("captured", C.c_uint64)]
+
+
 _lib = None
 _lib_lock = threading.Lock()
 
@@ -113,6 +118,10 @@ def lib() -> C.CDLL:
             "oeq_conv_backward_ex": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, u64, u64, vp, vp, vp, C.c_uint32]),
             "oeq_conv_double_backward": (C.c_int, [vp] * 14 + [u64, u64, vp, vp, vp]),
             "oeq_conv_double_backward_ex": (C.c_int, [vp] * 14 + [u64, u64, vp, vp, vp, C.c_uint32]),
+            "oeq_conv_forward_on": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, u64, u64, vp, vp, vp, C.c_uint32, C.POINTER(ConvCounters), u64]),
+            "oeq_conv_backward_on": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, u64, u64, vp, vp, vp, C.c_uint32,
+                                               C.POINTER(ConvCounters), u64]),
+            "oeq_conv_double_backward_on": (C.c_int, [vp] * 14 + [u64, u64, vp, vp, vp, C.c_uint32, C.POINTER(ConvCounters), u64]),
             "oeq_conv_set_forward_workspace": (C.c_int, [vp, u64, u64, u64]),
             "oeq_conv_forward_noalloc": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, u64, u64, vp, vp]),
             "oeq_module_load": (C.c_int, [vp, sz, C.POINTER(vp)]),
@@ -142,6 +151,7 @@ EXPORTED_SYMBOLS = [
     "oeq_tp_create", "oeq_tp_destroy", "oeq_tp_forward", "oeq_tp_backward", "oeq_tp_double_backward",
     "oeq_conv_create", "oeq_conv_destroy", "oeq_conv_forward", "oeq_conv_backward",
     "oeq_conv_forward_ex", "oeq_conv_backward_ex", "oeq_conv_double_backward", "oeq_conv_double_backward_ex",
+    "oeq_conv_forward_on", "oeq_conv_backward_on", "oeq_conv_double_backward_on",
     "oeq_conv_set_forward_workspace", "oeq_conv_forward_noalloc",
     "oeq_module_load", "oeq_module_unload", "oeq_module_launch",
     "oeq_timer_create", "oeq_timer_destroy", "oeq_timer_start", "oeq_timer_stop", "oeq_timer_clear_cache",
@@ -158,8 +168,8 @@ def _check(status: int) -> None:
 def entry_points() -> List[int]:
     """Addresses of the calls that the torch operators' C++ kernels make."""
     return [C.cast(getattr(lib(), name), C.c_void_p).value for name in
-            ("oeq_tp_forward", "oeq_tp_backward", "oeq_tp_double_backward", "oeq_conv_forward_ex", "oeq_conv_backward_ex",
-             "oeq_conv_double_backward_ex", "oeq_last_error")]
+            ("oeq_tp_forward", "oeq_tp_backward", "oeq_tp_double_backward", "oeq_conv_forward_on", "oeq_conv_backward_on",
+             "oeq_conv_double_backward_on", "oeq_last_error")]
 
 
 # --------------------------------------------------------------------------- device
@@ -311,6 +321,12 @@ class TPImpl:
             _lib.oeq_tp_destroy(h)
 
 
+def _knowledge(prepared, counters_zero):
+    """(call flags, record of the counters, kind) of a convolution's call."""
+    counters, kind, zero = counters_zero if isinstance(counters_zero, tuple) else (None, 0, counters_zero)
+    return (CALL_PREPARED if prepared else 0) | (CALL_COUNTERS_ZERO if zero else 0), counters, kind
+
+
 class ConvImpl:
     """Handle of a compiled fused convolution (reference type: JITConvImpl,
     extension/convolution.hpp:94-176)."""
@@ -331,9 +347,12 @@ class ConvImpl:
                           prepared=False, counters_zero=False):
         """``prepared``: the workspace still holds this graph's forward preparation (OEQ_CALL_PREPARED); the
         preparation kernels are then not launched.  ``counters_zero``: the operator's counters in the
-        workspace are known to be zero (OEQ_CALL_COUNTERS_ZERO); the step that clears them is skipped."""
-        flags = (CALL_PREPARED if prepared else 0) | (CALL_COUNTERS_ZERO if counters_zero else 0)
-        _check(lib().oeq_conv_forward_ex(self._h, L1, L2, W, L3, rows, cols, nnz, node_count, workspace, tperm, stream, flags))
+        workspace are known to be zero (OEQ_CALL_COUNTERS_ZERO); the step that clears them is skipped.
+        ``counters_zero`` may be (ConvCounters kept beside the workspace, kind of the kernel set, whether they are known to be zero
+        all the same): the call then finds that out itself and keeps the record."""
+        flags, counters, kind = _knowledge(prepared, counters_zero)
+        _check(lib().oeq_conv_forward_on(self._h, L1, L2, W, L3, rows, cols, nnz, node_count, workspace, tperm, stream, flags,
+                                         counters, kind))
 
     def exec_conv_noalloc(self, L1, L2, W, L3, rows, cols, nnz, node_count, tperm=0, stream=0):
         """The forward with the library's static scratch as its workspace: allocates nothing."""
@@ -341,16 +360,16 @@ class ConvImpl:
 
     def backward_rawptrs(self, L1, L1g, L2, L2g, W, Wg, L3g, rows, cols, nnz, node_count,
                          workspace=0, tperm=0, stream=0, prepared=False, counters_zero=False):
-        flags = (CALL_PREPARED if prepared else 0) | (CALL_COUNTERS_ZERO if counters_zero else 0)
-        _check(lib().oeq_conv_backward_ex(self._h, L1, L1g, L2, L2g, W, Wg, L3g, rows, cols, nnz, node_count, workspace,
-                                          tperm, stream, flags))
+        flags, counters, kind = _knowledge(prepared, counters_zero)
+        _check(lib().oeq_conv_backward_on(self._h, L1, L1g, L2, L2g, W, Wg, L3g, rows, cols, nnz, node_count, workspace,
+                                          tperm, stream, flags, counters, kind))
 
     def double_backward(self, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, rows, cols, nnz, node_count, workspace=0,
                         tperm=0, stream=0, prepared=False, counters_zero=False):
         """Of a handle created from a double backward's code object with its plan as the backward steps."""
-        flags = (CALL_PREPARED if prepared else 0) | (CALL_COUNTERS_ZERO if counters_zero else 0)
-        _check(lib().oeq_conv_double_backward_ex(self._h, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, rows, cols, nnz,
-                                                 node_count, workspace, tperm, stream, flags))
+        flags, counters, kind = _knowledge(prepared, counters_zero)
+        _check(lib().oeq_conv_double_backward_on(self._h, L1, L2, W, L3g, L1c, L2c, Wc, L1o, L2o, Wo, L3o, rows, cols, nnz,
+                                                 node_count, workspace, tperm, stream, flags, counters, kind))
 
     def __del__(self):
         h, self._h = getattr(self, "_h", None), None
