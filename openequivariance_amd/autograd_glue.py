@@ -34,7 +34,7 @@ class Native:
         self.id, self.ops = id, getattr(torch.ops, NAMESPACE)
 
     @classmethod
-    def create(cls, handles, dtype64, index64, dims, scratch=0, conv=False, shared=False, deterministic=False, tuned=False,
+    def create(cls, handles, dtype64, index64, dims, scratch=0, conv=False, shared=False, deterministic=False, overwrites=True,
                few_limits=(0, 0), first=(), second=()):
         """``handles``: kernel sets (main, for few rows, of the double backward; None where there is none).  None where the
         main one is not a handle of the C library."""
@@ -46,7 +46,7 @@ class Native:
         ops = getattr(torch.ops, NAMESPACE)
         ops.native_library(rt.entry_points())
         return cls(ops.native_operator([int(dtype64), int(index64), *dims, int(scratch), int(conv), int(shared), int(deterministic),
-                                        int(tuned), *raw, *few_limits], [int(v) for t in first for v in t],
+                                        int(overwrites), *raw, *few_limits], [int(v) for t in first for v in t],
                                        [int(v) for t in second for v in t]))
 
 

@@ -310,7 +310,8 @@ class TensorProductConv:
     # ------------------------------------------------------------------ what the C++ kernels have to know of
     def _native_enable(self) -> None:
         if self._native is not None:
-            self._native.ops.native_enable(self._native.id, not self._graph_cache, self._double is not None)
+            self._native.ops.native_enable(self._native.id, not self._graph_cache, self._double is not None,
+                                           self._autotune and not self.deterministic)
 
     @property
     def graph_cache(self) -> bool:
@@ -332,6 +333,7 @@ class TensorProductConv:
     def autotune(self, value: bool) -> None:
         self._autotune = bool(value)
         self._forget_native_variants()
+        self._native_enable()
 
     @property
     def _bwd_choice(self):
@@ -343,12 +345,14 @@ class TensorProductConv:
         self._forget_native_variants()
 
     def _forget_native_variants(self) -> None:
+        self._lent = set()                        # size classes whose variant the C++ kernels have
         if self._native is not None:
             self._native.ops.native_variant(self._native.id, 0, 0, 0, False, 0)
 
     def _lend_variant(self, size_class) -> None:
         """Tells the C++ kernels which backward a size class takes."""
-        if self._native is not None and self._autotune:
+        if self._native is not None and self._autotune and size_class not in self._lent:
+            self._lent.add(size_class)
             name = self._choices[size_class]
             impl, overwrites = self._backward_variant(name)
             self._native.ops.native_variant(self._native.id, *size_class, impl._h.value, overwrites, _StreamWorkspace.TAGS.index(name) + 1)
@@ -609,7 +613,7 @@ class TensorProductConv:
             self._check(x, y, w, rows, cols, tperm, g)
             E, N = rows.shape[0], x.shape[0]
             with _on_device(x.device):
-                if not self.autotune or E == 0:
+                if not self.autotune or det or E == 0:
                     return bwd_run(x, y, w, g, rows, cols, tperm, E, N)
                 size_class = (E.bit_length(), N.bit_length())
                 if size_class not in self._bwd_choice:
@@ -617,7 +621,7 @@ class TensorProductConv:
                         return bwd_run(x, y, w, g, rows, cols, tperm, E, N)
                     self._bwd_choice[size_class] = self._time_backward_variants(
                         lambda name: bwd_run(x, y, w, g, rows, cols, tperm, E, N, name))
-                    self._lend_variant(size_class)
+                self._lend_variant(size_class)
                 return bwd_run(x, y, w, g, rows, cols, tperm, E, N, self._bwd_choice[size_class])
 
         # the two variants differ only in the trailing transpose_perm argument, which the operators' schemas spell out
@@ -632,7 +636,7 @@ class TensorProductConv:
         if self.forward_overwrites and hasattr(self.generator, "workspace_terms"):
             native = Native.create(
                 (self.internal, None, self._double_built[0]), self.config.irrep_dtype == np.float64, self.idx_dtype == np.int64, self._dims,
-                conv=True, deterministic=det, tuned=not self.backward_overwrites or self.autotune,
+                conv=True, deterministic=det, overwrites=self.backward_overwrites,
                 first=[self.generator.workspace_terms()], second=[t for t in self._double_built[2:] if t])
         self._native = native
         self._native_enable()

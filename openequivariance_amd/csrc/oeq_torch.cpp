@@ -210,7 +210,7 @@ struct Variant {
 struct Native {
     at::ScalarType dtype, index;
     int64_t d1, d2, d3, wn, scratch;
-    bool conv, shared, deterministic, tuned;         // tuned: the backward's variant is measured per size class
+    bool conv, shared, deterministic, overwrites;    // overwrites: the main set's backward writes every row of dX
     std::atomic<void*> main, few;                    // kernel sets: general, for few rows,
     void* twice;                                     // ... of the double backward
     std::atomic<int64_t> few_forward, few_backward;  // largest batches of the kernels for few rows
@@ -219,7 +219,7 @@ struct Native {
     std::mutex mutex;                                // of everything below, and of a convolution's launches
     std::vector<Lease> leases;
     std::map<std::pair<int64_t, int64_t>, Variant> variants;
-    bool enabled = true, double_ready = false;
+    bool enabled = true, double_ready = false, tuned = false;      // tuned: the backward's variant is measured per size class
 
     Lease* lease(int64_t device, int64_t stream) {
         for (auto& l : leases)
@@ -360,7 +360,7 @@ struct NativeKernel final : c10::OperatorKernel {
             done(g_lib.conv_forward(static_cast<oeq_conv*>(n.main.load()), in(&x), in(&y), in(&w), to(out[0]), rows, cols, edges, nodes,
                                     to(buffer), perm, stream, 0, l->counters, 1));
         } else if (kind == CONV_BACKWARD) {
-            Variant v{n.main, true, 1};
+            Variant v{n.main, n.overwrites, 1};
             if (n.tuned) {
                 const auto found = n.variants.find({bits(edges), bits(nodes)});
                 if (found == n.variants.end()) return false;
@@ -417,7 +417,7 @@ void native_library(at::IntArrayRef address) {
     for (size_t i = 0; i < 7; ++i) *out[i] = reinterpret_cast<void*>(address[i]);
 }
 
-// Numbers of an operator -> its id.  ``v``: fp64, index64, d1, d2, d3, wn, scratch bytes, conv, shared, deterministic, tuned, handles
+// Numbers of an operator -> its id.  ``v``: fp64, index64, d1, d2, d3, wn, scratch bytes, conv, shared, deterministic, overwrites, handles
 // (main, few, double), limits of the kernels for few rows; ``first`` / ``second``: nine numbers (Bytes) for each workspace rule.
 int64_t native_operator(at::IntArrayRef v, at::IntArrayRef first, at::IntArrayRef second) {
     TORCH_CHECK(v.size() == 16 && first.size() % 9 == 0 && second.size() % 9 == 0, "bad argument");
@@ -425,7 +425,7 @@ int64_t native_operator(at::IntArrayRef v, at::IntArrayRef first, at::IntArrayRe
     n->dtype = v[0] ? at::kDouble : at::kFloat;
     n->index = v[1] ? at::kLong : at::kInt;
     n->d1 = v[2]; n->d2 = v[3]; n->d3 = v[4]; n->wn = v[5]; n->scratch = v[6];
-    n->conv = v[7]; n->shared = v[8]; n->deterministic = v[9]; n->tuned = v[10];
+    n->conv = v[7]; n->shared = v[8]; n->deterministic = v[9]; n->overwrites = v[10];
     n->main = reinterpret_cast<void*>(v[11]); n->few = reinterpret_cast<void*>(v[12]); n->twice = reinterpret_cast<void*>(v[13]);
     n->few_forward = n->few ? v[14] : 0;
     n->few_backward = n->few ? v[15] : 0;
@@ -475,11 +475,12 @@ void native_bytes(int64_t id, at::IntArrayRef more) {
     std::lock_guard<std::mutex> lock(n.mutex);
     n.first_order.push_back({more[0], more[1], more[2], more[3], more[4], more[5], more[6], more[7], more[8]});
 }
-void native_enable(int64_t id, bool enabled, bool double_ready) {
+void native_enable(int64_t id, bool enabled, bool double_ready, bool tuned) {
     Native& n = native(id);
     std::lock_guard<std::mutex> lock(n.mutex);
     n.enabled = enabled;
     n.double_ready = n.double_ready || double_ready;
+    n.tuned = tuned;
 }
 void native_kernels(int64_t id, int64_t main, int64_t few, int64_t forward, int64_t backward) {
     Native& n = native(id);
@@ -508,7 +509,7 @@ TORCH_LIBRARY_FRAGMENT(openequivariance_amd, m) {
     m.def("native_lease(int id, Tensor buffer, int device, int stream, int counters) -> ()", native_lease);
     m.def("native_variant(int id, int edge_bits, int node_bits, int handle, bool overwrites, int kind) -> ()", native_variant);
     m.def("native_bytes(int id, int[] more) -> ()", native_bytes);
-    m.def("native_enable(int id, bool enabled, bool double_ready) -> ()", native_enable);
+    m.def("native_enable(int id, bool enabled, bool double_ready, bool tuned) -> ()", native_enable);
     m.def("native_kernels(int id, int main, int few, int forward, int backward) -> ()", native_kernels);
     m.def("native_workspace_bytes(int id, bool second, int edges, int nodes) -> int", native_workspace_bytes);
 }

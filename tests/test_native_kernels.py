@@ -170,3 +170,37 @@ def test_switches_of_the_convolution_reach_the_kernels(cuda):
     conv.forward(x2, y, w, r, c)
     assert rec.zero_fwd == (nnz, 50 * nodes, "")
     check()
+
+
+@pytest.mark.gpu
+def test_autotune_reaches_the_kernels_both_ways(cuda, monkeypatch):
+    """An operator built without ``autotune``, and with either kernel set as its own: no call goes through Python; set later, the
+    next backward is measured and the calls after it are C++ again, also after off and on."""
+    from openequivariance_amd import tunables
+    prob, oprob = common.channelwise(common.NEQUIP)
+    nodes, nnz = 60, 900
+    rows, cols = common.random_graph(nodes, nnz, 5)
+    r, c = torch.tensor(rows, device=cuda), torch.tensor(cols, device=cuda)
+    host = common.conv_inputs(prob, nodes, nnz, 3)
+    x, y, w, g = (torch.tensor(t, device=cuda) for t in host)
+    want = common.conv_reference_on_valid_edges(otp, oprob, *host, rows, cols, np.ones(nnz, bool))[1:]
+    for default in ("atomic", "grouped"):
+        monkeypatch.setattr(tunables.current, "conv_backward", default)
+        conv = oeq.TensorProductConv(prob, torch_op=True)
+        monkeypatch.undo()
+        assert not conv.autotune and conv.backward_overwrites == (default == "grouped")
+        python = []
+        monkeypatch.setattr(conv, "backward_rawptrs", lambda *a, f=conv.backward_rawptrs, **k: python.append(1) or f(*a, **k))
+
+        def calls():
+            before = len(python)
+            for got, ref in zip(conv.backward_helper(x, y, w, g, r, c), want):
+                assert common.rel_err(got.cpu().numpy(), ref) < 1e-5
+            return len(python) - before
+        assert calls() == 1 and calls() == 0                       # (the first takes the workspace)
+        conv.autotune = True
+        assert calls() > 1 and len(conv._choices) == 1 and calls() == 0
+        conv.autotune = False
+        assert calls() == 0
+        conv.autotune = True
+        assert calls() == 1 and calls() == 0                       # the choice is known, and lent again
