@@ -79,7 +79,7 @@ enum { OEQ_GRID_FIXED = 0, OEQ_GRID_PER_ROW = 1, OEQ_GRID_PER_NODE = 2, OEQ_GRID
  * zeroed again: a call with OEQ_CALL_COUNTERS_ZERO skips it.
  * OEQ_STEP_FEW_NODES(n, d, m), of a convolution's plan: the step runs only on graphs of at most n < 4096 nodes, of more than m
  * (a multiple of 128 below 2048), and at least d < 256 times as many edges as nodes; OEQ_STEP_MANY_NODES(n, d): only on
- * graphs of more than n nodes or fewer than d times as many edges.  A plan holds the forms of a launch that way: one
+ * graphs of more than n nodes or fewer than d times as many edges (oeq_tp_create rejects both).  A plan holds the forms of a launch that way: one
  * wavefront per node, two and four. */
 enum { OEQ_STEP_NEEDS_WORKSPACE = 1, OEQ_STEP_NEEDS_TPERM = 2, OEQ_STEP_GRAPH_PREP = 4, OEQ_STEP_COUNTER_CLEAR = 8 };
 #define OEQ_STEP_FEW_NODES(n, d, m) (16u | (uint32_t)(n) << 8 | (uint32_t)(d) << 20 | (uint32_t)(m) / 128u << 28)
@@ -231,7 +231,7 @@ int  oeq_conv_double_backward_on(oeq_conv* conv, const void* L1_in, const void* 
                                  uint64_t node_count, void* workspace, const void* transpose_perm, void* stream,
                                  uint32_t call_flags, oeq_conv_counters* counters, uint64_t kind);
 
-/* Workspace bytes the forward steps use when every node is walked by one wavefront (no pieces):
+/* Workspace bytes the forward steps use when every node's edges are walked whole (no pieces):
  * fixed_bytes + bytes_per_node * node_count + bytes_per_edge * nnz.  The host sets it from the plan it
  * built the operator with; oeq_conv_forward_noalloc checks graphs against it.  (The reference sizes
  * its workspace on the Python side as well: implementations/convolution/LoopUnrollConv.py:61-72.) */
@@ -242,7 +242,7 @@ int  oeq_conv_set_forward_workspace(oeq_conv* conv, uint64_t fixed_bytes, uint64
  * tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.
  * The workspace is a static device array of OEQ_NOALLOC_SCRATCH_BYTES inside the library (one copy
  * per GPU, held until the process ends); the call allocates and frees nothing.  The forward kernels
- * use what oeq_conv_set_forward_workspace declared (every node is walked by one wavefront here: the
+ * use what oeq_conv_set_forward_workspace declared (every node's edges are walked whole here, by one wavefront or a team: the
  * pieces of long nodes would need partial rows beyond a static array); larger graphs are rejected
  * with an error.  All
  * calls on one GPU share the array: calls that overlap in time on one GPU (different streams or

@@ -274,6 +274,11 @@ void oeq_free(void* p) { free(p); }
 int oeq_tp_create(const void* code, size_t code_size, const oeq_step* fs, int nf, const oeq_step* bs,
                   int nb, oeq_tp** out) {
     if (!code || !out || nf < 0 || nb < 0 || (nf && !fs) || (nb && !bs)) return fail("bad argument");
+    for (int i = 0; i < nf + nb; ++i) {             // (a product has no nodes to choose by: every form of the launch would run)
+        const oeq_step& s = i < nf ? fs[i] : bs[i - nf];
+        if (s.flags & (OEQ_STEP_FEW_NODES(0, 0, 0) | OEQ_STEP_MANY_NODES(0, 0)))
+            return fail("step %d (%.63s): a size rule of graphs in the plan of a batch product", i, s.kernel);
+    }
     oeq_tp* tp = new oeq_tp();
     if (load_steps(tp->mod, code, code_size, fs, nf, tp->fwd) ||
         load_steps(tp->mod, code, code_size, bs, nb, tp->bwd)) {
@@ -531,7 +536,7 @@ int oeq_conv_forward_noalloc(oeq_conv* c, const void* L1, const void* L2, const 
         return fail("oeq_conv_forward_noalloc: the operator's forward workspace size is unknown "
                     "(call oeq_conv_set_forward_workspace after oeq_conv_create)");
     if (nnz > (1ull << 40) || node_count > (1ull << 40)) return fail("graph too large");
-    // what the forward steps of this operator's plan use with every node walked by one wavefront
+    // what the forward steps of this operator's plan use with every node's edges walked whole
     const uint64_t need = c->ws_fixed + c->ws_per_node * node_count + c->ws_per_edge * nnz;
     if (need > (uint64_t)OEQ_NOALLOC_SCRATCH_BYTES)
         return fail("oeq_conv_forward_noalloc: %llu edges and %llu nodes need %llu bytes of scratch, the static "

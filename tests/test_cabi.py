@@ -66,3 +66,11 @@ def test_error_reporting_without_device():
     assert b"null handle" in L.oeq_last_error()
     n = ctypes.c_int(-1)
     assert L.oeq_device_count(ctypes.byref(n)) == 0 and n.value >= 0
+
+
+def test_size_rules_of_graphs_are_rejected_in_a_products_plan():
+    L, h = rt.lib(), ctypes.c_void_p()
+    plain, few, many = (rt.Step.make("k", 64, flags=f) for f in (0, rt.step_few_nodes(100, 2), rt.step_many_nodes(100, 2)))
+    for fwd, bwd in ((few, plain), (plain, many)):
+        assert L.oeq_tp_create(b"code", 4, ctypes.byref(fwd), 1, ctypes.byref(bwd), 1, ctypes.byref(h)) != 0
+        assert b"size rule" in L.oeq_last_error()
