@@ -356,6 +356,8 @@ def run_tp(gen, steps: Sequence[Dict], X, Y, W, G=None, ws_bytes: int = 0):
     """Run TP steps; returns dict of outputs (Z or dX, dY, dW)."""
     dt = np.float32 if gen.T == "float" else np.float64
     extra = TP_EXTRA_UVW if gen.kind == "uvw" else TP_EXTRA_UVW_ROWS if gen.kind == "uvw_rows" else (TP_EXTRA_SHARED if gen.shared else "")
+    if gen.kind == "uvw" and not gen.separate_prep:
+        extra = "\n".join(line for line in extra.split("\n") if "prep_backward" not in line)
     main = TP_MAIN.replace("@EXTRA@", extra)
     exe = build(gen.render(prelude=emu_prelude(gen.T)), main)
     n = X.shape[0]
