@@ -50,9 +50,15 @@ class UVWBatchedGenerator(UVWGenerator):
         self.stream = self.batches is not None
         # the backward keeps its other walk where chunks are long and whole lines: 32 channels, 20 000 rows 112 us against 116.5, 48
         # channels 160 against 163, fp64, 24 channels, 6000 rows 117 against 120 (16 channels, chunks of 256 words: 81.9 / 79.8)
-        self.stream_backward = self.stream and not (self.WN >= 400 * sum(map(len, self.batches)) and all(
-            ul * wl * self.itemsize % 128 == 0 for b in self.batches for _, _, ul, _, wl, _ in b))
+        self.stream_backward = self.stream and self.WN <= self.STREAM_ROW[self.T] and not (
+            self.WN >= 400 * sum(map(len, self.batches)) and all(
+                ul * wl * self.itemsize % 128 == 0 for b in self.batches for _, _, ul, _, wl, _ in b))
 
+    # Words of a row up to which the backward's weights move in batches.  A long row of few is bound by what one wavefront has in
+    # flight, and the other walk has four chunks: fp32, batches / chunks, us, 46 channels, l <= 2 (23 276 words) 859 rows 41 / 44,
+    # 6444 rows 264 / 278; 52 (29 744) 672 rows 55 / 47, 5043 rows 249 / 257; 100 (110 000) 500 rows 142 / 108, 1363 rows 256 / 271.
+    # fp64, where that walk has two, does not lose: 38 880 words, 500 rows 82 / 83, 1929 rows 244 / 248.
+    STREAM_ROW = {"float": 25000, "double": 1 << 62}
     STREAM_UNROLL = 4             # steps of a chunk's loop in flight in the forward
     STREAM_BYTES = 4096           # of a batch at most (a chunk of 32 x 32 words; 8192 in fp64)
 
@@ -513,6 +519,25 @@ class UVWBatchedGenerator(UVWGenerator):
         E("}")
         return E.text()
 
+    # A path's dT goes into dX and dY with products that nothing waits for before the row ends, and left to itself the compiler
+    # keeps every dT until then: the registers grow with the paths.  Here they are taken after every four paths (of 32 channels;
+    # fp64: eight), after every two where outputs reach l = 3.  Left / taken, registers (bytes of scratch) and us:
+    #   fp32   44 channels of both parities, l <= 1, 7747 rows      512 (384) 367    248 240
+    #          44 channels, l <= 2, 7043 rows                       264 251          245 238
+    #          10 channels, l <= 3, 20 000 rows                     270 231          103 112
+    #   fp64   17 channels of both parities, l <= 2, 8650 rows      454 308          236 261
+    #          36 channels, l <= 3, 2516 rows                       512 (524) 323    324 268
+    # Problems whose sums fit lose a little of what the order gave them, 38 channels, l <= 2, 9443 rows 265 / 271, and more where
+    # they are taken after each path: DiffDock's layer, 20 000 rows 226 left, 227 after four, 231 after each.
+    PUT_OFF, PUT_OFF_L3 = {"float": 4, "double": 8}, 2
+
+    def _take_sums(self, E: Emitter, put_off) -> None:
+        """The dX (of these names) and dY of the paths are worked out here."""
+        sums = dict.fromkeys([f"{dx}{i}" for p, dx in put_off for i in range(p.a.D)]
+                             + [f"dy{p.b.off + j}" for p, _ in put_off for j in range(p.b.D) if p.b.off + j in self.used_y])
+        E(" ".join(f"OEQ_OPAQUE({v});" for v in sums))
+        put_off.clear()
+
     def backward_stream_body(self) -> str:
         """The row's weights as batches of whole chunks, in memory order: a batch moves 16 bytes per lane and instruction, whole cache
         lines, and the next one is in flight in registers while this one is worked on in LDS.  Chunk by chunk, an access
@@ -526,6 +551,8 @@ class UVWBatchedGenerator(UVWGenerator):
         E(f"__shared__ T gl[{max(1, self.D3)}];")
         E(f"T* __restrict__ Wgr = Wg + row * {self.WN};")
         now = [None]                                 # (path, uc, ul) whose t and dt the registers hold
+        put_off = []                                 # paths whose sums the compiler may still put off
+        names = max(p.o.D for p in self.paths)
 
         def work(job, at):
             p, uc, ul = job[:3]
@@ -599,7 +626,9 @@ class UVWBatchedGenerator(UVWGenerator):
                 s *= 2
             E(f"if (!act{ul} || ws{ul} != 0) {{ " + " ".join(f"dt{k} = (T)0;" for k in range(p.o.D)) + " }")
             self.emit_cg_backward(E, p, "dt", f"x{p.a.idx}_{uc}_", "y", f"dx{p.a.idx}_{uc}_", "dy")
-        names = max(p.o.D for p in self.paths)
+            put_off.append((p, f"dx{p.a.idx}_{uc}_"))
+            if len(put_off) == (self.PUT_OFF[self.T] if names <= 5 else self.PUT_OFF_L3):
+                self._take_sums(E, put_off)
         E("T " + ", ".join(f"{v}{k} = (T)0" for v in ("t", "dt") for k in range(names)) + ";")
         for _ in stream:
             pass

@@ -15,6 +15,7 @@ CASES = {
     "short_chunks": ("10x1o+10x1e+20x0e", "1x0e+1x1o", "10x1o+10x1e+20x0e"),
     "rows_of_32_16_8_4_words": ("34x0e+6x1o", "1x0e+1x1o", "32x0e+48x1o+8x0o+4x2e"),
     "copies": ("10x0e+40x1o", "3x0e+2x1o", "36x0e+10x1o"),
+    "l3": ("12x0e+6x1o+10x3o", "1x0e+1x1o+1x2e+1x3o", "12x0e+6x1o+4x2e+10x3o"),
     "odd_paths_even_row": ("3x0e+5x1o", "1x0e+1x1o", "4x0e+1x1o"),
 }
 TOL = {np.float32: 4e-6, np.float64: 1e-13}       # a few hundred roundings a value
@@ -35,6 +36,27 @@ def test_which_rows_stream():
     ragged, lines = (UVWBatchedGenerator(common.fully_connected(irreps, shared=False)[0]) for irreps in
                      (("5x0e+21x1o", "1x0e+1x1o+1x2e", "18x0e+7x1o+3x2e"), ("32x0e+32x1o", "1x0e+1x1o", "32x0e+32x1o")))
     assert not ragged.stream and not ragged.stream_backward and lines.stream and not lines.stream_backward
+
+
+@pytest.mark.parametrize("mul, lmax, parities, dtype, most", [(44, 1, "eo", np.float32, 256), (10, 3, "", np.float32, 128),
+                                                               (17, 2, "eo", np.float64, 256), (36, 3, "", np.float64, 512)])
+def test_registers_of_the_backward_are_bounded(mul, lmax, parities, dtype, most):
+    """Many paths between few channels: their sums are not all kept until the row ends (two wavefronts per SIMD have 256 registers
+    each), and none goes to memory."""
+    from openequivariance_amd import runtime as rt
+    irreps = "+".join(f"{mul}x{l}{p}" for l in range(lmax + 1) for p in (parities or "eo"[l % 2]))
+    g = UVWBatchedGenerator(common.fully_connected((irreps, "+".join(f"1x{l}{'eo'[l % 2]}" for l in range(lmax + 1)), irreps), shared=False,
+                                                   dtype=dtype)[0])
+    assert g.stream_backward
+    k = rt.kernel_metadata(rt.compile_source(g.render(), use_cache=False))["backward"]
+    assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_count"] <= most
+
+
+def test_long_rows_keep_the_walk_over_chunks():
+    """fp32, 25 000 words and more: a wavefront's four chunks in flight do more for few rows than one batch does."""
+    gens = [UVWBatchedGenerator(common.fully_connected((f"{m}x0e+{m}x1o+{m}x2e", "1x0e+1x1o+1x2e", f"{m}x0e+{m}x1o+{m}x2e"), shared=False, dtype=dtype)[0])
+            for m, dtype in ((46, np.float32), (52, np.float32), (50, np.float64))]
+    assert [(g.stream, g.stream_backward) for g in gens] == [(True, True), (True, False), (True, True)]
 
 
 @pytest.mark.parametrize("dtype", list(TOL))
