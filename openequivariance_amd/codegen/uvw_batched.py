@@ -369,14 +369,26 @@ class UVWBatchedGenerator(UVWGenerator):
         return E.text()
 
     # ---------------------------------------------------------------- backward
-    # Weight chunks whose loads are in flight ahead of the one being worked on, and steps of a chunk's row loop in flight (all 16 at
-    # once would take 100 more registers).  Many chunks are short - 100 words between two 10-channel blocks - and two of them
-    # ahead cover less than a memory latency.  2 and 4 steps / 4 and 8: DiffDock's layer, 50 000 rows 617 / 592 us; 30 channels,
-    # 15 000 rows 161 / 154; 42, 10 000 rows 155 / 150; 8, 20 000 rows 41.6 / 40.6.  More wavefronts per SIMD instead (96 registers)
-    # spill: 656.  fp64, where a word is two registers, gains nothing (465 / 463) and keeps two and 4 (48 channels, l <= 2: 248
-    # registers, 324 with the others).
-    PREFETCH = {"float": 4, "double": 2}
-    COMPUTE_UNROLL = {"float": 8, "double": 4}
+    # The walk over chunks: chunks whose loads are in flight ahead of the one being worked on, and steps of a chunk's row loop in
+    # flight (all 16 at once would take 100 more registers).  fp32 words whose chunks are short or ragged: two of them ahead cover
+    # less than a memory latency.  2 and 4 steps / 4 and 8, us, l <= 2, 0.6 GB of weights (20 000 rows at most) and 0.08: 17
+    # channels 123 / 118 and 45 / 43, 31 267 / 258 and 42 / 42, 47 287 / 279 and 46 / 44; l <= 1, 17 45.0 / 43.2 and 40 / 38.  Chunks that
+    # are 32 x 32 throughout, several to a block, are far enough ahead with two: 64 channels 241 / 254 and 43 / 45, of both parities
+    # 254 / 253 and 109 / 119.  fp64, where a word is two registers, gains nothing (DiffDock's layer 465 / 463).
+    AHEAD = {"float": (4, 8), "double": (2, 4)}
+    AHEAD_WHOLE = 2, 4
+
+    def _chunk_walk(self):
+        """((chunks ahead, steps in flight), whether a path's sums are taken when it is done with).  Left to the compiler they go
+        to the end of a block of the first operand (see PUT_OFF), which costs registers where its paths are many: fp32, 17 channels of
+        both parities, l <= 2, 17 301 rows, 259 registers 486 us, taken 291; fp64, 20 channels to l = 3, 8152 rows 400, 309 and
+        244, 48 of both parities, l <= 2, 1085 rows 313 and 272; and where a block is several chunks long: fp32, 80 channels, l <= 2,
+        2130 rows 273 / 258, 65 channels 310 / 291.  Few sums are better left: 47 channels of both parities, l <= 1, 266 / 276."""
+        muls = [b.mul for b in (*self.in1, *self.out) if b.dim]
+        whole = all(m % 32 == 0 for m in muls) and max(muls) > 32
+        sums = max(sum(p.o.D for p in self.paths_from(a.idx)) for a in self.in1 if a.dim)
+        return self.AHEAD_WHOLE if whole else self.AHEAD[self.T], sums >= 20 or max(muls) > 64
+
     NONTEMPORAL = True    # the weights and their gradient are touched once
     def backward_body(self) -> str:
         if self.stream_backward:
@@ -405,7 +417,7 @@ class UVWBatchedGenerator(UVWGenerator):
 
         def regs(job):
             return width(job) * _ceil(job[3], 64 * width(job))
-        ahead = self.PREFETCH[self.T]
+        (ahead, unroll), take = self._chunk_walk()
         nbuf = ahead + 1
         for b in range(min(nbuf, len(jobs))):
             E(f"T r{b}_[{max(regs(job) for job in jobs[b::nbuf])}];")
@@ -478,7 +490,7 @@ class UVWBatchedGenerator(UVWGenerator):
                             E(("  if (act) " if lp != ul else "  ") + f"tile[ur * {S} + {wq}] = "
                               + " + ".join(f"t{k} * g{k}" for k in range(o.D)) + ";")
                         if full:
-                            E(f"#pragma unroll {self.COMPUTE_UNROLL[self.T]}")
+                            E(f"#pragma unroll {unroll}")
                             E(f"for (int j = 0; j < {full}; ++j) {{")
                             step(f"ws + {ns} * j")
                             E("}")
@@ -504,6 +516,8 @@ class UVWBatchedGenerator(UVWGenerator):
                         s *= 2
                     E("if (!act || ws != 0) { " + " ".join(f"dt{k} = (T)0;" for k in range(o.D)) + " }")
                     self.emit_cg_backward(E, p, "dt", "x", "y", "dx", "dy")
+                    if take:
+                        self._take_sums(E, [(p, "dx")])
                     E.level -= 1
                     E("}")
                 E(f"if (act && ws == 0) {{ T* __restrict__ dp = Xg + row * {self.D1} + {a.off} + ({32 * uc} + uq) * {a.D}; "
@@ -606,7 +620,7 @@ class UVWBatchedGenerator(UVWGenerator):
                 E(("  if (act%d) " % ul if lp != ul else "  ") + f"tile[{at} + ur{ul} * {wl} + c_] = "
                   + " + ".join(f"t{k} * g{k}" for k in range(o.D)) + ";")
             if full:
-                E(f"#pragma unroll {self.COMPUTE_UNROLL[self.T]}")
+                E(f"#pragma unroll {self.AHEAD[self.T][1]}")
                 E(f"for (int j = 0; j < {full}; ++j) {{")
                 step(f"ws{ul} + {ns} * j")
                 E("}")

@@ -94,3 +94,33 @@ def test_on_the_gpu(cuda, case, dtype, monkeypatch):
             got = [t.cpu().numpy() for t in tp.backward_helper(x, y, v, dz)]
             for a, b in zip((*got[:2], ow.oeq_to_e3nn(oprob, got[2])), (dX, dY, dW)):
                 assert rel_err(a, b) < TOL[dtype]
+
+
+def test_walk_over_chunks(monkeypatch):
+    """Where it takes a path's sums, how far it looks ahead, and the registers of a problem of many paths (all sums kept: 259)."""
+    from openequivariance_amd import runtime as rt
+
+    def walk(irreps, in2="1x0e+1x1o+1x2e", dtype=np.float32):
+        return UVWBatchedGenerator(common.fully_connected((irreps, in2, irreps), shared=False, dtype=dtype)[0], stream=False)
+    seven = "+".join(f"17x{l}{p}" for l in range(3) for p in "eo")
+    assert walk("17x0e+17x1o+17x2e")._chunk_walk() == ((4, 8), False)
+    assert walk("17x0e+17x1o+17x2e", dtype=np.float64)._chunk_walk() == ((2, 4), False)
+    assert walk("65x0e+65x1o")._chunk_walk() == ((4, 8), True) and walk(seven)._chunk_walk() == ((4, 8), True)
+    assert walk("64x0e+64x1o")._chunk_walk() == ((2, 4), False) and walk("32x0e+32x1o")._chunk_walk() == ((4, 8), False)
+    k = rt.kernel_metadata(rt.compile_source(walk(seven).render(), use_cache=False))["backward"]
+    assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_count"] <= 128
+
+
+@pytest.mark.parametrize("dtype", list(TOL))
+@pytest.mark.parametrize("case", ["l3", "copies", "whole"])
+def test_walk_over_chunks_emulated(case, dtype, monkeypatch):
+    """With sums taken (many paths) and left, looking four and two chunks ahead, more and fewer of them than that."""
+    monkeypatch.setitem(CASES, "whole", ("64x0e", "1x0e", "64x0e"))
+    _, prob, oprob = generator(case, dtype)
+    g = UVWBatchedGenerator(prob, stream=False)
+    assert g._chunk_walk()[1] == (case == "l3")
+    X, Y, We, G = common.tp_inputs(prob, 3, 10, dtype=dtype, w_scale=0.3)
+    out = emu.run_tp(g, g.plan()[1], X, Y, ow.e3nn_to_oeq(oprob, We), G)
+    dX, dY, dW = otp.backward(oprob, X, Y, We, G)
+    assert rel_err(out["Xg"], dX) < TOL[dtype] and rel_err(out["Yg"], dY) < TOL[dtype]
+    assert rel_err(ow.oeq_to_e3nn(oprob, out["Wg"]), dW) < TOL[dtype]
