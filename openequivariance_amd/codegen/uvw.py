@@ -106,9 +106,17 @@ class UVWGenerator:
     #     66, l <= 2                   30.8 / 21.4  34.8 / 25.1   97 / 65     192 / 143   366 / 310
     #     80, l <= 1                   22.1 / 15.3  26.3 / 20.2   71 / 56     140 / 124   272 / 285
     #     90, l <= 1                   37.3 / 23.7  41.7 / 29.4  115 / 78     233 / 189   460 / 396
+    # Blocks of five tiles whose whole form leaves room for two wavefronts per SIMD (second operands up to l = 1: 212 - 252 registers;
+    # to l = 2 328 and more) are better whole on many rows, where the chip is full and a cut block's X is read and multiplied twice:
+    #     80, l <= 1      57 000 rows 164 / 159   65 000  186 / 188   100 000  275 / 286   200 000  529 / 561
+    #     72, l <= 1                  166 / 161           190 / 219            292 / 345            560 / 674
+    #     20 -> 80, l <= 1             95 / 85            105 / 96             156 / 178            304 / 366
+    # and from fewer rows on the longer their K loop: 100 -> 80 (50 steps) 20 000 rows 96 / 89, 35 000 140 / 144, 57 000 229 / 270.
+    # Operators give them the cut form up to ROWS_CUT rows, by the steps of the loop (few_rows_generator).
     # Beside outputs of l = 2, whose items are the longer ones, it goes either way (80 channels l <= 2 27 / 29 at 4097 rows, 253 / 263
     # at 50 000; 70 with l <= 2 55 / 63, 542 / 503), and so does cutting those (64 channels 20 / 18, 142 / 182).
     FWD_ACC_LIMIT_L1 = {4: 80, 8: 56}
+    ROWS_CUT = ((45, 57000), (1 << 30, 28000))
     FWD_PIPELINE = {4: (4, 2), 8: (1, 3)}
     # Steps of an fp64 path (one a batch, unrolled three times) that are a multiple of three cost more than another one: per
     # step and 100 000 rows 13 us with 20 or 19 of them, 18 us with 18.  66 channels l <= 1, 18 / 20 / 19 steps 316 / 267 /
@@ -116,7 +124,8 @@ class UVWGenerator:
     FWD_NO_MULTIPLE = {4: 0, 8: 3}
     BWD_LDS_LIMIT = 80 * 1024    # dZ tile of the backward: two workgroups per compute unit (gfx950: 160 KB)
 
-    def __init__(self, problem: TPProblem):
+    def __init__(self, problem: TPProblem, many_rows: bool = False):
+        """``many_rows``: the forward's blocks as they are best on many rows, where ``rows_cut`` names those they are cut for."""
         self.problem = problem
         self.kind = "uvw"
         self.T = {np.float32: "float", np.float64: "double"}[problem.irrep_dtype]
@@ -178,6 +187,12 @@ class UVWGenerator:
         # a work item of its own: fewer accumulators per wavefront buy a third wavefront per SIMD, which
         # hides one wavefront's vector-ALU phases behind another's matrix-core phases
         limits = {3: min(self.FWD_ACC_LIMIT, self.FWD_ACC_LIMIT_L1[self.itemsize])} if max(self.out[o].D for o in self.used_out) == 3 else {}
+        five = [o for o in self.used_out if self.out[o].D == 3 and limits and limits[3] < 12 * _ceil(self.out[o].mul, 16) <= 60]
+        self.rows_cut = 0                       # (0: one form for all)
+        if many_rows and five and max(p.b.l for p in self.paths) <= 1 and max(b.mul for b in self.out if b.idx in self.used_out and b.D == 3) <= 80:
+            steps = max(sum(p.SU for p in self.paths if p.o.idx == o) for o in five)
+            self.rows_cut = next(rows for most, rows in self.ROWS_CUT if steps <= most)
+            limits = {}
         self.fwd_order = []
         for o in sorted([o for o in self.out if o.dim > 0], key=lambda o: -cost(o)):
             nt_all = _ceil(o.mul, 16)

@@ -141,6 +141,12 @@ class UVWSmallGenerator(UVWGenerator):
         """What the dW phases of a workgroup hand over to each other, of the largest unit."""
         return max(uw * (self.DW_WAVES // uw // 2) * _ceil(p.NTU, uw) * (hi - lo) * 256 for p, lo, hi, uw in self.units)
 
+    forward_from = None          # the generator whose forward is this set's, in place of its own
+
+    def take_forward(self, g: UVWGenerator) -> None:
+        self.forward_from, self.has_forward = g, True
+        self.forward_body, self.forward_attr, self.prep_body = g.forward_body, g.forward_attr, g.prep_body
+
     def forward_attr(self) -> str:
         return " __attribute__((amdgpu_waves_per_eu(2)))"
 
@@ -282,4 +288,6 @@ class UVWSmallGenerator(UVWGenerator):
         _, dx, dw, reduce = bwd
         dw["num_blocks"] = sum(self.chunks)
         reduce["num_blocks"] = _ceil(self.WN, 64)
+        if self.forward_from is not None:
+            fwd = self.forward_from.plan()[0]
         return fwd, [dw, dx, reduce], ws               # (dW packs the weights that dX reads)

@@ -76,7 +76,7 @@ def select_generator(config: TPProblem):
     if mode == "uvw" and config.shared_weights:
         from .codegen.uvw_rows import UVWRowsGenerator
         # a few hundred weights on multiplicities far below a 16 x 16 tile: one row per lane on the vector ALU
-        return UVWRowsGenerator(config) if UVWRowsGenerator.suits(config) else UVWSplitGenerator.create(config) or UVWGenerator(config)
+        return UVWRowsGenerator(config) if UVWRowsGenerator.suits(config) else UVWSplitGenerator.create(config) or UVWGenerator(config, many_rows=True)
     if mode == "uvw":
         from .codegen.uvw_batched import UVWBatchedGenerator
         return UVWBatchedGenerator(config)
@@ -122,10 +122,14 @@ def few_rows_generator(config: TPProblem, generator: UVWGenerator):
     """(generator, largest batches forward and backward) of the kernels for few rows beside a dense uvw product's
     ``generator``: without a forward where they leave it none, (None, (0, 0)) where they have no batch at all."""
     small = UVWSmallGenerator.create(config)
+    cut = UVWGenerator(config) if generator.rows_cut else None        # the forward of fewer rows
     if small is None:
-        return None, (0, 0)
+        return cut, (generator.rows_cut, 0)
     limits = getattr(generator, "few_rows", tuple)(UVWSmallGenerator.row_limits(generator))
     small.has_forward = limits[0] > 0
+    if cut is not None:
+        small.take_forward(cut)
+        limits = generator.rows_cut, limits[1]
     return (small, limits) if any(limits) else (None, (0, 0))
 
 
