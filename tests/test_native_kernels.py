@@ -204,3 +204,35 @@ def test_autotune_reaches_the_kernels_both_ways(cuda, monkeypatch):
         assert calls() == 0
         conv.autotune = True
         assert calls() == 1 and calls() == 0                       # the choice is known, and lent again
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("problem", ["nequip", "mace"])
+def test_both_backwards_of_unsorted_edges(cuda, problem, monkeypatch):
+    """Each variant as the choice, whatever a stopwatch would say: from C++ (float atomics into zeros, groups by sender and - mace -
+    in receiver order), the kinds of their counters kept apart, sizes changing between calls."""
+    prob, oprob = common.channelwise(dict(nequip=common.NEQUIP, mace=common.MACE)[problem])
+    conv = oeq.TensorProductConv(prob, torch_op=True)
+    graphs = []
+    for nodes, nnz, seed in ((60, 900, 5), (61, 1001, 6)):
+        rows, cols = common.random_graph(nodes, nnz, seed)
+        host = common.conv_inputs(prob, nodes, nnz, seed)
+        want = common.conv_reference_on_valid_edges(otp, oprob, *host, rows, cols, np.ones(nnz, bool))
+        graphs.append(([torch.tensor(t, device=cuda) for t in (*host, rows, cols)], want))
+    assert conv._backward_variant("grouped")[0] is not conv._backward_variant("atomic")[0]
+    (x, y, w, g, r, c), _ = graphs[1]
+    conv.backward_helper(x, y, w, g, r, c)                                  # (the larger one's workspace; times the variants)
+    sizes = (int(r.numel()).bit_length(), int(x.shape[0]).bit_length())
+    python = []
+    for name in ("exec_conv_rawptrs", "backward_rawptrs"):
+        monkeypatch.setattr(conv, name, lambda *a, f=getattr(conv, name), n=name, **k: python.append(n) or f(*a, **k))
+    for choice in ("atomic", "grouped", "atomic"):
+        conv._bwd_choice = {sizes: choice}
+        conv._lend_variant(sizes)
+        for k in (0, 1, 1, 0, 0):
+            (x, y, w, g, r, c), want = graphs[k]
+            got = conv.forward(x, y, w, r, c), *conv.backward_helper(x, y, w, g, r, c)
+            for a, b in zip(got, want):
+                assert common.rel_err(a.cpu().numpy(), b) < 2e-5, (choice, k)
+            assert conv._workspace_record(int(r.numel()), int(x.shape[0])).zero_bwd == (int(r.numel()), int(x.shape[0]), choice)
+    assert not python, "a call went through Python"
