@@ -15,6 +15,7 @@ assumption about the graph.
 """
 from __future__ import annotations
 
+import collections
 import contextlib
 import ctypes
 import threading
@@ -139,6 +140,39 @@ def with_few_nodes(generator):
     return generator.add_few_nodes() if hasattr(generator, "add_few_nodes") else generator
 
 
+# Generators with the kernels for few nodes and what they write, by what that depends on.  Operators of one problem - the layers of
+# a model - share them (bounded): writing the kernels takes 1.3 ms of an operator's construction at 64 channels, and 1.9 ms of the
+# first backward over unsorted edges, which builds the other variant.
+_GENERATED: "collections.OrderedDict[tuple, tuple]" = collections.OrderedDict()
+_GENERATED_MAX = 64
+_generated_lock = threading.Lock()
+
+
+def _identity(generator) -> tuple:
+    """What tells the sources and plans of a generator from those of others: its problem, type, constants and choices."""
+    skip = ("problem", "in1", "in2", "out", "paths", "_lines")                # (follow from the problem)
+    return (getattr(generator, "problem", None) and generator.problem.signature(), type(generator),
+            tuple((k, repr(v)) for c in type(generator).__mro__ for k, v in vars(c).items() if k.isupper()),
+            tuple((k, _identity(v) if hasattr(v, "render") else repr(v)) for k, v in vars(generator).items() if k not in skip))
+
+
+def generated(generator) -> tuple:
+    """(key, generator, source): the generator ``with_few_nodes`` that writes what this one would, and its source."""
+    key = _identity(generator)
+    with _generated_lock:
+        got = _GENERATED.get(key)
+        if got is not None:
+            _GENERATED.move_to_end(key)
+    if got is None:
+        generator = with_few_nodes(generator)
+        got = (key, generator, generator.render())
+        with _generated_lock:
+            got = _GENERATED.setdefault(key, got)
+            if len(_GENERATED) > _GENERATED_MAX:
+                _GENERATED.popitem(last=False)
+    return got
+
+
 class _StreamWorkspace:
     """Device scratch of one operator on one stream, and which graph its preparation areas
     (CSR pointers, position lists, node order) currently describe."""
@@ -197,20 +231,19 @@ class TensorProductConv:
         if mode != "uvu":
             raise NotImplementedError("TensorProductConv supports uvu problems")
 
-        self.generator = with_few_nodes(select_conv_generator(config, deterministic, idx_dtype=self.idx_dtype))
+        _, self.generator, self.jit_kernel = generated(select_conv_generator(config, deterministic, idx_dtype=self.idx_dtype))
         # True: the forward writes every row of Z itself; False: it accumulates into a zeroed Z
         self.forward_overwrites = not isinstance(self.generator, UVUDirectGenerator) or deterministic
         # likewise for dX in the backward (the per-edge backward accumulates with atomics)
         self.backward_overwrites = deterministic or getattr(self.generator, "grouped_backward", False)
         # the deterministic backward walks the caller's transpose permutation
         self.backward_needs_tperm = deterministic
-        self.jit_kernel = self.generator.render()
         # held from the look at a stream's workspace until the launches in it are issued: threads share it
         self._lock = threading.RLock()
         self._native = None                       # the operator's part in the C++ kernels (torch_op=True)
         self._ws_fns = []
         self._ws_last = self._double_ws_last = (None, 0)          # (sizes, bytes) of the last workspace query
-        self.internal = self._build(self.generator, self.jit_kernel)
+        self.internal = self._build(None, self.generator, self.jit_kernel)
         self._workspaces: typing.Dict[tuple, _StreamWorkspace] = {}      # (device, stream) -> scratch
         # Unsorted edge lists: whether the backward scatters dX with float atomics or groups the edges by
         # sender first depends on the row length AND on the graph (atomics per edge against the gathers of
@@ -239,20 +272,24 @@ class TensorProductConv:
         if torch_op:
             self._setup_torch_module()
 
-    def _build(self, generator, source=None) -> "rt.ConvImpl":
-        """Compile one kernel set of this operator (``with_few_nodes``).  Every set shares the operator's workspace, which is
-        sized for the largest of them."""
+    def _build(self, key, generator, source: str) -> "rt.ConvImpl":
+        """Loads a kernel set of this operator (``generated``), with a ``key`` shared with the operators that have the same.  Every set
+        shares the operator's workspace, which is sized for the largest of them."""
         fwd, bwd, ws = getattr(generator, "plan_few", generator.plan)()
         self._ws_fns.append(ws)
         if self._native is not None:
             self._native.ops.native_bytes(self._native.id, generator.workspace_terms())
         need_ws = rt.STEP_NEEDS_WORKSPACE if ws(1, 1) > 0 else 0
         need_tp = rt.STEP_NEEDS_TPERM if self.backward_needs_tperm else 0
-        code = rt.compile_source(source if source is not None else generator.render())
-        impl = rt.ConvImpl(code, _make_steps(fwd, need_ws), _make_steps(bwd, need_ws | need_tp))
-        model = getattr(generator, "forward_workspace_model", None)
-        impl.set_forward_workspace(*(model() if model else (0, 0, 0)))
-        return impl
+
+        def load(code, _=None):
+            impl = rt.ConvImpl(code, _make_steps(fwd, need_ws), _make_steps(bwd, need_ws | need_tp))
+            model = getattr(generator, "forward_workspace_model", None)
+            impl.set_forward_workspace(*(model() if model else (0, 0, 0)))
+            return impl
+        if key is not None:
+            return rt.variant(("conv", key, need_tp), torch.cuda.current_device(), lambda: (source, None), load)[0]
+        return load(rt.compile_source(source))
 
     def _ws_bytes(self, nnz: int, node_count: int) -> int:
         key, last = (nnz, node_count, len(self._ws_fns)), self._ws_last       # (read once: other threads ask for other sizes)
@@ -264,9 +301,9 @@ class TensorProductConv:
         """(kernel set, whether its backward overwrites dX) of a backward variant of the unsorted operator,
         compiled on first need."""
         if name not in self._bwd_variants:
-            g = with_few_nodes(UVUSortedGenerator(self.config, grouped_backward=(name == "grouped"),
-                                                  idx_ctype="i64" if self.idx_dtype == np.int64 else "int"))
-            self._bwd_variants[name] = (self._build(g), name == "grouped")
+            g = UVUSortedGenerator(self.config, grouped_backward=(name == "grouped"),
+                                   idx_ctype="i64" if self.idx_dtype == np.int64 else "int")
+            self._bwd_variants[name] = (self._build(*generated(g)), name == "grouped")
             for rec in self._workspaces.values():            # the workspace may have to grow: sizes are re-checked per call
                 rec.bwd_key = None
         return self._bwd_variants[name]
@@ -451,9 +488,8 @@ class TensorProductConv:
             bits |= int(p)
         if bits % 16:
             if self._internal_unaligned is None:
-                g = with_few_nodes(select_conv_generator(self.config, self.deterministic, vector_stores=False,
-                                                         idx_dtype=self.idx_dtype))
-                self._internal_unaligned = self._build(g)
+                g = select_conv_generator(self.config, self.deterministic, vector_stores=False, idx_dtype=self.idx_dtype)
+                self._internal_unaligned = self._build(*generated(g))
             return self._internal_unaligned
         return self.internal
 

@@ -2,6 +2,7 @@
 last owner; an operator has them when it is constructed."""
 import gc
 
+import numpy as np
 import pytest
 import torch
 
@@ -123,3 +124,40 @@ def test_workspace_sizes_asked_for_by_several_threads(monkeypatch):
     for nnz in (1000, 1000, 7):
         assert conv._ws_bytes(nnz, 5) == 8 * nnz
         assert conv._double_ws_bytes(nnz, 5) == 16 * nnz
+
+
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_layers_of_one_problem_write_their_convolution_once(deterministic, monkeypatch):
+    """The kernels of a second operator, and the backward variant that its first pass builds, are there already; an operator
+    with other choices gets its own."""
+    from openequivariance_amd import conv as conv_mod, tunables
+    from openequivariance_amd.codegen.uvu_det import UVUDetGenerator
+    from openequivariance_amd.codegen.uvu_sorted import UVUSortedGenerator
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(rt, "compile_source", lambda source, *a, **k: source.encode())
+    monkeypatch.setattr(rt, "ConvImpl", Impl)
+    monkeypatch.setattr(rt, "_VARIANTS", type(rt._VARIANTS)())
+    monkeypatch.setattr(rt, "_LOADED", type(rt._LOADED)())
+    monkeypatch.setattr(conv_mod, "_GENERATED", type(conv_mod._GENERATED)())
+    written = []
+    for cls in (UVUDetGenerator, UVUSortedGenerator):
+        monkeypatch.setattr(cls, "render", lambda self, *a, f=cls.render, **k: written.append(type(self)) or f(self, *a, **k))
+
+    def layer(**kwargs):
+        op = oeq.TensorProductConv(common.channelwise(common.NEQUIP)[0], deterministic=deterministic, **kwargs)
+        sets = [op._pick(8)] if deterministic else [op._backward_variant(v)[0] for v in ("atomic", "grouped")] + [op._pick(8)]
+        return op, sets
+    (first, a), n = layer(), len(written)
+    (second, b) = layer()
+    assert n == len(written) == (2 if deterministic else 3)
+    assert first.jit_kernel == second.jit_kernel == first.internal.code.decode() and first.internal is not second.internal
+    assert sum(x is y for x, y in zip(a, b)) == len(a) - (not deterministic)        # (all but the operator's own set)
+    assert first._ws_bytes(5000, 300) == second._ws_bytes(5000, 300)
+    with monkeypatch.context() as m:
+        m.setattr(tunables.current, "long_node", 0)
+        assert layer()[0].jit_kernel != first.jit_kernel
+    with monkeypatch.context() as m:
+        m.setattr(UVUDetGenerator, "TEAMS", ())
+        assert "forward_few" not in layer()[0].jit_kernel and "forward_few" in first.jit_kernel
+    assert layer(idx_dtype=np.int32)[0].jit_kernel != first.jit_kernel
+    assert layer()[0].jit_kernel == first.jit_kernel
