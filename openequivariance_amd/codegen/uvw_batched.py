@@ -544,6 +544,23 @@ class UVWBatchedGenerator(UVWGenerator):
     # Problems whose sums fit lose a little of what the order gave them, 38 channels, l <= 2, 9443 rows 265 / 271, and more where
     # they are taken after each path: DiffDock's layer, 20 000 rows 226 left, 227 after four, 231 after each.
     PUT_OFF, PUT_OFF_L3 = {"float": 4, "double": 8}, 2
+    # A chunk whose rows are no longer than AHEAD's eight steps is one line to the compiler, together with those around it.  Where most
+    # of a row is such chunks and some take more than STEP_WORDS words of dZ, four steps are in flight, a loop, and sums are taken every
+    # two paths.  fp32, l <= 2, chunks / eight / four: 12 channels to 60 (190, 272 and 185 registers) 200 rows 16.2 / 14.8 / 16.7 us,
+    # 2500 45.5 / 47.0 / 44.6, 18 939 234 / 311 / 230; 10 to 40 12.8 / 10.8 / 12.0, 20.8 / 25.1 / 19.9, 34 090 230 / 237 / 220.  Where
+    # they are few, 42 channels, 7730 rows 263 / 252 / 257.
+    STEP_WORDS, FEWER_STEPS = 32, 4
+
+    def _stream_steps(self):
+        """(steps in flight of a chunk's row with these words of dZ a step, paths after which sums are taken) of the backward over
+        batches."""
+        most, names = self.AHEAD[self.T][1], max(p.o.D for p in self.paths)
+        put_off = self.PUT_OFF_L3 if names > 5 else self.PUT_OFF[self.T]
+        line = [(ul * wl, wl // self._split(ul)[2] * p.o.D) for batch in self.batches for p, _, ul, _, wl, _ in batch
+                if self.FEWER_STEPS < wl // self._split(ul)[2] <= most]
+        if line and 2 * sum(words for words, _ in line) > self.WN and max(g for _, g in line) > self.STEP_WORDS:
+            return (lambda words: self.FEWER_STEPS if most * words > self.STEP_WORDS else most), self.PUT_OFF_L3
+        return (lambda words: most), put_off
 
     def _take_sums(self, E: Emitter, put_off) -> None:
         """The dX (of these names) and dY of the paths are worked out here."""
@@ -567,6 +584,7 @@ class UVWBatchedGenerator(UVWGenerator):
         now = [None]                                 # (path, uc, ul) whose t and dt the registers hold
         put_off = []                                 # paths whose sums the compiler may still put off
         names = max(p.o.D for p in self.paths)
+        steps, put_off_most = self._stream_steps()
 
         def work(job, at):
             p, uc, ul = job[:3]
@@ -620,7 +638,7 @@ class UVWBatchedGenerator(UVWGenerator):
                 E(("  if (act%d) " % ul if lp != ul else "  ") + f"tile[{at} + ur{ul} * {wl} + c_] = "
                   + " + ".join(f"t{k} * g{k}" for k in range(o.D)) + ";")
             if full:
-                E(f"#pragma unroll {self.AHEAD[self.T][1]}")
+                E(f"#pragma unroll {steps(o.D)}")
                 E(f"for (int j = 0; j < {full}; ++j) {{")
                 step(f"ws{ul} + {ns} * j")
                 E("}")
@@ -641,7 +659,7 @@ class UVWBatchedGenerator(UVWGenerator):
             E(f"if (!act{ul} || ws{ul} != 0) {{ " + " ".join(f"dt{k} = (T)0;" for k in range(p.o.D)) + " }")
             self.emit_cg_backward(E, p, "dt", f"x{p.a.idx}_{uc}_", "y", f"dx{p.a.idx}_{uc}_", "dy")
             put_off.append((p, f"dx{p.a.idx}_{uc}_"))
-            if len(put_off) == (self.PUT_OFF[self.T] if names <= 5 else self.PUT_OFF_L3):
+            if len(put_off) == put_off_most:
                 self._take_sums(E, put_off)
         E("T " + ", ".join(f"{v}{k} = (T)0" for v in ("t", "dt") for k in range(names)) + ";")
         for _ in stream:

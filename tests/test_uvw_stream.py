@@ -16,6 +16,7 @@ CASES = {
     "rows_of_32_16_8_4_words": ("34x0e+6x1o", "1x0e+1x1o", "32x0e+48x1o+8x0o+4x2e"),
     "copies": ("10x0e+40x1o", "3x0e+2x1o", "36x0e+10x1o"),
     "l3": ("12x0e+6x1o+10x3o", "1x0e+1x1o+1x2e+1x3o", "12x0e+6x1o+4x2e+10x3o"),
+    "rows_in_one_line": ("12x0e+12x2e", "1x0e+1x1o+1x2e", "44x0e+64x2e"),
     "odd_paths_even_row": ("3x0e+5x1o", "1x0e+1x1o", "4x0e+1x1o"),
 }
 TOL = {np.float32: 4e-6, np.float64: 1e-13}       # a few hundred roundings a value
@@ -48,6 +49,16 @@ def test_registers_of_the_backward_are_bounded(mul, lmax, parities, dtype, most)
     g = UVWBatchedGenerator(common.fully_connected((irreps, "+".join(f"1x{l}{'eo'[l % 2]}" for l in range(lmax + 1)), irreps), shared=False,
                                                    dtype=dtype)[0])
     assert g.stream_backward
+    k = rt.kernel_metadata(rt.compile_source(g.render(), use_cache=False))["backward"]
+    assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_count"] <= most
+
+
+@pytest.mark.parametrize("mul, out, steps, most", [(12, 60, (4, 2), 192), (10, 40, (4, 2), 168), (42, 42, (8, 4), 256), (60, 12, (8, 4), 256)])
+def test_registers_of_chunks_in_one_line(mul, out, steps, most):
+    """Rows of eight steps with five words of dZ each (12 channels to 60: 272 registers with all of them in flight)."""
+    from openequivariance_amd import runtime as rt
+    g = UVWBatchedGenerator(common.fully_connected((f"{mul}x0e+{mul}x1o+{mul}x2e", "1x0e+1x1o+1x2e", f"{out}x0e+{out}x1o+{out}x2e"), shared=False)[0])
+    assert g.stream_backward and (g._stream_steps()[0](5), g._stream_steps()[1]) == steps and g._stream_steps()[0](3) == 8
     k = rt.kernel_metadata(rt.compile_source(g.render(), use_cache=False))["backward"]
     assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_count"] <= most
 
