@@ -47,12 +47,29 @@ class UVWBatchedGenerator(UVWGenerator):
         self.t_lds = max([sum(p.mu * o.D for o in ph for p in self.paths_into(o.idx)) for ph in self.forward_phases()] + [0])
         self.ws_elems = 0
         self.batches = self._batches() if stream else None
-        self.stream = self.batches is not None
+        self.stream_forward = self.batches is not None and not self._first_operand_too_wide(forward=True)
         # the backward keeps its other walk where chunks are long and whole lines: 32 channels, 20 000 rows 112 us against 116.5, 48
         # channels 160 against 163, fp64, 24 channels, 6000 rows 117 against 120 (16 channels, chunks of 256 words: 81.9 / 79.8)
-        self.stream_backward = self.stream and self.WN <= self.STREAM_ROW[self.T] and not (
+        self.stream_backward = self.batches is not None and self.WN <= self.STREAM_ROW[self.T] and not (
             self.WN >= 400 * sum(map(len, self.batches)) and all(
-                ul * wl * self.itemsize % 128 == 0 for b in self.batches for _, _, ul, _, wl, _ in b))
+                ul * wl * self.itemsize % 128 == 0 for b in self.batches for _, _, ul, _, wl, _ in b)
+        ) and not self._first_operand_too_wide(forward=False)
+        self.stream = self.stream_forward or self.stream_backward
+
+    # 32-bit words a lane holds of the first operand over a whole row, which the walks over chunks read block by block: in the forward
+    # X (and few sums Z beside it: a narrow output), in the backward X and dX.  Beyond these the batches lose their wavefronts, then
+    # their registers.  512 channels to 4, l <= 2, chunks / batches, us, 600 rows and 420 MB of weights: forward, fp32 (72 words) 15.1 /
+    # 15.9 and 69 / 89, fp64 (144) 22.9 / 26.9 and 75 / 90; backward, fp32 (288) 41 / 26 and 146 / 154, fp64 (576) 56 / 84 and 154 / 289;
+    # 2000x1o to 4, fp32 (378) 49 / 28 and 138 / 146, fp64 (756) 65 / 80 and 134 / 276.  256 channels, fp64: forward (72) 10.1 /
+    # 9.9 and 60 / 62, backward (288) 30 / 21 and 141 / 135.
+    FORWARD_WORDS, BACKWARD_WORDS = 64, 400
+
+    def _first_operand_too_wide(self, forward: bool) -> bool:
+        def held(blocks, lanes):
+            return sum(_ceil(b.mul, lanes) * b.D for b in blocks if b.dim) * self.itemsize // 4
+        if forward:
+            return held(self.in1, 64) > max(self.FORWARD_WORDS, 4 * held(self.out, 32))
+        return 2 * held(self.in1, 32) > self.BACKWARD_WORDS
 
     # Words of a row up to which the backward's weights move in batches.  A long row of few is bound by what one wavefront has in
     # flight, and the other walk has four chunks: fp32, batches / chunks, us, 46 channels, l <= 2 (23 276 words) 859 rows 41 / 44,
@@ -150,7 +167,7 @@ class UVWBatchedGenerator(UVWGenerator):
         return [ph for ph in phases if ph]
 
     def forward_body(self) -> str:
-        if self.stream:
+        if self.stream_forward:
             return self.forward_stream_body()
         E = Emitter()
         E("const int lane = threadIdx.x;")

@@ -63,6 +63,22 @@ def test_registers_of_chunks_in_one_line(mul, out, steps, most):
     assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_count"] <= most
 
 
+def test_wide_first_operands_keep_the_walk_over_chunks():
+    """A lane of a batch holds its channels' X (and dX) over the whole row."""
+    from openequivariance_amd import runtime as rt
+
+    def gen(irreps, dtype):
+        return UVWBatchedGenerator(common.fully_connected(irreps, shared=False, dtype=dtype)[0])
+    wide, half = ("512x0e+512x1o+512x2e", "1x0e+1x1o", "4x0e+4x1o+4x2e"), ("256x0e+256x1o+256x2e", "1x0e+1x1o+1x2e", "4x0e+4x1o")
+    for irreps, dtype, forward, backward in ((wide, np.float32, False, True), (wide, np.float64, False, False), (half, np.float32, True, True),
+                                             (half, np.float64, False, True), (("2000x1o", "1x0e+1x1o", "4x0e+4x1o"), np.float64, False, False),
+                                             (("100x0e+100x0o+100x1o+100x1e+100x2e+100x2o", "1x0e+1x1o+1x2e", "100x0e+100x1o+100x2e"), np.float64, True, False)):
+        g = gen(irreps, dtype)
+        assert (g.stream_forward, g.stream_backward, g.stream) == (forward, backward, forward or backward)
+    for k in rt.kernel_metadata(rt.compile_source(gen(wide, np.float64).render(), use_cache=False)).values():
+        assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_count"] <= 256
+
+
 def test_long_rows_keep_the_walk_over_chunks():
     """fp32, 25 000 words and more: a wavefront's four chunks in flight do more for few rows than one batch does."""
     gens = [UVWBatchedGenerator(common.fully_connected((f"{m}x0e+{m}x1o+{m}x2e", "1x0e+1x1o+1x2e", f"{m}x0e+{m}x1o+{m}x2e"), shared=False, dtype=dtype)[0])
