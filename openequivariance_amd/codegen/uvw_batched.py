@@ -322,7 +322,12 @@ class UVWBatchedGenerator(UVWGenerator):
         then lanes <-> (output channel, slice of u).  Against lanes that read the weights from memory chunk by chunk: DiffDock's
         layer, 50 000 rows 275 -> 252 us (5.9 TB/s), fp64, 20 000 rows 210 -> 197; 6 channels, 20 000 rows 26.5 -> 17.8, 12 31.7 ->
         26.4, 42, 10 000 rows 67.6 -> 60.2, 48, 4000 rows 65.8 -> 64.0 (eight steps at a time: 70.8), fp64, 2500 rows 141 -> 80
-        (that walk spilled); 32 channels, 20 000 rows 53.8 and 54.0."""
+        (that walk spilled); 32 channels, 20 000 rows 53.8 and 54.0.
+
+        Rows of no more than STREAM_UNROLL steps are no loop, and nothing waits for their sums before the row ends: left to itself the
+        compiler keeps the operands of every chunk until then.  There a path's sums are taken when the next one begins.  8 channels
+        to 36, both parities, l <= 2, 11 574 rows: chunks 89.7 us, sums left 122.6 (479 registers), taken 79.2 (120); fp64, 5787 rows
+        93 / 409 (512 and 1972 bytes of scratch) / 81 (218); 4 to 34, fp64, l <= 1 91 / 88 / 85; 8 to 8, fp32 158 / 109 / 108."""
         E = Emitter()
         words = [sum(ul * wl for _, _, ul, _, wl, _ in b) for b in self.batches]
         self._stream_header(E, words)
@@ -334,13 +339,14 @@ class UVWBatchedGenerator(UVWGenerator):
         for o, wc, _ in outs:
             E("T " + ", ".join(f"z{o.idx}_{wc}_{k} = (T)0" for k in range(o.D)) + ";")
         held = [(a, h) for a in self.in1 if a.dim for h in range(_ceil(a.mul, 64))]
-        now = [None]
+        now, put_off = [None], {}                     # the path whose T is in LDS; sums that the compiler may still put off
 
         def work(job, at):
             p, uc, ul, wc, wl, _ = job
             o = p.o
             if now[0] != p.t:
                 now[0] = p.t
+                self._take(E, put_off)
                 E("oeq_sync();")
                 for h in range(_ceil(p.mu, 64)):
                     E(f"{{ const int u = {64 * h} + lane;   // T of path {p.t}")
@@ -352,6 +358,8 @@ class UVWBatchedGenerator(UVWGenerator):
                 E("oeq_sync();")
             _, _, ns = self._split(wl)
             full, tail = divmod(ul, ns)
+            if full <= self.STREAM_UNROLL:
+                put_off.update((f"z{o.idx}_{wc}_{k}", None) for k in range(o.D))
             E(f"{{ // weights [{ul}][{wl}] of path {p.t}")
 
             def step(u):
@@ -579,11 +587,18 @@ class UVWBatchedGenerator(UVWGenerator):
             return (lambda words: self.FEWER_STEPS if most * words > self.STEP_WORDS else most), self.PUT_OFF_L3
         return (lambda words: most), put_off
 
+    @staticmethod
+    def _take(E: Emitter, names: dict) -> None:
+        """The values are worked out here."""
+        if names:
+            E(" ".join(f"OEQ_OPAQUE({v});" for v in names))
+            names.clear()
+
     def _take_sums(self, E: Emitter, put_off) -> None:
         """The dX (of these names) and dY of the paths are worked out here."""
         sums = dict.fromkeys([f"{dx}{i}" for p, dx in put_off for i in range(p.a.D)]
                              + [f"dy{p.b.off + j}" for p, _ in put_off for j in range(p.b.D) if p.b.off + j in self.used_y])
-        E(" ".join(f"OEQ_OPAQUE({v});" for v in sums))
+        self._take(E, sums)
         put_off.clear()
 
     def backward_stream_body(self) -> str:

@@ -17,6 +17,7 @@ CASES = {
     "copies": ("10x0e+40x1o", "3x0e+2x1o", "36x0e+10x1o"),
     "l3": ("12x0e+6x1o+10x3o", "1x0e+1x1o+1x2e+1x3o", "12x0e+6x1o+4x2e+10x3o"),
     "rows_in_one_line": ("12x0e+12x2e", "1x0e+1x1o+1x2e", "44x0e+64x2e"),
+    "few_to_many": ("4x0e+8x1o+6x1e", "1x0e+1x1o", "66x0e+40x1o+6x1e"),
     "odd_paths_even_row": ("3x0e+5x1o", "1x0e+1x1o", "4x0e+1x1o"),
 }
 TOL = {np.float32: 4e-6, np.float64: 1e-13}       # a few hundred roundings a value
@@ -60,6 +61,18 @@ def test_registers_of_chunks_in_one_line(mul, out, steps, most):
     g = UVWBatchedGenerator(common.fully_connected((f"{mul}x0e+{mul}x1o+{mul}x2e", "1x0e+1x1o+1x2e", f"{out}x0e+{out}x1o+{out}x2e"), shared=False)[0])
     assert g.stream_backward and (g._stream_steps()[0](5), g._stream_steps()[1]) == steps and g._stream_steps()[0](3) == 8
     k = rt.kernel_metadata(rt.compile_source(g.render(), use_cache=False))["backward"]
+    assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_count"] <= most
+
+
+@pytest.mark.parametrize("mul, out, dtype, most", [(8, 36, np.float32, 128), (8, 36, np.float64, 256), (4, 34, np.float64, 256), (6, 50, np.float32, 128),
+                                                    (8, 100, np.float64, 320)])
+def test_registers_of_the_forward_are_bounded(mul, out, dtype, most):
+    """Few channels: a chunk's rows are no loop (8 to 36, fp64: 512 registers and 1972 bytes of scratch where all sums wait for the end)."""
+    from openequivariance_amd import runtime as rt
+    irreps = tuple("+".join(f"{m}x{l}{p}" for l in range(3) for p in "eo") for m in (mul, out))
+    g = UVWBatchedGenerator(common.fully_connected((irreps[0], "1x0e+1x1o+1x2e", irreps[1]), shared=False, dtype=dtype)[0])
+    assert g.stream_forward
+    k = rt.kernel_metadata(rt.compile_source(g.render(), use_cache=False))["forward"]
     assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_count"] <= most
 
 
