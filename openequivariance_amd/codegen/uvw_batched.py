@@ -55,6 +55,20 @@ class UVWBatchedGenerator(UVWGenerator):
                 ul * wl * self.itemsize % 128 == 0 for b in self.batches for _, _, ul, _, wl, _ in b)
         ) and not self._first_operand_too_wide(forward=False)
         self.stream = self.stream_forward or self.stream_backward
+        self.rows_chunked = self.ROWS_CHUNKED if self.stream_forward and self.ROW_BYTES[0] <= self.WN * self.itemsize <= self.ROW_BYTES[1] else 0
+        self.has_backward = True
+
+    # Rows up to which the forward keeps the walk over chunks, as a kernel for few rows: a wavefront per SIMD, with nothing beside it to
+    # hide a batch's way through LDS.  Rows of 16 to 64 KB; short ones are a batch or two, and longer ones spill in that walk.  Chunks /
+    # batches, us, 256, 1024 and 2048 rows: DiffDock's layer 5.0 / 5.9, 7.0 / 7.8 and 10.6 / 10.5, fp64 5.8 / 7.0, 10.7 / 10.9 and 19.9 / 19.0;
+    # 10 channels to 50, l <= 2, 5.7 / 7.3, 7.5 / 8.7 and 10.7 / 10.3, fp64 5.5 / 8.8, 10.1 / 11.3 and 19.9 / 17.6; 60 of both parities
+    # to 26, l <= 1, 6.5 / 10.5, 11.5 / 15.0 and 20.8 / 21.6.  Below 16 KB, 34 channels, one scalar, 5.1 / 4.5, 6.4 / 5.9, 9.0 / 7.9.
+    ROWS_CHUNKED, ROW_BYTES = 1024, (16 << 10, 64 << 10)
+
+    def forward_of_few_rows(self) -> "UVWBatchedGenerator":
+        few = UVWBatchedGenerator(self.problem, stream=False)
+        few.has_backward = False
+        return few
 
     # 32-bit words a lane holds of the first operand over a whole row, which the walks over chunks read block by block: in the forward
     # X (and few sums Z beside it: a narrow output), in the backward X and dX.  Beyond these the batches lose their wavefronts, then
@@ -716,5 +730,5 @@ class UVWBatchedGenerator(UVWGenerator):
 
     def plan(self):
         fwd = [dict(kernel="forward", num_threads=64, grid_kind=1, work_per_block=1)]
-        bwd = [dict(kernel="backward", num_threads=64, grid_kind=1, work_per_block=1)]
+        bwd = [dict(kernel="backward", num_threads=64, grid_kind=1, work_per_block=1)] if self.has_backward else []
         return fwd, bwd, (lambda nnz=0, nodes=0: 0)

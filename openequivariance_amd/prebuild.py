@@ -14,6 +14,7 @@ from . import runtime as rt
 from .codegen.uvu_conv_double import conv_double_generator
 from .codegen.uvu_double import UVUDoubleGenerator
 from .codegen.uvw import UVWGenerator
+from .codegen.uvw_batched import UVWBatchedGenerator
 from .codegen.uvw_split import UVWSplitGenerator
 from .conv import select_conv_generator, with_few_nodes
 from .problem import ChannelwiseTPP, FullyConnectedTPProblem, TPProblem
@@ -31,7 +32,7 @@ def benchmark_generators():
     def tp(label, problem):
         g = select_generator(problem)
         gens.append((label, g))
-        if type(g) in (UVWGenerator, UVWSplitGenerator):
+        if type(g) in (UVWGenerator, UVWSplitGenerator, UVWBatchedGenerator):
             few, _ = few_rows_generator(problem, g)
             if few is not None:
                 gens.append((label + " few rows", few))

@@ -119,8 +119,10 @@ class TensorProductBase:
 
 
 def few_rows_generator(config: TPProblem, generator: UVWGenerator):
-    """(generator, largest batches forward and backward) of the kernels for few rows beside a dense uvw product's
+    """(generator, largest batches forward and backward) of the kernels for few rows beside a uvw product's
     ``generator``: without a forward where they leave it none, (None, (0, 0)) where they have no batch at all."""
+    if isinstance(generator, UVWBatchedGenerator):
+        return (generator.forward_of_few_rows(), (generator.rows_chunked, 0)) if generator.rows_chunked else (None, (0, 0))
     small = UVWSmallGenerator.create(config)
     cut = UVWGenerator(config) if generator.rows_cut else None        # the forward of fewer rows
     if small is None:
@@ -162,7 +164,7 @@ class TensorProduct(TensorProductBase):
         self._workspaces = {}                 # (device, stream) -> scratch tensor (fixed size, never regrown)
         self._internal_unaligned = None       # kernels without 16-byte vector stores, compiled on first need
         self._unaligned_batched = {}          # those of per-row uvw weights for tensors aligned to 8 bytes (True) or not
-        # dense uvw: kernels for few rows and their largest batch (forward, backward).  Built here like the double backward's,
+        # uvw: kernels for few rows and their largest batch (forward, backward).  Built here like the double backward's,
         # not by the call that first needs them: that call would wait for the compiler, and a stream capture cannot
         self._few_rows, self._few_rows_limits = self._few_row_kernels()
         # double backward in one launch: kernels by alignment of the outputs (misaligned ones are compiled on first need)
@@ -238,12 +240,12 @@ class TensorProduct(TensorProductBase):
     internal, _few_rows, _few_rows_limits = _kernel_set("internal"), _kernel_set("_few_rows"), _kernel_set("_few_rows_limits")
 
     def _few_row_kernels(self):
-        """(kernel set, limits) of the kernels for few rows of a dense uvw product."""
+        """(kernel set, limits) of the kernels for few rows of a uvw product."""
         def build():
             g, limits = few_rows_generator(self.config, self.generator)
             return (None, None) if g is None else (g.render(), (*g.plan()[:2], limits))
         none = None, (0, 0)
-        if type(self.generator) not in (UVWGenerator, UVWSplitGenerator):
+        if type(self.generator) not in (UVWGenerator, UVWSplitGenerator) and not getattr(self.generator, "rows_chunked", 0):
             return none
         impl, plan = rt.variant(("uvw few rows", self.config.signature()), torch.cuda.current_device(), build,
                                 lambda code, plan: rt.TPImpl(code, *(_make_steps(steps, self._step_flags) for steps in plan[:2])))
@@ -259,7 +261,9 @@ class TensorProduct(TensorProductBase):
 
     def forward_raw(self, batch, L1_in, L2_in, L3_out, weights, stream=None) -> None:
         """Device pointers as integers (reference: TensorProductBase.py:41-49)."""
-        impl = self._pick_rows(int(batch), False) or self._pick(L1_in, L2_in, L3_out, weights)
+        impl = self._pick(L1_in, L2_in, L3_out, weights)
+        if impl is self.internal:                       # (the kernels for few rows need the alignment that these do)
+            impl = self._pick_rows(int(batch), False) or impl
         impl.exec_tensor_product(int(batch), L1_in, L2_in, L3_out, weights, self._workspace_ptr(stream),
                                  self._stream() if stream is None else stream)
 

@@ -164,3 +164,45 @@ def test_walk_over_chunks_emulated(case, dtype, monkeypatch):
     dX, dY, dW = otp.backward(oprob, X, Y, We, G)
     assert rel_err(out["Xg"], dX) < TOL[dtype] and rel_err(out["Yg"], dY) < TOL[dtype]
     assert rel_err(ow.oeq_to_e3nn(oprob, out["Wg"]), dW) < TOL[dtype]
+
+
+DIFFDOCK = ("10x1o+10x1e+48x0e+48x0o", "1x0e+1x1o+1x2e", "10x1o+10x1e+48x0e+48x0o")
+
+
+@pytest.mark.parametrize("irreps, rows", [(DIFFDOCK, (1024, 1024)), (("10x0e+10x1o+10x2e", "1x0e+1x1o+1x2e", "10x0e+10x1o+10x2e"), (0, 0)),
+                                          (("44x0e+44x1o+44x2e", "1x0e+1x1o+1x2e", "44x0e+44x1o+44x2e"), (0, 0)),
+                                          (("30x0e+30x1o", "1x0e+1x1o", "30x0e+30x1o"), (0, 1024)), (("5x0e+31x1o", "1x0e+1x1o", "33x0e+31x1o"), (0, 0))])
+def test_forward_of_few_rows(irreps, rows):
+    """Rows of 16 to 64 KB that pass in batches; the set for few of them has a forward alone."""
+    from openequivariance_amd.tensor_product import few_rows_generator
+    for dtype, most in zip(TOL, rows):
+        prob = common.fully_connected(irreps, shared=False, dtype=dtype)[0]
+        g = UVWBatchedGenerator(prob)
+        few, limits = few_rows_generator(prob, g)
+        assert g.rows_chunked == most and limits == (most, 0) and (few is None) == (most == 0)
+        if few is not None:
+            assert not few.stream and few.plan()[1] == [] and "void backward(" not in few.render() and "void backward(" in g.render()
+            assert few.forward_body() == UVWBatchedGenerator(prob, stream=False).forward_body() != g.forward_body()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(TOL))
+def test_forward_of_few_rows_on_the_gpu(cuda, dtype, monkeypatch):
+    """Both sides of the line, through the C++ kernels and the raw entry point; a misaligned operand keeps its own kernels."""
+    import torch
+    import openequivariance_amd as oeq
+    prob, oprob = common.fully_connected(DIFFDOCK, shared=False, dtype=dtype)
+    tp = oeq.TensorProduct(prob, torch_op=True)
+    assert tp._few_rows_limits == (1024, 0) and tp._few_rows is not None
+    calls = []
+    monkeypatch.setattr(tp._few_rows, "exec_tensor_product", lambda *a, f=tp._few_rows.exec_tensor_product: calls.append(a[0]) or f(*a))
+    for n in (1, 1024, 1025):
+        X, Y, We, _ = common.tp_inputs(prob, n, n, dtype=dtype, w_scale=0.3)
+        x, y, w = (torch.tensor(a, device=cuda) for a in (X, Y, ow.e3nn_to_oeq(oprob, We)))
+        Z = otp.forward(oprob, X, Y, We)
+        z = torch.full((n, Z.shape[1]), float("nan"), device=cuda, dtype=x.dtype)
+        tp.forward_raw(n, x.data_ptr(), y.data_ptr(), z.data_ptr(), w.data_ptr())
+        off = torch.cat([w.new_zeros(1), w.reshape(-1)])[1:].view(w.shape)
+        for got in (tp.forward(x, y, w), z, tp.forward(x, y, off)):
+            assert rel_err(got.cpu().numpy(), Z) < TOL[dtype]
+    assert calls == [1, 1024]
