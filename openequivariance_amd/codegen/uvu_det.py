@@ -578,7 +578,7 @@ class UVUDetGenerator(UVUDirectGenerator):
         2000 nodes 26 / 17 / 15, 4000 32 / 29 / 27; 128 channels, 1000 nodes 55 / 50 / 50.  Sender pass, 32 channels: 760 nodes 31 / 25 / 24, 1500 42 / 41 / 43; fp64, 64
         channels, 760 nodes 100 / 95 / 101, 1001 143 / 162 / 156.  Double backward, 32 channels: 500 nodes 66 / 48 / 37, 1001
         81 / 69 / 77, 1500 87 / 90 / 94."""
-        needs = [k["need"] for k in self.few_sources[which]]
+        needs = [k["need"] for k in self.few_sources[which] if "need" in k]
         out, beyond = [], 0
         for team, groups in self.TEAMS:
             if not needs or any(self.team_bytes(team, n) + self.lds_elems * self.itemsize > self.TEAM_LDS for n in needs):

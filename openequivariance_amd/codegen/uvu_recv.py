@@ -24,6 +24,8 @@ tiles: the dZ row of a receiver whose edges span two tiles is then re-read from 
 """
 from __future__ import annotations
 
+import copy
+
 from ..problem import TPProblem
 from .common import Emitter, WAVE
 from .uvu_det import UVUDetGenerator
@@ -118,7 +120,13 @@ class UVURecvGenerator(UVUDetGenerator):
         # shortest has to hold half of the longest's words: two fp32 groups of 80 and 22 words of dZ take 281 apart and 314
         # together (the short one runs two wavefronts per SIMD instead of five).  fp32 stays at a launch per group: most of
         # its problems have one group (three of 110, 102 and 100 words: 753 apart, 700 together).
-        self.fused = self.staged_f64 and self.HR > 1 and 2 * min(held_by) >= max(held_by)
+        # So do groups that lose a wavefront per SIMD by it (those of less than three quarters of the longest) and are more than a
+        # third of all words: 128x0e+128x1o to l = 3, groups of 16 and 24 words, 140 and 180 registers apart: 8000 nodes / 240 000
+        # edges 1711 apart and 1925 together, 1000 / 30 000 241 and 262; 64 channels 848 and 934.  These go together on graphs that
+        # do not fill the chip (TOGETHER_NODES): 100 / 800 46 and 31, 64 channels, 300 / 7500 56 and 48, 24 channels, 520 / 10 000 52 and 43.
+        together = self.staged_f64 and self.HR > 1 and 2 * min(held_by) >= max(held_by)
+        self.fused = together and 3 * sum(h for h in held_by if 4 * h < 3 * max(held_by)) <= sum(held_by)
+        self.fused_few = together and not self.fused
         self.regroup_pairs = bool(self.REGROUP_STAGED and self.uses_stage)
         if self.uses_stage:
             self.waves_hint = 0
@@ -136,6 +144,27 @@ class UVURecvGenerator(UVUDetGenerator):
         return super().describe() + f" receiver-order backward (spill {self.spill_row} words/edge)"
 
     # ------------------------------------------------------------------ plan
+    TOGETHER_NODES = 512          # (nodes x chunks / row groups) up to which groups that otherwise have a launch each go in one (fused_few)
+
+    def add_few_nodes(self, which=("forward", "backward")):
+        super().add_few_nodes(which)
+        if self.fused_few and "backward" in which:
+            twin = copy.copy(self)
+            twin.fused = True
+            self.few_sources["backward"] = self.few_sources["backward"] + [dict(twin._edge_kernel_sources()[0], name="backward_together")]
+        return self
+
+    def few_steps(self, which: str, steps):
+        """As UVUDetGenerator.few_steps; pass 1 in one launch beside its launches, for graphs that do not fill the chip."""
+        steps = super().few_steps(which, steps)
+        most = min(4095, self.TOGETHER_NODES * self.R // self.NCH)
+        if which != "backward" or not self.fused_few or not most:
+            return steps
+        edges = [name for name, _ in self.backward_kernels()]
+        first = next(s for s in steps if s["kernel"] == edges[0])
+        together = dict(first, kernel="backward_together", grid_y=self.NCH * self.HR, few_nodes=(most, 0, 0))
+        return [t for s in steps for t in ([together] if s is first else []) + [dict(s, many_nodes=(most, 0)) if s["kernel"] in edges else s]]
+
     def backward_steps(self):
         steps = [dict(kernel=name, num_threads=WAVE, grid_kind=1, work_per_block=self.MIN_TILE_ITERS * self.R,
                       num_blocks=self.MAX_TILES, grid_y=self.NCH * (self.HR if self.fused else 1))
@@ -195,13 +224,16 @@ class UVURecvGenerator(UVUDetGenerator):
     def backward_kernels(self):
         return [("backward" if h == 0 else f"backward_g{h}", h) for h in range(1 if self.fused else self.HR)]
 
-    def backward_kernel_sources(self):
+    def _edge_kernel_sources(self):
         def attr(h):
             with self._group(h, self.recv_groups):
                 w = self.group_waves_hint()
             return f" __attribute__((amdgpu_waves_per_eu({w}, {w})))" if w else ""
         return [dict(name=name, threads=WAVE, attr=attr(h), body=self._fused_body() if self.fused else self._edges_body(h))
-                for name, h in self.backward_kernels()] \
+                for name, h in self.backward_kernels()]
+
+    def backward_kernel_sources(self):
+        return self._edge_kernel_sources() \
             + [self.with_team(dict(name="backward_dx", threads=WAVE * self.team, attr="", body=self._dx_body()))]
 
     # ---------------------------------------------------------------- pass 1

@@ -87,3 +87,52 @@ def test_on_the_gpu(cuda, case):
         for got, want in zip(runs[0], common.conv_reference_on_valid_edges(otp, oprob, X, Y, W, G, rows, cols, valid)[1:]):
             if np.abs(want).max():
                 assert rel(got.cpu().numpy(), want) < TOL
+
+
+TWO = ("64x0e+64x1o", SH3, "64x0e+64x1o+64x2e+64x3o")             # groups of 16 and 24 words
+
+
+def test_two_groups_go_together_on_few_nodes():
+    """Together, the shorter of two groups loses a wavefront per SIMD: a launch each, but on graphs that do not fill the chip."""
+    for irreps, chunks in ((TWO, 1), (tuple(s.replace("64x", "128x") if s != SH3 else s for s in TWO), 2)):
+        g = UVURecvGenerator(common.channelwise(irreps, dtype=np.float64)[0]).add_few_nodes()
+        assert not g.fused and g.fused_few and g.NCH == chunks and "void backward_together(" in g.render()
+        steps = {s["kernel"]: s for s in g.plan_few()[1] if s["kernel"] in ("backward", "backward_g1", "backward_together")}
+        assert list(steps) == ["backward_together", "backward", "backward_g1"] and steps["backward_together"]["grid_y"] == 2 * chunks
+        assert [s.get("few_nodes", s.get("many_nodes")) for s in steps.values()] == [(512 // chunks, 0, 0)] + [(512 // chunks, 0)] * 2
+        assert not any("few_nodes" in s or s["kernel"] == "backward_together" for s in g.plan()[1])
+    three = UVURecvGenerator(common.channelwise(CASES["two_row_groups"], dtype=np.float64)[0]).add_few_nodes()
+    assert three.fused and not three.fused_few and "backward_together" not in three.render()
+
+
+@pytest.mark.parametrize("together", [False, True])
+def test_two_groups_emulated(together):
+    prob, oprob = common.channelwise(TWO, dtype=np.float64)
+    g = UVURecvGenerator(prob)
+    g.fused = together                            # (what backward_together runs)
+    nodes, nnz = 5, 19
+    rows, cols, tperm, _ = otp.coord_graph(*common.random_graph(nodes, nnz, 7, self_loops=True))
+    X, Y, W, G = common.conv_inputs(prob, nodes, nnz, 8, dtype=np.float64)
+    _, bwd, ws = g.plan()
+    out = emu.run_conv(g, bwd, X, Y, W, rows, cols, G=G, tperm=tperm, ws_bytes=ws(nnz, nodes))
+    want = common.conv_reference_on_valid_edges(otp, oprob, X, Y, W, G, rows, cols, np.ones(nnz, bool))[1:]
+    for got, ref in zip((out["Xg"], out["Yg"], out["Wg"]), want):
+        assert rel(got, ref) < TOL
+
+
+@pytest.mark.gpu
+def test_two_groups_on_the_gpu(cuda):
+    """Both sides of the line in nodes, few and many edges."""
+    import torch
+    import openequivariance_amd as oeq
+    prob, oprob = common.channelwise(TWO, dtype=np.float64)
+    conv = oeq.TensorProductConv(prob, torch_op=True, deterministic=True)
+    assert conv.generator.fused_few
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    for nodes, nnz in ((1, 3), (512, 100), (512, 4000), (513, 100), (513, 4000)):
+        rows, cols, tperm, _ = otp.coord_graph(*common.random_graph(nodes, nnz, 5, self_loops=True))
+        X, Y, W, G = common.conv_inputs(prob, nodes, nnz, 6, dtype=np.float64)
+        x, y, w = (t(a).requires_grad_() for a in (X, Y, W))
+        got = torch.autograd.grad(conv(x, y, w, t(rows), t(cols), t(tperm)), (x, y, w), t(G))
+        for a, ref in zip(got, common.conv_reference_on_valid_edges(otp, oprob, X, Y, W, G, rows, cols, np.ones(nnz, bool))[1:]):
+            assert rel(a.cpu().numpy(), ref) < TOL
