@@ -80,7 +80,7 @@ enum { OEQ_GRID_FIXED = 0, OEQ_GRID_PER_ROW = 1, OEQ_GRID_PER_NODE = 2, OEQ_GRID
  * OEQ_STEP_FEW_NODES(n, d, m), of a convolution's plan: the step runs only on graphs of at most n < 4096 nodes, of more than m
  * (a multiple of 128 below 2048), and at least d < 256 times as many edges as nodes; OEQ_STEP_MANY_NODES(n, d): only on
  * graphs of more than n nodes or fewer than d times as many edges (oeq_tp_create rejects both).  A plan holds the forms of a launch that way: one
- * wavefront per node, two and four. */
+ * wavefront per node, two and four; a launch for each group of outputs, or one for all. */
 enum { OEQ_STEP_NEEDS_WORKSPACE = 1, OEQ_STEP_NEEDS_TPERM = 2, OEQ_STEP_GRAPH_PREP = 4, OEQ_STEP_COUNTER_CLEAR = 8 };
 #define OEQ_STEP_FEW_NODES(n, d, m) (16u | (uint32_t)(n) << 8 | (uint32_t)(d) << 20 | (uint32_t)(m) / 128u << 28)
 #define OEQ_STEP_MANY_NODES(n, d) (32u | (uint32_t)(n) << 8 | (uint32_t)(d) << 20)
