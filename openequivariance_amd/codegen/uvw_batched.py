@@ -55,15 +55,20 @@ class UVWBatchedGenerator(UVWGenerator):
                 ul * wl * self.itemsize % 128 == 0 for b in self.batches for _, _, ul, _, wl, _ in b)
         ) and not self._first_operand_too_wide(forward=False)
         self.stream = self.stream_forward or self.stream_backward
-        self.rows_chunked = self.ROWS_CHUNKED if self.stream_forward and self.ROW_BYTES[0] <= self.WN * self.itemsize <= self.ROW_BYTES[1] else 0
+        self.rows_chunked = 0
+        if self.stream_forward and self.WN * self.itemsize >= self.ROWS_CHUNKED_FROM:
+            self.rows_chunked = next(rows for most, rows in self.ROWS_CHUNKED if self.WN * self.itemsize <= most)
         self.has_backward = True
 
     # Rows up to which the forward keeps the walk over chunks, as a kernel for few rows: a wavefront per SIMD, with nothing beside it to
-    # hide a batch's way through LDS.  Rows of 16 to 64 KB; short ones are a batch or two, and longer ones spill in that walk.  Chunks /
-    # batches, us, 256, 1024 and 2048 rows: DiffDock's layer 5.0 / 5.9, 7.0 / 7.8 and 10.6 / 10.5, fp64 5.8 / 7.0, 10.7 / 10.9 and 19.9 / 19.0;
-    # 10 channels to 50, l <= 2, 5.7 / 7.3, 7.5 / 8.7 and 10.7 / 10.3, fp64 5.5 / 8.8, 10.1 / 11.3 and 19.9 / 17.6; 60 of both parities
-    # to 26, l <= 1, 6.5 / 10.5, 11.5 / 15.0 and 20.8 / 21.6.  Below 16 KB, 34 channels, one scalar, 5.1 / 4.5, 6.4 / 5.9, 9.0 / 7.9.
-    ROWS_CHUNKED, ROW_BYTES = 1024, (16 << 10, 64 << 10)
+    # hide a batch's way through LDS; half of them where a row is longer than 64 KB, none where the walk spills or a row is a batch or two.
+    # Chunks / batches, us, 256, 1024 and 2048 rows: DiffDock's layer (28 KB) 5.0 / 5.9, 7.0 / 7.8 and 10.6 / 10.5, fp64 5.8 / 7.0,
+    # 10.7 / 10.9 and 19.9 / 19.0; 10 channels to 50, l <= 2, 5.7 / 7.3, 7.5 / 8.7 and 10.7 / 10.3, fp64 5.5 / 8.8, 10.1 / 11.3 and 19.9 /
+    # 17.6; 60 of both parities to 26, l <= 1, 6.5 / 10.5, 11.5 / 15.0 and 20.8 / 21.6.  256, 512 and 1024 rows: 80 channels to 34, l <= 2
+    # (74 KB) 10.9 / 12.7, 12.1 / 16.4 and 17.0 / 19.8, 128 of both parities to 20, l <= 1 (100 KB) 11.1 / 17.8, 13.4 / 22.0 and 20.2 / 25.9, 34 to 100,
+    # fp64 (106 KB) 7.0 / 11.0, 10.4 / 13.3 and 18.9 / 18.5, 128 to 18, fp64 (72 KB) 8.5 / 9.2, 10.2 / 11.4 and 15.3 / 13.9.
+    # Below 16 KB, 34 channels, one scalar, 256, 1024 and 2048 rows 5.1 / 4.5, 6.4 / 5.9, 9.0 / 7.9.
+    ROWS_CHUNKED_FROM, ROWS_CHUNKED = 16 << 10, ((64 << 10, 1024), (128 << 10, 512), (1 << 62, 0))
 
     def forward_of_few_rows(self) -> "UVWBatchedGenerator":
         few = UVWBatchedGenerator(self.problem, stream=False)

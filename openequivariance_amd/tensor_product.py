@@ -122,7 +122,10 @@ def few_rows_generator(config: TPProblem, generator: UVWGenerator):
     """(generator, largest batches forward and backward) of the kernels for few rows beside a uvw product's
     ``generator``: without a forward where they leave it none, (None, (0, 0)) where they have no batch at all."""
     if isinstance(generator, UVWBatchedGenerator):
-        return (generator.forward_of_few_rows(), (generator.rows_chunked, 0)) if generator.rows_chunked else (None, (0, 0))
+        few = generator.forward_of_few_rows() if generator.rows_chunked else None
+        if few is None or rt.kernel_metadata(rt.compile_source(few.render()))["forward"][".private_segment_fixed_size"]:
+            return None, (0, 0)
+        return few, (generator.rows_chunked, 0)
     small = UVWSmallGenerator.create(config)
     cut = UVWGenerator(config) if generator.rows_cut else None        # the forward of fewer rows
     if small is None:
